@@ -213,6 +213,10 @@ struct IgemmDesc {
   // MFMA blocks, blockM 64 or 128; 2: 16-pixel MFMA blocks, blockM = pixels
   // per tile, any number up to 112.
   uint32_t patch = 0;
+  // 1 to kIgemmSmallTiles: the kernel for small problems runs (tiles of 16 x
+  // 16, 16 x 32, 32 x 32 or 64 x 32 pixels x channels; igemmSmallTakes); the
+  // packed weights then have its layout (launchPackIgemmSmallWeights).
+  uint32_t small = 0;
   // Patch rows the tallest tile of that kernel spans (igemmPatchMaxRows),
   // worked out once when the plan is made - it takes a walk over the tiles -
   // so that a launch does not repeat it; 0 = not known, work it out.
@@ -257,6 +261,33 @@ hipError_t launchIgemmPatch(const IgemmDesc &d, int inType, int outType,
                             const void *bias, void *out, const QuarterInfo &q,
                             hipStream_t stream);
 
+/// The same convolution by the kernel for problems too small to fill the chip
+/// with 128-pixel tiles: d.small names the tile, K is split over the waves of
+/// a workgroup.  Two field dimensions; a dilated input by arithmetic.
+constexpr uint32_t kIgemmSmallTiles = 4;
+bool igemmSmallTakes(const IgemmDesc &d, int inType, int outType);
+uint32_t igemmSmallTilePixels(uint32_t tile);
+uint32_t igemmSmallTileChans(uint32_t tile);
+uint64_t igemmSmallTileCount(const IgemmDesc &d);
+/// Waves of a workgroup, among which K is split.
+uint32_t igemmSmallWaves(const IgemmDesc &d, int inType);
+/// Elements of its packed weights:
+/// [G][16-channel block][64-byte k-step][lane][16 bytes].
+uint64_t igemmSmallPackedElems(const IgemmDesc &d, int inType);
+/// src as for launchPackIgemmWeights; sourceChans, sourceTaps: the stored
+/// kernel's input channels (d's may be padded) and taps.
+hipError_t launchPackIgemmSmallWeights(const IgemmDesc &d, int inType,
+                                       const void *src, void *dst,
+                                       uint32_t sourceChans,
+                                       uint32_t sourceTaps, hipStream_t stream,
+                                       bool chansTransposed = false,
+                                       const IgemmTapSelection *select =
+                                           nullptr);
+hipError_t launchIgemmSmall(const IgemmDesc &d, int inType, int outType,
+                            const void *in, const void *weightsPacked,
+                            const void *bias, void *out, const QuarterInfo &q,
+                            hipStream_t stream);
+
 /// Several convolutions that run the same igemm kernel (same tile width,
 /// types, fp8 formats, channel-block alignment; K not split) as ONE launch
 /// whose grid is the concatenation of their tiles - at most 8 at a time.
@@ -271,6 +302,10 @@ constexpr size_t kIgemmMaxFused = 8;
 bool igemmFusable(const IgemmFusedItem &x, const IgemmFusedItem &y);
 hipError_t launchIgemmFused(const IgemmFusedItem *items, size_t count,
                             hipStream_t stream);
+/// The same for convolutions of the small-problem kernel.
+bool igemmSmallFusable(const IgemmFusedItem &x, const IgemmFusedItem &y);
+hipError_t launchIgemmSmallFused(const IgemmFusedItem *items, size_t count,
+                                 hipStream_t stream);
 
 /// Pointwise convolution (every kernel extent 1, stride 1, no padding or
 /// truncation, half inputs) with a multiple of 8 up to 512 input channels per

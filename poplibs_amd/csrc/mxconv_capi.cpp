@@ -198,6 +198,10 @@ mxconv_status forward(const mxconv_plan *plan, const void *in, const void *w,
         return st;
       in = padded;
     }
+    if (plan->igemm.small)
+      return hipStatus(mxk::launchIgemmSmall(plan->igemm, inType, outType, in,
+                                             w, bias, out, q, s),
+                       "implicit-GEMM convolution launch (small tiles)");
     if (plan->igemm.patch)
       return hipStatus(mxk::launchIgemmPatch(plan->igemm, inType, outType, in,
                                              w, bias, out, q, s),
@@ -695,7 +699,8 @@ std::string packingSignature(const mxconv_plan &p) {
      << p.convGroupsPerGroup;
   if (p.kernel == mxconv_plan::Kernel::IGEMM) {
     os << "/pw" << p.pointwiseOn << "/thin" << p.thinInputOn << "/patch"
-       << p.igemm.patch << "/co"
+       << p.igemm.patch << "/small" << mxk::igemmSmallTileChans(p.igemm.small)
+       << "/co"
        << p.coPadded << "/k" << p.kPadded << "/ci" << p.paddedInputChans
        << "/sel" << p.kernelSelected;
     auto taps = [&](const mxk::IgemmTapSelection &t) {
@@ -770,6 +775,13 @@ mxconv_status mxconv_pack_weights(const mxconv_plan *plan,
       return hipStatus(mxk::launchPackPointwiseWeights(
                            plan->pointwise, weights_external, weights_packed, s),
                        "weight packing");
+    if (plan->igemm.small)
+      return hipStatus(
+          mxk::launchPackIgemmSmallWeights(
+              plan->igemm, p.inputType.id(), weights_external, weights_packed,
+              ci, uint32_t(taps), s, false,
+              plan->kernelSelected ? &plan->igemmTaps : nullptr),
+          "weight packing");
     for (const auto &phase : plan->igemmPhases) {
       const mxconv_status st = hipStatus(
           mxk::launchPackIgemmWeights(
@@ -1043,12 +1055,17 @@ mxconv_status mxconv_multi_fwd(size_t n, const mxconv_plan *const *plans,
     size_t member[mxk::kIgemmMaxFused] = {i};
     size_t members = 0;
     double alone = 0, together = 0;
+    const auto fusable = [&](const mxk::IgemmFusedItem &x,
+                             const mxk::IgemmFusedItem &y) {
+      return x.d->small || y.d->small ? mxk::igemmSmallFusable(x, y)
+                                      : mxk::igemmFusable(x, y);
+    };
     if (parallel && fusedItem(i, 0, group[0])) {
       members = 1;
       for (size_t j = i + 1; j != n && members != mxk::kIgemmMaxFused; ++j) {
         mxk::IgemmFusedItem item;
         if (!done[j] && fusedItem(j, members, item) &&
-            mxk::igemmFusable(group[0], item)) {
+            fusable(group[0], item)) {
           member[members] = j;
           group[members++] = item;
         }
@@ -1067,10 +1084,13 @@ mxconv_status mxconv_multi_fwd(size_t n, const mxconv_plan *const *plans,
       together = 6 + 0.3 * double(longest * ((tiles + 255) / 256));
     }
     mxconv_status st;
-    if (members >= 2 && together < alone) {
+    // (small-tile convolutions cost little but their launch)
+    const bool small = members != 0 && group[0].d->small;
+    if (members >= 2 && (small || together < alone)) {
       for (size_t k = 0; k != members; ++k)
         done[member[k]] = true;
-      st = hipStatus(mxk::launchIgemmFused(group, members, s),
+      st = hipStatus(small ? mxk::launchIgemmSmallFused(group, members, s)
+                           : mxk::launchIgemmFused(group, members, s),
                      "fused implicit-GEMM convolution launch");
     } else {
       st = forward(plans[i], in[i], weights_packed[i],
@@ -1216,6 +1236,11 @@ mxconv_status mxconv_matmul_pack_rhs(const mxconv_plan *plan, const void *rhs,
     if (plan->pointwiseOn)
       return hipStatus(mxk::launchPackPointwiseWeights(plan->pointwise, rhs,
                                                        weights_packed, s, true),
+                       "weight packing");
+    if (plan->igemm.small)
+      return hipStatus(mxk::launchPackIgemmSmallWeights(
+                           plan->igemm, p.inputType.id(), rhs, weights_packed,
+                           uint32_t(p.inputChannelsPerConvGroup), 1, s, true),
                        "weight packing");
     if (plan->igemm.patch)
       return hipStatus(mxk::launchPackIgemmPatchWeights(
@@ -1531,7 +1556,7 @@ mxconv_status fusedWeightDeltas(const mxconv_plan *plan, const void *zDeltas,
                       !plan->pointwiseOn && !plan->thinInputOn &&
                       !plan->paddedInputChans &&
                       plan->igemmPhases.empty() && !plan->kernelSelected &&
-                      !plan->igemm.patch &&
+                      !plan->igemm.patch && !plan->igemm.small &&
                       // (a padded output field - the forward kernel was
                       // truncated - is filled by the general path)
                       !plan->outputPadded;

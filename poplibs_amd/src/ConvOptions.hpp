@@ -64,6 +64,10 @@ struct PlanConstraints {
   /// pixels as one k-step, no padded copy of the input): -1 planner's choice
   /// (never with "kernel" or a tile named), 0 never, 1 required.
   int thinInput = -1;
+  /// The matrix-core kernel for small problems (tiles of 16 to 64 pixels, K
+  /// split over the waves of a workgroup): -1 planner's choice (never with
+  /// "kernel" or another tile named), 0 never, 1 to 4 the tile.
+  int smallTile = -1;
   /// A weight update pass's deltas: -1 planner's choice, 0 through the pass's
   /// own convolution (batch and channels exchanged), 1 by the kernel that
   /// reads the layer's own tensors (an error where none takes the layer), 2

@@ -326,6 +326,40 @@ double estimatePatch(std::size_t workgroups, std::size_t kSteps, unsigned mode,
   return kLaunchUs + rounds * (fixed + step * double(kSteps));
 }
 
+/// igemmSmallKernel, by its tile (kIgemmSmallTiles): a workgroup that has a CU
+/// to itself takes `first` and `group` for every further group of k-steps its
+/// waves go through; where there are more of them than half the CUs, each
+/// workgroup adds `tile` + `step` per k-step to its CU's time (times 1 +
+/// `window` where a window is worked out, + `fp32` for fp32's slower MFMAs).
+/// Fitted to 330 random layers and products of up to 6 GFLOP, four tiles each:
+/// the tile picked by it is on average within 3 % of the best of the four.
+double estimateSmall(const mxk::IgemmDesc &d, int inType) {
+  struct Fit {
+    double first, group, tile, step, window, fp32;
+    unsigned stepsPerGroup;
+  };
+  static constexpr Fit kFits[mxk::kIgemmSmallTiles + 1] = {
+      {},
+      {0.69, 1.56, 0.123, 0.0246, 0.02, 0.71, 4},
+      {1.04, 2.26, 0.213, 0.0379, 0.0, 0.89, 4},
+      {1.37, 1.45, 0.250, 0.0537, 0.0, 1.49, 2},
+      {2.04, 0.99, 0.661, 0.0337, 0.71, 7.14, 1}};
+  const Fit &f = kFits[d.small];
+  const unsigned eb = inType == mxk::kFloat ? 4 : inType == mxk::kHalf ? 2 : 1;
+  const double steps =
+      std::ceil(double(d.kH) * d.kW * d.inChansPerGroup * eb / 64.0);
+  const double tiles = double(mxk::igemmSmallTileCount(d));
+  const double perWave = std::ceil(steps / mxk::igemmSmallWaves(d, inType));
+  const bool window = d.kH * d.kW > 1 || d.inDilH != 1 || d.inDilW != 1;
+  return 2.1 + f.first +
+         f.group * (std::ceil(perWave / f.stepsPerGroup) - 1.0) *
+             (window ? 1.0 + 0.5 * f.window : 1.0) +
+         std::max(0.0, tiles / double(gfx950::numCUs) - 0.5) *
+             (f.tile + f.step * steps *
+                           (1.0 + (window ? f.window : 0.0) +
+                            (inType == mxk::kFloat ? f.fp32 : 0.0)));
+}
+
 } // namespace
 
 namespace {
@@ -1231,6 +1265,84 @@ mxconv_plan makePlanWith(const ConvParams &params,
         plan.weightPackedElems = mxk::igemmPatchPackedElems(g, inId);
       }
     }
+    // A problem too small for 128-pixel tiles to fill the chip: small tiles
+    // with K split over the waves of a workgroup.
+    {
+      const int inId = halfIn ? mxk::kHalf : floatIn ? mxk::kFloat
+                                                     : mxk::kQuarter;
+      const int outId =
+          params.outputType == poplar::HALF ? mxk::kHalf : mxk::kFloat;
+      const std::size_t eb = params.inputType.size();
+      auto asSmall = [&](uint32_t tile) {
+        mxk::IgemmDesc t = g;
+        t.small = tile, t.patch = 0, t.blockM = 128, t.splitK = 1;
+        return t;
+      };
+      uint32_t tile = 0;
+      if (pc.smallTile > 0) {
+        tile = uint32_t(pc.smallTile);
+        if (!mxk::igemmSmallTakes(asSmall(tile), inId, outId))
+          throw poplar::invalid_option(
+              "planConstraints gfx950 smallTile: that kernel takes "
+              "convolutions of up to two field dimensions");
+      } else if (pc.smallTile != 0 && pc.kernel.empty() &&
+                 pc.method == Method::ANY && !pc.blockM && !pc.blockN &&
+                 !pc.blockK && !pc.splitK && !pc.stages && pc.patch < 0 &&
+                 pc.pointwise < 0 && !pc.chanTiles &&
+                 !isWeightUpdatePass(options.pass) &&
+                 double(s.batch) * s.outH * s.outW * co * p.numConvGroups *
+                         double(k) <=
+                     3e9) {
+        // The planner's choice, for what the estimates were fitted to: the
+        // tile with the lowest estimate, where that is clearly below the
+        // kernel's chosen above.  (What the other
+        // estimates leave out at this end of the range: the pointwise kernel
+        // takes 1.9 us more than launch and bytes, fp32 MFMAs make the
+        // streaming kernel's k-steps longer, phases run side by side.)
+        const mxconv_plan::DetailedEstimate e = plan.detailedEstimate();
+        double planned = e.computeUs + e.reductionUs;
+        if (plan.pointwiseOn)
+          planned += 1.9;
+        else if (!plan.igemmPhases.empty()) {
+          std::size_t tiles = 0, steps = 0;
+          for (const auto &ph : plan.igemmPhases) {
+            tiles += (std::size_t(ph.d.batch) * ph.d.outH * ph.d.outW +
+                      g.blockM - 1) /
+                     g.blockM * (plan.coPadded / g.blockN) * g.groups;
+            steps = std::max(steps, ph.d.noTaps ? 0 : ph.kPadded / g.blockK);
+          }
+          planned = estimateStreaming(tiles, steps,
+                                      g.blockN == 64 || g.stages == 2 ? 2 : 1,
+                                      g.blockN, 1, 0);
+        }
+        if (floatIn && !plan.pointwiseOn)
+          planned *= 1.6;
+        double best = 0.9 * planned;
+        for (uint32_t t = 1; t <= mxk::kIgemmSmallTiles; ++t) {
+          const mxk::IgemmDesc d = asSmall(t);
+          if (!mxk::igemmSmallTakes(d, inId, outId))
+            continue;
+          const double us = estimateSmall(d, inId);
+          if (us < best)
+            best = us, tile = t;
+        }
+      }
+      if (tile) {
+        g = asSmall(tile);
+        plan.reason = "few output tiles: small ones, K shared by the waves of "
+                      "a workgroup";
+        plan.pointwiseOn = false;
+        plan.candidates.clear();
+        plan.igemmPhases.clear();
+        plan.workspaceBytes = 0;
+        if (plan.paddedInputChans) {
+          plan.paddedInputOffset = 0;
+          plan.workspaceBytes = s.batch * s.inH * s.inW * p.numConvGroups *
+                                ciPadded * eb;
+        }
+        plan.weightPackedElems = mxk::igemmSmallPackedElems(g, inId);
+      }
+    }
     if (!g.patch && g.blockM != 128)
       throw poplar::invalid_option(
           "planConstraints gfx950 blockM 64 goes with the resident-patch "
@@ -1346,6 +1458,8 @@ std::string mxconv_plan::constraintsJson() const {
     } else if (pointwiseOn) {
       os << ", \"pointwise\": 1, \"chanTiles\": "
          << mxk::pointwiseLaunchShape(pointwise, gfx950::numCUs).chansPerWorkgroup / 64;
+    } else if (igemm.small) {
+      os << ", \"smallTile\": " << igemm.small;
     } else if (igemm.patch) {
       os << ", \"pointwise\": 0, \"patch\": " << igemm.patch
          << ", \"blockM\": " << igemm.blockM;
@@ -1467,6 +1581,17 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
       spread(e, l.workgroups, 1);
       break;
     }
+    if (igemm.small) {
+      e.computeUs = std::max(
+          poplin::estimateSmall(igemm, params.inputType == poplar::FLOAT
+                                           ? mxk::kFloat
+                                       : params.inputType == poplar::HALF
+                                           ? mxk::kHalf
+                                           : mxk::kQuarter),
+          streamed(inputBytes() + outputBytes() + weightPackedBytes()));
+      spread(e, mxk::igemmSmallTileCount(igemm), 1);
+      break;
+    }
     if (pointwiseOn) {
       e.computeUs =
           streamed(inputBytes() + outputBytes() + weightPackedBytes());
@@ -1547,7 +1672,8 @@ std::string mxconv_plan::describe() const {
        << " operands, fp32 accumulate)"
        << (pointwiseOn ? ", pointwise streaming variant" : "")
        << (thinInputOn ? ", kernel rows as k-steps" : "")
-       << (igemm.patch ? ", input patch resident in LDS" : "");
+       << (igemm.patch ? ", input patch resident in LDS" : "")
+       << (igemm.small ? ", small tiles" : "");
     break;
   case Kernel::DEPTHWISE:
     os << (mxk::depthwiseDirectInBlocks(depthwise)
@@ -1614,7 +1740,28 @@ std::string mxconv_plan::describe() const {
          << canonical.outputChannelsPerConvGroup << " channels run as "
          << g.groups << " of " << g.inChansPerGroup << " -> "
          << g.outChansPerGroup << ", weights block-diagonal)\n";
-    if (pointwiseOn) {
+    if (g.small) {
+      const int inId = params.inputType == poplar::FLOAT  ? mxk::kFloat
+                       : params.inputType == poplar::HALF ? mxk::kHalf
+                                                          : mxk::kQuarter;
+      const std::size_t chans = mxk::igemmSmallTileChans(g.small);
+      os << "        block M x N x K            "
+         << mxk::igemmSmallTilePixels(g.small) << " x " << chans << " x "
+         << 64 / params.inputType.size() << "\n";
+      os << "        workgroups                 "
+         << mxk::igemmSmallTileCount(g) << " on " << gfx950::numCUs
+         << " CUs, K shared by the " << mxk::igemmSmallWaves(g, inId)
+         << " waves of each\n";
+      os << "        packed weights             [G=" << g.groups << "]["
+         << (g.outChansPerGroup + chans - 1) / chans * chans / 16 << " blocks of 16]["
+         << (k * params.inputType.size() + 63) / 64
+         << " k-steps][64 lanes][16 bytes]\n";
+      if (paddedInputChans)
+        os << "        input channels padded      "
+           << params.inputChannelsPerConvGroup << " -> " << paddedInputChans
+           << " per group (zero-filled copy in the workspace, every "
+              "launch)\n";
+    } else if (pointwiseOn) {
       const std::size_t nTiles = (g.outChansPerGroup + 63) / 64;
       const mxk::PointwiseLaunch l =
           mxk::pointwiseLaunchShape(pointwise, gfx950::numCUs);
@@ -1754,5 +1901,20 @@ std::string mxconv_plan::describe() const {
        << (tiling.empty() ? "" : "; " + tiling) << "\n";
   }
   os << "        workspaceBytes             " << workspaceBytes << "\n";
+  if (kernel == Kernel::IGEMM && igemm.small) {
+    // the plan without the small tiles, which they were weighed against
+    poplin::ConvOptions o = options;
+    o.planConstraints = poplin::PlanConstraints{};
+    o.planConstraints.smallTile = 0;
+    o.planConstraints.convGroupsPerGroup = convGroupsPerGroup;
+    const mxconv_plan other = poplin::makePlan(params, o);
+    char line[96];
+    std::snprintf(line, sizeof line,
+                  "  Left aside for it (estimates: %.1f us, above %.1f us):\n",
+                  other.estimatedMicroseconds(), estimatedMicroseconds());
+    // (without the heading, which names the chip again)
+    const std::string text = other.describe();
+    os << line << text.substr(text.find('\n') + 1);
+  }
   return os.str();
 }
