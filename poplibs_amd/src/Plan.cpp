@@ -295,9 +295,11 @@ double splitPenaltyUs(std::size_t partialBytes) {
 
 double estimateStreaming(std::size_t workgroups, std::size_t kSteps,
                          std::size_t perCU, unsigned blockN, unsigned splitK,
-                         std::size_t partialBytes) {
+                         std::size_t partialBytes, bool fp32) {
   const double rounds = roundsOf(workgroups, perCU);
-  const double step = blockN == 128 ? 0.345 : 0.24;
+  // (fp32 MFMAs: a 128 x 128 k-step of 32 values is 2 048 cycles of them)
+  const double step = fp32 ? (blockN == 128 ? 1.0 : 0.52)
+                           : (blockN == 128 ? 0.345 : 0.24);
   double tile = 2.95 + step * double(kSteps);
   if (perCU == 1 && rounds > 1)
     tile += 1.5;
@@ -330,34 +332,53 @@ double estimatePatch(std::size_t workgroups, std::size_t kSteps, unsigned mode,
 /// to itself takes `first` and `group` for every further group of k-steps its
 /// waves go through; where there are more of them than half the CUs, each
 /// workgroup adds `tile` + `step` per k-step to its CU's time (times 1 +
-/// `window` where a window is worked out, + `fp32` for fp32's slower MFMAs).
-/// Fitted to 330 random layers and products of up to 6 GFLOP, four tiles each:
-/// the tile picked by it is on average within 3 % of the best of the four.
+/// `window` where a window is worked out).  Fitted to 330 random layers and
+/// products of up to 6 GFLOP, and to 150 more in fp32, four tiles each: the
+/// tile picked by it is on average within 3 % of the best of the four.
+/// Nor is a launch faster than a CU's share of the operands arrives, at 60 KB
+/// per us: a product of a few rows, bound by its weights, wants tiles enough
+/// for every CU (16 x 4096 x 4096: 256 tiles of 16 x 16 take 7.9 us, 128 of
+/// 16 x 32 10.3).
 double estimateSmall(const mxk::IgemmDesc &d, int inType) {
   struct Fit {
-    double first, group, tile, step, window, fp32;
+    double first, group, tile, step, window;
     unsigned stepsPerGroup;
   };
-  static constexpr Fit kFits[mxk::kIgemmSmallTiles + 1] = {
+  static constexpr Fit kHalfFits[mxk::kIgemmSmallTiles + 1] = {
       {},
-      {0.69, 1.56, 0.123, 0.0246, 0.02, 0.71, 4},
-      {1.04, 2.26, 0.213, 0.0379, 0.0, 0.89, 4},
-      {1.37, 1.45, 0.250, 0.0537, 0.0, 1.49, 2},
-      {2.04, 0.99, 0.661, 0.0337, 0.71, 7.14, 1}};
-  const Fit &f = kFits[d.small];
+      {0.69, 1.56, 0.123, 0.0246, 0.02, 4},
+      {1.04, 2.26, 0.213, 0.0379, 0.0, 4},
+      {1.37, 1.45, 0.250, 0.0537, 0.0, 2},
+      {2.04, 0.99, 0.661, 0.0337, 0.71, 1}};
+  static constexpr Fit kFloatFits[mxk::kIgemmSmallTiles + 1] = {
+      {},
+      {0.63, 0.73, 0.171, 0.0376, 0.0, 4},
+      {0.97, 0.70, 0.329, 0.0652, 0.0, 4},
+      {1.61, 2.74, 0.605, 0.0652, 0.0, 2},
+      {2.74, 2.48, 0.867, 0.0771, 0.0, 1}};
+  const Fit &f = inType == mxk::kFloat ? kFloatFits[d.small]
+                                       : kHalfFits[d.small];
   const unsigned eb = inType == mxk::kFloat ? 4 : inType == mxk::kHalf ? 2 : 1;
   const double steps =
       std::ceil(double(d.kH) * d.kW * d.inChansPerGroup * eb / 64.0);
-  const double tiles = double(mxk::igemmSmallTileCount(d));
+  const double perCU =
+      double(mxk::igemmSmallTileCount(d)) / double(gfx950::numCUs);
   const double perWave = std::ceil(steps / mxk::igemmSmallWaves(d, inType));
-  const bool window = d.kH * d.kW > 1 || d.inDilH != 1 || d.inDilW != 1;
-  return 2.1 + f.first +
-         f.group * (std::ceil(perWave / f.stepsPerGroup) - 1.0) *
-             (window ? 1.0 + 0.5 * f.window : 1.0) +
-         std::max(0.0, tiles / double(gfx950::numCUs) - 0.5) *
-             (f.tile + f.step * steps *
-                           (1.0 + (window ? f.window : 0.0) +
-                            (inType == mxk::kFloat ? f.fp32 : 0.0)));
+  const double window =
+      d.kH * d.kW > 1 || d.inDilH != 1 || d.inDilW != 1 ? f.window : 0.0;
+  const double pixelBlocks =
+      std::min(double(mxk::igemmSmallTilePixels(d.small)) / 16.0,
+               std::ceil(double(d.batch) * d.outH * d.outW / 16.0));
+  const double arriveUs =
+      2.6 + (perCU <= 2.0 ? std::ceil(perCU) : perCU) * steps *
+                (pixelBlocks + mxk::igemmSmallTileChans(d.small) / 16.0) /
+                60.0;
+  const double computeUs =
+      2.1 + f.first +
+      f.group * (std::ceil(perWave / f.stepsPerGroup) - 1.0) *
+          (1.0 + 0.5 * window) +
+      std::max(0.0, perCU - 0.5) * (f.tile + f.step * steps * (1.0 + window));
+  return std::max(arriveUs, computeUs);
 }
 
 } // namespace
@@ -871,14 +892,14 @@ mxconv_plan makePlanWith(const ConvParams &params,
           parts * m * p.numConvGroups * ((co + 127) / 128 * 128) * 4;
       const double wideUs = std::min(
           estimateStreaming(wide, kSteps, wide > gfx950::numCUs ? 2 : 1, 128,
-                            1, 0),
+                            1, 0, floatIn),
           parts > 1 ? estimateStreaming(wide * parts,
                                         (kSteps + parts - 1) / parts, 1, 128,
-                                        unsigned(parts), partial)
+                                        unsigned(parts), partial, floatIn)
                     : 1e30);
       const double wideWholeUs = estimateStreaming(
-          wide, kSteps, wide > gfx950::numCUs ? 2 : 1, 128, 1, 0);
-      if (estimateStreaming(narrow, kSteps, 2, 64, 1, 0) < wideUs) {
+          wide, kSteps, wide > gfx950::numCUs ? 2 : 1, 128, 1, 0, floatIn);
+      if (estimateStreaming(narrow, kSteps, 2, 64, 1, 0, floatIn) < wideUs) {
         g.blockN = 64, narrowWhole = true;
       } else if (wideUs < wideWholeUs && narrow * 2 <= gfx950::numCUs) {
         // K split wins: then over narrow tiles, in half as many parts of at
@@ -934,11 +955,11 @@ mxconv_plan makePlanWith(const ConvParams &params,
       // 3 x 3, 512 -> 512 (52 tiles of 72 k-steps) 18.7 in four, 21.1 whole.
       if (!pc.splitK && !narrowSplit && parts > 1 &&
           estimateStreaming(tiles, kSteps, g.blockN == 64 ? 2 : 1, g.blockN, 1,
-                            0) <=
+                            0, floatIn) <=
               estimateStreaming(tiles * parts, (kSteps + parts - 1) / parts,
                                 1, g.blockN, unsigned(parts),
                                 parts * m * p.numConvGroups * plan.coPadded *
-                                    4))
+                                    4, floatIn))
         parts = 1;
       const std::size_t chans = p.numConvGroups * co;
       // partial tiles of more than 1 GB are not worth it
@@ -1227,7 +1248,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
               Tiling{0, 128}, streamTiles, streamPerCU, streamSteps,
               estimateStreaming(streamTiles, streamSteps, streamPerCU,
                                 g.blockN, g.splitK,
-                                mxk::igemmWorkspaceBytes(g)),
+                                mxk::igemmWorkspaceBytes(g), floatIn),
               roundsOf(streamTiles, streamPerCU));
       std::size_t best = iStream;
       if (pc.patch >= 1) {
@@ -1297,8 +1318,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
         // tile with the lowest estimate, where that is clearly below the
         // kernel's chosen above.  (What the other
         // estimates leave out at this end of the range: the pointwise kernel
-        // takes 1.9 us more than launch and bytes, fp32 MFMAs make the
-        // streaming kernel's k-steps longer, phases run side by side.)
+        // takes 1.9 us more than launch and bytes, phases run side by side.)
         const mxconv_plan::DetailedEstimate e = plan.detailedEstimate();
         double planned = e.computeUs + e.reductionUs;
         if (plan.pointwiseOn)
@@ -1313,11 +1333,9 @@ mxconv_plan makePlanWith(const ConvParams &params,
           }
           planned = estimateStreaming(tiles, steps,
                                       g.blockN == 64 || g.stages == 2 ? 2 : 1,
-                                      g.blockN, 1, 0);
+                                      g.blockN, 1, 0, floatIn);
         }
-        if (floatIn && !plan.pointwiseOn)
-          planned *= 1.6;
-        double best = 0.9 * planned;
+        double best = (plan.pointwiseOn ? 0.9 : 0.95) * planned;
         for (uint32_t t = 1; t <= mxk::kIgemmSmallTiles; ++t) {
           const mxk::IgemmDesc d = asSmall(t);
           if (!mxk::igemmSmallTakes(d, inId, outId))
@@ -1631,7 +1649,7 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
     const std::size_t perCU = g.blockN == 64 || g.stages == 2 ? 2 : 1;
     double us = poplin::estimateStreaming(tiles, steps, perCU, g.blockN,
                                           g.splitK,
-                                          mxk::igemmWorkspaceBytes(igemm));
+                                          mxk::igemmWorkspaceBytes(igemm), params.inputType == poplar::FLOAT);
     // No kernel is faster than its tensors stream.
     us = std::max(us, streamed(inputBytes() + outputBytes() +
                                weightPackedBytes()));
