@@ -477,53 +477,7 @@ __device__ __forceinline__ void igemmTile(
             (range(idBase, int(d.loD), int(d.hiD), int(d.dilD), int(d.kD), 8)
              << 16);
       } else {
-        uint32_t mask = 0;
-        if (d.dilD == 1 && d.dilH == 1 && d.dilW == 1) {
-          // Undilated kernel: the valid kernel columns are the interval
-          // [lo - base, hi - base) cut to the kernel, and so are the rows.
-          // Bits [first, last) of a word:
-          auto bitRange = [](int first, int last) {
-            return first < last ? uint32_t(((1ull << last) - 1) &
-                                           ~((1ull << first) - 1))
-                                : 0u;
-          };
-          auto cut = [](int v, int size) {
-            return v < 0 ? 0 : v > size ? size : v;
-          };
-          const int kW = int(d.kW), kH = int(d.kH), kD = int(d.kD);
-          const uint32_t kwMask = bitRange(cut(int(d.loW) - iwBase, kW),
-                                           cut(int(d.hiW) - iwBase, kW));
-          // one bit per valid kernel row, at that row's first tap; the
-          // product puts the column mask there (no carries: it is narrower
-          // than the distance between the bits)
-          const uint32_t rowStarts =
-              a.tapRowStarts & bitRange(cut(int(d.loH) - ihBase, kH) * kW,
-                                        cut(int(d.hiH) - ihBase, kH) * kW);
-          // likewise one bit per valid kernel plane, at its first tap
-          const uint32_t planeStarts =
-              a.tapPlaneStarts &
-              bitRange(cut(int(d.loD) - idBase, kD) * kH * kW,
-                       cut(int(d.hiD) - idBase, kD) * kH * kW);
-          mask = kwMask * rowStarts * planeStarts;
-        } else {
-          uint32_t kwMask = 0;
-          for (uint32_t kw = 0; kw != d.kW; ++kw) {
-            const int iw = iwBase + int(kw * d.dilW);
-            if (iw >= int(d.loW) && iw < int(d.hiW))
-              kwMask |= 1u << kw;
-          }
-          uint32_t planeMask = 0;
-          for (uint32_t kh = 0; kh != d.kH; ++kh) {
-            const int ih = ihBase + int(kh * d.dilH);
-            if (ih >= int(d.loH) && ih < int(d.hiH))
-              planeMask |= kwMask << (kh * d.kW);
-          }
-          for (uint32_t kd = 0; kd != d.kD; ++kd) {
-            const int id = idBase + int(kd * d.dilD);
-            if (id >= int(d.loD) && id < int(d.hiD))
-              mask |= planeMask << (kd * d.kH * d.kW);
-          }
-        }
+        const uint32_t mask = tapMaskOf(a, idBase, ihBase, iwBase);
         rowTable[t] = uint2{originOffset, rowValid ? mask : 0u};
       }
     }
@@ -883,7 +837,10 @@ hipError_t prepare(const IgemmDesc &d, int inType, bool haveWorkspace,
   const uint32_t bke = kRowBytes / eb;
   const int mode = igemmTapAddressing(d);
   const bool dilated = mode == kDilatedTaps;
-  if (d.blockM != kBlockM || (d.blockN != 64 && d.blockN != 128) ||
+  const bool wide = d.blockM == 256;
+  if ((!wide && (d.blockM != kBlockM ||
+                 (d.blockN != 64 && d.blockN != 128))) ||
+      (wide && !igemmWideTakes(d, inType, kHalf)) ||
       d.blockK != bke || d.inChansPerGroup % (16 / eb) != 0 ||
       (inType != kHalf && inType != kQuarter && inType != kFloat) ||
       d.splitK == 0 ||
@@ -947,10 +904,11 @@ hipError_t prepare(const IgemmDesc &d, int inType, bool haveWorkspace,
   a.divOutW = makeFastDiv(d.outW);
   a.divOutH = makeFastDiv(d.outH);
   a.divOutD = makeFastDiv(d.outD);
-  a.mTiles = (a.M + kBlockM - 1) / kBlockM;
+  a.mTiles = (a.M + d.blockM - 1) / d.blockM;
   a.nTiles = (d.outChansPerGroup + d.blockN - 1) / d.blockN;
   a.divNTiles = makeFastDiv(a.nTiles);
   a.divMTiles = makeFastDiv(a.mTiles);
+  a.divWideBlock = makeFastDiv(4 * a.nTiles);
   a.divGroups = makeFastDiv(d.groups);
   // bit kh * kW for every kernel row (tap mask mode: at most 32 taps)
   a.tapRowStarts = a.tapPlaneStarts = 0;
@@ -988,6 +946,9 @@ hipError_t launchIgemm(const IgemmDesc &d, int inType, int outType,
   hipError_t e = prepare(d, inType, workspace != nullptr, a);
   if (e != hipSuccess)
     return e;
+  if (d.blockM == 256)
+    return launchIgemmWide(a, inType, outType, in, weightsPacked, bias, out, q,
+                           stream);
   const float scale = inType == kQuarter ? q.scale : 1.0f;
   if (d.splitK == 1)
     return dispatch(kernelKey(d, inType, outType, q),
@@ -1018,6 +979,7 @@ hipError_t launchIgemm(const IgemmDesc &d, int inType, int outType,
 
 bool igemmFusable(const IgemmFusedItem &x, const IgemmFusedItem &y) {
   return x.d->splitK == 1 && y.d->splitK == 1 &&
+         x.d->blockM == kBlockM && y.d->blockM == kBlockM &&
          kernelKey(*x.d, x.inType, x.outType, x.q) ==
              kernelKey(*y.d, y.inType, y.outType, y.q);
 }

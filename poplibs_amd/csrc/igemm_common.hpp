@@ -30,7 +30,15 @@ struct IgemmArgs {
   uint64_t inBytes;    // size of the input tensor
   uint32_t imageBytes; // ... and of one image (batch element) of it
   uint32_t wBytes;   // size of the packed weights
+  FastDiv divWideBlock; // by 4 * nTiles (igemm_wide.hip)
 };
+
+/// igemm_wide.hip: tiles of 256 pixels; `a` as prepared for igemmKernel.
+bool igemmWideTakes(const IgemmDesc &d, int inType, int outType);
+hipError_t launchIgemmWide(const IgemmArgs &a, int inType, int outType,
+                           const void *in, const void *w, const void *bias,
+                           void *out, const QuarterInfo &q,
+                           hipStream_t stream);
 
 namespace {
 
@@ -188,6 +196,25 @@ template <> struct Mma<2> {
           between();
       }
   }
+  /// load<S> and mul<S> in pieces, for a caller that places each: operand K
+  /// of the set (the two of A, then B's), the K-th (i, j) of the products.
+  template <int S, int K, int TN>
+  static __device__ __forceinline__ void loadOne(const FragmentAddress &at,
+                                                 int lane, Frags<TN> &f) {
+    const int c = S * 2 + (lane >> 5);
+    if constexpr (K < 2)
+      f.a[S][K] = *reinterpret_cast<const half8 *>(
+          at.a[K] + (((at.chunkBase + c) ^ at.swizzleA[K]) << 4));
+    else
+      f.b[S][K - 2] = *reinterpret_cast<const half8 *>(
+          at.b + (K - 2) * 32 * kRowBytes + ((c ^ at.swizzleB) << 4));
+  }
+  template <int S, int K, int TN, int FA, int FB>
+  static __device__ __forceinline__ void mulOne(const Frags<TN> &f,
+                                                floatx16 (&acc)[2][TN]) {
+    acc[K / TN][K % TN] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+        f.b[S][K % TN], f.a[S][K / TN], acc[K / TN][K % TN], 0, 0, 0);
+  }
 };
 
 /// fp32: 4 sub-steps of 8 values, 32 bytes (two chunks, one per half-wave)
@@ -228,6 +255,26 @@ template <> struct Mma<4> {
           if (e == 0 && i == 0 && j == 0)
             between();
         }
+  }
+  template <int S, int K, int TN>
+  static __device__ __forceinline__ void loadOne(const FragmentAddress &at,
+                                                 int lane, Frags<TN> &f) {
+    const int c = S * 2 + (lane >> 5);
+    if constexpr (K < 2)
+      f.a[S][K] = *reinterpret_cast<const floatx4 *>(
+          at.a[K] + (((at.chunkBase + c) ^ at.swizzleA[K]) << 4));
+    else
+      f.b[S][K - 2] = *reinterpret_cast<const floatx4 *>(
+          at.b + (K - 2) * 32 * kRowBytes + ((c ^ at.swizzleB) << 4));
+  }
+  template <int S, int K, int TN, int FA, int FB>
+  static __device__ __forceinline__ void mulOne(const Frags<TN> &f,
+                                                floatx16 (&acc)[2][TN]) {
+    // (the four depend on each other; the other wave of the SIMD fills in)
+#pragma unroll
+    for (int e = 0; e != 4; ++e)
+      acc[K / TN][K % TN] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+          f.b[S][K % TN][e], f.a[S][K / TN][e], acc[K / TN][K % TN], 0, 0, 0);
   }
 };
 
@@ -271,7 +318,97 @@ template <> struct Mma<1> {
           between();
       }
   }
+  template <int S, int K, int TN>
+  static __device__ __forceinline__ void loadOne(const FragmentAddress &at,
+                                                 int lane, Frags<TN> &f) {
+    const int c = S * 4 + (lane >> 5) * 2 + (K < 2 ? at.chunkBase : 0);
+    const int swizzle = K < 2 ? at.swizzleA[K & 1] : at.swizzleB;
+    const char *row = K < 2 ? at.a[K & 1] : at.b + (K - 2) * 32 * kRowBytes;
+    const uintx4 lo =
+        *reinterpret_cast<const uintx4 *>(row + ((c ^ swizzle) << 4));
+    const uintx4 hi =
+        *reinterpret_cast<const uintx4 *>(row + (((c + 1) ^ swizzle) << 4));
+    const intx8 v = {int(lo.x), int(lo.y), int(lo.z), int(lo.w),
+                     int(hi.x), int(hi.y), int(hi.z), int(hi.w)};
+    if constexpr (K < 2)
+      f.a[S][K] = v;
+    else
+      f.b[S][K - 2] = v;
+  }
+  template <int S, int K, int TN, int FA, int FB>
+  static __device__ __forceinline__ void mulOne(const Frags<TN> &f,
+                                                floatx16 (&acc)[2][TN]) {
+    acc[K / TN][K % TN] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+        f.b[S][K % TN], f.a[S][K / TN], acc[K / TN][K % TN], FB, FA, 0, 0, 0,
+        0);
+  }
 };
+
+/// The kernel taps (at most 32, bit (kd * kH + kh) * kW + kw) that read inside
+/// the input for a window with its origin at (idBase, ihBase, iwBase).
+__device__ __forceinline__ uint32_t tapMaskOf(const IgemmArgs &a, int idBase,
+                                              int ihBase, int iwBase) {
+  const IgemmDesc &d = a.d;
+  if (d.dilD == 1 && d.dilH == 1 && d.dilW == 1) {
+    // Undilated kernel: the valid kernel columns are the interval
+    // [lo - base, hi - base) cut to the kernel, and so are the rows.
+    // Bits [first, last) of a word:
+    auto bitRange = [](int first, int last) {
+      return first < last
+                 ? uint32_t(((1ull << last) - 1) & ~((1ull << first) - 1))
+                 : 0u;
+    };
+    auto cut = [](int v, int size) { return v < 0 ? 0 : v > size ? size : v; };
+    const int kW = int(d.kW), kH = int(d.kH), kD = int(d.kD);
+    const uint32_t kwMask = bitRange(cut(int(d.loW) - iwBase, kW),
+                                     cut(int(d.hiW) - iwBase, kW));
+    // one bit per valid kernel row, at that row's first tap; the product puts
+    // the column mask there (no carries: it is narrower than the distance
+    // between the bits)
+    const uint32_t rowStarts =
+        a.tapRowStarts & bitRange(cut(int(d.loH) - ihBase, kH) * kW,
+                                  cut(int(d.hiH) - ihBase, kH) * kW);
+    // likewise one bit per valid kernel plane, at its first tap
+    const uint32_t planeStarts =
+        a.tapPlaneStarts & bitRange(cut(int(d.loD) - idBase, kD) * kH * kW,
+                                    cut(int(d.hiD) - idBase, kD) * kH * kW);
+    return kwMask * rowStarts * planeStarts;
+  }
+  uint32_t kwMask = 0, planeMask = 0, mask = 0;
+  for (uint32_t kw = 0; kw != d.kW; ++kw) {
+    const int iw = iwBase + int(kw * d.dilW);
+    if (iw >= int(d.loW) && iw < int(d.hiW))
+      kwMask |= 1u << kw;
+  }
+  for (uint32_t kh = 0; kh != d.kH; ++kh) {
+    const int ih = ihBase + int(kh * d.dilH);
+    if (ih >= int(d.loH) && ih < int(d.hiH))
+      planeMask |= kwMask << (kh * d.kW);
+  }
+  for (uint32_t kd = 0; kd != d.kD; ++kd) {
+    const int id = idBase + int(kd * d.dilD);
+    if (id >= int(d.loD) && id < int(d.hiD))
+      mask |= planeMask << (kd * d.kH * d.kW);
+  }
+  return mask;
+}
+
+/// The output pixel of row m: m itself, or - one phase of a convolution over a
+/// zero-stuffed input, a padded output field - every outStep-th pixel of a
+/// larger field.
+__device__ __forceinline__ size_t outPixel(const IgemmArgs &a, uint32_t m) {
+  if (!a.outMapped)
+    return m;
+  const IgemmDesc &d = a.d;
+  const uint32_t q = a.divOutW(m), ow = m - q * d.outW;
+  const uint32_t q2 = a.divOutH(q), oh = q - q2 * d.outH;
+  const uint32_t image = a.divOutD(q2), od = q2 - image * d.outD;
+  return ((size_t(image) * d.outFullD + od * d.outStepD + d.outOffD) *
+              d.outFullH +
+          oh * d.outStepH + d.outOffH) *
+             d.outFullW +
+         ow * d.outStepW + d.outOffW;
+}
 
 /// LDS bytes the epilogue needs for a 128 x BN tile of OutT.
 template <int BN, class OutT> constexpr int epilogueLdsBytes() {
@@ -349,19 +486,7 @@ igemmEpilogue(char *lds, const IgemmArgs &a, floatx16 (&acc)[2][BN / 64],
     if (m >= a.M || n >= d.outChansPerGroup)
       continue;
     const char *src = lds + mLocal * kOutRow + vec * 16;
-    // the output pixel of row m: m itself, or - one phase of a convolution
-    // over a zero-stuffed input - every outStep-th pixel of a larger field
-    size_t pixel = m;
-    if (a.outMapped) {
-      const uint32_t q = a.divOutW(m), ow = m - q * d.outW;
-      const uint32_t q2 = a.divOutH(q), oh = q - q2 * d.outH;
-      const uint32_t image = a.divOutD(q2), od = q2 - image * d.outD;
-      pixel = ((size_t(image) * d.outFullD + od * d.outStepD + d.outOffD) *
-                   d.outFullH +
-               oh * d.outStepH + d.outOffH) *
-                  d.outFullW +
-              ow * d.outStepW + d.outOffW;
-    }
+    const size_t pixel = outPixel(a, m);
     if (a.outTransposed) {
       // [channel][pixel]: element stores, for small outputs
       const OutT *e = reinterpret_cast<const OutT *>(src);

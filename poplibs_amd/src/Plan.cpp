@@ -309,6 +309,32 @@ double estimateStreaming(std::size_t workgroups, std::size_t kSteps,
          (splitK > 1 ? splitPenaltyUs(partialBytes) : 0.0);
 }
 
+/// ... nor is it faster than the chip's power lets the matrix cores run, the
+/// work on padding counted: 950 TFLOP/s on a plain product in 128 x 128 tiles
+/// (4096 x 4096 x 4096), 800 where taps are gathered (N = 64, 56 x 56, 3 x 3
+/// stride 2, 256 -> 512: 740), 720 in 128 x 64 tiles (N = 71, 35 x 35, 3 x 3,
+/// 624 -> 136: 730); twice that in fp8, whose k-steps hold twice as much.
+double streamingPowerUs(std::size_t workgroups, std::size_t kSteps,
+                        unsigned blockN, bool oneTap) {
+  const double rate = blockN == 64 ? 7.2e8 : oneTap ? 9.5e8 : 8.0e8;
+  return double(workgroups) * double(kSteps) * 128.0 * blockN * 64.0 * 2.0 /
+         rate;
+}
+
+/// igemmWideKernel: 10 us per round around the loop (256 x 256 outputs leave
+/// at its end), 1.3 us per k-step of a workgroup, and where all CUs are busy
+/// 1.7 us - the chip's power (4096 x 4096 x 4096 120 us, 4096 x 1024 x 4096
+/// 38, 2048 x 4096 x 4096 on half the CUs 84, N = 64, 56 x 56, 3 x 3 stride 2,
+/// 256 -> 512 in 392 tiles 122); four fifths of it for tiles of 192 channels.
+double estimateWide(std::size_t workgroups, std::size_t kSteps,
+                    unsigned blockN) {
+  const double rounds = roundsOf(workgroups, 1);
+  const double step =
+      std::max(1.3 * rounds, 1.7 * double(workgroups) / gfx950::numCUs);
+  return kLaunchUs + 10.0 * rounds +
+         step * double(kSteps) * (blockN == 192 ? 0.8 : 1.0);
+}
+
 /// igemmPatchKernel (mode 1): 1.9 us to the first MFMA + 0.5 us reduction and
 /// stores, 0.333 us per k-step of 128 pixels (half of that for 64); one
 /// workgroup per CU, so further rounds pay their start-up in full (4.5 us
@@ -918,12 +944,16 @@ mxconv_plan makePlanWith(const ConvParams &params,
       }
     }
     const bool anyHeight = pc.patch == 2 && g.blockM >= 1 && g.blockM <= 112;
-    if ((g.blockM != 128 && g.blockM != 64 && !anyHeight) ||
-        (g.blockN != 64 && g.blockN != 128) ||
+    // (tiles of 256 pixels: igemm_wide.hip)
+    const bool wideTile = g.blockM == 256 && pc.patch < 1;
+    if ((g.blockM != 128 && g.blockM != 64 && !anyHeight && !wideTile) ||
+        (!wideTile && g.blockN != 64 && g.blockN != 128) ||
+        (wideTile && ((g.blockN != 192 && g.blockN != 256) || floatIn)) ||
         g.blockK != stepElems)
       throw poplar::invalid_option(
           "planConstraints gfx950 tile not available: blockM must be 128 (64 "
-          "with patch 1, 1 to 112 with patch 2), blockN 64 or 128, blockK 32 "
+          "with patch 1, 1 to 112 with patch 2), blockN 64 or 128 (blockM "
+          "256, half and quarter: blockN 192 or 256), blockK 32 "
           "(float), 64 (half) or 128 (quarter)");
     const std::size_t k = std::size_t(s.kD) * s.kH * s.kW * ciPadded;
     plan.coPadded = (co + g.blockN - 1) / g.blockN * g.blockN;
@@ -941,7 +971,9 @@ mxconv_plan makePlanWith(const ConvParams &params,
                                 (plan.coPadded / g.blockN) * p.numConvGroups;
       const std::size_t kSteps = plan.kPadded / g.blockK;
       std::size_t parts = 1;
-      if (pc.splitK)
+      if (g.blockM == 256)
+        parts = 1;
+      else if (pc.splitK)
         parts = pc.splitK;
       else if (narrowSplit)
         parts = narrowSplit;
@@ -1286,6 +1318,57 @@ mxconv_plan makePlanWith(const ConvParams &params,
         plan.weightPackedElems = mxk::igemmPatchPackedElems(g, inId);
       }
     }
+    // A problem that fills the chip: tiles of 256 pixels, where they are
+    // estimated to be faster than what is chosen so far.
+    if (!plan.pointwiseOn && plan.igemmPhases.empty() && !floatIn &&
+        pc.kernel.empty() && pc.method == Method::ANY && !pc.blockM &&
+        !pc.blockN && !pc.blockK && !pc.splitK && !pc.stages && pc.patch < 0 &&
+        pc.pointwise < 0 && !pc.chanTiles && g.splitK == 1 &&
+        !isWeightUpdatePass(options.pass)) {
+      const std::size_t m = s.batch * s.outD * s.outH * s.outW;
+      const std::size_t kSteps = plan.kPadded / g.blockK;
+      double planned;
+      if (g.patch) {
+        planned = 1e30;
+        for (const auto &c : plan.candidates)
+          if (c.chosen)
+            planned = 0.9 * c.estimateUs; // (an estimate on the high side)
+      } else {
+        const std::size_t tiles =
+            (m + 127) / 128 * (plan.coPadded / g.blockN) * p.numConvGroups;
+        planned = std::max(
+            estimateStreaming(tiles, kSteps,
+                              g.blockN == 64 || g.stages == 2 ? 2 : 1,
+                              g.blockN, 1, 0, false),
+            kLaunchUs + streamingPowerUs(tiles, kSteps, g.blockN,
+                                         s.kD * s.kH * s.kW == 1));
+      }
+      for (uint32_t bn : {192u, 256u}) {
+        mxk::IgemmDesc t = g;
+        t.patch = 0, t.blockM = 256, t.blockN = bn;
+        const std::size_t tiles =
+            (m + 255) / 256 * ((co + bn - 1) / bn) * p.numConvGroups;
+        const double us = estimateWide(tiles, kSteps, bn);
+        if (us >= planned ||
+            p.numConvGroups * ((co + bn - 1) / bn * bn) * plan.kPadded *
+                    params.inputType.size() >=
+                (1ull << 31) ||
+            mxk::igemmTapAddressing(t) != mxk::kMaskTaps)
+          continue;
+        planned = us;
+        g = t;
+        plan.coPadded = (co + bn - 1) / bn * bn;
+        plan.weightPackedElems =
+            p.numConvGroups * plan.coPadded * plan.kPadded;
+        for (auto &c : plan.candidates)
+          c.chosen = false;
+        mxconv_plan::Candidate c;
+        c.name = "streaming 256 x " + std::to_string(bn);
+        c.workgroups = tiles, c.perCU = 1, c.kSteps = kSteps;
+        c.estimateUs = us, c.rounds = roundsOf(tiles, 1), c.chosen = true;
+        plan.candidates.push_back(c);
+      }
+    }
     // A problem too small for 128-pixel tiles to fill the chip: small tiles
     // with K split over the waves of a workgroup.
     {
@@ -1361,7 +1444,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
         plan.weightPackedElems = mxk::igemmSmallPackedElems(g, inId);
       }
     }
-    if (!g.patch && g.blockM != 128)
+    if (!g.patch && g.blockM != 128 && g.blockM != 256)
       throw poplar::invalid_option(
           "planConstraints gfx950 blockM 64 goes with the resident-patch "
           "kernel only");
@@ -1642,14 +1725,18 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
       break;
     const auto &g = igemm;
     const std::size_t m = std::size_t(g.batch) * g.outD * g.outH * g.outW;
-    const std::size_t tiles = (m + 127) / 128 * (coPadded / g.blockN) *
+    const std::size_t tiles = (m + g.blockM - 1) / g.blockM * (coPadded / g.blockN) *
                               g.groups * g.splitK;
     const std::size_t steps =
         (kPadded / g.blockK + g.splitK - 1) / g.splitK;
     const std::size_t perCU = g.blockN == 64 || g.stages == 2 ? 2 : 1;
-    double us = poplin::estimateStreaming(tiles, steps, perCU, g.blockN,
-                                          g.splitK,
-                                          mxk::igemmWorkspaceBytes(igemm), params.inputType == poplar::FLOAT);
+    double us =
+        g.blockM == 256
+            ? poplin::estimateWide(tiles, steps, g.blockN)
+            : poplin::estimateStreaming(tiles, steps, perCU, g.blockN,
+                                        g.splitK,
+                                        mxk::igemmWorkspaceBytes(igemm),
+                                        params.inputType == poplar::FLOAT);
     // No kernel is faster than its tensors stream.
     us = std::max(us, streamed(inputBytes() + outputBytes() +
                                weightPackedBytes()));
@@ -1810,6 +1897,10 @@ std::string mxconv_plan::describe() const {
                      "SIMD\n"
                    : "32 pixels, each k-step halved between the two waves of "
                      "a SIMD\n");
+      else if (g.blockM == 256)
+        os << "        data path                  8 waves, each fetching its "
+              "share and multiplying 64 x "
+           << g.blockN / 2 << "; 2 LDS stages, one workgroup per CU\n";
       else if (g.blockN == 128)
         os << "        LDS stages                 " << g.stages
            << (g.stages == 2 ? " (two workgroups per CU)\n"
