@@ -1031,64 +1031,6 @@ __global__ __launch_bounds__(kPatchThreads) void igemmPatch16Kernel(
 #endif
 }
 
-/// One element of the packed weights per thread:
-/// [group][block of kTN x 32 channels][k-step][K half][32 channels][operand j]
-/// [lane][16 bytes], or igemmPatch16Kernel's order of the same 4 KB per step
-/// and 32 channels.
-template <class T>
-__global__ __launch_bounds__(256) void packPatchWeightsKernel(
-    const T *__restrict__ src, T *__restrict__ dst, uint32_t co, uint32_t ci,
-    uint32_t taps, uint32_t blocks, uint32_t kSteps, uint32_t packedTaps,
-    uint64_t total, bool chansTransposed, bool selected,
-    IgemmTapSelection select, bool blocks16) {
-  constexpr uint32_t kVec = 16 / sizeof(T), kSlice = 128 / sizeof(T);
-  const uint64_t tid = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (tid >= total)
-    return;
-  const uint32_t e = uint32_t(tid % kVec);
-  const uint32_t lane = uint32_t(tid / kVec % 64);
-  const uint32_t j = uint32_t(tid / (kVec * 64) % 2);
-  const uint32_t c32 = uint32_t(tid / (kVec * 128) % kTN);
-  const uint32_t half = uint32_t(tid / (kVec * 128 * kTN) % 2);
-  const uint64_t rest = tid / (kVec * 256 * kTN);
-  const uint32_t kt = uint32_t(rest % kSteps);
-  const uint32_t block =
-      uint32_t(rest / kSteps % (blocks / kTN)) * kTN + c32;
-  const uint64_t g = rest / kSteps / (blocks / kTN);
-  uint32_t n, within;
-  if (blocks16) {
-    // igemmPatch16Kernel: operand `half * 2 + j` of the step is (K unit,
-    // column block) for fp16 and (column block, half of the lane's 32 bytes)
-    // for fp8; lane = (K quarter, channel of the column block)
-    const uint32_t quarter = lane >> 4;
-    n = block * 32 + (sizeof(T) == 2 ? j : half) * 16 + (lane & 15);
-    within = sizeof(T) == 2 ? half * 32 + quarter * 8 + e
-                            : j * 64 + quarter * 16 + e;
-  } else {
-    const uint32_t h = lane >> 5;
-    n = block * 32 + (lane & 31);
-    within = sizeof(T) == 2 ? half * 32 + j * 16 + h * 8 + e
-                            : half * 64 + h * 32 + j * 16 + e;
-  }
-  const uint32_t slice = kt / packedTaps;
-  uint32_t tap = kt % packedTaps;
-  const uint32_t c = slice * kSlice + within;
-  T v = T(0);
-  if (n < co && c < ci) {
-    if (selected) {
-      const uint32_t jw = tap % select.countW, r = tap / select.countW;
-      const uint32_t i = r % select.countH, plane = r / select.countH;
-      tap = ((select.firstD + plane * select.stepD) * select.kH +
-             select.firstH + i * select.stepH) *
-                select.kW +
-            select.firstW + jw * select.stepW;
-    }
-    v = chansTransposed ? src[((g * ci + c) * co + n) * taps + tap]
-                        : src[((g * co + n) * ci + c) * taps + tap];
-  }
-  dst[tid] = v;
-}
-
 uint32_t elemBytesOf(int type) {
   return type == kFloat ? 4 : type == kHalf ? 2 : 1;
 }
@@ -1282,41 +1224,13 @@ uint64_t igemmPatchPackedElems(const IgemmDesc &d, int inType) {
          (4096 / eb);
 }
 
-hipError_t launchPackIgemmPatchWeights(const IgemmDesc &d, int inType,
-                                       const void *src, void *dst,
-                                       uint32_t sourceTaps,
-                                       hipStream_t stream,
-                                       bool chansTransposed,
-                                       const IgemmTapSelection *select) {
-  const uint32_t eb = elemBytesOf(inType);
-  if (eb == 4 || (d.inChansPerGroup * eb) % 128 != 0)
-    return hipErrorInvalidValue;
-  const uint64_t total = igemmPatchPackedElems(d, inType);
-  if (total == 0)
-    return hipSuccess;
-  const uint32_t packedTaps = d.kH * d.kW;
-  const uint32_t kSteps = d.inChansPerGroup * eb / 128 * packedTaps;
-  const uint32_t blocks32 = (d.outChansPerGroup + 127) / 128 * 4;
-  const uint64_t blocks = (total + 255) / 256;
-  if (blocks > 0x7fffffffull)
-    return hipErrorInvalidConfiguration;
-  const IgemmTapSelection chosen = select ? *select : IgemmTapSelection{};
-  if (eb == 2)
-    hipLaunchKernelGGL(packPatchWeightsKernel<uint16_t>, dim3(uint32_t(blocks)),
-                       dim3(256), 0, stream,
-                       static_cast<const uint16_t *>(src),
-                       static_cast<uint16_t *>(dst), d.outChansPerGroup,
-                       d.inChansPerGroup, sourceTaps, blocks32, kSteps,
-                       packedTaps, total, chansTransposed, select != nullptr,
-                       chosen, d.patch == 2);
-  else
-    hipLaunchKernelGGL(packPatchWeightsKernel<uint8_t>, dim3(uint32_t(blocks)),
-                       dim3(256), 0, stream, static_cast<const uint8_t *>(src),
-                       static_cast<uint8_t *>(dst), d.outChansPerGroup,
-                       d.inChansPerGroup, sourceTaps, blocks32, kSteps,
-                       packedTaps, total, chansTransposed, select != nullptr,
-                       chosen, d.patch == 2);
-  return hipGetLastError();
+PackJob igemmPatchPackJob(const IgemmDesc &d, int inType) {
+  PackJob j;
+  j.taps = d.kH * d.kW;
+  j.steps = d.inChansPerGroup * elemBytesOf(inType) / 128 * j.taps;
+  j.blocks = (d.outChansPerGroup + 127) / 128 * 4;
+  j.ciPadded = d.inChansPerGroup;
+  return j;
 }
 
 hipError_t launchIgemmPatch(const IgemmDesc &d, int inType, int outType,

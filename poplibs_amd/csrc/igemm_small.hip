@@ -468,48 +468,6 @@ hipError_t launchSmall(int inType, uint32_t tile, const SmallLaunch &l) {
   return inType == kFloat ? launchType<4>(tile, l) : launchType<1>(tile, l);
 }
 
-/// One weight vector (a lane's 16 bytes of one k-step) per thread.
-template <class T>
-__global__ __launch_bounds__(256) void packSmallWeightsKernel(
-    const T *__restrict__ src, uint4 *__restrict__ dst, uint32_t co,
-    uint32_t ci, uint32_t ciPadded, uint32_t taps, uint32_t chunks,
-    uint32_t blocks, uint32_t steps, uint32_t total, bool chansTransposed,
-    bool selected, IgemmTapSelection select, FastDiv divSteps,
-    FastDiv divBlocks, FastDiv divChunks) {
-  const uint32_t id = blockIdx.x * 256 + threadIdx.x;
-  if (id >= total)
-    return;
-  constexpr uint32_t kVec = 16 / sizeof(T);
-  const uint32_t lane = id & 63;
-  const uint32_t q = divSteps(id >> 6), step = (id >> 6) - q * steps;
-  const uint32_t g = divBlocks(q), block = q - g * blocks;
-  const uint32_t n = block * 16 + (lane & 15);
-  const uint32_t c = step * 4 + (lane >> 4);
-  union {
-    T e[kVec];
-    uint4 u;
-  } v;
-  v.u = uint4{0, 0, 0, 0};
-  if (n < co && c < chunks) {
-    uint32_t tap = divChunks(c);
-    const uint32_t c0 = (c - tap * (ciPadded / kVec)) * kVec;
-    if (selected) {
-      const uint32_t i = tap / select.countW, j = tap - i * select.countW;
-      tap = (select.firstD * select.kH + select.firstH + i * select.stepH) *
-                select.kW +
-            select.firstW + j * select.stepW;
-    }
-#pragma unroll
-    for (uint32_t e = 0; e != kVec; ++e)
-      if (c0 + e < ci)
-        v.e[e] =
-            chansTransposed
-                ? src[(uint64_t(g * ci + c0 + e) * co + n) * taps + tap]
-                : src[(uint64_t(g * co + n) * ci + c0 + e) * taps + tap];
-  }
-  dst[id] = v.u;
-}
-
 } // namespace
 
 uint32_t igemmSmallTilePixels(uint32_t tile) {
@@ -569,40 +527,15 @@ bool igemmSmallTakes(const IgemmDesc &d, int inType, int outType) {
          igemmAddressable(d, inType);
 }
 
-hipError_t launchPackIgemmSmallWeights(const IgemmDesc &d, int inType,
-                                       const void *src, void *dst,
-                                       uint32_t sourceChans,
-                                       uint32_t sourceTaps,
-                                       hipStream_t stream,
-                                       bool chansTransposed,
-                                       const IgemmTapSelection *select) {
+PackJob igemmSmallPackJob(const IgemmDesc &d, int inType) {
   const uint32_t eb = elemBytesOf(inType);
-  const uint64_t vectors = igemmSmallPackedElems(d, inType) * eb / 16;
-  if (vectors == 0)
-    return hipSuccess;
-  if (vectors > 0x7fffffffull)
-    return hipErrorInvalidConfiguration;
-  const uint32_t steps = smallSteps(d, eb);
-  const uint32_t chunks = d.kH * d.kW * d.inChansPerGroup * eb / 16;
-  const uint32_t blocks = uint32_t(vectors / 64 / steps / d.groups);
-  const IgemmTapSelection chosen = select ? *select : IgemmTapSelection{};
-  auto go = [&](auto *from) {
-    using T = std::remove_const_t<std::remove_pointer_t<decltype(from)>>;
-    hipLaunchKernelGGL(packSmallWeightsKernel<T>,
-                       dim3(uint32_t((vectors + 255) / 256)), dim3(256), 0,
-                       stream, from, static_cast<uint4 *>(dst),
-                       d.outChansPerGroup, sourceChans, d.inChansPerGroup,
-                       sourceTaps, chunks, blocks, steps, uint32_t(vectors),
-                       chansTransposed, select != nullptr, chosen,
-                       makeFastDiv(steps), makeFastDiv(blocks),
-                       makeFastDiv(d.inChansPerGroup * eb / 16));
-    return hipGetLastError();
-  };
-  if (eb == 1)
-    return go(static_cast<const uint8_t *>(src));
-  if (eb == 2)
-    return go(static_cast<const uint16_t *>(src));
-  return go(static_cast<const uint32_t *>(src));
+  PackJob j;
+  j.steps = smallSteps(d, eb);
+  j.blocks = uint32_t(igemmSmallPackedElems(d, inType) * eb / 1024 / j.steps /
+                      d.groups);
+  j.ciPadded = d.inChansPerGroup;
+  j.taps = d.kH * d.kW;
+  return j;
 }
 
 namespace {

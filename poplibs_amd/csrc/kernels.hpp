@@ -56,14 +56,8 @@ hipError_t launchPermute4(const void *src, void *dst, const uint64_t srcDims[4],
 /// (strides in elements; elements of 2 or 4 bytes): channels-last activations
 /// with the batch axis moved innermost, as the weight update pass wants both
 /// of its operands.
-/// Weights in external order [groups][co][ci][taps] -> the block-diagonal
-/// weights [groups / perGroup][perGroup co][perGroup ci][taps] of the layer
-/// with `perGroup` neighbouring groups taken as one.
-hipError_t launchFuseGroupWeights(const void *src, void *dst, uint64_t groups,
-                                  uint64_t perGroup, uint64_t co, uint64_t ci,
-                                  uint64_t taps, int elemBytes,
-                                  hipStream_t stream);
-/// ... and back, for weight deltas: the diagonal blocks of
+/// Weight deltas of `perGroup` neighbouring groups taken as one (block-diagonal
+/// weights, launchPackWeights): the diagonal blocks of
 /// [groups / perGroup][perGroup co][perGroup ci][taps] -> [groups][co][ci][taps].
 hipError_t launchUnfuseGroupWeights(const void *src, void *dst,
                                     uint64_t groups, uint64_t perGroup,
@@ -129,14 +123,12 @@ hipError_t launchPadChans(const void *src, void *dst, uint64_t pixels,
                           uint32_t groups, uint32_t ci, uint32_t ciPadded,
                           int elemBytes, hipStream_t stream);
 
-/// Weights [G][Co][Ci][taps] -> [G][coPadded][kPadded] with k = tap * Ci + ci,
-/// zero-filled beyond Co and beyond taps * Ci: the B operand of the
-/// matrix-core kernel, K contiguous.  With ciPadded (not 0) every tap takes
-/// ciPadded places of k, the ones beyond Ci zero.
-/// `select` (optional) packs a sub-kernel: of a kH x kW kernel the taps
-/// (firstH + i * stepH, firstW + j * stepW), i < countH, j < countW, in that
-/// order; `taps` is then kH * kW of the source and K holds countH * countW of
-/// them (none: all zeros).
+/// Problems in one fused launch of the matrix-core kernels, and packings in
+/// one of launchPackWeights.
+constexpr size_t kIgemmMaxFused = 8;
+
+/// A sub-kernel: of a kH x kW kernel the taps (firstH + i * stepH,
+/// firstW + j * stepW), i < countH, j < countW, in that order.
 struct IgemmTapSelection {
   uint32_t kW;
   uint32_t firstH, stepH, countH, firstW, stepW, countW;
@@ -144,13 +136,38 @@ struct IgemmTapSelection {
   // kernel of kH rows per plane (1 plane, unselected, by default)
   uint32_t kH = 1, firstD = 0, stepD = 1, countD = 1;
 };
-hipError_t launchPackIgemmWeights(const void *src, void *dst, uint32_t groups,
-                                  uint32_t co, uint32_t ci, uint32_t taps,
-                                  uint32_t coPadded, uint32_t kPadded,
-                                  int elemBytes, hipStream_t stream,
-                                  bool chansTransposed = false,
-                                  uint32_t ciPadded = 0,
-                                  const IgemmTapSelection *select = nullptr);
+/// Weights to pack: [groups][co][ci][taps], or [groups][ci][co] (a matrix
+/// product's right-hand side, one tap) with chansTransposed.  `fuse` groups
+/// are packed as one of fuse x the channels, with the block-diagonal weights
+/// that keep the groups apart.
+struct PackSource {
+  const void *weights;
+  uint32_t groups, co, ci, taps, fuse;
+  int elemBytes;
+  bool chansTransposed;
+};
+/// Orders of packed weights, by what a vector of 16 bytes (of one tap's input
+/// channels) belongs to.
+enum PackLayout {
+  kPackRows,       // [group][channel][k]: K contiguous (igemm.hip)
+  kPackOperands16, // [group][16 channels][64-byte k-step][lane]
+  kPackOperands32, // [group][32 channels][32-byte k-step][lane]
+  kPackPatch16,    // igemm_patch.hip's operands, 16-pixel and 32-pixel blocks
+  kPackPatch32,
+};
+/// One packing: `steps` vectors (kPackRows) or k-steps of `blocks` rows or
+/// blocks of channels per group; K holds `taps` taps of ciPadded channels
+/// (whole vectors), all of the source's or the selected ones.  What is beyond
+/// the source's channels and the taps is zero.
+struct PackJob {
+  uint32_t blocks, steps, ciPadded, taps;
+  const IgemmTapSelection *select = nullptr;
+  uint64_t dstBytes = 0; // where in the destination it goes
+};
+/// Up to kIgemmMaxFused packings of the same weights in one launch.
+hipError_t launchPackWeights(const PackSource &source, PackLayout layout,
+                             const PackJob *jobs, size_t count, void *dst,
+                             hipStream_t stream);
 
 /// acts[outer][c] += bias[c] for `type` elements (kHalf or kFloat).
 hipError_t launchAddBias(int type, void *acts, const void *bias,
@@ -209,13 +226,13 @@ struct IgemmDesc {
   uint32_t stages = 4;
   // 1 or 2: the kernel that keeps a tile's input patch in LDS runs (unit
   // stride, channels in whole 128-byte slices; igemmPatchTakes); the packed
-  // weights then have its layout (launchPackIgemmPatchWeights).  1: 32-pixel
+  // weights then have its layout (igemmPatchPackJob).  1: 32-pixel
   // MFMA blocks, blockM 64 or 128; 2: 16-pixel MFMA blocks, blockM = pixels
   // per tile, any number up to 112.
   uint32_t patch = 0;
   // 1 to kIgemmSmallTiles: the kernel for small problems runs (tiles of 16 x
   // 16, 16 x 32, 32 x 32 or 64 x 32 pixels x channels; igemmSmallTakes); the
-  // packed weights then have its layout (launchPackIgemmSmallWeights).
+  // packed weights then have its layout (igemmSmallPackJob).
   uint32_t small = 0;
   // Patch rows the tallest tile of that kernel spans (igemmPatchMaxRows),
   // worked out once when the plan is made - it takes a walk over the tiles -
@@ -249,13 +266,7 @@ uint32_t igemmPatchMaxRows(const IgemmDesc &d);
 /// Elements of its packed weights:
 /// [G][32-channel block][K half][k-step][operand][lane][16 bytes].
 uint64_t igemmPatchPackedElems(const IgemmDesc &d, int inType);
-/// src as for launchPackIgemmWeights; sourceTaps: taps of the stored kernel.
-hipError_t launchPackIgemmPatchWeights(const IgemmDesc &d, int inType,
-                                       const void *src, void *dst,
-                                       uint32_t sourceTaps, hipStream_t stream,
-                                       bool chansTransposed = false,
-                                       const IgemmTapSelection *select =
-                                           nullptr);
+PackJob igemmPatchPackJob(const IgemmDesc &d, int inType);
 hipError_t launchIgemmPatch(const IgemmDesc &d, int inType, int outType,
                             const void *in, const void *weightsPacked,
                             const void *bias, void *out, const QuarterInfo &q,
@@ -274,15 +285,7 @@ uint32_t igemmSmallWaves(const IgemmDesc &d, int inType);
 /// Elements of its packed weights:
 /// [G][16-channel block][64-byte k-step][lane][16 bytes].
 uint64_t igemmSmallPackedElems(const IgemmDesc &d, int inType);
-/// src as for launchPackIgemmWeights; sourceChans, sourceTaps: the stored
-/// kernel's input channels (d's may be padded) and taps.
-hipError_t launchPackIgemmSmallWeights(const IgemmDesc &d, int inType,
-                                       const void *src, void *dst,
-                                       uint32_t sourceChans,
-                                       uint32_t sourceTaps, hipStream_t stream,
-                                       bool chansTransposed = false,
-                                       const IgemmTapSelection *select =
-                                           nullptr);
+PackJob igemmSmallPackJob(const IgemmDesc &d, int inType);
 hipError_t launchIgemmSmall(const IgemmDesc &d, int inType, int outType,
                             const void *in, const void *weightsPacked,
                             const void *bias, void *out, const QuarterInfo &q,
@@ -298,7 +301,6 @@ struct IgemmFusedItem {
   void *out;
   QuarterInfo q;
 };
-constexpr size_t kIgemmMaxFused = 8;
 bool igemmFusable(const IgemmFusedItem &x, const IgemmFusedItem &y);
 hipError_t launchIgemmFused(const IgemmFusedItem *items, size_t count,
                             hipStream_t stream);
@@ -328,9 +330,7 @@ bool pointwiseChanTilesOk(const PointwiseDesc &d, uint32_t chanTiles);
 /// Elements of the packed weights ([G][32-channel block][32-byte k-slice]
 /// [lane][16 bytes]).
 uint64_t pointwisePackedElems(const PointwiseDesc &d);
-hipError_t launchPackPointwiseWeights(const PointwiseDesc &d, const void *src,
-                                      void *dst, hipStream_t stream,
-                                      bool chansTransposed = false);
+PackJob pointwisePackJob(const PointwiseDesc &d);
 /// How launchPointwise runs a layer on a chip of `cus` compute units:
 /// persistent workgroups, each taking tiles of `tilePixels` pixels in turn
 /// through a ring of `ring` LDS buffers filled by `loaderWaves` waves.

@@ -7,40 +7,54 @@
 namespace mxk {
 namespace {
 
+/// Where element i of a permuted tensor comes from: the strides in the source
+/// of the destination's dimensions (backwards through it where negative, as
+/// wrapped numbers) from `srcBase` on.
 struct PermuteArgs {
   uint64_t dstDims[4];
-  uint64_t srcStride[4]; // stride in the source of each destination dimension
-  uint64_t total;
-  FastDiv div[4]; // by dstDims, for tensors of fewer than 2^31 elements
+  uint64_t srcStride[4];
+  uint64_t total, srcBase;
+};
+/// ... of fewer than 2^31 elements: 31-bit indices taken apart with
+/// multiply-high divisions instead of eight 64-bit ones per element, and
+/// arguments that a launch copies in a microsecond less.
+struct PermuteSmallArgs {
+  uint32_t total, srcBase;
+  uint32_t dstDims[3]; // the inner three
+  uint32_t srcStride[4];
+  FastDiv div[3];
 };
 
-/// Any permutation, one element per thread.  SMALL: 31-bit indices taken apart
-/// with multiply-high divisions instead of eight 64-bit ones per element.
-template <class T, bool SMALL>
+/// Any permutation, one element per thread.
+template <class T>
 __global__ __launch_bounds__(256) void permuteKernel(PermuteArgs a,
                                                      const T *__restrict__ src,
                                                      T *__restrict__ dst) {
-  const uint64_t tid = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const uint64_t tid = uint64_t(blockIdx.x) * 256 + threadIdx.x;
   if (tid >= a.total)
     return;
-  uint64_t srcIndex = 0;
-  if constexpr (SMALL) {
-    uint32_t rest = uint32_t(tid), index = 0;
-#pragma unroll
-    for (int j = 3; j > 0; --j) {
-      const uint32_t q = a.div[j](rest);
-      index += (rest - q * uint32_t(a.dstDims[j])) * uint32_t(a.srcStride[j]);
-      rest = q;
-    }
-    srcIndex = index + rest * uint32_t(a.srcStride[0]);
-  } else {
-    uint64_t rest = tid;
-    for (int j = 3; j >= 0; --j) {
-      srcIndex += (rest % a.dstDims[j]) * a.srcStride[j];
-      rest /= a.dstDims[j];
-    }
+  uint64_t srcIndex = a.srcBase, rest = tid;
+  for (int j = 3; j >= 0; --j) {
+    srcIndex += (rest % a.dstDims[j]) * a.srcStride[j];
+    rest /= a.dstDims[j];
   }
   dst[tid] = src[srcIndex];
+}
+template <class T>
+__global__ __launch_bounds__(256) void
+permuteSmallKernel(PermuteSmallArgs a, const T *__restrict__ src,
+                   T *__restrict__ dst) {
+  const uint32_t tid = blockIdx.x * 256 + threadIdx.x;
+  if (tid >= a.total)
+    return;
+  uint32_t srcIndex = a.srcBase, rest = tid;
+#pragma unroll
+  for (int j = 2; j >= 0; --j) {
+    const uint32_t q = a.div[j](rest);
+    srcIndex += (rest - q * a.dstDims[j]) * a.srcStride[j + 1];
+    rest = q;
+  }
+  dst[tid] = src[srcIndex + rest * a.srcStride[0]];
 }
 
 /// 16 bytes of neighbouring elements at any address: global memory takes such
@@ -231,41 +245,6 @@ __global__ __launch_bounds__(256) void interleaveKernel(
   }
 }
 
-template <class T>
-__global__ __launch_bounds__(256) void packIgemmWeightsKernel(
-    const T *__restrict__ src, T *__restrict__ dst, uint32_t co, uint32_t ci,
-    uint32_t ciPadded, uint32_t taps, uint32_t coPadded, uint32_t kPadded,
-    uint64_t total, bool chansTransposed, bool selected,
-    IgemmTapSelection select) {
-  const uint64_t tid = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (tid >= total)
-    return;
-  const uint32_t k = uint32_t(tid % kPadded);
-  const uint32_t n = uint32_t((tid / kPadded) % coPadded);
-  const uint64_t g = tid / (uint64_t(kPadded) * coPadded);
-  T v = T(0);
-  const uint32_t packedTaps =
-      selected ? select.countD * select.countH * select.countW : taps;
-  if (n < co && k < packedTaps * ciPadded) {
-    uint32_t tap = k / ciPadded;
-    const uint32_t c = k % ciPadded;
-    if (selected) {
-      const uint32_t j = tap % select.countW, rest = tap / select.countW;
-      const uint32_t i = rest % select.countH, plane = rest / select.countH;
-      tap = ((select.firstD + plane * select.stepD) * select.kH +
-             select.firstH + i * select.stepH) *
-                select.kW +
-            select.firstW + j * select.stepW;
-    }
-    // source [G][Co][Ci][taps], or [G][Ci][Co][taps] (a matrix
-    // multiplication's right-hand side)
-    if (c < ci)
-      v = chansTransposed ? src[((g * ci + c) * co + n) * taps + tap]
-                          : src[((g * co + n) * ci + c) * taps + tap];
-  }
-  dst[tid] = v;
-}
-
 /// One 16-byte vector of the padded tensor per thread.
 template <class T>
 __global__ __launch_bounds__(256) void padChansKernel(
@@ -286,37 +265,6 @@ __global__ __launch_bounds__(256) void padChansKernel(
   for (uint32_t i = 0; i != kVec; ++i)
     v.e[i] = c0 + i < ci ? src[pg * ci + c0 + i] : T(0);
   reinterpret_cast<uint4 *>(dst)[tid] = v.u;
-}
-
-struct FlipArgs {
-  uint64_t co, ci, taps, total;
-  uint32_t numDims;
-  uint32_t shape[kMaxDims];
-};
-
-template <class T>
-__global__ __launch_bounds__(256) void transposeChansFlipKernel(
-    FlipArgs a, const T *__restrict__ src, T *__restrict__ dst) {
-  const uint64_t tid = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (tid >= a.total)
-    return;
-  // tid indexes dst [g][ci][co][k]
-  uint64_t r = tid;
-  const uint64_t k = r % a.taps;
-  r /= a.taps;
-  const uint64_t co = r % a.co;
-  r /= a.co;
-  const uint64_t ci = r % a.ci;
-  const uint64_t g = r / a.ci;
-  // reverse every axis of the row-major tap index
-  uint64_t rem = k, flipped = 0, stride = 1;
-  for (int d = int(a.numDims) - 1; d >= 0; --d) {
-    const uint64_t x = rem % a.shape[d];
-    rem /= a.shape[d];
-    flipped += (a.shape[d] - 1 - x) * stride;
-    stride *= a.shape[d];
-  }
-  dst[tid] = src[((g * a.co + co) * a.ci + ci) * a.taps + flipped];
 }
 
 template <class T>
@@ -590,7 +538,7 @@ __global__ __launch_bounds__(256) void biasUpdateKernel(
   storeOut(biases, c, Load<T>::at(biases, c, 0) + scale * total);
 }
 
-/// The other way round, for weight deltas: the f diagonal blocks of every
+/// Weight deltas of groups that ran f as one: the f diagonal blocks of every
 /// fused group of [G / f][f co][f ci][taps] -> [G][co][ci][taps].  One element
 /// of the result per thread.
 template <class T>
@@ -612,30 +560,6 @@ unfuseGroupWeightsKernel(const T *__restrict__ src, T *__restrict__ dst,
                tap];
 }
 
-/// Weights [G][co][ci][taps] of G conv groups -> [G / f][f co][f ci][taps] of
-/// G / f groups that each take f of them as one: block (a, b) of a fused
-/// group's f x f blocks of co x ci channels is group (f g' + a)'s weights
-/// where a == b and zero elsewhere.  One element of the result per thread.
-template <class T>
-__global__ __launch_bounds__(256) void
-fuseGroupWeightsKernel(const T *__restrict__ src, T *__restrict__ dst,
-                       uint64_t f, uint64_t co, uint64_t ci, uint64_t taps,
-                       uint64_t total) {
-  const uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= total)
-    return;
-  const uint64_t tap = i % taps;
-  uint64_t rest = i / taps;
-  const uint64_t k = rest % (f * ci);
-  rest /= f * ci;
-  const uint64_t n = rest % (f * co);
-  const uint64_t fused = rest / (f * co);
-  const uint64_t a = n / co, b = k / ci;
-  dst[i] = a == b ? src[(((fused * f + a) * co + n % co) * ci + k % ci) * taps +
-                        tap]
-                  : T(0);
-}
-
 } // namespace
 
 namespace {
@@ -646,12 +570,22 @@ hipError_t permuteAny(const void *src, void *dst, const PermuteArgs &a,
   if (blocks > 0x7fffffffull)
     return hipErrorInvalidConfiguration;
   const dim3 grid{uint32_t(blocks)}, block{256};
-  if (a.total < 0x7fffffffull)
-    hipLaunchKernelGGL((permuteKernel<T, true>), grid, block, 0, stream, a,
+  if (a.total < 0x7fffffffull) {
+    PermuteSmallArgs s;
+    s.total = uint32_t(a.total), s.srcBase = uint32_t(a.srcBase);
+    for (int j = 0; j != 4; ++j) {
+      s.srcStride[j] = uint32_t(a.srcStride[j]);
+      if (j != 0) {
+        s.dstDims[j - 1] = uint32_t(a.dstDims[j]);
+        s.div[j - 1] = makeFastDiv(uint32_t(a.dstDims[j]));
+      }
+    }
+    hipLaunchKernelGGL(permuteSmallKernel<T>, grid, block, 0, stream, s,
                        static_cast<const T *>(src), static_cast<T *>(dst));
-  else
-    hipLaunchKernelGGL((permuteKernel<T, false>), grid, block, 0, stream, a,
+  } else {
+    hipLaunchKernelGGL(permuteKernel<T>, grid, block, 0, stream, a,
                        static_cast<const T *>(src), static_cast<T *>(dst));
+  }
   return hipGetLastError();
 }
 
@@ -788,14 +722,12 @@ hipError_t launchPermute4(const void *src, void *dst, const uint64_t srcDims[4],
     s *= dims[i];
   }
   PermuteArgs a;
-  a.total = s;
+  a.total = s, a.srcBase = 0;
   for (int j = 0; j != 4; ++j) {
     // destination dimensions, right-aligned
     const int d = j - (4 - n);
     a.dstDims[j] = d >= 0 ? dims[order[d]] : 1;
     a.srcStride[j] = d >= 0 ? stride[order[d]] : 0;
-    a.div[j] = makeFastDiv(
-        uint32_t(a.dstDims[j] < 0x7fffffffull ? a.dstDims[j] : 1));
   }
   switch (elemBytes) {
   case 1:
@@ -808,46 +740,6 @@ hipError_t launchPermute4(const void *src, void *dst, const uint64_t srcDims[4],
   return permuteAny<uint4>(src, dst, a, stream);
 }
 
-hipError_t launchPackIgemmWeights(const void *src, void *dst, uint32_t groups,
-                                  uint32_t co, uint32_t ci, uint32_t taps,
-                                  uint32_t coPadded, uint32_t kPadded,
-                                  int elemBytes, hipStream_t stream,
-                                  bool chansTransposed, uint32_t ciPadded,
-                                  const IgemmTapSelection *select) {
-  const IgemmTapSelection chosen = select ? *select : IgemmTapSelection{};
-  if (ciPadded == 0)
-    ciPadded = ci;
-  if (ciPadded < ci)
-    return hipErrorInvalidValue;
-  const uint64_t total = uint64_t(groups) * coPadded * kPadded;
-  if (total == 0)
-    return hipSuccess;
-  const uint64_t blocks = (total + 255) / 256;
-  if (blocks > 0x7fffffffull)
-    return hipErrorInvalidConfiguration;
-  const dim3 grid{uint32_t(blocks)}, block{256};
-  if (elemBytes == 1)
-    hipLaunchKernelGGL(packIgemmWeightsKernel<uint8_t>, grid, block, 0, stream,
-                       static_cast<const uint8_t *>(src),
-                       static_cast<uint8_t *>(dst), co, ci, ciPadded, taps,
-                       coPadded, kPadded, total, chansTransposed,
-                       select != nullptr, chosen);
-  else if (elemBytes == 2)
-    hipLaunchKernelGGL(packIgemmWeightsKernel<uint16_t>, grid, block, 0, stream,
-                       static_cast<const uint16_t *>(src),
-                       static_cast<uint16_t *>(dst), co, ci, ciPadded, taps,
-                       coPadded, kPadded, total, chansTransposed,
-                       select != nullptr, chosen);
-  else if (elemBytes == 4)
-    hipLaunchKernelGGL(packIgemmWeightsKernel<uint32_t>, grid, block, 0, stream,
-                       static_cast<const uint32_t *>(src),
-                       static_cast<uint32_t *>(dst), co, ci, ciPadded, taps,
-                       coPadded, kPadded, total, chansTransposed,
-                       select != nullptr, chosen);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
-}
 
 hipError_t launchPadChans(const void *src, void *dst, uint64_t pixels,
                           uint32_t groups, uint32_t ci, uint32_t ciPadded,
@@ -886,34 +778,32 @@ hipError_t launchWeightsTransposeChansFlipXY(const void *src, void *dst,
                                              hipStream_t stream) {
   if (numDims > uint32_t(kMaxDims))
     return hipErrorInvalidValue;
-  FlipArgs a{};
-  a.co = co, a.ci = ci, a.taps = 1, a.numDims = numDims;
-  for (uint32_t d = 0; d != numDims; ++d) {
-    a.shape[d] = kernelShape[d];
-    a.taps *= kernelShape[d];
-  }
-  a.total = groups * co * ci * a.taps;
+  uint64_t taps = 1;
+  for (uint32_t d = 0; d != numDims; ++d)
+    taps *= kernelShape[d];
+  PermuteArgs a;
+  a.total = groups * co * ci * taps;
   if (a.total == 0)
     return hipSuccess;
-  const uint64_t blocks = (a.total + 255) / 256;
-  if (blocks > 0x7fffffffull)
-    return hipErrorInvalidConfiguration;
-  const dim3 grid{uint32_t(blocks)}, block{256};
+  if (taps == 1) {
+    const uint64_t dims[4] = {1, groups, co, ci};
+    const int perm[4] = {0, 1, 3, 2};
+    return launchPermute4(src, dst, dims, perm, elemBytes, stream);
+  }
+  // dst [g][ci][co][k] = src [g][co][ci][taps - 1 - k]: every axis of the
+  // window reversed is its row-major index read from the end
+  const uint64_t dims[4] = {groups, ci, co, taps};
+  const uint64_t stride[4] = {co * ci * taps, taps, ci * taps, ~0ull};
+  for (int j = 0; j != 4; ++j)
+    a.dstDims[j] = dims[j], a.srcStride[j] = stride[j];
+  a.srcBase = taps - 1;
   if (elemBytes == 1)
-    hipLaunchKernelGGL(transposeChansFlipKernel<uint8_t>, grid, block, 0,
-                       stream, a, static_cast<const uint8_t *>(src),
-                       static_cast<uint8_t *>(dst));
-  else if (elemBytes == 2)
-    hipLaunchKernelGGL(transposeChansFlipKernel<uint16_t>, grid, block, 0,
-                       stream, a, static_cast<const uint16_t *>(src),
-                       static_cast<uint16_t *>(dst));
-  else if (elemBytes == 4)
-    hipLaunchKernelGGL(transposeChansFlipKernel<uint32_t>, grid, block, 0,
-                       stream, a, static_cast<const uint32_t *>(src),
-                       static_cast<uint32_t *>(dst));
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
+    return permuteAny<uint8_t>(src, dst, a, stream);
+  if (elemBytes == 2)
+    return permuteAny<uint16_t>(src, dst, a, stream);
+  if (elemBytes == 4)
+    return permuteAny<uint32_t>(src, dst, a, stream);
+  return hipErrorInvalidValue;
 }
 
 hipError_t launchAddBias(int type, void *acts, const void *bias,
@@ -1279,37 +1169,6 @@ hipError_t launchUnfuseGroupWeights(const void *src, void *dst,
     hipLaunchKernelGGL(unfuseGroupWeightsKernel<uint16_t>, grid, block, 0,
                        stream, static_cast<const uint16_t *>(src),
                        static_cast<uint16_t *>(dst), perGroup, co, ci, taps,
-                       total);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-
-hipError_t launchFuseGroupWeights(const void *src, void *dst, uint64_t groups,
-                                  uint64_t perGroup, uint64_t co, uint64_t ci,
-                                  uint64_t taps, int elemBytes,
-                                  hipStream_t stream) {
-  const uint64_t total = groups * perGroup * co * ci * taps;
-  if (total == 0)
-    return hipSuccess;
-  const uint64_t blocks = (total + 255) / 256;
-  if (blocks > 0x7fffffffull || groups % perGroup != 0)
-    return hipErrorInvalidConfiguration;
-  const dim3 grid{uint32_t(blocks)}, block{256};
-  if (elemBytes == 4)
-    hipLaunchKernelGGL(fuseGroupWeightsKernel<uint32_t>, grid, block, 0, stream,
-                       static_cast<const uint32_t *>(src),
-                       static_cast<uint32_t *>(dst), perGroup, co, ci, taps,
-                       total);
-  else if (elemBytes == 2)
-    hipLaunchKernelGGL(fuseGroupWeightsKernel<uint16_t>, grid, block, 0, stream,
-                       static_cast<const uint16_t *>(src),
-                       static_cast<uint16_t *>(dst), perGroup, co, ci, taps,
-                       total);
-  else if (elemBytes == 1)
-    hipLaunchKernelGGL(fuseGroupWeightsKernel<uint8_t>, grid, block, 0, stream,
-                       static_cast<const uint8_t *>(src),
-                       static_cast<uint8_t *>(dst), perGroup, co, ci, taps,
                        total);
   else
     return hipErrorInvalidValue;

@@ -14,6 +14,7 @@
 #include "poputil/exceptions.hpp"
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -731,6 +732,72 @@ mxconv_status mxconv_plans_pack_alike(const mxconv_plan *plan,
   return MXCONV_OK;
 }
 
+/// Packs the weights of a plan of one of the matrix-core kernels: of the conv
+/// groups it runs as one, of all the phases it runs.
+static hipError_t packIgemmWeights(const mxconv_plan &plan,
+                                   const void *weights, uint32_t taps,
+                                   bool chansTransposed, void *packed,
+                                   hipStream_t stream) {
+  const auto &p = plan.params;
+  const int inType = p.inputType.id();
+  if (plan.thinInputOn)
+    return mxk::launchPackThinInputWeights(plan.thinInput, weights, packed,
+                                           stream);
+  const mxk::PackSource source{weights,
+                               uint32_t(p.numConvGroups),
+                               uint32_t(p.outputChannelsPerConvGroup),
+                               uint32_t(p.inputChannelsPerConvGroup),
+                               taps,
+                               plan.convGroupsPerGroup,
+                               int(p.inputType.size()),
+                               chansTransposed};
+  const uint32_t vectorElems = 16 / source.elemBytes;
+  const uint32_t ciPadded = plan.paddedInputChans
+                                ? uint32_t(plan.paddedInputChans)
+                                : source.ci * source.fuse;
+  std::array<mxk::PackJob, mxk::kIgemmMaxFused> jobs;
+  size_t count = 0;
+  mxk::PackLayout layout = mxk::kPackRows;
+  if (!plan.igemmPhases.empty()) {
+    // (no plan has more of them than a launch takes)
+    if (plan.igemmPhases.size() > jobs.size())
+      return hipErrorInvalidValue;
+    for (const auto &phase : plan.igemmPhases) {
+      mxk::PackJob &j = jobs[count++];
+      j.blocks = uint32_t(plan.coPadded);
+      j.steps = uint32_t(phase.kPadded) / vectorElems;
+      j.ciPadded = ciPadded;
+      j.taps = phase.taps.countD * phase.taps.countH * phase.taps.countW;
+      j.select = &phase.taps;
+      j.dstBytes = phase.packedOffset * source.elemBytes;
+    }
+    return mxk::launchPackWeights(source, layout, jobs.data(), count, packed,
+                                  stream);
+  }
+  mxk::PackJob j;
+  if (plan.pointwiseOn) {
+    layout = mxk::kPackOperands32;
+    j = mxk::pointwisePackJob(plan.pointwise);
+  } else if (plan.igemm.small) {
+    layout = mxk::kPackOperands16;
+    j = mxk::igemmSmallPackJob(plan.igemm, inType);
+  } else if (plan.igemm.patch) {
+    layout = plan.igemm.patch == 2 ? mxk::kPackPatch16 : mxk::kPackPatch32;
+    j = mxk::igemmPatchPackJob(plan.igemm, inType);
+  } else {
+    j.blocks = uint32_t(plan.coPadded);
+    j.steps = uint32_t(plan.kPadded) / vectorElems;
+    j.ciPadded = ciPadded;
+    j.taps = taps;
+  }
+  if (plan.kernelSelected && !plan.pointwiseOn) {
+    const auto &t = plan.igemmTaps;
+    j.select = &t;
+    j.taps = t.countD * t.countH * t.countW;
+  }
+  return mxk::launchPackWeights(source, layout, &j, 1, packed, stream);
+}
+
 mxconv_status mxconv_pack_weights(const mxconv_plan *plan,
                                   const void *weights_external,
                                   void *weights_packed, mxconv_stream stream) {
@@ -748,69 +815,9 @@ mxconv_status mxconv_pack_weights(const mxconv_plan *plan,
   if (plan->kernel == mxconv_plan::Kernel::IGEMM) {
     if (plan->weightElems != 0)
       REQUIRE_ARG(weights_external);
-    // Conv groups run as one: their block-diagonal weights, in external
-    // order, are laid out behind the packed weights first and packed from
-    // there as the weights of the fused groups.
-    uint32_t groups = uint32_t(p.numConvGroups);
-    uint32_t co = uint32_t(p.outputChannelsPerConvGroup);
-    uint32_t ci = uint32_t(p.inputChannelsPerConvGroup);
-    if (plan->convGroupsPerGroup > 1) {
-      const uint32_t f = plan->convGroupsPerGroup;
-      void *fused = static_cast<char *>(weights_packed) +
-                    plan->weightPackedElems * elemBytes;
-      const mxconv_status st = hipStatus(
-          mxk::launchFuseGroupWeights(weights_external, fused, groups, f, co,
-                                      ci, taps, elemBytes, s),
-          "weight packing");
-      if (st != MXCONV_OK)
-        return st;
-      weights_external = fused;
-      groups /= f, co *= f, ci *= f;
-    }
-    if (plan->thinInputOn)
-      return hipStatus(mxk::launchPackThinInputWeights(
-                           plan->thinInput, weights_external, weights_packed, s),
-                       "weight packing");
-    if (plan->pointwiseOn)
-      return hipStatus(mxk::launchPackPointwiseWeights(
-                           plan->pointwise, weights_external, weights_packed, s),
-                       "weight packing");
-    if (plan->igemm.small)
-      return hipStatus(
-          mxk::launchPackIgemmSmallWeights(
-              plan->igemm, p.inputType.id(), weights_external, weights_packed,
-              ci, uint32_t(taps), s, false,
-              plan->kernelSelected ? &plan->igemmTaps : nullptr),
-          "weight packing");
-    for (const auto &phase : plan->igemmPhases) {
-      const mxconv_status st = hipStatus(
-          mxk::launchPackIgemmWeights(
-              weights_external,
-              static_cast<char *>(weights_packed) +
-                  phase.packedOffset * elemBytes,
-              groups, co, ci, uint32_t(taps),
-              uint32_t(plan->coPadded), uint32_t(phase.kPadded), elemBytes, s,
-              false, uint32_t(plan->paddedInputChans), &phase.taps),
-          "weight packing");
-      if (st != MXCONV_OK)
-        return st;
-    }
-    if (!plan->igemmPhases.empty())
-      return MXCONV_OK;
-    if (plan->igemm.patch)
-      return hipStatus(
-          mxk::launchPackIgemmPatchWeights(
-              plan->igemm, p.inputType.id(), weights_external, weights_packed,
-              uint32_t(taps), s, false,
-              plan->kernelSelected ? &plan->igemmTaps : nullptr),
-          "weight packing");
-    return hipStatus(
-        mxk::launchPackIgemmWeights(
-            weights_external, weights_packed, groups, co, ci, uint32_t(taps),
-            uint32_t(plan->coPadded), uint32_t(plan->kPadded), elemBytes, s,
-            false, uint32_t(plan->paddedInputChans),
-            plan->kernelSelected ? &plan->igemmTaps : nullptr),
-        "weight packing");
+    return hipStatus(packIgemmWeights(*plan, weights_external, uint32_t(taps),
+                                      false, weights_packed, s),
+                     "weight packing");
   }
   REQUIRE_ARG(weights_external);
   // [G][Co][Ci][K] -> [G][K][Ci][Co]; with Co = Ci = 1 this is also the
@@ -1231,30 +1238,9 @@ mxconv_status mxconv_matmul_pack_rhs(const mxconv_plan *plan, const void *rhs,
     REQUIRE_ARG(rhs);
   const auto &p = plan->params;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int elemBytes = int(p.inputType.size());
   if (plan->kernel == mxconv_plan::Kernel::IGEMM) {
-    if (plan->pointwiseOn)
-      return hipStatus(mxk::launchPackPointwiseWeights(plan->pointwise, rhs,
-                                                       weights_packed, s, true),
-                       "weight packing");
-    if (plan->igemm.small)
-      return hipStatus(mxk::launchPackIgemmSmallWeights(
-                           plan->igemm, p.inputType.id(), rhs, weights_packed,
-                           uint32_t(p.inputChannelsPerConvGroup), 1, s, true),
-                       "weight packing");
-    if (plan->igemm.patch)
-      return hipStatus(mxk::launchPackIgemmPatchWeights(
-                           plan->igemm, p.inputType.id(), rhs, weights_packed,
-                           1, s, true),
-                       "weight packing");
-    return hipStatus(
-        mxk::launchPackIgemmWeights(
-            rhs, weights_packed, uint32_t(p.numConvGroups),
-            uint32_t(p.outputChannelsPerConvGroup),
-            uint32_t(p.inputChannelsPerConvGroup), 1, uint32_t(plan->coPadded),
-            uint32_t(plan->kPadded), elemBytes, s, true,
-            uint32_t(plan->paddedInputChans)),
-        "weight packing");
+    return hipStatus(packIgemmWeights(*plan, rhs, 1, true, weights_packed, s),
+                     "weight packing");
   }
   // Generic kernel: packed = [G][1][Ci][Co], which is B itself.  Depthwise
   // kernel (k = n = 1): packed = [1][G], again B itself.

@@ -403,34 +403,6 @@ __global__ __launch_bounds__(TM * 4 + 64 * LW) void pointwiseKernel(
   }
 }
 
-/// Weights [G][Co][Ci] -> [G][32-channel block][k-slice][lane][16 bytes]:
-/// lane l of a slice holds channel l % 32 of the block, and of its input
-/// channels the E = 8 (fp16) or 16 (fp8) from 2 E slice + E (l / 32) on - the
-/// row operand of pwMma.  Channels past Co are zero, and so are input channels
-/// past Ci (the slices run to the padded row, `slices` of 32 bytes).
-template <class T>
-__global__ __launch_bounds__(256) void packPointwiseWeightsKernel(
-    const T *__restrict__ src, T *__restrict__ dst, uint32_t co, uint32_t ci,
-    uint32_t slices, uint32_t nBlocks, uint64_t total, bool chansTransposed) {
-  constexpr uint32_t E = 16 / sizeof(T);
-  const uint64_t tid = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (tid >= total)
-    return;
-  const uint32_t e = uint32_t(tid % E), lane = uint32_t(tid / E) & 63;
-  uint64_t r = tid / (64 * E);
-  const uint32_t ks = uint32_t(r % slices);
-  r /= slices;
-  const uint32_t block = uint32_t(r % nBlocks);
-  const uint64_t g = r / nBlocks;
-  const uint32_t n = block * 32 + (lane & 31);
-  const uint32_t k = ks * 2 * E + E * (lane >> 5) + e;
-  // source [G][Co][Ci], or [G][Ci][Co] (a matrix multiplication's right-hand
-  // side)
-  dst[tid] = n >= co || k >= ci ? T(0)
-             : chansTransposed  ? src[(g * ci + k) * co + n]
-                                : src[(g * co + n) * ci + k];
-}
-
 /// Workgroups that share the pixel tiles of one (group, channel tile) pair:
 /// as many workgroups as fit the chip at once (LDS allows 160 KB / ldsBytes
 /// per CU), shared out over the pairs - and no more than give every walker
@@ -643,32 +615,16 @@ uint64_t pointwisePackedElems(const PointwiseDesc &d) {
          (1024 / d.elemBytes);
 }
 
-hipError_t launchPackPointwiseWeights(const PointwiseDesc &d, const void *src,
-                                      void *dst, hipStream_t stream,
-                                      bool chansTransposed) {
-  const uint64_t total = pointwisePackedElems(d);
-  if (total == 0)
-    return hipSuccess;
-  const uint64_t blocks = (total + 255) / 256;
-  if (blocks > 0x7fffffffull)
-    return hipErrorInvalidConfiguration;
-  const uint32_t nBlocks = (d.outChansPerGroup + kPwChans - 1) / kPwChans * 2;
-  const uint32_t slices = pwPaddedChans(pwRowChans(d)) / 16;
-  if (d.elemBytes == 2)
-    hipLaunchKernelGGL(packPointwiseWeightsKernel<uint16_t>,
-                       dim3(uint32_t(blocks)), dim3(256), 0, stream,
-                       static_cast<const uint16_t *>(src),
-                       static_cast<uint16_t *>(dst), d.outChansPerGroup,
-                       d.inChansPerGroup, slices, nBlocks, total,
-                       chansTransposed);
-  else
-    hipLaunchKernelGGL(packPointwiseWeightsKernel<uint8_t>,
-                       dim3(uint32_t(blocks)), dim3(256), 0, stream,
-                       static_cast<const uint8_t *>(src),
-                       static_cast<uint8_t *>(dst), d.outChansPerGroup,
-                       d.inChansPerGroup, slices, nBlocks, total,
-                       chansTransposed);
-  return hipGetLastError();
+/// Lane l of a slice holds channel l % 32 of the block, and of its input
+/// channels the E = 8 (fp16) or 16 (fp8) from 2 E slice + E (l / 32) on - the
+/// row operand of pwMma (the slices run to the padded row).
+PackJob pointwisePackJob(const PointwiseDesc &d) {
+  PackJob j;
+  j.blocks = (d.outChansPerGroup + kPwChans - 1) / kPwChans * 2;
+  j.steps = pwPaddedChans(pwRowChans(d)) / 16;
+  j.ciPadded = j.steps * 32 / d.elemBytes;
+  j.taps = 1;
+  return j;
 }
 
 PointwiseLaunch pointwiseLaunchShape(const PointwiseDesc &d, uint32_t cus) {

@@ -117,9 +117,9 @@ struct mxconv_plan {
   // already, so only the weight packing knows.  The role of the reference
   // planner's convGroupsPerGroup (lib/poplin/ConvPlan.cpp, the AMP and SLIC
   // vertices that take several conv groups at once).  The packed-weights
-  // buffer then has room behind the packed weights for the block-diagonal
-  // weights in external order, `weightExpandElems` elements, which the
-  // packing fills first.
+  // buffer's size, which callers know, has room for the block-diagonal
+  // weights in external order behind the packed ones (`weightExpandElems`
+  // elements), though the packing works them out as it goes.
   unsigned convGroupsPerGroup = 1;
   std::size_t weightExpandElems = 0;
   // A weight update pass planned for the layer with that many conv groups
