@@ -145,15 +145,15 @@ __global__ __launch_bounds__(256) void transposeKernel(
 
 /// The same where one side is only N elements - an image's channels: TO_LAST
 /// [batch][N][pixels] -> [batch][pixels][N], else the other way round.  A
-/// workgroup takes 256 vectors of pixels; a thread turns N vectors round in
+/// workgroup takes a vector of pixels per thread; a thread turns N vectors round in
 /// registers, and LDS makes both sides' accesses consecutive 16-byte pieces.
 /// Bound by HBM (N = 32 images of 3 x 224 x 224 halves: 18.5 -> 5.6 us).
-template <class T, int N, bool TO_LAST>
-__global__ __launch_bounds__(256) void interleaveKernel(
+template <class T, int N, bool TO_LAST, uint32_t THREADS>
+__global__ __launch_bounds__(THREADS) void interleaveKernel(
     const T *__restrict__ src, T *__restrict__ dst, uint64_t pixels,
     uint32_t blocksPerImage) {
-  constexpr uint32_t kVec = 16 / sizeof(T), kPixels = 256 * kVec;
-  __shared__ uint4 packed[256 * N];
+  constexpr uint32_t kVec = 16 / sizeof(T), kPixels = THREADS * kVec;
+  __shared__ uint4 packed[THREADS * N];
   const uint32_t image = blockIdx.x / blocksPerImage;
   const uint64_t p0 =
       uint64_t(blockIdx.x - image * blocksPerImage) * kPixels;
@@ -190,12 +190,12 @@ __global__ __launch_bounds__(256) void interleaveKernel(
     T *to = dst + base + p0 * N;
 #pragma unroll
     for (int n = 0; n != N; ++n) {
-      const uint32_t i = (n * 256 + threadIdx.x) * kVec;
+      const uint32_t i = (n * THREADS + threadIdx.x) * kVec;
       union {
         uint4 raw;
         Piece<T> p;
       } v;
-      v.raw = packed[n * 256 + threadIdx.x];
+      v.raw = packed[n * THREADS + threadIdx.x];
       if (i + kVec <= left) {
         storePiece(to + i, v.p);
       } else {
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(256) void interleaveKernel(
     const T *from = src + base + p0 * N;
 #pragma unroll
     for (int n = 0; n != N; ++n) {
-      const uint32_t i = (n * 256 + threadIdx.x) * kVec;
+      const uint32_t i = (n * THREADS + threadIdx.x) * kVec;
       union {
         uint4 raw;
         Piece<T> p;
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256) void interleaveKernel(
         for (uint32_t e = 0; e != kVec; ++e)
           v.p.e[e] = i + e < left ? from[i + e] : T(0);
       }
-      packed[n * 256 + threadIdx.x] = v.raw;
+      packed[n * THREADS + threadIdx.x] = v.raw;
     }
     __syncthreads();
 #pragma unroll
@@ -592,16 +592,24 @@ hipError_t permuteAny(const void *src, void *dst, const PermuteArgs &a,
 template <class T, int N, bool TO_LAST>
 hipError_t interleave(const void *src, void *dst, uint64_t batch,
                       uint64_t pixels, hipStream_t stream) {
-  const uint64_t perImage =
-      (pixels + 256 * (16 / sizeof(T)) - 1) / (256 * (16 / sizeof(T)));
-  const uint64_t blocks = batch * perImage;
-  if (blocks > 0x7fffffffull)
-    return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((interleaveKernel<T, N, TO_LAST>),
-                     dim3{uint32_t(blocks)}, dim3{256}, 0, stream,
-                     static_cast<const T *>(src), static_cast<T *>(dst), pixels,
-                     uint32_t(perImage));
-  return hipGetLastError();
+  constexpr uint32_t kVec = 16 / sizeof(T);
+  auto launch = [&](auto threads) {
+    constexpr uint32_t THREADS = decltype(threads)::value;
+    const uint64_t perImage =
+        (pixels + THREADS * kVec - 1) / (THREADS * kVec);
+    const uint64_t blocks = batch * perImage;
+    if (blocks > 0x7fffffffull)
+      return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL((interleaveKernel<T, N, TO_LAST, THREADS>),
+                       dim3{uint32_t(blocks)}, dim3{THREADS}, 0, stream,
+                       static_cast<const T *>(src), static_cast<T *>(dst),
+                       pixels, uint32_t(perImage));
+    return hipGetLastError();
+  };
+  // Few images: single-wave workgroups, or a handful of CUs do all the work.
+  if (batch * pixels < 256ull * 256 * kVec)
+    return launch(std::integral_constant<uint32_t, 64>{});
+  return launch(std::integral_constant<uint32_t, 256>{});
 }
 
 /// [batch][rows][cols] -> [batch][cols][rows]; *taken = false and nothing
@@ -612,9 +620,13 @@ hipError_t transposeBatches(const void *src, void *dst, uint64_t batch,
                             bool *taken) {
   *taken = true;
   // Two to four elements on one side (an image's channels): tiles of 64 would
-  // be nearly empty.  Worth it from half a workgroup of pixels on.
+  // be nearly empty.  Worth it from half a workgroup of pixels on, and from a
+  // few vectors for every CU: below, an element per thread is the shorter
+  // chain (halves of three channels, 191 x 191 pixels: 2.8 against 3.5 us;
+  // three images of 239 x 239: 3.7 against 3.4).
   const uint64_t fewest = 128 * (16 / sizeof(T));
-  if (cols >= fewest) {
+  const bool many = batch * rows * cols >= 256 * 1024;
+  if (many && cols >= fewest) {
     if (rows == 2)
       return interleave<T, 2, true>(src, dst, batch, cols, stream);
     if (rows == 3)
@@ -622,7 +634,7 @@ hipError_t transposeBatches(const void *src, void *dst, uint64_t batch,
     if (rows == 4)
       return interleave<T, 4, true>(src, dst, batch, cols, stream);
   }
-  if (rows >= fewest) {
+  if (many && rows >= fewest) {
     if (cols == 2)
       return interleave<T, 2, false>(src, dst, batch, rows, stream);
     if (cols == 3)

@@ -42,7 +42,7 @@ struct ThinArgs {
   uint32_t tilesPerImage, tiles;
   uint32_t colBlocks;  // blocks of 16 output pixels per row
   FastDiv divTilesPerImage, divColBlocks;
-  FastDiv divRowUnits; // by the 16-byte vectors (or dwords) of an input row
+  FastDiv divRowUnits; // by the 16-byte vectors (rows below 16 bytes: dwords) of a row
   FastDiv divBorder;   // by the dwords of zeros left and right of a row
   uint32_t biasByte;   // where the fp32 bias lies in LDS
   uint32_t weightByte; // ... and the packed weights, on their way to registers
@@ -104,13 +104,25 @@ __global__ void packThinWeightsKernel(const __half *__restrict__ src,
   dst[i] = v;
 }
 
+/// Sixteen bytes at any even address.
+typedef uintx4 uintx4Unaligned __attribute__((aligned(2)));
+
 /// Input rows ih0 .. ih0 + ldsRows - 1 of an image into LDS in units of V
-/// (16 or 4 bytes), zeros for rows outside [loH, hiH).
-template <class V>
+/// (16 or 4 bytes), zeros for rows outside [loH, hiH).  RAGGED: rows of no
+/// whole vectors - of an odd field's three channels, say, which start at any
+/// even byte - are read in vectors all the same; a row's last one is the 16
+/// bytes up to the row's end, moved down to where it belongs, with zeros
+/// behind.  (Odd fields took the padded copy and the streaming kernel before:
+/// N = 32, 223 x 223, 3 x 3, 3 -> 64: 146 -> 42 us; N = 16, 129 x 129, 7 x 7:
+/// 46 -> 18.  Rows of whole dwords, copied in dwords before: 5.9 -> 5.7 us for
+/// N = 3, 122 x 122, 7 x 7 stride 2, 3 -> 48.)
+template <class V, bool RAGGED>
 __device__ __forceinline__ void copyRows(const ThinArgs &a, char *lds,
                                          const char *img, int32_t ih0, int t) {
+  static_assert(!RAGGED || sizeof(V) == 16, "whole vectors");
   constexpr int kBatch = 8;
-  const uint32_t units = a.rowBytes / uint32_t(sizeof(V));
+  const uint32_t units =
+      (a.rowBytes + (RAGGED ? 15 : 0)) / uint32_t(sizeof(V));
   const uint32_t total = a.ldsRows * units;
   for (uint32_t first = 0; first < total; first += kBatch * kThinThreads) {
     V v[kBatch];
@@ -123,8 +135,28 @@ __device__ __forceinline__ void copyRows(const ThinArgs &a, char *lds,
       at[u] = i < total ? row * a.pitch + a.dataOff + c * uint32_t(sizeof(V))
                         : ~0u;
       v[u] = V{};
-      if (i < total && ih >= int32_t(a.d.loH) && ih < int32_t(a.d.hiH))
-        v[u] = reinterpret_cast<const V *>(img + size_t(ih) * a.rowBytes)[c];
+      if (i < total && ih >= int32_t(a.d.loH) && ih < int32_t(a.d.hiH)) {
+        const char *rowAt = img + size_t(ih) * a.rowBytes;
+        if constexpr (RAGGED) {
+          const uint32_t last = a.rowBytes - 16;
+          v[u] = *reinterpret_cast<const uintx4Unaligned *>(
+              rowAt + (c * 16 < last ? c * 16 : last));
+        } else {
+          v[u] = reinterpret_cast<const V *>(rowAt)[c];
+        }
+      }
+    }
+    if constexpr (RAGGED) {
+      const uint32_t down = (units * 16 - a.rowBytes) * 8; // bits, < 128
+#pragma unroll
+      for (int u = 0; u != kBatch; ++u) {
+        const uint32_t i = first + u * kThinThreads + t;
+        const uint32_t c = i - a.divRowUnits(i) * units;
+        unsigned __int128 bits;
+        __builtin_memcpy(&bits, &v[u], 16);
+        bits >>= c + 1 == units ? down : 0u;
+        __builtin_memcpy(&v[u], &bits, 16);
+      }
     }
 #pragma unroll
     for (int u = 0; u != kBatch; ++u)
@@ -166,7 +198,8 @@ __global__ __launch_bounds__(kThinThreads)
     for (uint32_t i = t; i < a.ldsRows * per; i += kThinThreads) {
       const uint32_t row = a.divBorder(i), c = i - row * per;
       const uint32_t byte =
-          c < left ? c * 4 : a.dataOff + a.rowBytes + (c - left) * 4;
+          c < left ? c * 4
+                   : a.dataOff + ((a.rowBytes + 3) & ~3u) + (c - left) * 4;
       *reinterpret_cast<uint32_t *>(lds + row * a.pitch + byte) = 0;
     }
   }
@@ -230,9 +263,11 @@ __global__ __launch_bounds__(kThinThreads)
     const char *img = reinterpret_cast<const char *>(
         in + size_t(image) * d.inH * d.inW * d.inChans);
     if (vec16)
-      copyRows<uintx4>(a, lds, img, ih0, t);
+      copyRows<uintx4, false>(a, lds, img, ih0, t);
+    else if (a.rowBytes >= 16)
+      copyRows<uintx4, true>(a, lds, img, ih0, t);
     else
-      copyRows<uint32_t>(a, lds, img, ih0, t);
+      copyRows<uint32_t, false>(a, lds, img, ih0, t);
     if (a.cutElems) {
       // truncated columns read as zeros: wiped once the rows are in
       __syncthreads();
@@ -464,8 +499,8 @@ bool thinInputTakes(const ThinInputDesc &d, int inType, int outType) {
     return false;
   if (d.outChans % 16 != 0 || d.outChans > 64)
     return false;
-  // rows are copied in dwords
-  if ((d.inW * d.inChans) % 2 != 0)
+  // rows are copied in 16-byte vectors, those shorter than one in dwords
+  if ((d.inW * d.inChans) % 2 != 0 && d.inW * d.inChans < 8)
     return false;
   if (d.strideH == 0 || d.strideW == 0 || d.strideW > 64 ||
       d.padW > 4096 || d.padW < -4096 || d.padH > (1 << 20) ||
@@ -527,7 +562,7 @@ hipError_t launchThinInput(const ThinInputDesc &d, int inType, int outType,
   a.divTilesPerImage = makeFastDiv(a.tilesPerImage);
   a.divColBlocks = makeFastDiv(a.colBlocks);
   a.divRowUnits =
-      makeFastDiv((s.rowBytes & 15) == 0 ? s.rowBytes / 16 : s.rowBytes / 4);
+      makeFastDiv(s.rowBytes >= 16 ? (s.rowBytes + 15) / 16 : s.rowBytes / 4);
   a.divBorder = makeFastDiv((s.pitch - s.rowBytes) / 4);
   a.biasByte = s.ldsRows * s.pitch;
   a.weightByte = a.biasByte + 256;

@@ -17,6 +17,11 @@ TYPES = {pa.QUARTER: torch.uint8, pa.HALF: torch.int16, pa.FLOAT: torch.int32}
     (2, 3, 2048), (3, 3, 2049), (2, 3, 4097), (2, 2, 5001), (2, 4, 4095),
     (2, 2047, 3), (2, 2049, 3), (1, 6001, 2), (1, 8193, 4),
     (4, 3, 130), (4, 1, 77), (4, 77, 1), (1, 5, 5),
+    # ... and in numbers that fill the chip, with workgroups of one wave
+    # (up to 512 Ki elements to a side's vector of 16 bytes) and of four
+    (43, 3, 2049), (70, 2, 2047), (1, 4, 65537), (19, 4097, 4),
+    (1, 100001, 3), (131, 3, 4097), (300, 2, 4095), (2, 4, 299999),
+    (270, 4097, 3),
 ])
 @pytest.mark.parametrize("t", TYPES)
 def test_transpose(groups, rows, cols, t):

@@ -177,3 +177,36 @@ def test_thin_input_random_params(oracle):
         assert rel_l2(got, want) <= tol, (case, kw, rel_l2(got, want))
         ran += 1
     assert ran >= 150, ran
+
+
+# Rows of an odd number of elements start at any even byte and end inside a
+# 16-byte vector: every length of the last vector, rows of a single one, a
+# row's worth of tiles that goes round, truncated columns.
+ODD_ROWS = [dict(batch=2, field=(9, w), kernel=(3, 3), ci=3, co=16, pad=1)
+            for w in (3, 5, 7, 9, 11, 13, 15, 17, 19)] + [
+    dict(batch=3, field=(12, 9), kernel=(2, 5), ci=1, co=32, pad=1),
+    dict(batch=2, field=(31, 199), kernel=(7, 7), ci=3, co=48, pad=3,
+         stride=2),
+    dict(batch=40, field=(65, 33), kernel=(3, 3), ci=3, co=16, pad=1),
+    dict(batch=2, field=(12, 15), kernel=(3, 3), ci=3, co=64, itl=(1, 2),
+         itu=(2, 1), pad=2),
+    # rows of whole dwords that are no whole vector
+    dict(batch=2, field=(9, 6), kernel=(3, 3), ci=3, co=16, pad=1),
+]
+
+
+@pytest.mark.parametrize("kw", ODD_ROWS)
+def test_thin_input_rows_of_no_whole_vectors(oracle, kw):
+    from gpu_helpers import quantize, run_conv
+    p = make_params(pa.HALF, pa.FLOAT, **kw)
+    print("case", p, flush=True)
+    acts, weights, biases = random_data(p, 45, "normal")
+    aq, ad = quantize(acts, pa.HALF)
+    wq, wd = quantize(weights * 0.2, pa.HALF)
+    got, plan = run_conv(p, aq, wq, biases.astype(np.float32), FORCED,
+                         return_plan=True)
+    assert THIN in plan.describe(), plan.describe()
+    want = oracle.convolution(p, ad, wd, biases.astype(np.float32),
+                              threads=8)
+    # fp32 sums of at most 147 products
+    assert rel_l2(got, want) <= 1e-5, rel_l2(got, want)
