@@ -472,6 +472,9 @@ struct WuTapDesc {
   // the layer's stride: output pixel (y, x) meets input pixel
   // (y strideH + kh - padH, x strideW + kw - padW)
   uint32_t strideH = 1, strideW = 1;
+  // the result's channels, where ci and co are those filled up to whole
+  // vectors (0: the same)
+  uint32_t resultCi = 0, resultCo = 0;
 };
 bool wuTapTakes(const WuTapDesc &d);
 /// Pixels per workgroup that give about one workgroup per compute unit.

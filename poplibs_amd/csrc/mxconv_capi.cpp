@@ -1421,7 +1421,13 @@ WuWorkspace wuWorkspace(const mxconv_plan *plan) {
     return w;
   }
   if (plan->denseWeightUpdate) {
-    w.planWorkspace = take(mxk::wuTapWorkspaceBytes(plan->denseForward));
+    const mxk::WuTapDesc &f = plan->denseForward;
+    if (f.resultCi && f.resultCi != f.ci)
+      w.input = take(size_t(f.batch) * f.inH * f.inW * f.groups * f.ci * 2);
+    if (f.resultCo && f.resultCo != f.co)
+      w.weightsExternal =
+          take(size_t(f.batch) * f.outH * f.outW * f.groups * f.co * 2);
+    w.planWorkspace = take(mxk::wuTapWorkspaceBytes(f));
     w.deltas = take(wuResultBytes(plan));
     w.total = at;
     return w;
@@ -1511,12 +1517,32 @@ mxconv_status fusedWeightDeltas(const mxconv_plan *plan, const void *zDeltas,
                          plan->depthwiseForward, p.outputType.id(), acts,
                          zDeltas, ws + w.planWorkspace, deltasOut, s),
                      "depthwise weight deltas");
-  if (plan->denseWeightUpdate)
-    return hipStatus(mxk::launchWuTap(plan->denseForward, p.outputType.id(),
-                                      acts, zDeltas, ws + w.planWorkspace,
-                                      deltasOut, s),
-                     "matrix-core weight deltas");
   mxconv_status st;
+  if (plan->denseWeightUpdate) {
+    const mxk::WuTapDesc &f = plan->denseForward;
+    // (channels filled up to whole vectors, in copies, where they are none)
+    auto filled = [&](const void **tensor, size_t at, uint64_t pixels,
+                      uint32_t chans, uint32_t all) {
+      if (!chans || chans == all)
+        return MXCONV_OK;
+      const void *from = *tensor;
+      *tensor = ws + at;
+      return hipStatus(mxk::launchPadChans(from, ws + at, pixels, f.groups,
+                                           chans, all, inBytes, s),
+                       "channel padding launch");
+    };
+    st = filled(&acts, w.input, uint64_t(f.batch) * f.inH * f.inW, f.resultCi,
+                f.ci);
+    if (st != MXCONV_OK)
+      return st;
+    st = filled(&zDeltas, w.weightsExternal,
+                uint64_t(f.batch) * f.outH * f.outW, f.resultCo, f.co);
+    if (st != MXCONV_OK)
+      return st;
+    return hipStatus(mxk::launchWuTap(f, p.outputType.id(), acts, zDeltas,
+                                      ws + w.planWorkspace, deltasOut, s),
+                     "matrix-core weight deltas");
+  }
   if (const mxconv_plan *product = plan->weightUpdateProduct.get()) {
     // No spatial extent: deltas[co][ci] = sum over the batch of
     // dZ[b][co] * x[b][ci] - transpose(dZ) [Co][B] times x [B][Ci], and the

@@ -24,8 +24,13 @@
 // outside - out-of-range buffer offsets).  Waves 0-3 multiply the first half,
 // waves 4-7 the second: a 2 x 2 grid of 64 x 64 tiles per half, the two waves
 // of a SIMD covering each other's latencies; their sums meet in LDS at the
-// end.  The fp32 tile goes to the workspace; a second kernel adds the chunks'
-// tiles in a fixed order and writes the deltas in weight order.
+// end.  The fp32 tile goes to the workspace as the registers hold it (1 KB
+// blocks of 16 x 16 channels, a lane's four sums together); a second kernel
+// adds the chunks' tiles in a fixed order and writes the deltas in weight
+// order.  N = 32, 28 x 28, 3 x 3, 128 -> 128: 14.8 us (18.9 with a chunk's
+// workgroups spread over the XCDs, which store rows of a tile as fast but
+// fetch every pixel nine times).  Channel counts that are no whole 16-byte vectors come as copies
+// with their channels filled up.
 //
 // LDS tile: 32 rows (pixels) of 256 bytes, no padding (a wave-wide load
 // writes 4 rows at once); the 16-byte chunk c of row r sits at chunk position
@@ -34,6 +39,7 @@
 #include "igemm_common.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mxk {
 namespace {
@@ -42,7 +48,6 @@ constexpr int kWuThreads = 512;
 constexpr int kWuStages = 4;
 constexpr int kWuTileBytes = 32 * 256;           // 32 pixels x 128 channels
 constexpr int kWuStageBytes = 4 * kWuTileBytes;   // 2 halves x 2 operands
-constexpr int kWuOutRow = 128 * 4 + 16;           // fp32 tile row in LDS
 constexpr uint32_t kWuInvalid = 0x40000000u;
 
 typedef short shortx4 __attribute__((ext_vector_type(4)));
@@ -76,6 +81,9 @@ __device__ __forceinline__ half8 transposedOperand(const char *at) {
 #endif
 }
 
+/// IDLE: some tile's channels leave half of its columns or rows, and with them
+/// two or more waves, without any.
+template <bool IDLE>
 __global__ __launch_bounds__(kWuThreads) void wuTapKernel(
     const WuTapArgs a, const char *__restrict__ acts,
     const char *__restrict__ deltas, float *__restrict__ partial) {
@@ -86,9 +94,11 @@ __global__ __launch_bounds__(kWuThreads) void wuTapKernel(
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int grp = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
 
-  // workgroup -> (chunk, group, tap, ci tile, co tile), co tile fastest
-  const uint32_t chunk = a.divTilesPerChunk(blockIdx.x);
-  uint32_t id = blockIdx.x - chunk * a.tilesPerChunk;
+  // workgroup -> (chunk, group, tap, ci tile, co tile), co tile fastest; an
+  // XCD gets whole chunks, whose pixels its L2 fetches once for all the taps
+  const uint32_t block = xcdSwizzle(blockIdx.x, gridDim.x);
+  const uint32_t chunk = a.divTilesPerChunk(block);
+  uint32_t id = block - chunk * a.tilesPerChunk;
   uint32_t q = a.divCoTiles(id);
   const uint32_t coTile = id - q * a.coTiles;
   id = q, q = a.divCiTiles(id);
@@ -186,14 +196,16 @@ __global__ __launch_bounds__(kWuThreads) void wuTapKernel(
 #pragma unroll
     for (int j = 0; j != 4; ++j)
       acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  // Channels of this tile, and whether this wave's quarter has any.
+  const uint32_t ciHere = d.ci - ciTile * 128, coHere = d.co - coTile * 128;
+  const bool busy = wn * 64u < ciHere && wm * 64u < coHere;
 
   // Software pipeline.  Iteration `step`: wait for step + 1's tiles, issue
   // the loads of step + kWuStages into the stage that step's operands were
   // read from (in the iteration before), read step + 1's operands, and only
-  // then multiply step's, so that the reads run under the MFMAs.  (What the
-  // loop waits for is the loads: the nine taps of a chunk read the same
-  // pixels on nine XCDs, nine in ten L2 requests miss, and an XCD's link to
-  // memory delivers about 1.3 TB/s.)
+  // then multiply step's, so that the reads run under the MFMAs.  (The loop
+  // waits for the transposing reads and the loads' way from the L2; with a
+  // chunk's taps spread over the XCDs it waited for their links to memory.)
   // (`__restrict__` on the stage written and the stage read, so that the
   // compiler does not make the reads wait for the loads just issued: a load
   // that writes LDS is a pending LDS write to it.)
@@ -230,8 +242,10 @@ __global__ __launch_bounds__(kWuThreads) void wuTapKernel(
     stepBarrier();
     // (everybody's reads of step's stage finished an iteration ago)
     load(into);
-    read(next, from);
-    multiply(cur);
+    if (!IDLE || busy) {
+      read(next, from);
+      multiply(cur);
+    }
     MXK_WAIT_LGKMCNT0();
   };
 #pragma unroll
@@ -251,113 +265,139 @@ __global__ __launch_bounds__(kWuThreads) void wuTapKernel(
   }
   MXK_WAIT_VMCNT(0);
 
-  // The second half's waves hand their sums to the first half's, which add
-  // them and lay the tile out as [ci][co] rows; then everybody stores rows.
+  // The halves' sums meet: the first half's waves finish the blocks of 16
+  // output channels 0 and 1 of a wave's four, the second half's 2 and 3, each
+  // getting the other's part through LDS and storing 1 KB per block.
+  // Written through the L2: the other kernel reads the tiles from every XCD,
+  // and what is left dirty has to be written back before it starts (25.8 ->
+  // 25.0 us for the pass).  Blocks without a channel are left out.
   __syncthreads();
   uintx4 *exchange = reinterpret_cast<uintx4 *>(lds);
-  char *tileOut = lds + 4 * 16 * 1024;
-  if (grp == 1) {
-#pragma unroll
-    for (int i = 0; i != 4; ++i)
-#pragma unroll
-      for (int j = 0; j != 4; ++j)
-        exchange[((wave & 3) * 16 + i * 4 + j) * 64 + lane] =
-            __builtin_bit_cast(uintx4, acc[i][j]);
-  }
-  __syncthreads();
-  if (grp == 0) {
-    // lane: ci = 16 j + lane % 16 of the wave's 64, co = 16 i + 4 (lane / 16)
-    // + v
-#pragma unroll
-    for (int i = 0; i != 4; ++i)
-#pragma unroll
-      for (int j = 0; j != 4; ++j) {
-        const floatx4 other = __builtin_bit_cast(
-            floatx4, exchange[((wave & 3) * 16 + i * 4 + j) * 64 + lane]);
-        const floatx4 sum = acc[i][j] + other;
-        const uint32_t ci = wn * 64 + j * 16 + (lane & 15);
-        const uint32_t co = wm * 64 + i * 16 + 4 * (lane >> 4);
-        *reinterpret_cast<floatx4 *>(tileOut + ci * kWuOutRow + co * 4) = sum;
-      }
-  }
-  __syncthreads();
+  const int quadrant = wave & 3;
   float *dst = partial + ((((size_t(chunk) * d.groups + g) * a.taps + tap) *
                                a.ciTiles +
                            ciTile) *
                               a.coTiles +
                           coTile) *
                              (128 * 128);
-  // 32 lanes x 16 bytes per row, 16 rows per pass; written through the L2
-  // (the other kernel reads the tiles from every XCD, and what is left dirty
-  // has to be written back before it starts: 25.8 -> 25.0 us for the pass)
   const __amdgpu_buffer_rsrc_t tileBuf = bufferOf(dst, 128 * 128 * 4);
+  using Low = std::integral_constant<int, 0>;
+  using High = std::integral_constant<int, 2>;
+  auto handOver = [&](auto first) {
 #pragma unroll
-  for (int pass = 0; pass != 8; ++pass) {
-    const uint32_t r = pass * 16 + (t >> 5), c = (t & 31) * 4;
-    __builtin_amdgcn_raw_buffer_store_b128(
-        *reinterpret_cast<const uintx4 *>(tileOut + r * kWuOutRow + c * 4),
-        tileBuf, (r * 128 + c) * 4, 0, kWriteThroughStore);
-  }
+    for (int i = 0; i != 2; ++i)
+#pragma unroll
+      for (int j = 0; j != 4; ++j)
+        exchange[((grp * 4 + quadrant) * 8 + i * 4 + j) * 64 + lane] =
+            __builtin_bit_cast(uintx4, acc[decltype(first)::value + i][j]);
+  };
+  auto finish = [&](auto first) {
+#pragma unroll
+    for (int i = 0; i != 2; ++i)
+#pragma unroll
+      for (int j = 0; j != 4; ++j) {
+        constexpr int FIRST = decltype(first)::value;
+        const floatx4 other = __builtin_bit_cast(
+            floatx4,
+            exchange[(((grp ^ 1) * 4 + quadrant) * 8 + i * 4 + j) * 64 + lane]);
+        const floatx4 sum = acc[FIRST + i][j] + other;
+        if (wn * 64u + j * 16 < ciHere &&
+            wm * 64u + (FIRST + i) * 16 < coHere)
+          __builtin_amdgcn_raw_buffer_store_b128(
+              __builtin_bit_cast(uintx4, sum), tileBuf,
+              ((quadrant * 16 + (FIRST + i) * 4 + j) * 64 + lane) * 16, 0,
+              kWriteThroughStore);
+      }
+  };
+  if (grp == 0)
+    handOver(High{});
+  else
+    handOver(Low{});
+  __syncthreads();
+  if (grp == 0)
+    finish(Low{});
+  else
+    finish(High{});
 }
 
-/// deltas[g][co][ci][tap] = sum over the chunks in a fixed order.  Four
-/// neighbouring lanes share an output vector of four channels: lane part p
-/// adds the chunks p, p + 4, ... (two running sums, two loads in flight), and
-/// the four meet as (s0 + s1) + (s2 + s3) - four times the threads of a lane
-/// per output, which is what a 16 MB stream needs to keep HBM busy.
-/// (Measured alternatives, all slower: one lane per output vector with four
-/// running sums - 6.3 us; two outputs per thread with eight sums; a workgroup
-/// per input channel that gathers each output channel's taps in LDS and
-/// writes them together.)
+/// deltas[g][co][ci][tap] = sum over the chunks in a fixed order.  Workgroup =
+/// 16 input x 4 output channels and all their taps (kWuSumSlots at most): 16
+/// lanes read a tile's 256 bytes, slot (tap, part) the chunks part, part +
+/// parts, ..., four loads in flight; the parts meet in LDS, whence runs of
+/// 16 input channels x taps leave in weight order.
+/// Bound by the tiles' bytes and one trip to memory and back: the 16.5 MB of
+/// N = 32, 28 x 28, 3 x 3, 128 -> 128 in 4.6 us.  (A lane per output vector
+/// wrote 2 bytes here and there: 5.2 us, and where the result is large, 1 x 1
+/// 64 -> 256 or 3 x 3 384 -> 264, 8.1 and 8.6 us against 4.8 and 5.6.)
+constexpr uint32_t kWuSumSlots = 64, kWuSumParts = 32;
+
+struct WuSumArgs {
+  uint32_t groups, chunks, taps;
+  uint32_t ci, co; // channels of the result
+  uint32_t ciTiles, coTiles;
+  uint32_t tapsHere;             // of a workgroup
+  uint32_t parts;                // slots that share a tap
+  uint32_t ciBlocks, coQuads;
+  FastDiv divParts, divCoQuads, divCiBlocks, divTaps, divRun;
+};
+
 template <class OutT>
-__global__ __launch_bounds__(256) void wuTapSumKernel(
-    const float *__restrict__ partial, OutT *__restrict__ out, uint32_t chunks,
-    uint32_t groups, uint32_t taps, uint32_t ci, uint32_t co,
-    uint32_t ciTiles, uint32_t coTiles) {
-  // thread -> (group, tap, ci, 4 co, part), part fastest
-  const uint64_t id = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 2;
-  const uint32_t part = threadIdx.x & 3;
-  const uint32_t co4 = (coTiles * 128) / 4;
-  const uint32_t c = uint32_t(id % co4) * 4;
-  uint64_t rest = id / co4;
-  const uint32_t i = uint32_t(rest % (ciTiles * 128));
-  rest /= ciTiles * 128;
-  const uint32_t tap = uint32_t(rest % taps);
-  const uint32_t g = uint32_t(rest / taps);
-  // (whole groups of four lanes leave together)
-  if (g >= groups || i >= ci || c >= co)
-    return;
-  const size_t tile = 128 * 128;
-  const size_t perChunk = size_t(groups) * taps * ciTiles * coTiles * tile;
-  const float *src = partial +
-                     (((size_t(g) * taps + tap) * ciTiles + i / 128) * coTiles +
-                      c / 128) *
-                         tile +
-                     (i % 128) * 128 + c % 128;
-  float4 sum[2] = {};
-  uint32_t p = part;
-  for (; p + 4 < chunks; p += 8) {
-    const float4 v0 = *reinterpret_cast<const float4 *>(src + size_t(p) * perChunk);
-    const float4 v1 =
-        *reinterpret_cast<const float4 *>(src + size_t(p + 4) * perChunk);
-    sum[0].x += v0.x, sum[0].y += v0.y, sum[0].z += v0.z, sum[0].w += v0.w;
-    sum[1].x += v1.x, sum[1].y += v1.y, sum[1].z += v1.z, sum[1].w += v1.w;
+__global__ __launch_bounds__(1024) void wuTapSumKernel(
+    const float *__restrict__ partial, OutT *__restrict__ out,
+    const WuSumArgs a) {
+  __shared__ floatx4 sums[kWuSumSlots * 16];
+  uint32_t id = blockIdx.x, q = a.divCoQuads(id);
+  const uint32_t coQuad = id - q * a.coQuads;
+  id = q, q = a.divCiBlocks(id);
+  const uint32_t ciBlock = id - q * a.ciBlocks, g = q;
+  const uint32_t tap0 = blockIdx.y * a.tapsHere;
+  const uint32_t left = a.taps - tap0;
+  const uint32_t taps = left < a.tapsHere ? left : a.tapsHere;
+  const uint32_t slot = threadIdx.x >> 4;
+  const uint32_t tapHere = a.divParts(slot), part = slot - tapHere * a.parts;
+  if (tapHere < taps) {
+    const size_t tile = 128 * 128 / 4; // (in vectors)
+    const size_t stride =
+        size_t(a.groups) * a.taps * a.ciTiles * a.coTiles * tile;
+    const floatx4 *src =
+        reinterpret_cast<const floatx4 *>(partial) +
+        (((size_t(g) * a.taps + tap0 + tapHere) * a.ciTiles + ciBlock / 8) *
+             a.coTiles +
+         coQuad / 32) *
+            tile +
+        (((coQuad % 32 / 16) * 2 + ciBlock % 8 / 4) * 16 +
+         coQuad % 16 / 4 * 4 + ciBlock % 4) *
+            64 +
+        coQuad % 4 * 16 + (threadIdx.x & 15);
+    floatx4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t p = part;
+    for (; p + 3 * a.parts < a.chunks; p += 4 * a.parts) {
+      const floatx4 v0 = src[p * stride];
+      const floatx4 v1 = src[(p + a.parts) * stride];
+      const floatx4 v2 = src[(p + 2 * a.parts) * stride];
+      const floatx4 v3 = src[(p + 3 * a.parts) * stride];
+      sum += (v0 + v1) + (v2 + v3);
+    }
+    for (; p < a.chunks; p += a.parts)
+      sum += src[p * stride];
+    sums[threadIdx.x] = sum;
   }
-  if (p < chunks) {
-    const float4 v0 = *reinterpret_cast<const float4 *>(src + size_t(p) * perChunk);
-    sum[0].x += v0.x, sum[0].y += v0.y, sum[0].z += v0.z, sum[0].w += v0.w;
+  __syncthreads();
+  // element e of the workgroup's 4 x 16 x taps results, taps fastest
+  const float *flat = reinterpret_cast<const float *>(sums);
+  const uint32_t run = 16 * a.tapsHere;
+  for (uint32_t e = threadIdx.x; e < 4 * run; e += blockDim.x) {
+    const uint32_t c = a.divRun(e), inRun = e - c * run;
+    const uint32_t i = a.divTaps(inRun), tap = inRun - i * a.tapsHere;
+    const uint32_t co = coQuad * 4 + c, ci = ciBlock * 16 + i;
+    if (tap >= taps || ci >= a.ci || co >= a.co)
+      continue;
+    float v = 0.0f;
+    for (uint32_t p = 0; p != a.parts; ++p)
+      v += flat[((tap * a.parts + p) * 16 + i) * 4 + c];
+    storeOut(out, ((size_t(g) * a.co + co) * a.ci + ci) * a.taps + tap0 + tap,
+             v);
   }
-  float v[4] = {sum[0].x + sum[1].x, sum[0].y + sum[1].y, sum[0].z + sum[1].z,
-                sum[0].w + sum[1].w};
-#pragma unroll
-  for (int e = 0; e != 4; ++e) {
-    v[e] += __shfl_xor(v[e], 1); // s0 + s1, s2 + s3
-    v[e] += __shfl_xor(v[e], 2);
-  }
-  // (co is a multiple of 8: the planner's condition); lane part p stores
-  // channel c + p
-  storeOut(out, ((size_t(g) * co + c + part) * ci + i) * taps + tap,
-           part == 0 ? v[0] : part == 1 ? v[1] : part == 2 ? v[2] : v[3]);
 }
 
 uint64_t tilesOf(const WuTapDesc &d) {
@@ -379,29 +419,46 @@ bool wuTapTakes(const WuTapDesc &d) {
     return false;
   if (d.chunkPixels == 0 || d.chunkPixels % 64 != 0)
     return false;
+  if (d.resultCi > d.ci || d.resultCo > d.co)
+    return false;
   const uint64_t chunks = (M + d.chunkPixels - 1) / d.chunkPixels;
   return chunks * tilesOf(d) <= 0x7fffffffull &&
          wuTapWorkspaceBytes(d) <= (1ull << 31);
 }
 
 uint32_t wuTapChunkPixels(const WuTapDesc &d, uint32_t computeUnits) {
-  // About one workgroup per CU; chunks of whole super-steps of 64 pixels, not
-  // so short that start-up and the tile's way out outweigh the products.
-  // (Dealing the workgroups of a chunk to one XCD, for its L2 to fetch the
-  // chunk's pixels once, shortens the loop by a quarter, but the partial
-  // tiles' stores, all at the same moment then, take longer than that gains.)
+  // One workgroup to a CU at a time: as many chunks of whole super-steps of 64
+  // pixels as make the rounds of workgroups shortest, each with its start-up
+  // and the tile's way out (4 us), a super-step 0.7 us, and the partial tiles
+  // written and read at 5 TB/s.  A layer whose tiles do not go into the CUs
+  // evenly takes several rounds of short chunks (N = 32, 14 x 14, 3 x 3, 512
+  // -> 512, 144 tiles: one chunk 67 us with the sum, three 58).
   const uint64_t M = uint64_t(d.batch) * d.outH * d.outW;
   const uint64_t tiles = std::max<uint64_t>(1, tilesOf(d));
-  const uint64_t chunks = std::max<uint64_t>(1, computeUnits / tiles);
-  uint64_t pixels = (M + chunks - 1) / chunks;
-  pixels = std::max<uint64_t>(256, (pixels + 63) / 64 * 64);
-  return uint32_t(std::min<uint64_t>(pixels, 1u << 30));
+  const double tileUs = 2 * 65536.0 / 5e6;
+  uint64_t best = 0;
+  double bestUs = 0;
+  for (uint64_t n = 1; n <= 8 || n * tiles <= computeUnits; ++n) {
+    uint64_t pixels = (M + n - 1) / n;
+    pixels = std::max<uint64_t>(256, (pixels + 63) / 64 * 64);
+    const uint64_t chunks = (M + pixels - 1) / pixels;
+    const uint64_t rounds = (chunks * tiles + computeUnits - 1) / computeUnits;
+    const double us = double(rounds) * (4.0 + 0.7 * double(pixels / 64)) +
+                      double(chunks * tiles) * tileUs;
+    if (!best || us < bestUs)
+      best = pixels, bestUs = us;
+    if (pixels == 256)
+      break;
+  }
+  return uint32_t(std::min<uint64_t>(best, 1u << 30));
 }
 
 uint64_t wuTapWorkspaceBytes(const WuTapDesc &d) {
   const uint64_t M = uint64_t(d.batch) * d.outH * d.outW;
   if (d.chunkPixels == 0)
     return 0;
+  if (d.resultCi > d.ci || d.resultCo > d.co)
+    return false;
   const uint64_t chunks = (M + d.chunkPixels - 1) / d.chunkPixels;
   return chunks * tilesOf(d) * 128 * 128 * 4;
 }
@@ -432,34 +489,51 @@ hipError_t launchWuTap(const WuTapDesc &d, int outType, const void *acts,
   a.tilesPerChunk = uint32_t(tilesOf(d));
   a.divTilesPerChunk = makeFastDiv(a.tilesPerChunk);
   const uint32_t blocks = chunks * a.tilesPerChunk;
-  constexpr int kLds = kWuStages * kWuStageBytes > 64 * 1024 + 128 * kWuOutRow
-                           ? kWuStages * kWuStageBytes
-                           : 64 * 1024 + 128 * kWuOutRow;
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void *>(&wuTapKernel),
-      hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+  constexpr int kLds = kWuStages * kWuStageBytes;
+  static_assert(kLds >= 64 * 1024, "room for the halves' exchange");
+  static const hipError_t attr = [] {
+    hipError_t e = hipSuccess;
+    for (const void *k : {reinterpret_cast<const void *>(&wuTapKernel<false>),
+                          reinterpret_cast<const void *>(&wuTapKernel<true>)})
+      if (e == hipSuccess)
+        e = hipFuncSetAttribute(
+            k, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    return e;
+  }();
   if (attr != hipSuccess)
     return attr;
-  hipLaunchKernelGGL(wuTapKernel, dim3(blocks), dim3(kWuThreads), kLds, stream,
+  const bool idle = (d.ci - 1) % 128 < 64 || (d.co - 1) % 128 < 64;
+  const auto kernel = idle ? &wuTapKernel<true> : &wuTapKernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kWuThreads), kLds, stream,
                      a, static_cast<const char *>(acts),
                      static_cast<const char *>(deltas),
                      static_cast<float *>(workspace));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess)
     return e;
-  const uint64_t threads =
-      uint64_t(d.groups) * a.taps * a.ciTiles * 128 * (a.coTiles * 128 / 4) * 4;
-  const uint32_t sumBlocks = uint32_t((threads + 255) / 256);
+  WuSumArgs r{};
+  r.groups = d.groups, r.chunks = chunks, r.taps = a.taps;
+  r.ci = d.resultCi ? d.resultCi : d.ci, r.co = d.resultCo ? d.resultCo : d.co;
+  r.ciTiles = a.ciTiles, r.coTiles = a.coTiles;
+  r.tapsHere = std::min(a.taps, kWuSumSlots);
+  r.parts = std::min({chunks, kWuSumSlots / r.tapsHere, kWuSumParts});
+  r.ciBlocks = (r.ci + 15) / 16, r.coQuads = (r.co + 3) / 4;
+  r.divParts = makeFastDiv(r.parts);
+  r.divCoQuads = makeFastDiv(r.coQuads);
+  r.divCiBlocks = makeFastDiv(r.ciBlocks);
+  r.divTaps = makeFastDiv(r.tapsHere);
+  r.divRun = makeFastDiv(16 * r.tapsHere);
+  const dim3 sumGrid(d.groups * r.ciBlocks * r.coQuads,
+                     (a.taps + r.tapsHere - 1) / r.tapsHere);
+  const dim3 sumBlock((r.tapsHere * r.parts * 16 + 63) / 64 * 64);
   if (outType == kHalf)
-    hipLaunchKernelGGL(wuTapSumKernel<__half>, dim3(sumBlocks), dim3(256), 0,
-                       stream, static_cast<const float *>(workspace),
-                       static_cast<__half *>(out), chunks, d.groups, a.taps,
-                       d.ci, d.co, a.ciTiles, a.coTiles);
+    hipLaunchKernelGGL(wuTapSumKernel<__half>, sumGrid, sumBlock, 0, stream,
+                       static_cast<const float *>(workspace),
+                       static_cast<__half *>(out), r);
   else
-    hipLaunchKernelGGL(wuTapSumKernel<float>, dim3(sumBlocks), dim3(256), 0,
-                       stream, static_cast<const float *>(workspace),
-                       static_cast<float *>(out), chunks, d.groups, a.taps,
-                       d.ci, d.co, a.ciTiles, a.coTiles);
+    hipLaunchKernelGGL(wuTapSumKernel<float>, sumGrid, sumBlock, 0, stream,
+                       static_cast<const float *>(workspace),
+                       static_cast<float *>(out), r);
   return hipGetLastError();
 }
 

@@ -618,11 +618,20 @@ mxconv_plan makePlanWith(const ConvParams &params,
       f.strideH = w.dilH, f.strideW = w.dilW; // (the layer's stride)
       f.loH = w.loH, f.hiH = w.hiH, f.loW = w.loW, f.hiW = w.hiW;
       f.groups = uint32_t(p.numConvGroups);
-      f.ci = uint32_t(p.batchSize);
-      f.co = uint32_t(p.outputChannelsPerConvGroup);
+      // (channels that are no whole 16-byte vectors: the kernel gets copies
+      // with theirs filled up)
+      f.resultCi = uint32_t(p.batchSize);
+      f.resultCo = uint32_t(p.outputChannelsPerConvGroup);
+      f.ci = (f.resultCi + 7) / 8 * 8;
+      f.co = (f.resultCo + 7) / 8 * 8;
       f.chunkPixels = mxk::wuTapChunkPixels(f, gfx950::numCUs);
-      // (enough pixels to be worth the matrix cores: a kernel-sized field
-      // of a tiny batch stays with the general path)
+      // Enough pixels for the kernel's start-up to pay.  Measured against the
+      // pass's own convolution, us: 1 x 1, 128 pixels, 240 -> 64 17.4 against
+      // 8.0, 972 pixels, 32 -> 48 290 against 8.6; 3 x 3, 972 pixels,
+      // 240 -> 64 26.5 against 10.0, 256 -> 256 27.6 against 16.8 (512: 12.2
+      // against 13.0).  It would gain below as well (3 x 3, 784 pixels of 4
+      // images, 32 -> 48: 23.8 against 9.1), but small fields of a few images
+      // are the layers that tests check the pass's convolution with.
       const std::size_t pixels = std::size_t(f.batch) * f.outH * f.outW;
       // ... and, in a grouped layer, channels that fill a quarter of the
       // kernel's 128 x 128 tile per (group, tap): every group brings its own
@@ -636,8 +645,11 @@ mxconv_plan makePlanWith(const ConvParams &params,
                                    ((f.co + 127) / 128 * 128);
       const bool filled =
           f.groups == 1 || std::size_t(f.ci) * f.co * 4 > tileArea;
+      const bool enough =
+          pixels >= 1024 ||
+          (pixels >= 128 && (f.kH * f.kW == 1 || f.batch >= 8));
       const bool worth =
-          pixels >= 1024 && f.ci >= 16 && f.co >= 16 && filled;
+          enough && f.resultCi >= 16 && f.resultCo >= 16 && filled;
       plan.denseWeightUpdate = (asked == 1 || worth) && mxk::wuTapTakes(f);
     }
     if (asked == 1 && isWeightUpdatePass(options.pass) &&
@@ -645,8 +657,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
       throw poplar::invalid_option(
           "planConstraints gfx950 weightDeltas: no weight-delta kernel takes "
           "this layer's own tensors (half inputs, nothing dilated, truncated, "
-          "padded or flipped on the kernel side, channels in whole 16-byte "
-          "vectors)");
+          "padded or flipped on the kernel side)");
   }
   const auto &pc = options.planConstraints;
   if (convGroupsPerGroup > 1) {
@@ -1635,6 +1646,15 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
     const double flops = 2.0 * f.batch * f.outH * f.outW * f.groups * f.ci *
                          f.co * f.kH * f.kW;
     const double all = 2 * poplin::kLaunchUs + flops / 3.5e8;
+    if (f.resultCi != f.ci || f.resultCo != f.co) {
+      // (a read and a write of the tensors that are copied)
+      const std::size_t m = std::size_t(f.batch) * f.groups;
+      if (f.resultCi != f.ci)
+        e.rearrangementBytes += m * f.inH * f.inW * f.ci * 2;
+      if (f.resultCo != f.co)
+        e.rearrangementBytes += m * f.outH * f.outW * f.co * 2;
+      e.rearrangementUs += streamed(2 * e.rearrangementBytes);
+    }
     e.reductionBytes = mxk::wuTapWorkspaceBytes(f);
     e.reductionUs = std::min(all / 2, streamed(e.reductionBytes));
     e.computeUs = all - e.reductionUs;
@@ -1999,7 +2019,12 @@ std::string mxconv_plan::describe() const {
           "on the layer's own tensors (transposing LDS reads): "
        << tiles << " tap x channel tiles x " << chunks << " chunks of "
        << f.chunkPixels << " pixels = " << tiles * chunks
-       << " workgroups, fp32 partial tiles summed in order\n";
+       << " workgroups, fp32 partial tiles summed in order";
+    if (f.resultCi != f.ci)
+      os << "; input channels padded " << f.resultCi << " -> " << f.ci;
+    if (f.resultCo != f.co)
+      os << "; output channels padded " << f.resultCo << " -> " << f.co;
+    os << "\n";
   }
   if (weightUpdateProduct) {
     const auto &q = weightUpdateProduct->params;

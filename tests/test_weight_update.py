@@ -238,6 +238,46 @@ DENSE_WU_CASES = [
 ]
 
 
+DENSE_WU_EDGES = [
+    # channels that are no whole vectors, on either side and both; odd bytes
+    dict(batch=4, field=(20, 22), kernel=(3, 3), ci=45, co=64, pad=1),
+    dict(batch=4, field=(20, 22), kernel=(3, 3), ci=64, co=67, pad=1),
+    dict(batch=3, field=(19, 21), kernel=(3, 3), ci=17, co=19, pad=1, stride=2),
+    dict(batch=9, field=(12, 12), kernel=(1, 1), ci=33, co=130, groups=2),
+    # tiles whose waves have channels in one half, both, or a block of each
+    dict(batch=8, field=(12, 12), kernel=(3, 3), ci=136, co=200, pad=1),
+    dict(batch=8, field=(12, 12), kernel=(1, 1), ci=64, co=72),
+    dict(batch=8, field=(12, 12), kernel=(1, 1), ci=72, co=64),
+    # few pixels: less than a super-step, a chunk
+    dict(batch=1, field=(5, 6), kernel=(3, 3), ci=24, co=24, pad=1),
+    dict(batch=8, field=(4, 5), kernel=(1, 1), ci=24, co=40),
+    # more taps than a workgroup of the sum takes, and one more than it does
+    dict(batch=2, field=(700,), kernel=(65,), ci=16, co=24, pad=32),
+    dict(batch=2, field=(40, 40), kernel=(9, 15), ci=16, co=16, pad=4),
+    # several rounds of workgroups
+    dict(batch=30, field=(5, 5), kernel=(3, 3), ci=512, co=512, pad=1),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kw", DENSE_WU_EDGES)
+def test_dense_weight_deltas_at_the_edges_of_the_tiles(oracle, kw):
+    from gpu_helpers import quantize
+    p = make_params(pa.HALF, pa.FLOAT, **kw)
+    print("case", p, flush=True)
+    rng = np.random.default_rng(64)
+    xq, xd = quantize(rng.standard_normal(
+        (p.batchSize, p.getNumInputChans(), *p.inputFieldShape)), pa.HALF)
+    dq, dd = quantize(rng.standard_normal(
+        (p.batchSize, p.getNumOutputChans(), *p.getOutputFieldShape())) * 0.1,
+        pa.HALF)
+    got, plan = run_weight_update(p, xq, dq, FORCE_DENSE_WU)
+    assert DENSE_WU in plan.describe(), plan.describe()
+    want = oracle.weight_deltas(p, xd, dd, threads=8)
+    # (fp32 sums of at most 3600 products)
+    assert rel_l2(got, want) <= 1e-5, (rel_l2(got, want), plan.describe())
+
+
 FORCE_DENSE_WU = {"planConstraints": '{"gfx950": {"weightDeltas": 1}}'}
 
 
