@@ -7,6 +7,7 @@ canonicalisation, size and range algebra all run in the C++ library.
 """
 import ctypes
 import os
+import struct
 import subprocess
 from ctypes import (POINTER, Structure, byref, c_char_p, c_int, c_int32,
                     c_size_t, c_uint8, c_uint32, c_uint64, c_void_p)
@@ -71,6 +72,15 @@ class CParams(Structure):
                 ("input_transform", _CInputTransform),
                 ("kernel_transform", _CInputTransform),
                 ("output_transform", _COutputTransform)]
+
+
+# CParams as one record: native types and alignment, closed by that of a
+# 64-bit field.
+_PARAMS_RECORD = struct.Struct(
+    "@iiIIQ{m}Q{m}QQQQ{i}{i}{o}0Q".format(
+        m=MAX_FIELD_DIMS, i=f"{5 * MAX_FIELD_DIMS}I{MAX_FIELD_DIMS}B",
+        o=f"{5 * MAX_FIELD_DIMS}I"))
+assert _PARAMS_RECORD.size == ctypes.sizeof(CParams)
 
 
 class _CPhaseCost(Structure):
@@ -317,6 +327,49 @@ class ConvParams:
         if n > MAX_FIELD_DIMS:
             raise MxconvError(Status.INVALID_PARAMS,
                               "too many field dimensions")
+        if len(self.kernelShape) != n:
+            raise MxconvError(
+                Status.INVALID_PARAMS,
+                "Number of kernel field dimensions does not match the number "
+                "of input field dimensions")
+        # One record packed at once (a training step makes this call: field
+        # by field it was a tenth of a small layer's step).
+        rest = [0] * (MAX_FIELD_DIMS - n)
+        values = [self.inputType, self.outputType, n, 0, self.batchSize,
+                  *self.inputFieldShape, *rest, *self.kernelShape, *rest,
+                  self.inputChannelsPerConvGroup,
+                  self.outputChannelsPerConvGroup, self.numConvGroups]
+        t, k, o = self.inputTransform, self.kernelTransform, \
+            self.outputTransform
+        for src, what in (
+                (t.truncationLower, "input truncation"),
+                (t.truncationUpper, "input truncation"),
+                (t.dilation, "input dilation"),
+                (t.paddingLower, "input padding"),
+                (t.paddingUpper, "input padding"), (t.flip, "input flip"),
+                (k.truncationLower, "kernel truncation"),
+                (k.truncationUpper, "kernel truncation"),
+                (k.dilation, "kernel dilation"),
+                (k.paddingLower, "kernel padding"),
+                (k.paddingUpper, "kernel padding"), (k.flip, "kernel flip"),
+                (o.truncationLower, "output truncation"),
+                (o.truncationUpper, "output truncation"),
+                (o.stride, "stride"), (o.paddingLower, "output padding"),
+                (o.paddingUpper, "output padding")):
+            if len(src) != n:
+                raise MxconvError(
+                    Status.INVALID_PARAMS,
+                    f"Number of {what} dimensions ({len(src)}) does not match "
+                    f"the number of field dimensions ({n})")
+            values += src
+            values += rest
+        try:
+            return CParams.from_buffer_copy(_PARAMS_RECORD.pack(*values))
+        except struct.error:
+            # (values a field takes modulo its size, or that int() takes)
+            return self._to_c_by_field(n)
+
+    def _to_c_by_field(self, n):
         c = CParams()
         c.input_type, c.output_type = self.inputType, self.outputType
         c.num_field_dims = n
@@ -324,39 +377,28 @@ class ConvParams:
         c.input_channels_per_conv_group = self.inputChannelsPerConvGroup
         c.output_channels_per_conv_group = self.outputChannelsPerConvGroup
         c.num_conv_groups = self.numConvGroups
-        if len(self.kernelShape) != n:
-            raise MxconvError(
-                Status.INVALID_PARAMS,
-                "Number of kernel field dimensions does not match the number "
-                "of input field dimensions")
         for d in range(n):
             c.input_field_shape[d] = self.inputFieldShape[d]
             c.kernel_shape[d] = self.kernelShape[d]
 
-        def put(dst, src, what):
-            if len(src) != n:
-                raise MxconvError(
-                    Status.INVALID_PARAMS,
-                    f"Number of {what} dimensions ({len(src)}) does not match "
-                    f"the number of field dimensions ({n})")
+        def put(dst, src):
             for d in range(n):
                 dst[d] = int(src[d])
 
-        for ct, t, name in ((c.input_transform, self.inputTransform, "input"),
-                            (c.kernel_transform, self.kernelTransform,
-                             "kernel")):
-            put(ct.truncation_lower, t.truncationLower, name + " truncation")
-            put(ct.truncation_upper, t.truncationUpper, name + " truncation")
-            put(ct.dilation, t.dilation, name + " dilation")
-            put(ct.padding_lower, t.paddingLower, name + " padding")
-            put(ct.padding_upper, t.paddingUpper, name + " padding")
-            put(ct.flip, t.flip, name + " flip")
+        for ct, t in ((c.input_transform, self.inputTransform),
+                      (c.kernel_transform, self.kernelTransform)):
+            put(ct.truncation_lower, t.truncationLower)
+            put(ct.truncation_upper, t.truncationUpper)
+            put(ct.dilation, t.dilation)
+            put(ct.padding_lower, t.paddingLower)
+            put(ct.padding_upper, t.paddingUpper)
+            put(ct.flip, t.flip)
         ot, o = c.output_transform, self.outputTransform
-        put(ot.truncation_lower, o.truncationLower, "output truncation")
-        put(ot.truncation_upper, o.truncationUpper, "output truncation")
-        put(ot.stride, o.stride, "stride")
-        put(ot.padding_lower, o.paddingLower, "output padding")
-        put(ot.padding_upper, o.paddingUpper, "output padding")
+        put(ot.truncation_lower, o.truncationLower)
+        put(ot.truncation_upper, o.truncationUpper)
+        put(ot.stride, o.stride)
+        put(ot.padding_lower, o.paddingLower)
+        put(ot.padding_upper, o.paddingUpper)
         return c
 
     @staticmethod

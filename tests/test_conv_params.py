@@ -808,3 +808,27 @@ def test_depthwise_7x7_tiles_fill_the_workgroup():
         pa.Plan(make_params(pa.HALF, batch=4, field=(64, 64), kernel=(7, 7),
                             groups=128, pad=3),
                 {"planConstraints": '{"gfx950": {"tileH": 32, "tileW": 16}}'})
+
+
+@pytest.mark.parametrize("edit", [
+    lambda p: None,
+    lambda p: setattr(p.inputTransform, "paddingLower", [-1, 2, 3]),  # wraps
+    lambda p: setattr(p.outputTransform, "stride", [2.0, 1.0, 3.0]),
+    lambda p: setattr(p.inputTransform, "flip", [True, 0, True]),
+    lambda p: setattr(p, "batchSize", np.int64(1 << 33)),
+])
+def test_params_record_is_what_the_fields_hold(edit):
+    p = pa.ConvParams(pa.HALF, pa.FLOAT, 2, [9, 8, 7], [3, 2, 1], 4, 5, 6)
+    p.inputTransform.paddingUpper = [7, 8, 9]
+    p.kernelTransform.dilation = [10, 11, 12]
+    p.outputTransform.truncationLower = [13, 14, 15]
+    p.outputTransform.paddingUpper = [16, 17, 18]
+    edit(p)
+    assert bytes(p.to_c()) == bytes(p._to_c_by_field(3))
+
+
+def test_params_of_unequal_dimensions_are_refused():
+    p = pa.ConvParams(pa.HALF, pa.FLOAT, 2, [9, 8], [3, 2], 4, 5, 6)
+    p.kernelTransform.paddingLower = [0]
+    with pytest.raises(MxconvError, match="kernel padding dimensions"):
+        p.to_c()
