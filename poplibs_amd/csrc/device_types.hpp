@@ -94,6 +94,26 @@ inline FastDiv makeFastDiv(uint32_t d) {
   return {uint32_t(m), s - 1, 0};
 }
 
+/// 16 bytes of neighbouring elements at any address: global memory takes such
+/// accesses, at full speed where the address happens to be a multiple of 16.
+typedef uint32_t AnyWords
+    __attribute__((ext_vector_type(4), aligned(1), may_alias));
+template <class T> union Piece {
+  T e[16 / sizeof(T)];
+  uint32_t w[4];
+};
+template <class T>
+__device__ __forceinline__ Piece<T> loadPiece(const T *at) {
+  const AnyWords v = *reinterpret_cast<const AnyWords *>(at);
+  Piece<T> p;
+  p.w[0] = v.x, p.w[1] = v.y, p.w[2] = v.z, p.w[3] = v.w;
+  return p;
+}
+template <class T>
+__device__ __forceinline__ void storePiece(T *at, const Piece<T> &p) {
+  *reinterpret_cast<AnyWords *>(at) = AnyWords{p.w[0], p.w[1], p.w[2], p.w[3]};
+}
+
 /// Four consecutive outputs as one vector store; p is aligned to the vector.
 __device__ __forceinline__ void storeOut4(float *p, const float (&v)[4]) {
   *reinterpret_cast<float4 *>(p) = float4{v[0], v[1], v[2], v[3]};

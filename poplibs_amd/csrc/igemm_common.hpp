@@ -475,10 +475,8 @@ igemmEpilogue(char *lds, const IgemmArgs &a, floatx16 (&acc)[2][BN / 64],
   __syncthreads();
   constexpr int kVecElems = 16 / int(sizeof(OutT));
   constexpr int kVecsPerRow = BN / kVecElems;
-  // 16-byte stores need the channel count (hence every row start) to be a
-  // multiple of the vector; otherwise fall back to single elements.
-  const bool vectorOk = outChans % kVecElems == 0 &&
-                        d.outChansPerGroup % kVecElems == 0;
+  // (16-byte stores whatever the rows start at; the channels beyond the last
+  // whole vector one by one)
   for (int idx = t; idx < kBlockM * kVecsPerRow; idx += kThreads) {
     const uint32_t mLocal = idx / kVecsPerRow, vec = idx % kVecsPerRow;
     const uint32_t m = mTile * kBlockM + mLocal;
@@ -495,8 +493,9 @@ igemmEpilogue(char *lds, const IgemmArgs &a, floatx16 (&acc)[2][BN / 64],
       continue;
     }
     OutT *dst = out + pixel * outChans + g * d.outChansPerGroup + n;
-    if (vectorOk) {
-      *reinterpret_cast<uintx4 *>(dst) = *reinterpret_cast<const uintx4 *>(src);
+    if (n + kVecElems <= d.outChansPerGroup) {
+      const uintx4 whole = *reinterpret_cast<const uintx4 *>(src);
+      *reinterpret_cast<AnyWords *>(dst) = whole;
     } else {
       const OutT *e = reinterpret_cast<const OutT *>(src);
       for (int k = 0; k != kVecElems && n + k < d.outChansPerGroup; ++k)

@@ -297,8 +297,6 @@ wideTile(const IgemmArgs &a, const char *__restrict__ in,
   constexpr int kVecElems = 16 / int(sizeof(OutT));
   constexpr int kVecsPerRow = BN / kVecElems;
   const uint32_t outChans = d.groups * d.outChansPerGroup;
-  const bool vectorOk = outChans % kVecElems == 0 &&
-                        d.outChansPerGroup % kVecElems == 0;
   // (the tile's bias as fp32, behind the rows)
   float *biasLds = reinterpret_cast<float *>(lds + 128 * kOutRow);
   __syncthreads();
@@ -341,9 +339,9 @@ wideTile(const IgemmArgs &a, const char *__restrict__ in,
         continue;
       const char *src = lds + mLocal * kOutRow + vec * 16;
       OutT *dst = out + outPixel(a, m) * outChans + g * d.outChansPerGroup + n;
-      if (vectorOk) {
-        *reinterpret_cast<uintx4 *>(dst) =
-            *reinterpret_cast<const uintx4 *>(src);
+      if (n + kVecElems <= d.outChansPerGroup) {
+        const uintx4 whole = *reinterpret_cast<const uintx4 *>(src);
+        *reinterpret_cast<AnyWords *>(dst) = whole;
       } else {
         const OutT *e = reinterpret_cast<const OutT *>(src);
         for (int k = 0; k != kVecElems && n + k < d.outChansPerGroup; ++k)

@@ -57,26 +57,6 @@ permuteSmallKernel(PermuteSmallArgs a, const T *__restrict__ src,
   dst[tid] = src[srcIndex + rest * a.srcStride[0]];
 }
 
-/// 16 bytes of neighbouring elements at any address: global memory takes such
-/// accesses, at full speed where the address happens to be a multiple of 16.
-typedef uint32_t AnyWords
-    __attribute__((ext_vector_type(4), aligned(1), may_alias));
-template <class T> union Piece {
-  T e[16 / sizeof(T)];
-  uint32_t w[4];
-};
-template <class T>
-__device__ __forceinline__ Piece<T> loadPiece(const T *at) {
-  const AnyWords v = *reinterpret_cast<const AnyWords *>(at);
-  Piece<T> p;
-  p.w[0] = v.x, p.w[1] = v.y, p.w[2] = v.z, p.w[3] = v.w;
-  return p;
-}
-template <class T>
-__device__ __forceinline__ void storePiece(T *at, const Piece<T> &p) {
-  *reinterpret_cast<AnyWords *>(at) = AnyWords{p.w[0], p.w[1], p.w[2], p.w[3]};
-}
-
 /// [batch][rows][cols] -> [batch][cols][rows] in tiles of 64 x 64 turned round
 /// in LDS: 16-byte loads along the columns, 16-byte stores along the rows.
 /// Bound by HBM.  The LDS pitch of an odd number of words keeps both the
@@ -245,7 +225,9 @@ __global__ __launch_bounds__(THREADS) void interleaveKernel(
   }
 }
 
-/// One 16-byte vector of the padded tensor per thread.
+/// One 16-byte vector of the padded tensor per thread, read as one where the
+/// source's channels fill it.  Bound by HBM: N = 13, 15 x 15, 327 channels
+/// 4.4 us element by element, 3.6 so.
 template <class T>
 __global__ __launch_bounds__(256) void padChansKernel(
     const T *__restrict__ src, T *__restrict__ dst, uint64_t vectors,
@@ -261,9 +243,15 @@ __global__ __launch_bounds__(256) void padChansKernel(
     T e[kVec];
     uint4 u;
   } v;
+  const T *at = src + pg * ci + c0;
+  if (c0 + kVec <= ci) {
+    const Piece<T> p = loadPiece(at);
+    v.u = uint4{p.w[0], p.w[1], p.w[2], p.w[3]};
+  } else {
 #pragma unroll
-  for (uint32_t i = 0; i != kVec; ++i)
-    v.e[i] = c0 + i < ci ? src[pg * ci + c0 + i] : T(0);
+    for (uint32_t i = 0; i != kVec; ++i)
+      v.e[i] = c0 + i < ci ? at[i] : T(0);
+  }
   reinterpret_cast<uint4 *>(dst)[tid] = v.u;
 }
 

@@ -65,3 +65,32 @@ def test_planner_takes_wide_tiles_for_products_that_fill_the_chip():
     assert again.packs_like(plan)
     small = pa.MatMulPlan(pa.HALF, pa.HALF, 1, 1024, 1024, 1024)
     assert "256 x 256" not in small.describe()
+
+
+# Rows of outputs that start at any element: whole vectors at every offset and
+# the channels behind the last one, in tiles of every width, with groups (whose
+# channels start inside a vector) and with input channels that are padded in a
+# copy at every offset.
+RAGGED = [
+    dict(batch=2, field=(11, 12), kernel=(1, 1), ci=64, co=7),
+    dict(batch=2, field=(11, 12), kernel=(3, 3), ci=33, co=67, pad=1),
+    dict(batch=2, field=(9, 9), kernel=(1, 1), ci=71, co=131),
+    dict(batch=1, field=(13, 12), kernel=(1, 1), ci=64, co=301),
+    dict(batch=2, field=(8, 9), kernel=(3, 3), ci=19, co=13, groups=3, pad=1),
+]
+
+
+@pytest.mark.parametrize("tile", [(128, 64), (128, 128), (256, 192),
+                                  (256, 256)])
+@pytest.mark.parametrize("kw", RAGGED)
+@pytest.mark.parametrize("out_type", [pa.FLOAT, pa.HALF])
+def test_rows_of_no_whole_vectors(oracle, kw, tile, out_type):
+    from test_fast_gpu import _run
+    p = make_params(pa.HALF, out_type, **kw)
+    options = {"planConstraints": '{"gfx950": {"kernel": "igemm", "patch": 0, '
+                                  '"pointwise": 0, "blockM": %d, "blockN": '
+                                  '%d}}' % tile}
+    assert "%d x %d x 64" % tile in pa.Plan(p, options).describe()
+    exact = out_type == pa.FLOAT
+    _run(oracle, p, 72, 0 if exact else 1e-3, "implicit GEMM",
+         dist="pm1" if exact else "normal", options=options)
