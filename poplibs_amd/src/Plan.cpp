@@ -293,13 +293,23 @@ double splitPenaltyUs(std::size_t partialBytes) {
   return 4.5 + 2.0 * double(partialBytes) / 6.4e6;
 }
 
+/// What a k-step is: fp16's or fp8's; fp32's (a 128 x 128 k-step of 32 values
+/// is 2 048 cycles of MFMAs); fp32's where the taps are looked up in ranges
+/// (more than 32 of them, a weight update pass mostly), which the loading
+/// threads take as long again for: N = 8, 16 x 16, 3 x 3, 96 -> 96 147 us in
+/// 64 k-steps of 128 x 128, 88 in 128 x 64.
+enum StepKind { kStep16, kStep32, kStep32Ranges };
+StepKind stepKindOf(bool fp32, std::size_t taps) {
+  return !fp32 ? kStep16 : taps > 32 ? kStep32Ranges : kStep32;
+}
+
 double estimateStreaming(std::size_t workgroups, std::size_t kSteps,
                          std::size_t perCU, unsigned blockN, unsigned splitK,
-                         std::size_t partialBytes, bool fp32) {
+                         std::size_t partialBytes, StepKind kind) {
   const double rounds = roundsOf(workgroups, perCU);
-  // (fp32 MFMAs: a 128 x 128 k-step of 32 values is 2 048 cycles of them)
-  const double step = fp32 ? (blockN == 128 ? 1.0 : 0.52)
-                           : (blockN == 128 ? 0.345 : 0.24);
+  const double step = kind == kStep32Ranges ? (blockN == 128 ? 2.1 : 1.2)
+                      : kind == kStep32     ? (blockN == 128 ? 1.0 : 0.52)
+                                            : (blockN == 128 ? 0.345 : 0.24);
   double tile = 2.95 + step * double(kSteps);
   if (perCU == 1 && rounds > 1)
     tile += 1.5;
@@ -916,6 +926,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
     // estimates (N = 32, 14 x 14, 1024 -> 256: 8.9 -> 7.1 us; 7 x 7, 2048 ->
     // 512: 12.8 -> 10.2; but 14 x 14, 1024 -> 512, 392 narrow tiles: 10.2
     // against 12.1, and the estimate keeps the wide tile there).
+    const StepKind stepKind =
+        stepKindOf(floatIn, std::size_t(s.kD) * s.kH * s.kW);
     bool narrowWhole = false;    // ... chosen: K stays whole
     std::size_t narrowSplit = 0; // ... or narrow tiles with K in this many parts
     if (!pc.blockN && !pc.splitK && !pc.stages && co > 64 &&
@@ -935,14 +947,14 @@ mxconv_plan makePlanWith(const ConvParams &params,
           parts * m * p.numConvGroups * ((co + 127) / 128 * 128) * 4;
       const double wideUs = std::min(
           estimateStreaming(wide, kSteps, wide > gfx950::numCUs ? 2 : 1, 128,
-                            1, 0, floatIn),
+                            1, 0, stepKind),
           parts > 1 ? estimateStreaming(wide * parts,
                                         (kSteps + parts - 1) / parts, 1, 128,
-                                        unsigned(parts), partial, floatIn)
+                                        unsigned(parts), partial, stepKind)
                     : 1e30);
       const double wideWholeUs = estimateStreaming(
-          wide, kSteps, wide > gfx950::numCUs ? 2 : 1, 128, 1, 0, floatIn);
-      if (estimateStreaming(narrow, kSteps, 2, 64, 1, 0, floatIn) < wideUs) {
+          wide, kSteps, wide > gfx950::numCUs ? 2 : 1, 128, 1, 0, stepKind);
+      if (estimateStreaming(narrow, kSteps, 2, 64, 1, 0, stepKind) < wideUs) {
         g.blockN = 64, narrowWhole = true;
       } else if (wideUs < wideWholeUs && narrow * 2 <= gfx950::numCUs) {
         // K split wins: then over narrow tiles, in half as many parts of at
@@ -1004,11 +1016,11 @@ mxconv_plan makePlanWith(const ConvParams &params,
       // 3 x 3, 512 -> 512 (52 tiles of 72 k-steps) 18.7 in four, 21.1 whole.
       if (!pc.splitK && !narrowSplit && parts > 1 &&
           estimateStreaming(tiles, kSteps, g.blockN == 64 ? 2 : 1, g.blockN, 1,
-                            0, floatIn) <=
+                            0, stepKind) <=
               estimateStreaming(tiles * parts, (kSteps + parts - 1) / parts,
                                 1, g.blockN, unsigned(parts),
                                 parts * m * p.numConvGroups * plan.coPadded *
-                                    4, floatIn))
+                                    4, stepKind))
         parts = 1;
       const std::size_t chans = p.numConvGroups * co;
       // partial tiles of more than 1 GB are not worth it
@@ -1297,7 +1309,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
               Tiling{0, 128}, streamTiles, streamPerCU, streamSteps,
               estimateStreaming(streamTiles, streamSteps, streamPerCU,
                                 g.blockN, g.splitK,
-                                mxk::igemmWorkspaceBytes(g), floatIn),
+                                mxk::igemmWorkspaceBytes(g), stepKind),
               roundsOf(streamTiles, streamPerCU));
       std::size_t best = iStream;
       if (pc.patch >= 1) {
@@ -1356,7 +1368,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
         planned = std::max(
             estimateStreaming(tiles, kSteps,
                               g.blockN == 64 || g.stages == 2 ? 2 : 1,
-                              g.blockN, 1, 0, false),
+                              g.blockN, 1, 0, kStep16),
             kLaunchUs + streamingPowerUs(tiles, kSteps, g.blockN,
                                          s.kD * s.kH * s.kW == 1));
       }
@@ -1433,7 +1445,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
           }
           planned = estimateStreaming(tiles, steps,
                                       g.blockN == 64 || g.stages == 2 ? 2 : 1,
-                                      g.blockN, 1, 0, floatIn);
+                                      g.blockN, 1, 0,
+                                      stepKindOf(floatIn, 0));
         }
         double best = (plan.pointwiseOn ? 0.9 : 0.95) * planned;
         for (uint32_t t = 1; t <= mxk::kIgemmSmallTiles; ++t) {
@@ -1762,7 +1775,9 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
             : poplin::estimateStreaming(tiles, steps, perCU, g.blockN,
                                         g.splitK,
                                         mxk::igemmWorkspaceBytes(igemm),
-                                        params.inputType == poplar::FLOAT);
+                                        poplin::stepKindOf(
+                                            params.inputType == poplar::FLOAT,
+                                            std::size_t(g.kD) * g.kH * g.kW));
     // No kernel is faster than its tensors stream.
     us = std::max(us, streamed(inputBytes() + outputBytes() +
                                weightPackedBytes()));
