@@ -16,6 +16,8 @@ pytestmark = pytest.mark.gpu
     (700, 8 * 65),       # two blocks of channels, an odd vector each
     (700, 8 * 64 + 4),   # whole vectors of float, not of half
     (5000, 3), (333, 1), (4097, 144),
+    # the last row that goes in one launch; around its row lanes' passes
+    (4096, 144), (1024, 33), (1025, 33), (2047, 40), (2049, 24), (256, 32), (257, 31),
 ])
 @pytest.mark.parametrize("dt,bt", [(pa.HALF, pa.HALF), (pa.HALF, pa.FLOAT),
                                    (pa.FLOAT, pa.FLOAT)])
