@@ -442,6 +442,9 @@ uint32_t wuTapChunkPixels(const WuTapDesc &d, uint32_t computeUnits) {
     uint64_t pixels = (M + n - 1) / n;
     pixels = std::max<uint64_t>(256, (pixels + 63) / 64 * 64);
     const uint64_t chunks = (M + pixels - 1) / pixels;
+    // (no more than the workspace may hold: wuTapTakes)
+    if (best && chunks * tiles * 65536 > (1ull << 31))
+      break;
     const uint64_t rounds = (chunks * tiles + computeUnits - 1) / computeUnits;
     const double us = double(rounds) * (4.0 + 0.7 * double(pixels / 64)) +
                       double(chunks * tiles) * tileUs;
