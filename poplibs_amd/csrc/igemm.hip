@@ -811,12 +811,12 @@ bool igemmAddressable(const IgemmDesc &d, int inType) {
                               d.inW +
                           uint64_t(d.padW > 0 ? d.padW : 0)) *
                          d.groups * d.inChansPerGroup * eb;
-  // images a tile of 128 output rows can touch: its rows' own, one more when
-  // it starts inside an image
+  // images a tile of blockM output rows can touch: its rows' own, one more
+  // when it starts inside an image
   const uint64_t rowsPerImage = uint64_t(d.outD) * d.outH * d.outW;
   if (rowsPerImage == 0)
     return true;
-  uint64_t images = (kBlockM - 1) / rowsPerImage + 2;
+  uint64_t images = (uint64_t(d.blockM) - 1) / rowsPerImage + 2;
   if (images > d.batch)
     images = d.batch;
   return images * imageBytes + shift < kOutOfRange - (1u << 20);

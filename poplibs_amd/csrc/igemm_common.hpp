@@ -34,7 +34,6 @@ struct IgemmArgs {
 };
 
 /// igemm_wide.hip: tiles of 256 pixels; `a` as prepared for igemmKernel.
-bool igemmWideTakes(const IgemmDesc &d, int inType, int outType);
 hipError_t launchIgemmWide(const IgemmArgs &a, int inType, int outType,
                            const void *in, const void *w, const void *bias,
                            void *out, const QuarterInfo &q,

@@ -383,9 +383,10 @@ hipError_t launchKernel(const IgemmArgs &a, uint32_t blocks, const void *in,
 bool igemmWideTakes(const IgemmDesc &d, int inType, int outType) {
   return (outType == kHalf || outType == kFloat) &&
          (inType == kHalf || inType == kQuarter) &&
+         d.blockM == uint32_t(kWideM) &&
          (d.blockN == 192 || d.blockN == 256) &&
          d.splitK == 1 && !d.noTaps && !d.outTransposed &&
-         igemmTapAddressing(d) == kMaskTaps;
+         igemmTapAddressing(d) == kMaskTaps && igemmAddressable(d, inType);
 }
 
 hipError_t launchIgemmWide(const IgemmArgs &a, int inType, int outType,

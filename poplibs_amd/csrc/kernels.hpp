@@ -245,9 +245,12 @@ struct IgemmDesc {
 /// input).
 enum : int { kMaskTaps = 0, kRangeTaps = 1, kDilatedTaps = 2 };
 /// Whether the kernel can address the input: it uses 32-bit offsets from the
-/// first image (batch element) a tile of 128 output rows reads, so those few
-/// images - not the tensor - have to stay under 2^31 bytes.
+/// first image (batch element) a tile of d.blockM output rows reads, so those
+/// few images - not the tensor - have to stay under 2^31 bytes.
 bool igemmAddressable(const IgemmDesc &d, int inType);
+/// Whether the kernel of 256-pixel tiles (d.blockM 256; d.blockN 192 or 256)
+/// takes the convolution, its tiles' images included.
+bool igemmWideTakes(const IgemmDesc &d, int inType, int outType);
 int igemmTapAddressing(const IgemmDesc &d);
 size_t igemmWorkspaceBytes(const IgemmDesc &d);
 hipError_t launchIgemm(const IgemmDesc &d, int inType, int outType,

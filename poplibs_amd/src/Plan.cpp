@@ -691,6 +691,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
   // first image a tile reads.
   auto inputAddressable = [&] {
     mxk::IgemmDesc g{};
+    g.blockM = 128; // (the tiles of 256 pixels ask for themselves)
     g.batch = uint32_t(s.batch), g.groups = uint32_t(p.numConvGroups);
     g.inChansPerGroup = uint32_t(ciPadded);
     g.inD = s.inD, g.inH = s.inH, g.inW = s.inW;
@@ -1174,6 +1175,23 @@ mxconv_plan makePlanWith(const ConvParams &params,
         ph.d.stages = stages;
       g.stages = stages;
     }
+    const int inId = halfIn ? mxk::kHalf : floatIn ? mxk::kFloat
+                                                   : mxk::kQuarter;
+    const int outId =
+        params.outputType == poplar::HALF ? mxk::kHalf : mxk::kFloat;
+    // (a weight update pass on the layer's own tensors runs none of this)
+    if (wideTile && !plan.denseWeightUpdate && !plan.depthwiseWeightUpdate) {
+      bool takes = !plan.igemmPhases.empty() ||
+                   mxk::igemmWideTakes(g, inId, outId);
+      for (const auto &ph : plan.igemmPhases)
+        takes = takes && mxk::igemmWideTakes(ph.d, inId, outId);
+      if (!takes)
+        throw poplar::invalid_option(
+            "planConstraints gfx950 blockM 256: that kernel takes kernels of "
+            "at most 32 taps on an input of which the images that 256 output "
+            "pixels meet stay under 2^31 bytes (a zero-stuffed input where "
+            "every phase has taps)");
+    }
     // A pointwise convolution with few input channels is bound by HBM, not
     // by the matrix cores: unless the big tile was asked for explicitly, the
     // streaming kernel of small workgroups takes it.
@@ -1242,10 +1260,6 @@ mxconv_plan makePlanWith(const ConvParams &params,
         !plan.paddedInputChans &&
         (g.splitK == 1 || !pc.splitK) && pc.patch != 0 &&
         !pc.blockN && !pc.blockK && !pc.stages) {
-      const int inId = halfIn ? mxk::kHalf : floatIn ? mxk::kFloat
-                                                     : mxk::kQuarter;
-      const int outId =
-          params.outputType == poplar::HALF ? mxk::kHalf : mxk::kFloat;
       const std::size_t m = std::size_t(s.batch) * s.outH * s.outW;
       const std::size_t nTiles128 = (co + 127) / 128 * p.numConvGroups;
       const std::size_t stepBytes = 128;
@@ -1382,7 +1396,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
             p.numConvGroups * ((co + bn - 1) / bn * bn) * plan.kPadded *
                     params.inputType.size() >=
                 (1ull << 31) ||
-            mxk::igemmTapAddressing(t) != mxk::kMaskTaps)
+            !mxk::igemmWideTakes(t, inId, outId))
           continue;
         planned = us;
         g = t;
@@ -1401,10 +1415,6 @@ mxconv_plan makePlanWith(const ConvParams &params,
     // A problem too small for 128-pixel tiles to fill the chip: small tiles
     // with K split over the waves of a workgroup.
     {
-      const int inId = halfIn ? mxk::kHalf : floatIn ? mxk::kFloat
-                                                     : mxk::kQuarter;
-      const int outId =
-          params.outputType == poplar::HALF ? mxk::kHalf : mxk::kFloat;
       const std::size_t eb = params.inputType.size();
       auto asSmall = [&](uint32_t tile) {
         mxk::IgemmDesc t = g;
