@@ -485,6 +485,53 @@ mxconv_plan makePlanWith(const ConvParams &params,
                          const ConvOptions &optionsIn,
                          unsigned convGroupsPerGroup);
 
+/// A weight update pass of fewer than 1024 pixels that was planned for
+/// wuTapKernel: back to the pass's own convolution where that is estimated to
+/// be faster.  Fitted to 2472 random layers of 1 to 64 images, kernels of up to
+/// 49 taps, 1 to 800 channels and up to 32 groups: what is picked by the two
+/// estimates is on average 0.4 % slower than the faster of the two; the kernel
+/// for all of them would be 2.5 % slower, the convolution takes 2.6 times it.
+///  * A batch that is no whole vector is the convolution's padded copy and two
+///    rearrangements more; only kernels of 25 taps and more over many poorly
+///    filled groups are faster so (3 images of 7 x 7, 7 x 7, 32 groups of 48 ->
+///    64 39.1 us, the kernel 52.6; but 4 of 14 x 14, 3 x 3, 32 -> 48 23.8
+///    against 9.1, one of 10 x 10, 504 -> 144 25.9 against 10.2).
+///  * With whole vectors of images it takes fewer taps to bring it ahead: 8
+///    images of 8 x 8, 5 x 5, 256 -> 256 12.3 against 22.7, 3 x 3, 512 -> 256
+///    12.5 against 17.8, 3 x 3, 64 -> 64 11.7 against 9.7.
+void settleFewPixelWeightDeltas(mxconv_plan &plan) {
+  const mxk::WuTapDesc &f = plan.denseForward;
+  const std::size_t pixels = std::size_t(f.batch) * f.outH * f.outW;
+  if (!plan.denseWeightUpdate || pixels >= 1024 ||
+      plan.options.planConstraints.weightDeltas == 1)
+    return;
+  plan.denseWeightUpdate = false;
+  const mxconv_plan::DetailedEstimate e = plan.detailedEstimate();
+  const bool wholeVectors =
+      f.batch % (16 / plan.params.inputType.size()) == 0;
+  const bool fused = plan.wuGroupsPerGroup > 1;
+  const double tensorsMB =
+      double(plan.inputBytes() + plan.weightBytes()) * 1e-6;
+  const double resultMB = double(plan.outputBytes()) * 1e-6;
+  const double partialBytes = double(mxk::wuTapWorkspaceBytes(f));
+  const double rounds =
+      std::ceil(partialBytes / 65536.0 / double(gfx950::numCUs));
+  const double steps = std::ceil(
+      double(std::min<std::size_t>(f.chunkPixels, pixels)) / 64.0);
+  const double kernelUs =
+      std::max(8.9, 6.8 + rounds * (0.6 + 0.52 * steps) +
+                        0.12e-6 * partialBytes + 1.5 * resultMB +
+                        (fused ? 2.2 + 0.17 * resultMB : 0.0));
+  const double blocksUs = fused ? 2.1 + 0.5 * resultMB : 0.0;
+  const double convolutionUs =
+      wholeVectors
+          ? std::max(11.8, 3.9 + 1.39 * e.totalUs() + 1.26 * tensorsMB +
+                               blocksUs)
+          : std::max(20.0, 11.7 + 1.3 * e.totalUs() + 2.5 * tensorsMB +
+                               blocksUs);
+  plan.denseWeightUpdate = !e.known || kernelUs <= convolutionUs;
+}
+
 } // namespace
 
 mxconv_plan makePlan(const ConvParams &params, const ConvOptions &optionsIn) {
@@ -498,6 +545,7 @@ mxconv_plan makePlan(const ConvParams &params, const ConvOptions &optionsIn) {
     fused.outputChannelsPerConvGroup *= fuse;
     mxconv_plan plan = makePlanWith(fused, optionsIn, 1);
     plan.wuGroupsPerGroup = fuse;
+    settleFewPixelWeightDeltas(plan);
     return plan;
   }
   if (fuse > 1) {
@@ -506,7 +554,9 @@ mxconv_plan makePlan(const ConvParams &params, const ConvOptions &optionsIn) {
     if (plan.kernel == mxconv_plan::Kernel::IGEMM)
       return plan;
   }
-  return makePlanWith(params, optionsIn, 1);
+  mxconv_plan plan = makePlanWith(params, optionsIn, 1);
+  settleFewPixelWeightDeltas(plan);
+  return plan;
 }
 
 namespace {
@@ -635,18 +685,10 @@ mxconv_plan makePlanWith(const ConvParams &params,
       f.ci = (f.resultCi + 7) / 8 * 8;
       f.co = (f.resultCo + 7) / 8 * 8;
       f.chunkPixels = mxk::wuTapChunkPixels(f, gfx950::numCUs);
-      // Enough pixels for the kernel's start-up to pay.  Measured against the
-      // pass's own convolution, us: 1 x 1, 128 pixels, 240 -> 64 17.4 against
-      // 8.0, 972 pixels, 32 -> 48 290 against 8.6; 3 x 3, 972 pixels,
-      // 240 -> 64 26.5 against 10.0, 256 -> 256 27.6 against 16.8 (512: 12.2
-      // against 13.0).  It would gain below as well (3 x 3, 784 pixels of 4
-      // images, 32 -> 48: 23.8 against 9.1), but small fields of a few images
-      // are the layers that tests check the pass's convolution with.
-      const std::size_t pixels = std::size_t(f.batch) * f.outH * f.outW;
-      // ... and, in a grouped layer, channels that fill a quarter of the
-      // kernel's 128 x 128 tile per (group, tap): every group brings its own
-      // tiles, and poorly filled ones lose to the pass's own convolution
-      // (N = 32, 28 x 28, 3 x 3: 32 groups of 16 -> 16 channels 420 against
+      // Of 1024 pixels or more: 16 channels and more and, in a grouped layer,
+      // a quarter of the kernel's 128 x 128 tile per (group, tap): every group
+      // brings its own tiles, and poorly filled ones lose to the pass's own
+      // convolution (N = 32, 28 x 28, 3 x 3: 32 groups of 16 -> 16 channels 420 against
       // 117 us, 8 groups of 32 -> 32 78 against 49, 2 groups of 64 -> 64 26
       // against 26.5, 4 groups of 64 -> 64 41 against 34 and 2 such groups on
       // 56 x 56 70 against 52; without groups 16 -> 16 on 56 x 56 ties at
@@ -655,11 +697,10 @@ mxconv_plan makePlanWith(const ConvParams &params,
                                    ((f.co + 127) / 128 * 128);
       const bool filled =
           f.groups == 1 || std::size_t(f.ci) * f.co * 4 > tileArea;
-      const bool enough =
-          pixels >= 1024 ||
-          (pixels >= 128 && (f.kH * f.kW == 1 || f.batch >= 8));
-      const bool worth =
-          enough && f.resultCi >= 16 && f.resultCo >= 16 && filled;
+      // Of fewer pixels: by estimate, once both are planned
+      // (settleFewPixelWeightDeltas).
+      const bool worth = std::size_t(f.batch) * f.outH * f.outW < 1024 ||
+                         (f.resultCi >= 16 && f.resultCo >= 16 && filled);
       plan.denseWeightUpdate = (asked == 1 || worth) && mxk::wuTapTakes(f);
     }
     if (asked == 1 && isWeightUpdatePass(options.pass) &&

@@ -360,17 +360,25 @@ def test_dense_weight_update_plan_choice():
     assert DENSE_WU in pa.WeightUpdatePlan(
         make_params(pa.HALF, batch=32, field=(28, 28), kernel=(3, 3), ci=128,
                     co=128, pad=1, stride=2)).describe()
-    # dilated kernels, tiny pixel counts and fp32 tensors stay with the
-    # pass's own convolution
+    # dilated kernels, large kernels over few pixels of whole vectors of
+    # images and fp32 tensors stay with the pass's own convolution
     for kw in (dict(batch=32, field=(28, 28), kernel=(3, 3), ci=128, co=128,
                     pad=2, kdil=2),
-               dict(batch=1, field=(8, 8), kernel=(3, 3), ci=128, co=128,
-                    pad=1)):
+               dict(batch=8, field=(8, 8), kernel=(5, 5), ci=256, co=256,
+                    pad=2)):
         assert DENSE_WU not in pa.WeightUpdatePlan(
             make_params(pa.HALF, **kw)).describe()
     assert DENSE_WU not in pa.WeightUpdatePlan(
         make_params(pa.FLOAT, batch=32, field=(28, 28), kernel=(3, 3), ci=128,
                     co=128, pad=1)).describe()
+    # (few pixels otherwise: the kernel, at any batch)
+    for kw in (dict(batch=4, field=(14, 14), kernel=(3, 3), ci=32, co=48,
+                    pad=1),
+               dict(batch=1, field=(8, 8), kernel=(3, 3), ci=128, co=128,
+                    pad=1),
+               dict(batch=16, field=(5, 5), kernel=(1, 1), ci=256, co=64)):
+        assert DENSE_WU in pa.WeightUpdatePlan(
+            make_params(pa.HALF, **kw)).describe()
     # ... and a kernel named in planConstraints is honoured
     opts = {"planConstraints": '{"gfx950": {"kernel": "igemm"}}'}
     assert DENSE_WU not in pa.WeightUpdatePlan(big, opts).describe()
@@ -386,10 +394,46 @@ def test_weight_deltas_of_a_small_batch_run_on_the_matrix_cores(oracle):
     rng = np.random.default_rng(26)
     xq, xd = quantize(rng.standard_normal((4, 32, 14, 14)), pa.HALF)
     dq, dd = quantize(rng.standard_normal((4, 48, 14, 14)) * 0.1, pa.HALF)
-    got, plan = run_weight_update(p, xq, dq)
+    got, plan = run_weight_update(
+        p, xq, dq, {"planConstraints": '{"gfx950": {"weightDeltas": 0}}'})
     assert "implicit GEMM" in plan.describe(), plan.describe()
     assert "input channels padded      4 -> 8" in plan.describe()
+    assert DENSE_WU not in plan.describe()
     assert rel_l2(got, oracle.weight_deltas(p, xd, dd, threads=8)) <= 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("deltas", [None, 0, 1])
+@pytest.mark.parametrize("kw", [
+    # one pixel; a few; a chunk of 256 and one more; around whole vectors of
+    # images, whole vectors of channels, groups taken as one
+    dict(batch=1, field=(3, 3), kernel=(3, 3), ci=40, co=24),
+    dict(batch=2, field=(2, 2), kernel=(1, 1), ci=5, co=3),
+    dict(batch=1, field=(17, 17), kernel=(3, 3), ci=24, co=131, pad=1),
+    dict(batch=7, field=(6, 5), kernel=(3, 3), ci=64, co=40, pad=1),
+    dict(batch=8, field=(6, 5), kernel=(3, 3), ci=64, co=40, pad=1),
+    dict(batch=8, field=(8, 8), kernel=(5, 5), ci=48, co=160, pad=2),
+    dict(batch=3, field=(9, 9), kernel=(3, 3), ci=4, co=8, groups=16, pad=1),
+    dict(batch=8, field=(11, 9), kernel=(3, 3), ci=16, co=4, groups=8, pad=1,
+         stride=2),
+])
+def test_weight_deltas_of_few_pixels(oracle, kw, deltas):
+    # the pass's own convolution, the kernel on the layer's tensors, and
+    # whichever the planner takes: +-1 tensors, exact sums
+    p = make_params(pa.HALF, pa.FLOAT, **kw)
+    rng = np.random.default_rng(64)
+    x = rng.choice([-1.0, 1.0],
+                   (p.batchSize, p.getNumInputChans(), *p.inputFieldShape))
+    dz = rng.choice([-1.0, 1.0], (p.batchSize, p.getNumOutputChans(),
+                                  *p.getOutputFieldShape()))
+    options = None if deltas is None else {
+        "planConstraints": '{"gfx950": {"weightDeltas": %d}}' % deltas}
+    got, plan = run_weight_update(p, x.astype(np.float16),
+                                  dz.astype(np.float16), options)
+    if deltas is not None:
+        assert (DENSE_WU in plan.describe()) == bool(deltas)
+    np.testing.assert_array_equal(got, oracle.weight_deltas(p, x, dz,
+                                                            threads=8))
 
 
 @pytest.mark.gpu
