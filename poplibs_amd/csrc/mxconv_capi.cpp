@@ -1569,6 +1569,8 @@ mxconv_status fusedWeightDeltas(const mxconv_plan *plan, const void *zDeltas,
                       !plan->paddedInputChans &&
                       plan->igemmPhases.empty() && !plan->kernelSelected &&
                       !plan->igemm.patch && !plan->igemm.small &&
+                      // (tiles of 256 pixels do not write it transposed)
+                      plan->igemm.blockM != 256 &&
                       // (a padded output field - the forward kernel was
                       // truncated - is filled by the general path)
                       !plan->outputPadded;

@@ -437,6 +437,25 @@ def test_weight_deltas_of_few_pixels(oracle, kw, deltas):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("width", [192, 256])
+@pytest.mark.parametrize("batch", [8, 3])
+def test_weight_deltas_by_a_named_tile_of_256_pixels(oracle, batch, width):
+    # the pass's convolution in tiles that write [pixel][channel] only
+    p = make_params(pa.HALF, pa.FLOAT, batch=batch, field=(5, 6),
+                    kernel=(3, 3), ci=40, co=24, pad=1)
+    rng = np.random.default_rng(65)
+    x = rng.choice([-1.0, 1.0], (batch, 40, 5, 6))
+    dz = rng.choice([-1.0, 1.0], (batch, 24, 5, 6))
+    got, plan = run_weight_update(
+        p, x.astype(np.float16), dz.astype(np.float16),
+        {"planConstraints": '{"gfx950": {"weightDeltas": 0, "kernel": "igemm",'
+                            ' "blockM": 256, "blockN": %d}}' % width})
+    assert "256 x %d x 64" % width in plan.describe(), plan.describe()
+    np.testing.assert_array_equal(got, oracle.weight_deltas(p, x, dz,
+                                                            threads=8))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("co", [3, 5])
 @pytest.mark.parametrize("dt", [pa.HALF, pa.FLOAT])
 def test_weight_deltas_of_a_layer_with_few_output_channels(oracle, co, dt):
