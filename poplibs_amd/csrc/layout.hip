@@ -529,17 +529,28 @@ __global__ __launch_bounds__(256) void biasUpdateKernel(
 /// The same in one launch, for few rows: a workgroup takes 32 channels (64
 /// bytes of halves, four lanes to a row; one channel per lane where they are
 /// no whole vectors) through all the rows, eight rows' loads in flight per
-/// thread; the row lanes' sums meet in LDS.  A single CU reads 64 bytes a
-/// cycle at best, which the second launch outweighs up to 4 096 rows (1 024
-/// of no whole vectors).  The call, host and all, with two kernels 5.9 us
-/// whatever the rows; with this one 144 halves in 1 024 rows 3.4, in 2 048 3.7,
-/// in 4 096 5.1, 45 halves in 1 024 rows 4.0, in 2 048 5.9.
-constexpr uint32_t kDirectRows = 4096, kDirectRaggedRows = 1024;
+/// thread; the row lanes' sums meet in LDS.  Of halves that is half a 128-byte
+/// line, so the two workgroups of a line are `paired`: dealt to one XCD, whose
+/// L2 fetches it once (8192 halves in 2 048 rows 13.3 -> 9.9 us).
+/// A single CU reads 64 bytes a cycle at best, which the second launch
+/// outweighs up to 2 048 rows - 3 200 of 1 MB in all, 4 096 of a single line,
+/// but 1 024 of no whole vectors.  The call, host and all, us, on rows from
+/// memory and on rows just read, with this kernel and with two:
+///   halves   64 x 4 096   7.1, 4.6   6.8, 6.6     144 x 2 048  5.3, 4.1   6.5, 6.5
+///           144 x 3 072   7.2, 4.5   6.6, 6.6   1 024 x 2 048  5.8, 3.8   6.8, 6.6
+///         1 024 x 4 096  10.9, 4.9   7.2, 6.5   8 192 x 2 048  9.9, 4.8  11.1, 7.8
+///   floats  144 x 2 048   5.4, 4.0   6.7, 6.6   2 048 x 2 048  8.8, 4.0   8.7, 6.4
+/// In a layer's training step the rows are somewhere between: 16 images of
+/// 14 x 14, 1 x 1, 512 -> 1024 (3 136 rows) 55.1 us with this kernel, 52.4 with
+/// two, 64 of 8 x 8, 3 x 3, 256 -> 512 (4 096) 74.8 and 71.2, but 4 of 28 x 28,
+/// 1 x 1, 64 -> 144 (3 136) 33.0 and 35.4.
+constexpr uint32_t kDirectRows = 2048, kDirectRaggedRows = 1024;
+constexpr uint32_t kDirectSmallRows = 3200, kDirectLineRows = 4096;
 constexpr uint32_t kDirectChans = 32;
 template <typename T, int VEC, typename B>
 __global__ __launch_bounds__(1024) void biasDirectKernel(
     const T *__restrict__ z, B *biases, float scale, uint32_t rows,
-    uint64_t channels) {
+    uint64_t channels, uint32_t paired) {
   constexpr uint32_t kVecLanes = kDirectChans / VEC;
   constexpr uint32_t kRowLanes = 1024 / kVecLanes, kParts = 32;
   constexpr uint32_t kPerPart = (kRowLanes + kParts - 1) / kParts;
@@ -547,7 +558,11 @@ __global__ __launch_bounds__(1024) void biasDirectKernel(
   __shared__ float parts[kParts][kDirectChans];
   const uint32_t vec = threadIdx.x % kVecLanes;
   const uint32_t rowLane = threadIdx.x / kVecLanes;
-  const uint64_t c0 = uint64_t(blockIdx.x) * kDirectChans;
+  // (workgroups b and b + 8 of every 16 run on one XCD)
+  const uint32_t b = blockIdx.x;
+  const uint32_t block =
+      b < paired ? (b & ~15u) | ((b & 7u) << 1) | ((b >> 3) & 1u) : b;
+  const uint64_t c0 = uint64_t(block) * kDirectChans;
   const uint64_t c = c0 + vec * VEC;
   struct alignas(sizeof(T) * VEC) Vec {
     T e[VEC];
@@ -1193,19 +1208,26 @@ hipError_t launchBiasUpdate(int deltasType, const void *zDeltas, uint64_t rows,
   const uint64_t vecElems = deltasType == kFloat ? 4 : 8;
   const bool vectors = channels % vecElems == 0 &&
                        reinterpret_cast<uintptr_t>(zDeltas) % 16 == 0;
-  if (rows <= (vectors ? kDirectRows : kDirectRaggedRows)) {
+  const uint64_t rowBytes = channels * (deltasType == kFloat ? 4 : 2);
+  if (rows <= (!vectors                        ? kDirectRaggedRows
+               : rowBytes <= 128               ? kDirectLineRows
+               : rows * rowBytes <= (1u << 20) ? kDirectSmallRows
+                                               : kDirectRows)) {
     auto direct = [&](auto *z, auto *b) {
       using T = std::remove_const_t<std::remove_pointer_t<decltype(z)>>;
       using B = std::remove_pointer_t<decltype(b)>;
       constexpr int kVec = 16 / sizeof(T);
-      const dim3 grid{
-          uint32_t((channels + kDirectChans - 1) / kDirectChans)};
+      const uint32_t n =
+          uint32_t((channels + kDirectChans - 1) / kDirectChans);
+      const uint32_t paired = sizeof(T) == 2 ? n & ~15u : 0;
       if (vectors)
-        hipLaunchKernelGGL((biasDirectKernel<T, kVec, B>), grid, dim3{1024}, 0,
-                           stream, z, b, scale, uint32_t(rows), channels);
+        hipLaunchKernelGGL((biasDirectKernel<T, kVec, B>), dim3{n}, dim3{1024},
+                           0, stream, z, b, scale, uint32_t(rows), channels,
+                           paired);
       else
-        hipLaunchKernelGGL((biasDirectKernel<T, 1, B>), grid, dim3{1024}, 0,
-                           stream, z, b, scale, uint32_t(rows), channels);
+        hipLaunchKernelGGL((biasDirectKernel<T, 1, B>), dim3{n}, dim3{1024}, 0,
+                           stream, z, b, scale, uint32_t(rows), channels,
+                           paired);
       return hipGetLastError();
     };
     auto ofBias = [&](auto *z) {

@@ -18,6 +18,11 @@ pytestmark = pytest.mark.gpu
     (5000, 3), (333, 1), (4097, 144),
     # the last row that goes in one launch; around its row lanes' passes
     (4096, 144), (1024, 33), (1025, 33), (2047, 40), (2049, 24), (256, 32), (257, 31),
+    (2048, 144), (2049, 144), (4096, 64), (4096, 32), (4097, 64), (4097, 32),
+    (3200, 144), (3201, 144), (3200, 168),
+    # workgroups in pairs: one short of 16, 16, one more, the last one partial
+    (300, 15 * 32), (300, 16 * 32), (300, 17 * 32), (300, 31 * 32 + 8),
+    (300, 33 * 32 - 1), (2048, 32 * 32),
 ])
 @pytest.mark.parametrize("dt,bt", [(pa.HALF, pa.HALF), (pa.HALF, pa.FLOAT),
                                    (pa.FLOAT, pa.FLOAT)])
