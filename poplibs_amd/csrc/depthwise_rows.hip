@@ -36,7 +36,6 @@ constexpr int kSlotBytes = kRowLoads * 1024;
 constexpr int kLoaderWaves = 4;
 constexpr int kComputeWaves = 6;
 constexpr int kComputeThreads = 64 * kComputeWaves;
-constexpr int kRowsThreads = 64 * (kComputeWaves + kLoaderWaves);
 constexpr int kOwnLoads = kRowLoads / kLoaderWaves; // per loader wave and row
 constexpr uint32_t kNoByte = 0x80000000u;           // beyond any buffer here
 

@@ -255,26 +255,6 @@ template <> struct Mma<4> {
             between();
         }
   }
-  template <int S, int K, int TN>
-  static __device__ __forceinline__ void loadOne(const FragmentAddress &at,
-                                                 int lane, Frags<TN> &f) {
-    const int c = S * 2 + (lane >> 5);
-    if constexpr (K < 2)
-      f.a[S][K] = *reinterpret_cast<const floatx4 *>(
-          at.a[K] + (((at.chunkBase + c) ^ at.swizzleA[K]) << 4));
-    else
-      f.b[S][K - 2] = *reinterpret_cast<const floatx4 *>(
-          at.b + (K - 2) * 32 * kRowBytes + ((c ^ at.swizzleB) << 4));
-  }
-  template <int S, int K, int TN, int FA, int FB>
-  static __device__ __forceinline__ void mulOne(const Frags<TN> &f,
-                                                floatx16 (&acc)[2][TN]) {
-    // (the four depend on each other; the other wave of the SIMD fills in)
-#pragma unroll
-    for (int e = 0; e != 4; ++e)
-      acc[K / TN][K % TN] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-          f.b[S][K % TN][e], f.a[S][K / TN][e], acc[K / TN][K % TN], 0, 0, 0);
-  }
 };
 
 /// fp8: 2 sub-steps of K=64, 64 bytes (four chunks, two per half-wave) each.

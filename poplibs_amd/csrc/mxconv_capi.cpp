@@ -1236,7 +1236,6 @@ mxconv_status mxconv_matmul_pack_rhs(const mxconv_plan *plan, const void *rhs,
   REQUIRE_ARG(weights_packed);
   if (plan->weightElems != 0)
     REQUIRE_ARG(rhs);
-  const auto &p = plan->params;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (plan->kernel == mxconv_plan::Kernel::IGEMM) {
     return hipStatus(packIgemmWeights(*plan, rhs, 1, true, weights_packed, s),

@@ -460,8 +460,6 @@ uint64_t wuTapWorkspaceBytes(const WuTapDesc &d) {
   const uint64_t M = uint64_t(d.batch) * d.outH * d.outW;
   if (d.chunkPixels == 0)
     return 0;
-  if (d.resultCi > d.ci || d.resultCo > d.co)
-    return false;
   const uint64_t chunks = (M + d.chunkPixels - 1) / d.chunkPixels;
   return chunks * tilesOf(d) * 128 * 128 * 4;
 }

@@ -1769,10 +1769,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
   } else {
     plan.weightPackedElems = plan.weightElems; // [G][K][Ci][Co]
   }
-  if (convGroupsPerGroup > 1 && chosen == Kernel::IGEMM) {
+  if (convGroupsPerGroup > 1 && chosen == Kernel::IGEMM)
     plan.convGroupsPerGroup = convGroupsPerGroup;
-    plan.weightExpandElems = plan.weightElems * convGroupsPerGroup;
-  }
   return plan;
 }
 

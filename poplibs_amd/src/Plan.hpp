@@ -116,12 +116,8 @@ struct mxconv_plan {
   // block-diagonal - the groups' channels are neighbours in the tensors
   // already, so only the weight packing knows.  The role of the reference
   // planner's convGroupsPerGroup (lib/poplin/ConvPlan.cpp, the AMP and SLIC
-  // vertices that take several conv groups at once).  The packed-weights
-  // buffer's size, which callers know, has room for the block-diagonal
-  // weights in external order behind the packed ones (`weightExpandElems`
-  // elements), though the packing works them out as it goes.
+  // vertices that take several conv groups at once).
   unsigned convGroupsPerGroup = 1;
-  std::size_t weightExpandElems = 0;
   // A weight update pass planned for the layer with that many conv groups
   // taken as one (1: as it is): `params` are that fused layer's weight update
   // parameters, the pass forms the fused layer's weight deltas
@@ -141,7 +137,7 @@ struct mxconv_plan {
     return weightElems * params.inputType.size();
   }
   std::size_t weightPackedBytes() const {
-    return (weightPackedElems + weightExpandElems) * params.inputType.size();
+    return weightPackedElems * params.inputType.size();
   }
   std::size_t biasBytes() const { return biasElems * params.outputType.size(); }
 

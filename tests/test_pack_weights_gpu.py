@@ -60,3 +60,29 @@ def test_transpose_chans_flip(kw, dtype):
     axes = list(range(3, w.dim()))
     want = w.cpu().transpose(1, 2).flip(axes)
     assert torch.equal(out.cpu(), want)
+
+
+@pytest.mark.parametrize("gfx", [dict(smallTile=2), dict(patch=1),
+                                 dict(patch=2), dict(patch=0, blockN=64),
+                                 dict(patch=0, blockN=128, splitK=2)])
+@pytest.mark.parametrize("groups", [2, 8])
+def test_packed_weights_end_with_their_buffer(gfx, groups):
+    # groups taken as one: the buffer is the fused groups' packed weights and
+    # nothing behind them is written
+    import torch
+    from poplibs_amd import capi
+    p = make_params(pa.HALF, pa.HALF, batch=2, field=(14, 14), kernel=(3, 3),
+                    ci=64 // groups, co=24, groups=16, pad=1)
+    plan = pa.Plan(p, {"planConstraints": json.dumps(
+        {"convGroupsPerGroup": groups, "gfx950": dict(gfx, kernel="igemm")})})
+    assert "conv groups per group      %d" % groups in plan.describe()
+    n = plan.buffer_bytes(capi.BUF_WEIGHTS_PACKED)
+    fused = 16 // groups * (64 * 9) * (24 * groups) * 2
+    assert fused <= n <= fused * 8 // 3  # (channels to whole tiles)
+    w = torch.randn(16 * 24 * 64 // groups * 9, device="cuda").half()
+    packed = torch.full((n + 4096,), 0xa5, dtype=torch.uint8, device="cuda")
+    plan.pack_weights(w.data_ptr(), packed.data_ptr())
+    torch.cuda.synchronize()
+    assert bool((packed[n:] == 0xa5).all())
+    assert int((packed[:n].view(torch.int16) != 0).sum()) == w.numel() - int(
+        (w == 0).sum())
