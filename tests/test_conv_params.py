@@ -763,15 +763,14 @@ def test_planner_runs_small_conv_groups_as_one():
     assert per_group(forced(1), ci=4, co=4, groups=32) == 1
     assert per_group(forced(5), ci=4, co=4, groups=32) == 1
     assert per_group(forced(2), ci=32, co=32, groups=8) == 2
-    # room for the block-diagonal weights behind the packed ones
+    # the packed buffer: the fused groups' weights and nothing behind them
     p = make_params(pa.HALF, batch=4, field=(14, 14), kernel=(3, 3), ci=4,
                     co=4, groups=32, pad=1)
     plan, alone = pa.Plan(p), pa.Plan(p, forced(1))
     external = 32 * 4 * 4 * 9 * 2
     assert plan.buffer_bytes(pa.capi.BUF_WEIGHTS_EXTERNAL) == external
     packed = 2 * 64 * 576 * 2
-    assert plan.buffer_bytes(pa.capi.BUF_WEIGHTS_PACKED) == \
-        packed + 16 * external
+    assert plan.buffer_bytes(pa.capi.BUF_WEIGHTS_PACKED) == packed
     assert not plan.packs_like(alone)
 
 
