@@ -475,6 +475,18 @@ double estimateManySmall(const mxk::IgemmDesc &d, int inType) {
                                  (f.tile + f.wave * waves +
                                   f.step * steps * (1.0 + lookup))});
 }
+/// What the host's share of a call and the launch's start add to what
+/// estimateSmall and the others count from.
+constexpr double kCallOverKernelUs = 1.5;
+/// Whether estimateManySmall holds for a layer.
+bool manySmallTiles(mxk::IgemmDesc d, int inType) {
+  d.small = 1;
+  const std::uint64_t tiles = mxk::igemmSmallTileCount(d);
+  if (inType != mxk::kHalf)
+    return tiles > 3 * gfx950::numCUs;
+  return tiles > 8 * gfx950::numCUs &&
+         std::uint64_t(d.kH) * d.kW * d.inChansPerGroup * 2 <= 64 * 64;
+}
 /// ... and igemmKernel's on the same scale: one tile alone, or a CU's tiles one
 /// behind the other.  `ragged`: channels that fill no whole k-steps.
 struct ManyTiles {
@@ -1580,7 +1592,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
                                        double(plan.outputBytes()));
         }
         if (g.blockM == 256 || g.splitK > 1)
-          return plan.detailedEstimate().totalUs() + (g.splitK > 1 ? 1.5 : 0);
+          return plan.detailedEstimate().totalUs() +
+                 (g.splitK > 1 ? kCallOverKernelUs : 0.0);
         if (g.patch) {
           const double steps = double(s.kH * s.kW) * chanBytes / 128.0;
           const double perCU = std::ceil(pixels / g.blockM) *
@@ -1645,9 +1658,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
           if (us < best)
             best = us, tile = t;
         }
-        const std::uint64_t tiles16 = mxk::igemmSmallTileCount(asSmall(1));
-        if (halfIn ? tiles16 > 8 * gfx950::numCUs && k * eb <= 64 * 64
-                   : tiles16 > 3 * gfx950::numCUs) {
+        if (manySmallTiles(asSmall(1), inId)) {
           auto manyUs = [&](uint32_t t) {
             const mxk::IgemmDesc d = asSmall(t);
             if (t == 0)
@@ -1939,12 +1950,14 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
       break;
     }
     if (igemm.small) {
+      const int inId = params.inputType == poplar::FLOAT  ? mxk::kFloat
+                       : params.inputType == poplar::HALF ? mxk::kHalf
+                                                          : mxk::kQuarter;
       e.computeUs = std::max(
-          poplin::estimateSmall(igemm, params.inputType == poplar::FLOAT
-                                           ? mxk::kFloat
-                                       : params.inputType == poplar::HALF
-                                           ? mxk::kHalf
-                                           : mxk::kQuarter),
+          poplin::manySmallTiles(igemm, inId)
+              ? poplin::estimateManySmall(igemm, inId) -
+                    poplin::kCallOverKernelUs
+              : poplin::estimateSmall(igemm, inId),
           streamed(inputBytes() + outputBytes() + weightPackedBytes()));
       spread(e, mxk::igemmSmallTileCount(igemm), 1);
       break;
