@@ -321,15 +321,22 @@ __global__ __launch_bounds__(kWuThreads) void wuTapKernel(
 }
 
 /// deltas[g][co][ci][tap] = sum over the chunks in a fixed order.  Workgroup =
-/// 16 input x 4 output channels and all their taps (kWuSumSlots at most): 16
-/// lanes read a tile's 256 bytes, slot (tap, part) the chunks part, part +
-/// parts, ..., four loads in flight; the parts meet in LDS, whence runs of
-/// 16 input channels x taps leave in weight order.
+/// ciPer blocks of 16 input channels x 4 output channels and all their taps
+/// (kWuSumSlots slots at most): 16 lanes read a tile's 256 bytes, slot (block,
+/// tap, part) the chunks part, part + parts, ..., four loads in flight; the
+/// parts meet in LDS, whence runs of 16 ciPer input channels x taps leave in
+/// weight order.
 /// Bound by the tiles' bytes and one trip to memory and back: the 16.5 MB of
 /// N = 32, 28 x 28, 3 x 3, 128 -> 128 in 4.6 us.  (A lane per output vector
 /// wrote 2 bytes here and there: 5.2 us, and where the result is large, 1 x 1
 /// 64 -> 256 or 3 x 3 384 -> 264, 8.1 and 8.6 us against 4.8 and 5.6.)
+/// Large results of few taps and chunks make thousands of small workgroups,
+/// whose turnover then sets the pace: as many blocks to a workgroup as leave
+/// 2 048 of them (1 024 -> 2 048 channels, 1 x 1, two chunks, 32 768 workgroups
+/// of a wave each, the pass 32.4 -> 21.2 us; 512 -> 2 048, 7 x 7, 23.1 -> 18.8; a
+/// limit of 512, 1 024 or 4 096 is within 3 % over 17 layers).
 constexpr uint32_t kWuSumSlots = 64, kWuSumParts = 32;
+constexpr uint32_t kWuSumWorkgroups = 2048;
 
 struct WuSumArgs {
   uint32_t groups, chunks, taps;
@@ -338,7 +345,8 @@ struct WuSumArgs {
   uint32_t tapsHere;             // of a workgroup
   uint32_t parts;                // slots that share a tap
   uint32_t ciBlocks, coQuads;
-  FastDiv divParts, divCoQuads, divCiBlocks, divTaps, divRun;
+  uint32_t ciPer, ciGroups;      // blocks of a workgroup, groups of them
+  FastDiv divParts, divCoQuads, divCiGroups, divTaps, divRun;
 };
 
 template <class OutT>
@@ -348,14 +356,17 @@ __global__ __launch_bounds__(1024) void wuTapSumKernel(
   __shared__ floatx4 sums[kWuSumSlots * 16];
   uint32_t id = blockIdx.x, q = a.divCoQuads(id);
   const uint32_t coQuad = id - q * a.coQuads;
-  id = q, q = a.divCiBlocks(id);
-  const uint32_t ciBlock = id - q * a.ciBlocks, g = q;
+  id = q, q = a.divCiGroups(id);
+  const uint32_t ciBlock0 = (id - q * a.ciGroups) * a.ciPer, g = q;
   const uint32_t tap0 = blockIdx.y * a.tapsHere;
   const uint32_t left = a.taps - tap0;
   const uint32_t taps = left < a.tapsHere ? left : a.tapsHere;
   const uint32_t slot = threadIdx.x >> 4;
-  const uint32_t tapHere = a.divParts(slot), part = slot - tapHere * a.parts;
-  if (tapHere < taps) {
+  const uint32_t sum = a.divParts(slot), part = slot - sum * a.parts;
+  const uint32_t blockHere = a.divTaps(sum);
+  const uint32_t tapHere = sum - blockHere * a.tapsHere;
+  const uint32_t ciBlock = ciBlock0 + blockHere;
+  if (blockHere < a.ciPer && ciBlock < a.ciBlocks && tapHere < taps) {
     const size_t tile = 128 * 128 / 4; // (in vectors)
     const size_t stride =
         size_t(a.groups) * a.taps * a.ciTiles * a.coTiles * tile;
@@ -369,32 +380,33 @@ __global__ __launch_bounds__(1024) void wuTapSumKernel(
          coQuad % 16 / 4 * 4 + ciBlock % 4) *
             64 +
         coQuad % 4 * 16 + (threadIdx.x & 15);
-    floatx4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    floatx4 total = {0.0f, 0.0f, 0.0f, 0.0f};
     uint32_t p = part;
     for (; p + 3 * a.parts < a.chunks; p += 4 * a.parts) {
       const floatx4 v0 = src[p * stride];
       const floatx4 v1 = src[(p + a.parts) * stride];
       const floatx4 v2 = src[(p + 2 * a.parts) * stride];
       const floatx4 v3 = src[(p + 3 * a.parts) * stride];
-      sum += (v0 + v1) + (v2 + v3);
+      total += (v0 + v1) + (v2 + v3);
     }
     for (; p < a.chunks; p += a.parts)
-      sum += src[p * stride];
-    sums[threadIdx.x] = sum;
+      total += src[p * stride];
+    sums[threadIdx.x] = total;
   }
   __syncthreads();
-  // element e of the workgroup's 4 x 16 x taps results, taps fastest
+  // element e of the workgroup's 4 x 16 ciPer x taps results, taps fastest
   const float *flat = reinterpret_cast<const float *>(sums);
-  const uint32_t run = 16 * a.tapsHere;
+  const uint32_t run = 16 * a.ciPer * a.tapsHere;
   for (uint32_t e = threadIdx.x; e < 4 * run; e += blockDim.x) {
     const uint32_t c = a.divRun(e), inRun = e - c * run;
     const uint32_t i = a.divTaps(inRun), tap = inRun - i * a.tapsHere;
-    const uint32_t co = coQuad * 4 + c, ci = ciBlock * 16 + i;
+    const uint32_t co = coQuad * 4 + c, ci = ciBlock0 * 16 + i;
     if (tap >= taps || ci >= a.ci || co >= a.co)
       continue;
     float v = 0.0f;
+    const uint32_t first = ((i >> 4) * a.tapsHere + tap) * a.parts;
     for (uint32_t p = 0; p != a.parts; ++p)
-      v += flat[((tap * a.parts + p) * 16 + i) * 4 + c];
+      v += flat[((first + p) * 16 + (i & 15)) * 4 + c];
     storeOut(out, ((size_t(g) * a.co + co) * a.ci + ci) * a.taps + tap0 + tap,
              v);
   }
@@ -521,12 +533,18 @@ hipError_t launchWuTap(const WuTapDesc &d, int outType, const void *acts,
   r.ciBlocks = (r.ci + 15) / 16, r.coQuads = (r.co + 3) / 4;
   r.divParts = makeFastDiv(r.parts);
   r.divCoQuads = makeFastDiv(r.coQuads);
-  r.divCiBlocks = makeFastDiv(r.ciBlocks);
+  const uint32_t tapBlocks = (a.taps + r.tapsHere - 1) / r.tapsHere;
+  const uint64_t single =
+      uint64_t(d.groups) * r.ciBlocks * r.coQuads * tapBlocks;
+  r.ciPer = uint32_t(std::min<uint64_t>(
+      {kWuSumSlots / (r.tapsHere * r.parts), r.ciBlocks,
+       std::max<uint64_t>(1, single / kWuSumWorkgroups)}));
+  r.ciGroups = (r.ciBlocks + r.ciPer - 1) / r.ciPer;
+  r.divCiGroups = makeFastDiv(r.ciGroups);
   r.divTaps = makeFastDiv(r.tapsHere);
-  r.divRun = makeFastDiv(16 * r.tapsHere);
-  const dim3 sumGrid(d.groups * r.ciBlocks * r.coQuads,
-                     (a.taps + r.tapsHere - 1) / r.tapsHere);
-  const dim3 sumBlock((r.tapsHere * r.parts * 16 + 63) / 64 * 64);
+  r.divRun = makeFastDiv(16 * r.ciPer * r.tapsHere);
+  const dim3 sumGrid(d.groups * r.ciGroups * r.coQuads, tapBlocks);
+  const dim3 sumBlock((r.ciPer * r.tapsHere * r.parts * 16 + 63) / 64 * 64);
   if (outType == kHalf)
     hipLaunchKernelGGL(wuTapSumKernel<__half>, sumGrid, sumBlock, 0, stream,
                        static_cast<const float *>(workspace),

@@ -437,6 +437,32 @@ def test_weight_deltas_of_few_pixels(oracle, kw, deltas):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("out_type", [pa.FLOAT, pa.HALF])
+@pytest.mark.parametrize("kw", [
+    # more results than 2048 workgroups of 16 x 4: two blocks of input channels
+    # to one, an odd count of them; seven, the last workgroup with six, in two
+    # chunks; two with all nine taps; ragged channels at the end of a block
+    dict(batch=3, field=(5, 7), kernel=(1, 1), ci=1040, co=260),
+    dict(batch=2, field=(20, 15), kernel=(1, 1), ci=984, co=1030),
+    dict(batch=1, field=(6, 6), kernel=(3, 3), ci=512, co=512, pad=1),
+    dict(batch=1, field=(4, 9), kernel=(2, 1), ci=773, co=347),
+])
+def test_weight_deltas_of_many_channels(oracle, kw, out_type):
+    p = make_params(pa.HALF, out_type, **kw)
+    rng = np.random.default_rng(66)
+    # (sums of at most 600 signs: exact in half too)
+    x = rng.choice([-1.0, 1.0],
+                   (p.batchSize, p.getNumInputChans(), *p.inputFieldShape))
+    dz = rng.choice([-1.0, 1.0], (p.batchSize, p.getNumOutputChans(),
+                                  *p.getOutputFieldShape()))
+    got, plan = run_weight_update(p, x.astype(np.float16),
+                                  dz.astype(np.float16), FORCE_DENSE_WU)
+    assert DENSE_WU in plan.describe()
+    np.testing.assert_array_equal(got, oracle.weight_deltas(p, x, dz,
+                                                            threads=8))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("width", [192, 256])
 @pytest.mark.parametrize("batch", [8, 3])
 def test_weight_deltas_by_a_named_tile_of_256_pixels(oracle, batch, width):
