@@ -57,6 +57,18 @@ def test_a_named_tile_the_kernel_cannot_run_is_refused_by_the_plan(kw):
         pa.Plan(make_params(H, **kw), WIDE)
 
 
+@pytest.mark.parametrize("kw", [
+    # a short K under large outputs: us in 256-pixel and in 128-pixel tiles
+    dict(batch=15, field=(57, 57), kernel=(1, 1), ci=192, co=960),  # 51.1 36.4
+    dict(batch=114, field=(38, 38), kernel=(1, 1), ci=144, co=960,
+         stride=2),                                                 # 45.8 35.1
+    dict(batch=32, field=(56, 56), kernel=(1, 1), ci=256, co=512,
+         stride=2),                                                 # 17.4 15.8
+])
+def test_a_short_sum_keeps_narrow_tiles(kw):
+    assert _tile(pa.Plan(make_params(H, **kw))) == "128 x 128 x 64"
+
+
 def test_products_that_fill_the_chip_keep_it():
     plan = pa.MatMulPlan(H, H, 1, 4096, 4096, 4096)
     assert _tile(plan) == "256 x 256 x 64"
