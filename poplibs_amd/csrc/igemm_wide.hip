@@ -18,14 +18,14 @@
 // Workgroups are dealt to an XCD in blocks of 4 M tiles, whose input rows and
 // weights its L2 then fetches once for all of them.
 //
-// Measured, fp16: 4096 x 4096 x 4096 138 -> 120 us (1.14 PFLOP/s; the 128 x 128
-// tile before), 4096 x 1024 x 4096 47 -> 38, N = 64, 56 x 56, 3 x 3 stride 2,
-// 256 -> 512 157 -> 122, and N = 71, 35 x 35, 3 x 3, 624 -> 136 in tiles of 192
-// channels 257 -> 223.  What bounds it is the chip's power: the matrix pipe is
-// busy 57 % of the cycles, but with the loads taken out of the loop the clock
-// rises with every cycle saved, and priorities that save 6 % of the cycles
-// lower the clock by as much.  Tiles of 256 x 128 gained nothing over 128 x
-// 128 ones with two workgroups to a CU.
+// Measured, fp16, us, tiles of 128 x 128 (two to a CU) and these in turn: 4096 x
+// 4096 x 4096 133.0 -> 118.6 (1.16 PFLOP/s), 8192 x 8192 x 8192 1263 -> 866
+// (1.27), N = 64, 56 x 56, 3 x 3 stride 2, 256 -> 512 137 -> 124, and N = 71,
+// 35 x 35, 3 x 3, 624 -> 136 in tiles of 192 channels 258 -> 213.  What bounds
+// it: in 4096 x 4096 x 4096 the matrix pipe is busy 64 % of the chip's cycles,
+// at a clock of 1.71 GHz where the chip goes to 2.4 - its power limit, under
+// which a loop of nothing but MFMAs holds 1.97.  Tiles of 256 x 128 gained
+// nothing over 128 x 128 ones with two workgroups to a CU.
 #include "igemm_common.hpp"
 
 namespace mxk {

@@ -333,9 +333,9 @@ double streamingPowerUs(std::size_t workgroups, std::size_t kSteps,
 
 /// igemmWideKernel: 10 us per round around the loop (256 x 256 outputs leave
 /// at its end), 1.3 us per k-step of a workgroup, and where all CUs are busy
-/// 1.7 us - the chip's power (4096 x 4096 x 4096 120 us, 4096 x 1024 x 4096
-/// 38, 2048 x 4096 x 4096 on half the CUs 84, N = 64, 56 x 56, 3 x 3 stride 2,
-/// 256 -> 512 in 392 tiles 122); four fifths of it for tiles of 192 channels.
+/// 1.7 us - the chip's power (4096 x 4096 x 4096 119 us, 4096 x 1024 x 4096
+/// 38, 2048 x 4096 x 4096 on half the CUs 90, N = 64, 56 x 56, 3 x 3 stride 2,
+/// 256 -> 512 in 392 tiles 124); four fifths of it for tiles of 192 channels.
 double estimateWide(std::size_t workgroups, std::size_t kSteps,
                     unsigned blockN) {
   const double rounds = roundsOf(workgroups, 1);
