@@ -478,11 +478,16 @@ struct WuTapDesc {
   // the result's channels, where ci and co are those filled up to whole
   // vectors (0: the same)
   uint32_t resultCi = 0, resultCo = 0;
+  // wuWindowKernel's tile of output x input channels (32 or 64 each; 0: it is
+  // not that kernel's) and the k-steps of 32 columns a workgroup sums over
+  uint32_t windowCo = 0, windowCi = 0, windowSteps = 0;
 };
 bool wuTapTakes(const WuTapDesc &d);
 /// Pixels per workgroup that give about one workgroup per compute unit.
 uint32_t wuTapChunkPixels(const WuTapDesc &d, uint32_t computeUnits);
 uint64_t wuTapWorkspaceBytes(const WuTapDesc &d);
+/// Estimated microseconds of the pass, both launches.
+double wuTapEstimateUs(const WuTapDesc &d, uint32_t computeUnits);
 /// weightDeltas [groups][co][ci][kH][kW] in outType (half or float) from acts
 /// [batch][inH][inW][groups][ci] and deltas [batch][outH][outW][groups][co],
 /// both fp16; fp32 partial tiles of the pixel chunks go through `workspace`
@@ -490,6 +495,19 @@ uint64_t wuTapWorkspaceBytes(const WuTapDesc &d);
 hipError_t launchWuTap(const WuTapDesc &d, int outType, const void *acts,
                        const void *deltas, void *workspace, void *out,
                        hipStream_t stream);
+
+/// The same by wuWindowKernel: kernels of one or three columns, strides of one
+/// or two along a row, channels in whole words of two, groups of any width.
+bool wuWindowTakes(const WuTapDesc &d);
+/// Sets the tile and the chunks that are estimated to be the fastest (and
+/// flattens the field of a 1 x 1 kernel); the estimate in microseconds, or a
+/// very large number where the kernel does not take the layer.
+double wuWindowChoose(WuTapDesc &d, uint32_t computeUnits);
+uint64_t wuWindowWorkspaceBytes(const WuTapDesc &d);
+uint64_t wuWindowWorkgroups(const WuTapDesc &d);
+hipError_t launchWuWindow(const WuTapDesc &d, int outType, const void *acts,
+                          const void *deltas, void *workspace, void *out,
+                          hipStream_t stream);
 
 /// Gradient with respect to the weights of the depthwise FORWARD convolution
 /// `d` (undilated input): weightDeltas [channels][kH * kW] in outType from

@@ -1408,7 +1408,7 @@ WuWorkspace wuWorkspace(const mxconv_plan *plan) {
   };
   // (groups taken as one: the fused layer's deltas, whose diagonal blocks
   // are the result)
-  if (plan->wuGroupsPerGroup > 1)
+  if (plan->wuGroupsPerGroup > 1 && !plan->wuOwnGroups)
     w.fusedDeltas = take(plan->outputBytes());
   if (plan->depthwiseWeightUpdate) {
     // the depthwise weight-delta kernel reads the layer's tensors as they
@@ -1426,7 +1426,8 @@ WuWorkspace wuWorkspace(const mxconv_plan *plan) {
     if (f.resultCo && f.resultCo != f.co)
       w.weightsExternal =
           take(size_t(f.batch) * f.outH * f.outW * f.groups * f.co * 2);
-    w.planWorkspace = take(mxk::wuTapWorkspaceBytes(f));
+    w.planWorkspace = take(f.windowCo ? mxk::wuWindowWorkspaceBytes(f)
+                                      : mxk::wuTapWorkspaceBytes(f));
     w.deltas = take(wuResultBytes(plan));
     w.total = at;
     return w;
@@ -1471,7 +1472,7 @@ mxconv_status weightDeltas(const mxconv_plan *plan, const void *zDeltas,
                            const void *acts, void *deltasOut, char *ws,
                            mxconv_stream stream) {
   const unsigned f = plan->wuGroupsPerGroup;
-  if (f == 1)
+  if (f == 1 || plan->wuOwnGroups)
     return fusedWeightDeltas(plan, zDeltas, acts, deltasOut, ws, stream);
   // Planned for the layer with f groups taken as one: that layer's deltas
   // into the workspace, their diagonal blocks out.
@@ -1538,8 +1539,9 @@ mxconv_status fusedWeightDeltas(const mxconv_plan *plan, const void *zDeltas,
                 uint64_t(f.batch) * f.outH * f.outW, f.resultCo, f.co);
     if (st != MXCONV_OK)
       return st;
-    return hipStatus(mxk::launchWuTap(f, p.outputType.id(), acts, zDeltas,
-                                      ws + w.planWorkspace, deltasOut, s),
+    const auto launch = f.windowCo ? &mxk::launchWuWindow : &mxk::launchWuTap;
+    return hipStatus(launch(f, p.outputType.id(), acts, zDeltas,
+                            ws + w.planWorkspace, deltasOut, s),
                      "matrix-core weight deltas");
   }
   if (const mxconv_plan *product = plan->weightUpdateProduct.get()) {

@@ -226,6 +226,11 @@ void checkGfx950(const std::string &path, const Value &v, PlanConstraints &pc) {
       if (v > 2)
         throw invalid_option("'" + sub + "': Must be 0, 1 or 2");
       pc.weightDeltas = int(v);
+    } else if (m.first == "deltaWindow") {
+      const unsigned v = requireUnsigned(sub, m.second);
+      if (v > 1)
+        throw invalid_option("'" + sub + "': Must be 0 or 1");
+      pc.deltaWindow = int(v);
     } else if (m.first == "chanTiles") {
       pc.chanTiles = requireUnsigned(sub, m.second);
       if (pc.chanTiles < 1 || pc.chanTiles > 4)

@@ -74,6 +74,11 @@ struct PlanConstraints {
   /// as one matrix product on the transposed deltas (a layer without spatial
   /// extent; an error for any other).
   int weightDeltas = -1;
+  /// ... of the two kernels that read a dense layer's own tensors, the one that
+  /// gathers pixels in registers (wuWindowKernel; 1: an error where it does not
+  /// take the layer) or the one of transposing LDS reads (0); -1 planner's
+  /// choice, which is 0 where weightDeltas is 1.
+  int deltaWindow = -1;
   std::string text; // the JSON as given, kept for reporting and cache keys
 };
 

@@ -604,6 +604,63 @@ mxconv_plan makePlanWith(const ConvParams &params,
                          const ConvOptions &optionsIn,
                          unsigned convGroupsPerGroup);
 
+/// The weight deltas of `layer` (channels of a group as the layer has them, in
+/// resultCi and resultCo) by wuWindowKernel, where that is named or estimated
+/// to be faster than what `plan` has; `fuse`: groups that plan takes as one.
+/// Of 4 500 random layers that both kernels take, the estimates' choice was
+/// 0.6 % slower than the faster of the two on average and 20 % faster than
+/// wuTapKernel for all.  The line at 0.93: wide layers (128 -> 128 channels, 28 x
+/// 28, 3 x 3, 32 images: 20.5 us by taps, 21.3 by windows) are estimated that
+/// much too slow by taps.
+void windowWeightDeltas(mxconv_plan &plan, const mxk::WuTapDesc &layer,
+                        unsigned fuse) {
+  const auto &pc = plan.options.planConstraints;
+  const int asked = pc.deltaWindow;
+  if (asked == 0 || pc.weightDeltas == 0 ||
+      (pc.weightDeltas == 1 && asked != 1))
+    return;
+  mxk::WuTapDesc w = layer;
+  w.chunkPixels = 64;
+  w.ci = w.resultCi, w.co = w.resultCo;
+  double us = mxk::wuWindowChoose(w, gfx950::numCUs);
+  if (!w.windowCo) {
+    // (channels filled up to whole vectors, in copies, as wuTapKernel's are)
+    w = layer;
+    w.chunkPixels = 64;
+    w.ci = (w.resultCi + 7) / 8 * 8, w.co = (w.resultCo + 7) / 8 * 8;
+    us = mxk::wuWindowChoose(w, gfx950::numCUs);
+    if (!w.windowCo)
+      return;
+  }
+  auto copiesUs = [](const mxk::WuTapDesc &d) {
+    double sum = 0.0;
+    if (d.resultCi != d.ci)
+      sum += 2.6 + double(d.batch) * d.inH * d.inW * d.groups * d.ci * 0.8e-6;
+    if (d.resultCo != d.co)
+      sum += 2.6 + double(d.batch) * d.outH * d.outW * d.groups * d.co * 0.8e-6;
+    return sum;
+  };
+  us += copiesUs(w);
+  if (asked != 1 && plan.denseWeightUpdate) {
+    double otherUs;
+    if (plan.denseForward.windowCo) {
+      otherUs = plan.windowUs;
+    } else {
+      otherUs = mxk::wuTapEstimateUs(plan.denseForward, gfx950::numCUs) +
+                copiesUs(plan.denseForward);
+    }
+    // (the diagonal blocks of groups taken as one are a launch of their own)
+    if (fuse > 1)
+      otherUs += 2.2;
+    if (us >= 0.93 * otherUs)
+      return;
+  }
+  plan.denseWeightUpdate = true;
+  plan.denseForward = w;
+  plan.windowUs = us;
+  plan.wuOwnGroups = fuse > 1;
+}
+
 /// A weight update pass of fewer than 1024 pixels that was planned for
 /// wuTapKernel: back to the pass's own convolution where that is estimated to
 /// be faster.  Fitted to 2472 random layers of 1 to 64 images, kernels of up to
@@ -622,7 +679,8 @@ void settleFewPixelWeightDeltas(mxconv_plan &plan) {
   const mxk::WuTapDesc &f = plan.denseForward;
   const std::size_t pixels = std::size_t(f.batch) * f.outH * f.outW;
   if (!plan.denseWeightUpdate || pixels >= 1024 ||
-      plan.options.planConstraints.weightDeltas == 1)
+      plan.options.planConstraints.weightDeltas == 1 ||
+      plan.options.planConstraints.deltaWindow == 1)
     return;
   plan.denseWeightUpdate = false;
   const mxconv_plan::DetailedEstimate e = plan.detailedEstimate();
@@ -638,6 +696,7 @@ void settleFewPixelWeightDeltas(mxconv_plan &plan) {
   const double steps = std::ceil(
       double(std::min<std::size_t>(f.chunkPixels, pixels)) / 64.0);
   const double kernelUs =
+      f.windowCo ? plan.windowUs :
       std::max(8.9, 6.8 + rounds * (0.6 + 0.52 * steps) +
                         0.12e-6 * partialBytes + 1.5 * resultMB +
                         (fused ? 2.2 + 0.17 * resultMB : 0.0));
@@ -649,6 +708,7 @@ void settleFewPixelWeightDeltas(mxconv_plan &plan) {
           : std::max(20.0, 11.7 + 1.3 * e.totalUs() + 2.5 * tensorsMB +
                                blocksUs);
   plan.denseWeightUpdate = !e.known || kernelUs <= convolutionUs;
+  plan.wuOwnGroups = plan.wuOwnGroups && plan.denseWeightUpdate;
 }
 
 } // namespace
@@ -664,6 +724,14 @@ mxconv_plan makePlan(const ConvParams &params, const ConvOptions &optionsIn) {
     fused.outputChannelsPerConvGroup *= fuse;
     mxconv_plan plan = makePlanWith(fused, optionsIn, 1);
     plan.wuGroupsPerGroup = fuse;
+    if (plan.wuOwnTensors) {
+      // (wuWindowKernel takes the layer's own groups, as many to a tile as
+      // have room in it)
+      mxk::WuTapDesc own = plan.wuLayer;
+      own.groups *= fuse;
+      own.resultCi /= fuse, own.resultCo /= fuse;
+      windowWeightDeltas(plan, own, fuse);
+    }
     settleFewPixelWeightDeltas(plan);
     return plan;
   }
@@ -804,6 +872,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
       f.ci = (f.resultCi + 7) / 8 * 8;
       f.co = (f.resultCo + 7) / 8 * 8;
       f.chunkPixels = mxk::wuTapChunkPixels(f, gfx950::numCUs);
+      plan.wuOwnTensors = true;
+      plan.wuLayer = f;
       // Of 1024 pixels or more: 16 channels and more and, in a grouped layer,
       // a quarter of the kernel's 128 x 128 tile per (group, tap): every group
       // brings its own tiles, and poorly filled ones lose to the pass's own
@@ -821,6 +891,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
       const bool worth = std::size_t(f.batch) * f.outH * f.outW < 1024 ||
                          (f.resultCi >= 16 && f.resultCo >= 16 && filled);
       plan.denseWeightUpdate = (asked == 1 || worth) && mxk::wuTapTakes(f);
+      // ... or by the kernel that gathers pixels in registers
+      windowWeightDeltas(plan, f, 1);
     }
     if (asked == 1 && isWeightUpdatePass(options.pass) &&
         !plan.denseWeightUpdate && !plan.depthwiseWeightUpdate)
@@ -828,6 +900,13 @@ mxconv_plan makePlanWith(const ConvParams &params,
           "planConstraints gfx950 weightDeltas: no weight-delta kernel takes "
           "this layer's own tensors (half inputs, nothing dilated, truncated, "
           "padded or flipped on the kernel side)");
+    if (options.planConstraints.deltaWindow == 1 &&
+        isWeightUpdatePass(options.pass) &&
+        !(plan.denseWeightUpdate && plan.denseForward.windowCo))
+      throw poplar::invalid_option(
+          "planConstraints gfx950 deltaWindow: that kernel takes weightDeltas "
+          "1 of half layers whose kernel has one or three columns and whose "
+          "stride along a row is one or two");
   }
   const auto &pc = options.planConstraints;
   if (convGroupsPerGroup > 1) {
@@ -1876,6 +1955,8 @@ std::string mxconv_plan::constraintsJson() const {
        << (weightUpdateProduct                           ? 2
            : denseWeightUpdate || depthwiseWeightUpdate ? 1
                                                         : 0);
+    if (denseWeightUpdate)
+      os << ", \"deltaWindow\": " << (denseForward.windowCo ? 1 : 0);
     if (depthwiseWeightUpdate && kernel != Kernel::DEPTHWISE)
       os << ", \"rowRing\": " << (depthwiseForward.dense3x3 == 2 ? 1 : 0);
   }
@@ -1936,6 +2017,17 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
       if (f.resultCo != f.co)
         e.rearrangementBytes += m * f.outH * f.outW * f.co * 2;
       e.rearrangementUs += streamed(2 * e.rearrangementBytes);
+    }
+    if (f.windowCo) {
+      e.reductionBytes = mxk::wuWindowWorkspaceBytes(f);
+      e.reductionUs =
+          e.reductionBytes
+              ? std::min(windowUs / 2, 2.7 + streamed(e.reductionBytes))
+              : 0.0;
+      e.computeUs =
+          std::max(0.0, windowUs - e.reductionUs - e.rearrangementUs);
+      spread(e, mxk::wuWindowWorkgroups(f), 1);
+      return e;
     }
     e.reductionBytes = mxk::wuTapWorkspaceBytes(f);
     e.reductionUs = std::min(all / 2, streamed(e.reductionBytes));
@@ -2295,7 +2387,29 @@ std::string mxconv_plan::describe() const {
     }
     os << "\n";
   }
-  if (denseWeightUpdate) {
+  if (denseWeightUpdate && denseForward.windowCo) {
+    const auto &f = denseForward;
+    // (groups that leave most of a 128 x 128 tile empty: what the kernel of
+    // such tiles is not for)
+    const bool narrow = f.groups > 1 && std::size_t(f.ci) * f.co * 4 <=
+                                            std::size_t((f.ci + 127) / 128) *
+                                                ((f.co + 127) / 128) * 16384;
+    os << "        as a weight update pass    "
+       << (narrow ? "kernel of narrow groups" : "matrix-core weight-delta kernel")
+       << " on the layer's own tensors (pixels gathered in registers): tiles "
+          "of "
+       << f.windowCo << " output x " << f.windowCi
+       << " input channels and a kernel row, chunks of " << f.windowSteps
+       << " k-steps of 32 columns = " << mxk::wuWindowWorkgroups(f)
+       << " workgroups"
+       << (mxk::wuWindowWorkspaceBytes(f) ? ", fp32 partial sums added in order"
+                                          : ", the result written at once");
+    if (f.resultCi != f.ci)
+      os << "; input channels padded " << f.resultCi << " -> " << f.ci;
+    if (f.resultCo != f.co)
+      os << "; output channels padded " << f.resultCo << " -> " << f.co;
+    os << "\n";
+  } else if (denseWeightUpdate) {
     const auto &f = denseForward;
     const std::size_t m = std::size_t(f.batch) * f.outH * f.outW;
     const std::size_t chunks = (m + f.chunkPixels - 1) / f.chunkPixels;

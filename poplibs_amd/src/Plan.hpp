@@ -72,9 +72,15 @@ struct mxconv_plan {
   bool depthwiseWeightUpdate = false;
   mxk::DepthwiseDesc depthwiseForward{};
   // ... or of a dense layer (any stride): the matrix-core kernel that reads
-  // the layer's tensors as they are (mxk::launchWuTap).
+  // the layer's tensors as they are (mxk::launchWuTap, or mxk::launchWuWindow
+  // where denseForward.windowCo is set, in an estimated windowUs).
   bool denseWeightUpdate = false;
   mxk::WuTapDesc denseForward{};
+  double windowUs = 0.0;
+  // The layer as those kernels would take it, whether they do or not; and
+  // that denseForward is the layer's own groups, not those taken as one.
+  bool wuOwnTensors = false, wuOwnGroups = false;
+  mxk::WuTapDesc wuLayer{};
 
   // Packed weights of the matrix-core kernel: [G][coPadded][kPadded].
   std::size_t coPadded = 0, kPadded = 0;
