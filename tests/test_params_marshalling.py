@@ -1,0 +1,61 @@
+"""The short ways of a call made on every training step: parameters of two
+field dimensions marshalled as one record, and weightsTransposeChansFlipXY's
+check of parameters without building the class."""
+from ctypes import byref
+
+import numpy as np
+import pytest
+
+import poplibs_amd as pa
+from poplibs_amd.capi import Status
+
+
+def _random_params(rng):
+    n = int(rng.integers(0, 4))
+
+    def ints(lo, hi):
+        return [int(v) for v in rng.integers(lo, hi, n)]
+
+    p = pa.ConvParams(pa.HALF, pa.FLOAT, 2, ints(0, 9), ints(0, 5), 3, 4, 2)
+    for t in (p.inputTransform, p.kernelTransform):
+        t.truncationLower = ints(0, 2) if rng.random() < .3 else [0] * n
+        t.truncationUpper = ints(0, 2) if rng.random() < .3 else [0] * n
+        t.dilation = ints(0, 4) if rng.random() < .3 else [1] * n
+        t.paddingLower, t.paddingUpper = ints(0, 3), ints(0, 3)
+        t.flip = [bool(v) for v in ints(0, 2)]
+    o = p.outputTransform
+    o.truncationLower = ints(0, 3) if rng.random() < .3 else [0] * n
+    o.truncationUpper = ints(0, 2) if rng.random() < .3 else [0] * n
+    o.stride = ints(0, 4) if rng.random() < .3 else [1] * n
+    o.paddingLower, o.paddingUpper = ints(0, 3), ints(0, 2)
+    return p
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_records_and_checks_agree_with_the_long_way(seed):
+    rng = np.random.default_rng(seed)
+    L = pa.lib()
+    seen = set()
+    for _ in range(500):
+        p = _random_params(rng)
+        c = p.to_c()
+        assert bytes(c) == bytes(p._to_c_by_field(len(p.inputFieldShape)))
+        valid = L.mxconv_params_validate(byref(c))
+        got = L.mxconv_weights_transpose_chans_flip_xy(byref(c), None, None,
+                                                       None)
+        empty = 0 in p.kernelShape
+        seen.add(valid)
+        # (valid ones go on to ask for the tensors, unless there is nothing
+        # to do)
+        assert got == (valid if valid != Status.OK else
+                       Status.OK if empty else Status.NULL_ARGUMENT), p
+    assert len(seen) == 2
+
+
+def test_lists_of_other_lengths_are_refused():
+    for change in ("stride", "paddingUpper"):
+        p = pa.ConvParams(pa.HALF, pa.HALF, 1, [4, 4], [3, 3], 8, 8)
+        getattr(p.outputTransform, change).append(1)
+        p.outputTransform.truncationLower.pop()
+        with pytest.raises(pa.MxconvError):
+            p.to_c()
