@@ -961,8 +961,15 @@ hipError_t launchIgemm(const IgemmDesc &d, int inType, int outType,
                          stream});
   if (e != hipSuccess)
     return e;
+  return launchSplitKSum(d, outType, workspace, bias, out, stream);
+}
+
+hipError_t launchSplitKSum(const IgemmDesc &d, int outType,
+                           const void *workspace, const void *bias, void *out,
+                           hipStream_t stream) {
   const uint32_t channels = d.groups * d.outChansPerGroup;
-  const uint64_t elems = uint64_t(a.M) * channels;
+  const uint64_t elems =
+      uint64_t(d.batch) * d.outD * d.outH * d.outW * channels;
   if (elems == 0)
     return hipSuccess;
   if ((elems + 63) / 64 > 0x7fffffffull)

@@ -1,6 +1,5 @@
 // Implicit-GEMM forward convolution with the input patch of a tile resident
-// in LDS: the kernel for unit-stride layers whose channels come in whole
-// 128-byte slices (a ResNet-style 3x3 layer).
+// in LDS: the kernel for unit-stride layers (a ResNet-style 3x3 layer).
 //
 // Same GEMM view as igemm.hip (M = output pixels, N = output channels,
 // K = taps x input channels), different data path.  A kernel of kH x kW taps
@@ -32,6 +31,18 @@
 // left and right; the pitch of the rows continues the pixels' progression
 // through the banks (modulo 256 bytes).  Patch rows are the rows, padding
 // rows included, of consecutive images that the tile's pixels read.
+//
+// Channels come in slices of 128 bytes; the last may be a partial one, whose
+// missing chunks are loaded as zeros (packed weights hold zeros there too).  A
+// long K is cut along its slices into parts, one workgroup each, their fp32
+// tiles summed by splitKReduceKernel; a part with more slices than the LDS has
+// room for passes them through a ring.  Against the streaming kernel, which
+// works out a tap per lane where a k-step is no whole slice, us: fp16, 3 x 3, 28
+// x 28, 32 images, 96 -> 128 12.5 -> 9.1, 184 -> 128 18.5 -> 12.2; 33 of 13 x
+// 13, 552 -> 160 (ring, two parts) 30.8 -> 23.0; 32 of 7 x 7, 512 -> 512 (four
+// parts) 19.7 -> 15.0; fp8, 49 of 38 x 38, 400 -> 96 57 -> 42.  Over 3 800 random
+// layers of 0.2 to 40 GFLOP what the planner picks takes 0.81 of the streaming
+// kernel's time.
 //
 // Takes the role of PopLibs' AMP vertex ConvPartialnx1
 // (lib/poplin/codelets/ConvPartialnx1.cpp:52-246) for these shapes; the fp8
@@ -95,7 +106,7 @@ struct PatchArgs {
   uint32_t inH;
   int32_t padH, padW;
   uint32_t loH, spanH, loW, spanW;
-  uint32_t kW, taps, slices, kSteps;
+  uint32_t kW, taps, slices, kSteps; // of the whole of K
   uint32_t tapRowBytes, tapColBytes; // LDS bytes per kernel row / column
   uint32_t rowLoads;   // wave loads (1 KB, the last one partial) per patch row
   uint32_t rowUnits;   // units of a patch row
@@ -108,6 +119,11 @@ struct PatchArgs {
   uint32_t wBytes;
   FastDiv divOutW, divOutH, divNTiles, divMTiles, divRowLoads, divRowsPerImage;
   FastDiv divTaps, divKW;
+  // K cut along its slices into parts, one workgroup each; slices in LDS at a
+  // time (a later one takes the place of one that all waves are through with).
+  // (Last, out of the way of what the other kernels fetch.)
+  uint32_t slicesPart, ring;
+  FastDiv divGroups, divRing;
 };
 
 /// LDS the reduction of the two K halves and the output tile need.
@@ -148,25 +164,20 @@ __device__ __forceinline__ uint32_t patchByteOf(const PatchArgs &a,
          ow * (16 * UNITS);
 }
 
-/// Loads the patch of a tile, all waves together.  Column blocks of all
-/// slices, slice 0 first, are dealt out to the waves in turn.  Slice 0 is what
-/// the k loop waits for: its loads go out before anything else, then
-/// `between()` runs (the first weight loads - WEIGHT_LOADS of them per wave -
-/// and address arithmetic, which fill the wait), then the wave waits for its
-/// part of slice 0 and meets the others at a barrier; the later slices' loads
-/// follow and are waited for inside the k loop.
-template <int WEIGHT_LOADS, int UNITS, class Between, class Behind>
-__device__ __forceinline__ void
-loadPatch(const PatchArgs &a, const char *__restrict__ in, char *lds, int wave,
-          int lane, uint32_t g, const TileSpan &span, Between &&between,
-          Behind &&behind MXK_STAMP_PARAM) {
+/// What a wave needs to load columns of a tile's patch.
+struct PatchLoader {
+  __amdgpu_buffer_rsrc_t inBuf;
   // Patch row `lane`: where its input row starts, from the first image the
   // tile reads (32-bit offsets), or kInvalid for a row of padding.  A load
   // adds the lane's own offset, itself kInvalid for padding columns: any sum
   // with a kInvalid in it lies beyond the buffer, which the range check
   // limits to kInvalid bytes, and reads as zeros.
-  uint32_t rowBase;
-  {
+  uint32_t rowBase, rows, slice0;
+
+  __device__ __forceinline__ PatchLoader(const PatchArgs &a,
+                                         const char *__restrict__ in, int lane,
+                                         uint32_t g, const TileSpan &span,
+                                         uint32_t firstSlice) {
     const uint32_t r = span.firstRow + lane;
     const uint32_t image = a.divRowsPerImage(r);
     const uint32_t ih = r - image * a.rowsPerImage - uint32_t(a.padH);
@@ -174,28 +185,34 @@ loadPatch(const PatchArgs &a, const char *__restrict__ in, char *lds, int wave,
                   ? ((image - span.image0) * a.inH + ih) * a.inRowBytes +
                         g * a.ciBytes
                   : kInvalid;
+    const uint64_t skipped = uint64_t(span.image0) * a.imageBytes;
+    const uint64_t left = a.inBytes - skipped;
+    inBuf = bufferOf(in + skipped, uint32_t(left < kInvalid ? left : kInvalid));
+    rows = span.rows, slice0 = firstSlice;
   }
-  const uint64_t skipped = uint64_t(span.image0) * a.imageBytes;
-  const uint64_t left = a.inBytes - skipped;
-  const __amdgpu_buffer_rsrc_t inBuf =
-      bufferOf(in + skipped, uint32_t(left < kInvalid ? left : kInvalid));
-  const uint32_t rows = span.rows;
-  // One wave loads column block q (units 64 q .. 64 q + 63 of every patch
-  // row: chunk u % UNITS of the pixel in padded column u / UNITS) of a
-  // slice.
-  auto loadColumns = [&](uint32_t slice, uint32_t q) {
+
+  /// Column block q (units 64 q .. 64 q + 63 of every patch row: chunk u %
+  /// UNITS of the pixel in padded column u / UNITS) of a slice.
+  /// RAGGED: the last slice may be a partial one.
+  template <int UNITS, bool RAGGED>
+  __device__ __forceinline__ void columns(const PatchArgs &a, char *lds,
+                                          int lane, uint32_t slice,
+                                          uint32_t slot, uint32_t q) const {
     const uint32_t u = q * 64 + lane;
     const uint32_t col = u / UNITS, c = u - col * UNITS;
     const uint32_t iw = col - uint32_t(a.padW);
+    const uint32_t at = (slice0 + slice) * 128; // within the pixel
     const uint32_t laneOff =
-        c < 8 && iw - a.loW < a.spanW ? iw * a.pixelBytes + c * 16 : kInvalid;
+        c < 8 && (!RAGGED || at + c * 16 < a.ciBytes) && iw - a.loW < a.spanW
+            ? iw * a.pixelBytes + c * 16
+            : kInvalid;
     // (the last block of a row is a partial one: lanes beyond it write
     // nothing)
     if (u < a.rowUnits) {
-      char *dst = lds + slice * a.sliceBytes + q * 1024;
+      char *dst = lds + slot * a.sliceBytes + q * 1024;
       auto loadRow = [&](uint32_t row) {
         const uint32_t base = __builtin_amdgcn_readlane(rowBase, row);
-        loadToLds(inBuf, (LdsPtr)dst, laneOff + base, slice * 128);
+        loadToLds(inBuf, (LdsPtr)dst, laneOff + base, at);
         dst += a.rowPitch;
       };
       // (four at a time: a taken branch costs as much as a load)
@@ -206,15 +223,31 @@ loadPatch(const PatchArgs &a, const char *__restrict__ in, char *lds, int wave,
       for (; row < rows; ++row)
         loadRow(row);
     }
-  };
+  }
+};
+
+/// Loads the patch of a tile, all waves together.  Column blocks of `slices`
+/// slices, slice 0 first, are dealt out to the waves in turn.  Slice 0 is what
+/// the k loop waits for: its loads go out before anything else, then
+/// `between()` runs (the first weight loads - WEIGHT_LOADS of them per wave -
+/// and address arithmetic, which fill the wait), then the wave waits for its
+/// part of slice 0 and meets the others at a barrier; the later slices' loads
+/// follow and are waited for inside the k loop.  (FIRST_ONLY: they are another
+/// wave's.)
+template <int WEIGHT_LOADS, int UNITS, bool RAGGED, bool FIRST_ONLY,
+          class Between, class Behind>
+__device__ __forceinline__ void
+loadPatch(const PatchArgs &a, const PatchLoader &from, char *lds, int wave,
+          int lane, uint32_t slices, Between &&between,
+          Behind &&behind MXK_STAMP_PARAM) {
   // A wave with no block of slice 0 issues its first block of a later slice
   // right away (behind `between`, so that slice 0 gets ahead); the others do
   // so after the barrier.
   MXK_STAMP(1); // set-up done: the first load of the patch goes out
-  const uint32_t blocks = a.slices * a.rowLoads;
+  const uint32_t blocks = FIRST_ONLY ? 0 : slices * a.rowLoads;
   uint32_t next = wave;
   for (; next < a.rowLoads; next += kPatchWaves)
-    loadColumns(0, next);
+    from.columns<UNITS, RAGGED>(a, lds, lane, 0, 0, next);
   MXK_STAMP(2); // slice 0 requested
   const bool early = uint32_t(wave) >= a.rowLoads;
   between();
@@ -222,7 +255,7 @@ loadPatch(const PatchArgs &a, const char *__restrict__ in, char *lds, int wave,
   if (early) {
     if (next < blocks) {
       const uint32_t s = a.divRowLoads(next);
-      loadColumns(s, next - s * a.rowLoads);
+      from.columns<UNITS, RAGGED>(a, lds, lane, s, s, next - s * a.rowLoads);
       next += kPatchWaves;
     }
   } else {
@@ -240,12 +273,12 @@ loadPatch(const PatchArgs &a, const char *__restrict__ in, char *lds, int wave,
   // without standing in the queue of the vector memory path (22 cycles per
   // load of 1 KB: 1 600 cycles for three slices of a 112-pixel tile).
   // Issued so far: slice 0's blocks and one block per wave without any.
-  if (wave < kWavesN) {
+  if (!FIRST_ONLY && wave < kWavesN) {
     const uint32_t issued =
         a.rowLoads > uint32_t(kPatchWaves) ? a.rowLoads : uint32_t(kPatchWaves);
     for (next = issued + wave; next < blocks; next += kWavesN) {
       const uint32_t s = a.divRowLoads(next);
-      loadColumns(s, next - s * a.rowLoads);
+      from.columns<UNITS, RAGGED>(a, lds, lane, s, s, next - s * a.rowLoads);
     }
   }
 }
@@ -328,7 +361,7 @@ template <> struct PatchMma<1> {
 /// EB: bytes per input element (2 half, 1 quarter); FA / FB: fp8 formats of
 /// activations / weights; RB: 32-row blocks per tile; D: k-steps the weight
 /// loads run ahead.
-template <int EB, int FA, int FB, int RB, int D, class OutT>
+template <int EB, int FA, int FB, int RB, int D, bool RAGGED, class OutT>
 __global__ __launch_bounds__(kPatchThreads) void igemmPatchKernel(
     const PatchArgs a, const char *__restrict__ in, const char *__restrict__ w,
     const OutT *__restrict__ bias, OutT *__restrict__ out, float scale) {
@@ -376,7 +409,9 @@ __global__ __launch_bounds__(kPatchThreads) void igemmPatchKernel(
   // k-step, at tap (0, 0) of slice 0.  (Worked out while the first loads are
   // in flight.)
   uint32_t pixelByte[RB];
-  loadPatch<2 * kTN * D, kPixelUnits>(a, in, lds, wave, lane, g, span, [&] {
+  const PatchLoader loader(a, in, lane, g, span, 0);
+  loadPatch<2 * kTN * D, kPixelUnits, RAGGED, false>(
+      a, loader, lds, wave, lane, a.slices, [&] {
 #pragma unroll
     for (int u = 0; u != D; ++u)
       loadB(bf[u]);
@@ -689,8 +724,21 @@ template <> struct PatchMma16<1> {
 };
 
 /// D: k-steps of its own (every second one) a wave's weight loads run ahead.
-template <int EB, int FA, int FB, int D, class OutT>
-__global__ __launch_bounds__(kPatchThreads) void igemmPatch16Kernel(
+/// RING: more slices than the LDS has room for.  A slice comes into the place
+/// of the last but one as soon as the waves start on the next: the barrier they
+/// meet at there tells that nobody reads that one any more (the last step of
+/// the slice before is still under way).  kRingWave: a ninth wave brings those
+/// behind the first, so that the compute waves' counts of outstanding loads
+/// stay those of their weights.  kRingOwn: the older wave of each SIMD does and
+/// waits a trip to memory per slice for it, the younger one multiplying
+/// meanwhile - for fp8, whose operands take more registers than nine waves have.
+/// kSlices: no ring, but a partial last slice or K in parts; kWhole: neither
+/// (what those add to a workgroup's start is 0.15 us in fp16, 0.3 in fp8, of
+/// 8.6 us in all).
+constexpr int kWhole = 0, kRingWave = 1, kRingOwn = 2, kSlices = 3;
+template <int EB, int FA, int FB, int D, int RING, class OutT>
+__global__ __launch_bounds__(
+    kPatchThreads + (RING == kRingWave ? 64 : 0)) void igemmPatch16Kernel(
     const PatchArgs a, const char *__restrict__ in, const char *__restrict__ w,
     const OutT *__restrict__ bias, OutT *__restrict__ out, float scale) {
   static_assert(kTN == 1 && D % 2 == 0 && 64 % D == 0, "");
@@ -715,18 +763,54 @@ __global__ __launch_bounds__(kPatchThreads) void igemmPatch16Kernel(
                "s"(a.inRowBytes), "s"(a.outChans), "s"(a.outChansPerGroup));
   const uint32_t overN = a.divNTiles(tile);
   const uint32_t nTile = tile - overN * a.nTiles;
-  const uint32_t g = a.divMTiles(overN);
+  constexpr bool kInRing = RING == kRingWave || RING == kRingOwn;
+  uint32_t g = a.divMTiles(overN);
   const uint32_t mTile = overN - g * a.mTiles;
   const TileSpan span = tileSpan(a, mTile);
+  uint32_t part = 0, slice0 = 0, slices = a.slices;
+  if constexpr (RING != kWhole) {
+    part = a.divGroups(g), g -= part * a.groups;
+    slice0 = part * a.slicesPart;
+    slices = slices - slice0 < a.slicesPart ? slices - slice0 : a.slicesPart;
+  }
+  if constexpr (RING == kRingWave) {
+    if (wave == kPatchWaves) {
+      const PatchLoader loader(a, in, lane, g, span, slice0);
+      // slice s lives in place s % ring
+      auto bring = [&](uint32_t s) {
+        const uint32_t slot = s - a.divRing(s) * a.ring;
+        for (uint32_t q = 0; q != a.rowLoads; ++q)
+          loader.columns<kPixelUnits16, true>(a, lds, lane, s, slot, q);
+      };
+      __builtin_amdgcn_s_barrier(); // slice 0 is there
+      for (uint32_t s = 1; s < a.ring && s < slices; ++s)
+        bring(s);
+      for (uint32_t s = 1; s < slices; ++s) {
+        MXK_WAIT_VMCNT(0);
+        __builtin_amdgcn_s_barrier(); // slice s is there, s - 2's place free
+        if (s >= 2 && s - 2 + a.ring < slices)
+          bring(s - 2 + a.ring);
+      }
+      // (the barriers of the sums' exchange)
+      if (a.exchangeByte == 0)
+        __syncthreads();
+      __syncthreads();
+      __syncthreads();
+      return;
+    }
+  }
+  const uint32_t kSteps = RING == kWhole ? a.kSteps : slices * a.taps;
+  if constexpr (RING != kWhole)
+    out += size_t(part) * a.M * a.outChans;
 
   // This wave's k-steps: grp, grp + 2, ... - `own` of them (at least one: the
   // kernel has two taps or more).  Their weights: 4 KB per step, lane l's four
   // operands 1 KB apart; the buffer ends with the wave's last step, so the
   // loads that run ahead beyond it read zeros.
-  const uint32_t own = (a.kSteps + 1 - grp) >> 1;
+  const uint32_t own = (kSteps + 1 - grp) >> 1;
   const uint32_t waveBlock = (g * a.nTiles + nTile) * kWavesN + wn;
   const __amdgpu_buffer_rsrc_t wBuf =
-      bufferOf(w + (size_t(waveBlock) * a.kSteps + grp) * 4096,
+      bufferOf(w + (size_t(waveBlock) * a.kSteps + slice0 * a.taps + grp) * 4096,
                (own - 1) * 8192 + 4096);
   uint32_t wOff = lane * 16;
   uintx4 bf[D][kUnits][2][kReads];
@@ -747,10 +831,13 @@ __global__ __launch_bounds__(kPatchThreads) void igemmPatch16Kernel(
   // Per row block: the LDS byte of the first chunk this lane reads of a
   // k-step, at tap (0, 0) of slice 0.
   uint32_t pixelByte[RB];
+  const PatchLoader loader(a, in, lane, g, span, slice0);
   // (the first step's weights before the barrier, the others behind it: the
   // vector memory path is what bounds the time to the barrier)
   constexpr int kFirst = 1;
-  loadPatch<4 * kFirst, kPixelUnits16>(a, in, lds, wave, lane, g, span, [&] {
+  loadPatch<4 * kFirst, kPixelUnits16, RING != kWhole, RING == kRingWave>(
+      a, loader, lds, wave, lane, kInRing && a.ring < slices ? a.ring : slices,
+      [&] {
 #pragma unroll
     for (int u = 0; u != kFirst; ++u)
       loadB(bf[u]);
@@ -792,8 +879,9 @@ __global__ __launch_bounds__(kPatchThreads) void igemmPatch16Kernel(
   auto fillTable = [&] {
     const uint32_t kt = 2 * (tableBase + 1 + lane) + grp;
     const uint32_t slice = a.divTaps(kt), tap = kt - slice * a.taps;
+    const uint32_t slot = kInRing ? slice - a.divRing(slice) * a.ring : slice;
     const uint32_t kh = a.divKW(tap), kw = tap - kh * a.kW;
-    tapTable = (slice * a.sliceBytes + kh * a.tapRowBytes +
+    tapTable = (slot * a.sliceBytes + kh * a.tapRowBytes +
                 kw * a.tapColBytes) |
                (tap < 2 ? 0x80000000u : 0u);
   };
@@ -825,14 +913,19 @@ __global__ __launch_bounds__(kPatchThreads) void igemmPatch16Kernel(
   // MFMAs and the LDS reads of the next unit in turn (a wave issues in order
   // and an MFMA behind another waits for the pipe: what stands between two
   // of them costs nothing).
+  // (kRingWave: an address at a time; the registers nine waves have are few)
   auto interleave = [&] {
-    __builtin_amdgcn_sched_group_barrier(0x002, RB, 0);
+    if constexpr (RING != kRingWave)
+      __builtin_amdgcn_sched_group_barrier(0x002, RB, 0);
 #pragma unroll
     for (int k = 0; k != RB * kReads; ++k) {
+      if constexpr (RING == kRingWave)
+        __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x008, 2 / kReads, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
   };
+  uint32_t sliceAt = 0; // of the next step
   // One own step: kUnits units of MFMAs; `first` holds unit 0's operands and
   // gets the next step's on the way out when the step has two units, else
   // `second` does.  GUARD: the steps behind the last whole group of D.
@@ -848,11 +941,21 @@ __global__ __launch_bounds__(kPatchThreads) void igemmPatch16Kernel(
         // A new slice: its loads were issued before the loop, so they are
         // older than the weight loads of the last D steps (loads complete in
         // order); the barrier tells that the other waves' have landed too.
-        if (j >= uint32_t(D))
+        // (GUARD: no weight loads are behind those of a ring any more)
+        if (j >= uint32_t(D) && !(GUARD && RING == kRingOwn))
           MXK_WAIT_VMCNT(4 * (D - 1));
         else
           MXK_WAIT_VMCNT(0);
         __builtin_amdgcn_s_barrier();
+        if constexpr (RING == kRingOwn) {
+          ++sliceAt;
+          const uint32_t next = sliceAt - 2 + a.ring;
+          if (wave < kWavesN && sliceAt >= 2 && next < slices) {
+            const uint32_t slot = next - a.divRing(next) * a.ring;
+            for (uint32_t q = wave; q < a.rowLoads; q += kWavesN)
+              loader.columns<kPixelUnits16, true>(a, lds, lane, next, slot, q);
+          }
+        }
       }
     }
     if constexpr (!GUARD) {
@@ -1062,6 +1165,8 @@ uint32_t maxPatchRows(const IgemmDesc &d) {
 
 struct PatchShape {
   uint32_t eb, slices, taps, kSteps, rowLoads, rowPitch, maxRows, ldsBytes, rb;
+  uint32_t slicesPart, ring;
+  bool ragged; // the last slice is a partial one
   uint32_t exchangeByte, tileByte;
 };
 
@@ -1072,7 +1177,7 @@ bool patchShape(const IgemmDesc &d, int inType, int outType, PatchShape &s) {
   s.eb = elemBytesOf(inType);
   if (d.inD != 1 || d.outD != 1 || d.kD != 1 || d.strideH != 1 ||
       d.strideW != 1 || d.inDilH != 1 || d.inDilW != 1 || d.outFullH != 0 ||
-      d.outFullW != 0 || d.outTransposed || d.noTaps || d.splitK != 1)
+      d.outFullW != 0 || d.outTransposed || d.noTaps || d.splitK == 0)
     return false;
   const bool blocks16 = d.patch == 2;
   if (blocks16 ? d.blockM == 0 || d.blockM > uint32_t(kRows16) ||
@@ -1084,12 +1189,20 @@ bool patchShape(const IgemmDesc &d, int inType, int outType, PatchShape &s) {
   if (M == 0 || M > 0x7fffffffull || d.kH == 0 || d.kW == 0 ||
       d.inChansPerGroup == 0)
     return false;
-  if ((d.inChansPerGroup * s.eb) % 128 != 0)
+  // (whole 16-byte vectors; the last slice may be a partial one)
+  if ((d.inChansPerGroup * s.eb) % 16 != 0)
     return false;
-  const uint32_t outVec = outType == kHalf ? 8 : 4;
+  if (!blocks16 && d.splitK != 1)
+    return false;
+  const uint32_t outVec = outType == kHalf && d.splitK == 1 ? 8 : 4;
   if (d.outChansPerGroup % outVec != 0)
     return false;
-  s.slices = d.inChansPerGroup * s.eb / 128;
+  s.slices = (d.inChansPerGroup * s.eb + 127) / 128;
+  s.ragged = d.inChansPerGroup * s.eb % 128 != 0;
+  s.slicesPart = (s.slices + d.splitK - 1) / d.splitK;
+  // (no part without any)
+  if (s.slicesPart * (d.splitK - 1) >= s.slices)
+    return false;
   s.taps = d.kH * d.kW;
   s.kSteps = s.slices * s.taps;
   const uint64_t cols = uint64_t(d.outW) + uint64_t(d.kW - 1) * d.dilW;
@@ -1106,15 +1219,19 @@ bool patchShape(const IgemmDesc &d, int inType, int outType, PatchShape &s) {
   // (a lane per patch row works out where the rows start)
   if (s.maxRows > 64)
     return false;
-  const uint64_t patch = uint64_t(s.slices) * s.maxRows * pitch;
-  if (patch > uint64_t(kLdsLimit))
+  // All slices of a part, or a ring of three or more of them.
+  const uint64_t slice = uint64_t(s.maxRows) * pitch;
+  s.ring = uint32_t(std::min<uint64_t>(s.slicesPart, kLdsLimit / slice));
+  if (s.ring < s.slicesPart && (s.ring < 3 || !blocks16))
     return false;
+  const uint64_t patch = s.ring * slice;
   s.rowPitch = uint32_t(pitch);
   const uint64_t exchange =
       blocks16 ? uint64_t(kPatchWaves) * kKeep16 * 2 * 1024
                : uint64_t(kPatchWaves) * (s.rb / 2) * kTN * 4 * 1024;
-  const uint64_t tile = (blocks16 ? 128 : 32 * s.rb) *
-                        (kPatchBN * (outType == kHalf ? 2 : 4) + 16);
+  const uint64_t tile =
+      (blocks16 ? 128 : 32 * s.rb) *
+      (kPatchBN * (outType == kHalf && d.splitK == 1 ? 2 : 4) + 16);
   const uint64_t patchEnd = (patch + 1023) / 1024 * 1024;
   // Beside the patch where there is room (the waves then hand over their
   // sums as they finish, without waiting for the others to leave the patch);
@@ -1146,15 +1263,16 @@ bool patchShape(const IgemmDesc &d, int inType, int outType, PatchShape &s) {
     return false;
   // tiles and weight blocks are numbered in 32 bits
   const uint64_t tiles = (M + d.blockM - 1) / d.blockM *
-                         ((d.outChansPerGroup + 127) / 128) * d.groups;
+                         ((d.outChansPerGroup + 127) / 128) * d.groups *
+                         d.splitK;
   return tiles <= 0x7fffffffull;
 }
 
-template <int EB, int FA, int FB, int RB, int D, class OutT>
+template <int EB, int FA, int FB, int RB, int D, bool RAGGED, class OutT>
 hipError_t launchPatchKernel(const PatchArgs &a, uint32_t ldsBytes,
                              const void *in, const void *w, const void *bias,
                              void *out, float scale, hipStream_t stream) {
-  auto kernel = &igemmPatchKernel<EB, FA, FB, RB, D, OutT>;
+  auto kernel = &igemmPatchKernel<EB, FA, FB, RB, D, RAGGED, OutT>;
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void *>(kernel),
       hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit);
@@ -1174,25 +1292,39 @@ hipError_t dispatchPatchShape(const PatchShape &s, const PatchArgs &a,
                               const void *in, const void *w, const void *bias,
                               void *out, float scale, hipStream_t stream) {
   if (s.rb == 0) {
-    auto kernel = &igemmPatch16Kernel<EB, FA, FB, kAhead16, OutT>;
-    static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(kernel),
-        hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit);
-    if (attr != hipSuccess)
-      return attr;
-    hipLaunchKernelGGL(kernel, dim3(a.mTiles * a.nTiles * a.groups),
-                       dim3(kPatchThreads), s.ldsBytes, stream, a,
-                       static_cast<const char *>(in),
-                       static_cast<const char *>(w),
-                       static_cast<const OutT *>(bias),
-                       static_cast<OutT *>(out), scale);
-    return hipGetLastError();
+    auto launch = [&](auto ring) {
+      constexpr int RING = decltype(ring)::value;
+      auto kernel = &igemmPatch16Kernel<EB, FA, FB, kAhead16, RING, OutT>;
+      static const hipError_t attr = hipFuncSetAttribute(
+          reinterpret_cast<const void *>(kernel),
+          hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit);
+      if (attr != hipSuccess)
+        return attr;
+      const uint32_t parts = (s.slices + s.slicesPart - 1) / s.slicesPart;
+      hipLaunchKernelGGL(kernel, dim3(a.mTiles * a.nTiles * a.groups * parts),
+                         dim3(kPatchThreads + (RING == kRingWave ? 64 : 0)),
+                         s.ldsBytes,
+                         stream, a, static_cast<const char *>(in),
+                         static_cast<const char *>(w),
+                         static_cast<const OutT *>(bias),
+                         static_cast<OutT *>(out), scale);
+      return hipGetLastError();
+    };
+    if (s.ring < s.slicesPart)
+      return launch(std::integral_constant<int, EB == 2 ? kRingWave
+                                                        : kRingOwn>{});
+    if (s.slicesPart < s.slices || s.ragged)
+      return launch(std::integral_constant<int, kSlices>{});
+    return launch(std::integral_constant<int, kWhole>{});
   }
-  if (s.rb == 4)
-    return launchPatchKernel<EB, FA, FB, 4, 4, OutT>(a, s.ldsBytes, in, w,
-                                                     bias, out, scale, stream);
-  return launchPatchKernel<EB, FA, FB, 2, 4, OutT>(a, s.ldsBytes, in, w, bias,
-                                                   out, scale, stream);
+  auto launch = [&](auto ragged) {
+    constexpr bool RAGGED = decltype(ragged)::value;
+    return s.rb == 4 ? launchPatchKernel<EB, FA, FB, 4, 4, RAGGED, OutT>(
+                           a, s.ldsBytes, in, w, bias, out, scale, stream)
+                     : launchPatchKernel<EB, FA, FB, 2, 4, RAGGED, OutT>(
+                           a, s.ldsBytes, in, w, bias, out, scale, stream);
+  };
+  return s.ragged ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 template <int EB, int FA, int FB>
@@ -1219,7 +1351,7 @@ bool igemmPatchTakes(const IgemmDesc &d, int inType, int outType) {
 uint64_t igemmPatchPackedElems(const IgemmDesc &d, int inType) {
   const uint32_t eb = elemBytesOf(inType);
   const uint64_t kSteps =
-      uint64_t(d.inChansPerGroup) * eb / 128 * d.kH * d.kW;
+      (uint64_t(d.inChansPerGroup) * eb + 127) / 128 * d.kH * d.kW;
   return uint64_t(d.groups) * ((d.outChansPerGroup + 127) / 128) * 4 * kSteps *
          (4096 / eb);
 }
@@ -1227,25 +1359,26 @@ uint64_t igemmPatchPackedElems(const IgemmDesc &d, int inType) {
 PackJob igemmPatchPackJob(const IgemmDesc &d, int inType) {
   PackJob j;
   j.taps = d.kH * d.kW;
-  j.steps = d.inChansPerGroup * elemBytesOf(inType) / 128 * j.taps;
+  j.steps = (d.inChansPerGroup * elemBytesOf(inType) + 127) / 128 * j.taps;
   j.blocks = (d.outChansPerGroup + 127) / 128 * 4;
   j.ciPadded = d.inChansPerGroup;
   return j;
 }
 
-hipError_t launchIgemmPatch(const IgemmDesc &d, int inType, int outType,
-                            const void *in, const void *weightsPacked,
-                            const void *bias, void *out, const QuarterInfo &q,
+namespace {
+hipError_t launchPatchTiles(const IgemmDesc &d, const PatchShape &s,
+                            int inType, int outType, const void *in,
+                            const void *weightsPacked, const void *bias,
+                            void *out, const QuarterInfo &q,
                             hipStream_t stream) {
-  PatchShape s;
-  if (!patchShape(d, inType, outType, s))
-    return hipErrorInvalidValue;
   PatchArgs a{};
   a.M = d.batch * d.outH * d.outW;
   a.tileM = d.blockM;
   a.mTiles = (a.M + d.blockM - 1) / d.blockM;
   a.nTiles = (d.outChansPerGroup + 127) / 128;
   a.groups = d.groups;
+  a.slicesPart = s.slicesPart, a.ring = s.ring;
+  a.divGroups = makeFastDiv(d.groups), a.divRing = makeFastDiv(s.ring);
   a.outW = d.outW, a.outH = d.outH;
   a.rowsPerImage = d.outH + (d.kH - 1) * d.dilH;
   a.inH = d.inH;
@@ -1294,6 +1427,31 @@ hipError_t launchIgemmPatch(const IgemmDesc &d, int inType, int outType,
                                      out, scale, stream);
   return dispatchPatchOut<1, 1, 1>(outType, s, a, in, weightsPacked, bias, out,
                                    scale, stream);
+}
+} // namespace
+
+hipError_t launchIgemmPatch(const IgemmDesc &d, int inType, int finalType,
+                            const void *in, const void *weightsPacked,
+                            const void *finalBias, void *finalOut,
+                            void *workspace, const QuarterInfo &q,
+                            hipStream_t stream) {
+  PatchShape s;
+  if (!patchShape(d, inType, finalType, s))
+    return hipErrorInvalidValue;
+  if (d.splitK > 1) {
+    // fp32 partial tiles per part (scaled, without bias), then their sum
+    if (!workspace)
+      return hipErrorInvalidValue;
+    const hipError_t e = launchPatchTiles(d, s, inType, kFloat, in,
+                                          weightsPacked, nullptr, workspace, q,
+                                          stream);
+    return e != hipSuccess
+               ? e
+               : launchSplitKSum(d, finalType, workspace, finalBias, finalOut,
+                                 stream);
+  }
+  return launchPatchTiles(d, s, inType, finalType, in, weightsPacked,
+                          finalBias, finalOut, q, stream);
 }
 
 } // namespace mxk

@@ -272,8 +272,13 @@ uint64_t igemmPatchPackedElems(const IgemmDesc &d, int inType);
 PackJob igemmPatchPackJob(const IgemmDesc &d, int inType);
 hipError_t launchIgemmPatch(const IgemmDesc &d, int inType, int outType,
                             const void *in, const void *weightsPacked,
-                            const void *bias, void *out, const QuarterInfo &q,
-                            hipStream_t stream);
+                            const void *bias, void *out, void *workspace,
+                            const QuarterInfo &q, hipStream_t stream);
+/// The sum of d.splitK parts' fp32 outputs in `workspace`
+/// [part][pixel][channel], with the bias, as launchIgemm ends with.
+hipError_t launchSplitKSum(const IgemmDesc &d, int outType,
+                           const void *workspace, const void *bias, void *out,
+                           hipStream_t stream);
 
 /// The same convolution by the kernel for problems too small to fill the chip
 /// with 128-pixel tiles: d.small names the tile, K is split over the waves of

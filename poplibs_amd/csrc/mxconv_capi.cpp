@@ -205,7 +205,7 @@ mxconv_status forward(const mxconv_plan *plan, const void *in, const void *w,
                        "implicit-GEMM convolution launch (small tiles)");
     if (plan->igemm.patch)
       return hipStatus(mxk::launchIgemmPatch(plan->igemm, inType, outType, in,
-                                             w, bias, out, q, s),
+                                             w, bias, out, workspace, q, s),
                        "implicit-GEMM convolution launch (resident patch)");
     if (!plan->igemmPhases.empty()) {
       // one convolution per phase of the zero-stuffed input, in one launch

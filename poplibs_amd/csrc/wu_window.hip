@@ -517,11 +517,11 @@ double wuWindowChoose(WuTapDesc &d, uint32_t computeUnits) {
     // (four workgroups for every CU at most: more lose to their own start)
     const uint64_t most =
         std::max<uint64_t>(1, 4ull * computeUnits / one.tiles);
-    for (uint32_t n = 1; n <= std::min<uint64_t>(steps, most); ++n) {
+    // (every count of chunks up to 16, then one in sixteen)
+    for (uint32_t n = 1; n <= std::min<uint64_t>(steps, most);
+         n += std::max(1u, n / 16)) {
       t.windowSteps = (steps + n - 1) / n;
       const WinShape s = winShape(t);
-      if (s.chunks != n)
-        continue;
       const double us = winEstimateUs(t, s, computeUnits);
       if (us < bestUs && wuWindowTakes(t))
         bestUs = us, best = t;

@@ -370,23 +370,36 @@ double fillingUs(unsigned blockM, unsigned blockN, unsigned stages,
          f.byte * mb;
 }
 
-/// igemmPatchKernel (mode 1): 1.9 us to the first MFMA + 0.5 us reduction and
-/// stores, 0.333 us per k-step of 128 pixels (half of that for 64); one
-/// workgroup per CU, so further rounds pay their start-up in full (4.5 us
-/// instead of 2.4).  igemmPatch16Kernel (mode 2): seven blocks of 16 pixels
-/// whatever the tile's height, 0.29 us per k-step and 1.5 us around them in
-/// a launch of one round (8.6 us measured for 224 tiles of 18 k-steps, 17.1
-/// for 50 k-steps), 0.34 and 2.6 us in launches of several (55 us for 4
-/// rounds of 36, 110 us for 7 rounds of 36, 35 us for 4 rounds of 18).
+/// igemmPatchKernel (mode 1) and igemmPatch16Kernel (mode 2, seven blocks of 16
+/// pixels whatever the tile's height): start and end of a workgroup and its
+/// k-steps, again for every further round of workgroups on a CU, and the way
+/// out of `outMB` megabytes of outputs.  Fitted to 17 000 measurements of 3 800
+/// random layers (fp16, 1 to 128 images, fields of 7 to 64, 32 to 768 channels,
+/// two to 25 taps; 5 500 in fp8), mode 2 within 10 % (fp8 3 %), mode 1 within 8
+/// % and, for tiles of 64, of which two may share a CU, 17 %.
 double estimatePatch(std::size_t workgroups, std::size_t kSteps, unsigned mode,
-                     unsigned blockM) {
-  const double rounds = roundsOf(workgroups, 1);
-  if (mode == 2)
-    return kLaunchUs + rounds * ((rounds > 1 ? 2.6 : 1.5) +
-                                 (rounds > 1 ? 0.34 : 0.29) * double(kSteps));
-  const double step = blockM == 128 ? 0.333 : 0.167;
-  const double fixed = rounds > 1 ? 4.5 : 2.4;
-  return kLaunchUs + rounds * (fixed + step * double(kSteps));
+                     unsigned blockM, bool quarter, double outMB) {
+  struct Fit {
+    double first, step, round, roundStep, byte;
+  };
+  static constexpr Fit kFits[2][3] = {
+      {{1.97, 0.173, 2.92, 0.163, 0.0},
+       {2.48, 0.286, 1.88, 0.377, 0.2},
+       {1.98, 0.259, 1.99, 0.281, 0.205}},
+      {{1.95, 0.154, 2.93, 0.129, 0.0},
+       {2.26, 0.280, 1.54, 0.377, 0.17},
+       {1.41, 0.283, 1.35, 0.312, 0.18}}};
+  const Fit &f = kFits[quarter][mode == 2 ? 2 : blockM == 128 ? 1 : 0];
+  return kLaunchUs + f.first + f.step * double(kSteps) +
+         (roundsOf(workgroups, 1) - 1.0) *
+             (f.round + f.roundStep * double(kSteps)) +
+         f.byte * outMB;
+}
+
+/// What K split adds to it (the same measurements): the second kernel, and
+/// the fp32 partial tiles out and in again, mostly from the caches.
+double patchSplitUs(std::size_t partialBytes) {
+  return 2.75 + 0.29e-6 * double(partialBytes);
 }
 
 /// igemmSmallKernel, by its tile (kIgemmSmallTiles): a workgroup that has a CU
@@ -1492,24 +1505,27 @@ mxconv_plan makePlanWith(const ConvParams &params,
           "does not take this convolution with that many 64-channel tiles "
           "per workgroup (they divide the layer's; at most 4 with up to 64 "
           "input channels, 2 with up to 256, 1 beyond)");
-    // Unit stride and whole 128-byte slices of channels: the kernel that
-    // keeps the tile's input patch in LDS reads every input element once
-    // instead of once per tap.
+    // Unit stride: the kernel that keeps the tile's input patch in LDS reads
+    // every input element once instead of once per tap.
+    // (A weight update pass's own convolution, whose channels are its images,
+    // takes it for whole 128-byte slices of them only: the streaming kernel
+    // writes its result in weight order.)
     if (!plan.pointwiseOn && plan.igemmPhases.empty() &&
-        !plan.paddedInputChans &&
-        (g.splitK == 1 || !pc.splitK) && pc.patch != 0 &&
+        (!isWeightUpdatePass(options.pass) ||
+         (!plan.paddedInputChans &&
+          ciPadded * params.inputType.size() % 128 == 0)) &&
+        (g.splitK == 1 || !pc.splitK || pc.patch == 2) && pc.patch != 0 &&
         !pc.blockN && !pc.blockK && !pc.stages) {
       const std::size_t m = std::size_t(s.batch) * s.outH * s.outW;
       const std::size_t nTiles128 = (co + 127) / 128 * p.numConvGroups;
-      const std::size_t stepBytes = 128;
-      const std::size_t patchSteps =
-          ciPadded * params.inputType.size() / stepBytes * s.kH * s.kW;
+      const std::size_t slices =
+          (ciPadded * params.inputType.size() + 127) / 128;
       // Weigh the tilings by estimated time: the streaming kernel as planned
       // above against this kernel with tiles of 128 and 64 pixels (32-pixel
       // MFMA blocks) and with the layer cut into as many equal tiles of at
       // most 112 pixels as there are CUs (16-pixel blocks).
       struct Tiling {
-        uint32_t patch, blockM;
+        uint32_t patch, blockM, parts;
       };
       std::vector<Tiling> tilings;
       auto add = [&](const std::string &name, Tiling tiling,
@@ -1523,30 +1539,39 @@ mxconv_plan makePlanWith(const ConvParams &params,
         return plan.candidates.size() - 1;
       };
       const std::size_t none = ~std::size_t(0);
-      auto addPatch = [&](uint32_t mode, uint32_t bm) -> std::size_t {
+      auto addPatch = [&](uint32_t mode, uint32_t bm,
+                          uint32_t parts) -> std::size_t {
         mxk::IgemmDesc t = g;
-        t.patch = mode, t.blockM = bm;
-        t.splitK = 1; // (asked for by name, it runs K whole)
+        t.patch = mode, t.blockM = bm, t.splitK = parts;
         if (!mxk::igemmPatchTakes(t, inId, outId))
           return none;
-        const std::size_t tiles = (m + bm - 1) / bm * nTiles128;
+        const std::size_t tiles = (m + bm - 1) / bm * nTiles128 * parts;
+        const std::size_t steps =
+            (slices + parts - 1) / parts * s.kH * s.kW;
         return add("resident patch " + std::to_string(bm) + " x 128" +
-                       (mode == 2 ? ", 16-pixel blocks" : ""),
-                   Tiling{mode, bm}, tiles, 1, patchSteps,
-                   estimatePatch(tiles, patchSteps, mode, bm),
+                       (mode == 2 ? ", 16-pixel blocks" : "") +
+                       (parts > 1 ? ", K in " + std::to_string(parts) +
+                                        " parts"
+                                  : ""),
+                   Tiling{mode, bm, parts}, tiles, 1, steps,
+                   estimatePatch(tiles, steps, mode, bm, quarterIn,
+                                 1e-6 * double(plan.outputBytes())) +
+                       (parts > 1 ? patchSplitUs(mxk::igemmWorkspaceBytes(t))
+                                  : 0.0),
                    roundsOf(tiles, 1));
       };
       // Equal tiles, one per CU, in whole 16-pixel MFMA blocks - a tile of 98
       // pixels costs its workgroup the seven blocks a tile of 112 does, and
       // 224 workgroups of 112 are through sooner than 256 of 98 (c2: 8.7
       // against 9.1 us); 112 pixels where that takes several rounds.
-      const std::size_t across = gfx950::numCUs / std::max<std::size_t>(
-                                                      1, nTiles128);
-      const uint32_t equalM =
-          across == 0
-              ? 112u
-              : uint32_t(std::min<std::size_t>(
-                    112, ((m + across - 1) / across + 15) / 16 * 16));
+      auto equalTiles = [&](std::size_t parts) {
+        const std::size_t across =
+            gfx950::numCUs / std::max<std::size_t>(1, nTiles128 * parts);
+        return across == 0
+                   ? 112u
+                   : uint32_t(std::min<std::size_t>(
+                         112, ((m + across - 1) / across + 15) / 16 * 16));
+      };
       const std::size_t streamTiles =
           (m + 127) / 128 * (plan.coPadded / g.blockN) * p.numConvGroups *
           g.splitK;
@@ -1567,9 +1592,12 @@ mxconv_plan makePlanWith(const ConvParams &params,
       std::size_t best = iStream;
       if (pc.patch >= 1) {
         // planConstraints: whenever the kernel can, with the tile asked for
-        const uint32_t bm = pc.blockM ? pc.blockM
-                                      : pc.patch == 2 ? equalM : 128u;
-        const std::size_t i = addPatch(uint32_t(pc.patch), bm);
+        // (K whole unless its parts are named as well)
+        const uint32_t parts = pc.patch == 2 && pc.splitK ? pc.splitK : 1;
+        const uint32_t bm = pc.blockM         ? pc.blockM
+                            : pc.patch == 2 ? equalTiles(parts)
+                                            : 128u;
+        const std::size_t i = addPatch(uint32_t(pc.patch), bm, parts);
         if (i != none)
           best = i;
       } else if (s.kH * s.kW > 1 && co > 64) {
@@ -1577,11 +1605,19 @@ mxconv_plan makePlanWith(const ConvParams &params,
         // equal tiles fill the chip without the second kernel - N = 32,
         // 14 x 14, 256 -> 256 channels 20.4 -> 12.4 us, N = 8, 28 x 28,
         // 128 -> 128 15.0 -> 7.7)
-        for (Tiling t : {Tiling{1, 128}, Tiling{1, 64}, Tiling{2, equalM}}) {
+        std::vector<Tiling> weighed{
+            {1, 128, 1}, {1, 64, 1}, {2, equalTiles(1), 1}};
+        // ... and K cut along its slices, where the tiles leave CUs idle
+        const std::size_t tiles112 = (m + 111) / 112 * nTiles128;
+        if (!s.outputPadded() && !isWeightUpdatePass(options.pass))
+          for (uint32_t parts = 2;
+               parts <= slices && tiles112 * parts <= gfx950::numCUs; ++parts)
+            weighed.push_back({2, equalTiles(parts), parts});
+        for (Tiling t : weighed) {
           // (a forced tile height picks among the patch tilings only)
           if (pc.blockM && pc.blockM != t.blockM)
             continue;
-          const std::size_t i = addPatch(t.patch, t.blockM);
+          const std::size_t i = addPatch(t.patch, t.blockM, t.parts);
           if (i != none && plan.candidates[i].estimateUs <
                                plan.candidates[best].estimateUs)
             best = i;
@@ -1591,11 +1627,18 @@ mxconv_plan makePlanWith(const ConvParams &params,
       if (best != iStream) {
         g.patch = tilings[best].patch;
         g.blockM = tilings[best].blockM;
-        g.splitK = 1;
+        g.splitK = tilings[best].parts;
         g.blockN = 128;
         g.patchMaxRows = 0;
         g.patchMaxRows = mxk::igemmPatchMaxRows(g);
-        plan.workspaceBytes = 0;
+        plan.workspaceBytes = mxk::igemmWorkspaceBytes(g);
+        if (plan.paddedInputChans) {
+          const std::size_t copy =
+              s.batch * s.inD * s.inH * s.inW * p.numConvGroups * ciPadded *
+              params.inputType.size();
+          plan.paddedInputOffset = (plan.workspaceBytes + 255) / 256 * 256;
+          plan.workspaceBytes = plan.paddedInputOffset + copy;
+        }
         plan.coPadded = (co + 127) / 128 * 128;
         plan.weightPackedElems = mxk::igemmPatchPackedElems(g, inId);
       }
@@ -1614,7 +1657,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
         planned = 1e30;
         for (const auto &c : plan.candidates)
           if (c.chosen)
-            planned = 0.9 * c.estimateUs; // (an estimate on the high side)
+            planned = c.estimateUs;
       } else {
         const std::size_t tiles =
             (m + 127) / 128 * (plan.coPadded / g.blockN) * p.numConvGroups;
@@ -1715,7 +1758,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
           return plan.detailedEstimate().totalUs() +
                  (g.splitK > 1 ? kCallOverKernelUs : 0.0);
         if (g.patch) {
-          const double steps = double(s.kH * s.kW) * chanBytes / 128.0;
+          const double steps =
+              double(s.kH * s.kW) * std::ceil(chanBytes / 128.0);
           const double perCU = std::ceil(pixels / g.blockM) *
                                double((co + 127) / 128 * p.numConvGroups) /
                                gfx950::numCUs;
@@ -1940,6 +1984,8 @@ std::string mxconv_plan::constraintsJson() const {
     } else if (igemm.small) {
       os << ", \"smallTile\": " << igemm.small;
     } else if (igemm.patch) {
+      if (igemm.splitK > 1)
+        os << ", \"splitK\": " << igemm.splitK;
       os << ", \"pointwise\": 0, \"patch\": " << igemm.patch
          << ", \"blockM\": " << igemm.blockM;
     } else {
@@ -2109,14 +2155,15 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
              1);
       break;
     }
-    // (the streaming kernel's K split: the fp32 partial tiles' way out and
-    // in again and the second kernel, see splitPenaltyUs)
-    const double kSplitUs =
-        igemm.splitK > 1 && !igemm.patch
-            ? poplin::splitPenaltyUs(mxk::igemmWorkspaceBytes(igemm))
-            : 0.0;
+    // (K split: the fp32 partial tiles' way out and in again and the second
+    // kernel, see splitPenaltyUs)
+    const std::size_t partialBytes = mxk::igemmWorkspaceBytes(igemm);
+    const double kSplitUs = igemm.splitK <= 1 ? 0.0
+                            : igemm.patch
+                                ? poplin::patchSplitUs(partialBytes)
+                                : poplin::splitPenaltyUs(partialBytes);
     e.reductionUs = kSplitUs;
-    e.reductionBytes = kSplitUs > 0 ? mxk::igemmWorkspaceBytes(igemm) : 0;
+    e.reductionBytes = kSplitUs > 0 ? partialBytes : 0;
     bool weighed = false;
     for (const auto &c : candidates)
       if (c.chosen) {
@@ -2181,7 +2228,10 @@ std::string mxconv_plan::describe() const {
        << " operands, fp32 accumulate)"
        << (pointwiseOn ? ", pointwise streaming variant" : "")
        << (thinInputOn ? ", kernel rows as k-steps" : "")
-       << (igemm.patch ? ", input patch resident in LDS" : "")
+       << (!igemm.patch ? ""
+           : igemm.inChansPerGroup * params.inputType.size() % 128 == 0
+               ? ", input patch resident in LDS"
+               : ", input patch in LDS, its last channel slice a partial one")
        << (igemm.small ? ", small tiles" : "");
     break;
   case Kernel::DEPTHWISE:
@@ -2324,7 +2374,9 @@ std::string mxconv_plan::describe() const {
               "input)\n";
       if (g.patch)
         os << "        packed weights             [G=" << g.groups << "]["
-           << coPadded / 32 << " blocks of 32][" << k * params.inputType.size() / 128
+           << coPadded / 32 << " blocks of 32]["
+           << (std::size_t(g.inChansPerGroup) * params.inputType.size() + 127) /
+                  128 * g.kH * g.kW
            << " k-steps]"
            << (g.patch == 2 ? "[4 operands]" : "[2 halves][2]")
            << "[64 lanes][16 bytes]\n";
@@ -2441,11 +2493,15 @@ std::string mxconv_plan::describe() const {
        << (tiling.empty() ? "" : "; " + tiling) << "\n";
   }
   os << "        workspaceBytes             " << workspaceBytes << "\n";
-  if (kernel == Kernel::IGEMM && igemm.small) {
-    // the plan without the small tiles, which they were weighed against
+  if (kernel == Kernel::IGEMM &&
+      (igemm.small || (igemm.patch && igemm.splitK > 1))) {
+    // the plan without the small tiles, or without a resident patch and its
+    // parts of K, which they were weighed against
     poplin::ConvOptions o = options;
     o.planConstraints = poplin::PlanConstraints{};
     o.planConstraints.smallTile = 0;
+    if (!igemm.small)
+      o.planConstraints.patch = 0;
     o.planConstraints.convGroupsPerGroup = convGroupsPerGroup;
     const mxconv_plan other = poplin::makePlan(params, o);
     char line[96];
