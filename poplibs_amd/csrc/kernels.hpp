@@ -409,6 +409,9 @@ struct DepthwiseDesc {
   // pixels of a row at once (7 x 7 taps, unit stride and dilation:
   // depthwiseStripTakes): 4 or 7; 0 = a pixel at a time.
   uint32_t stripPixels = 0;
+  // depthwiseColumnsKernel's output columns per lane (4 or 8; 0: it is not that
+  // kernel's) and output rows of a band
+  uint32_t columns = 0, columnRows = 0;
   // Bytes of an input element: 2 (fp16: every depthwise kernel), 4 (fp32) or
   // 1 (fp8) - those two by the LDS-tiled kernel only.
   uint32_t elemBytes = 2;
@@ -419,6 +422,16 @@ bool depthwiseStripTakes(const DepthwiseDesc &d);
 /// and, with strips, the taps; what it may take at most.
 uint64_t depthwiseTileLdsBytes(const DepthwiseDesc &d);
 constexpr uint32_t kDepthwiseTileLdsMost = 80 * 1024;
+/// fp16, 5 x 5 or 7 x 7 taps, stride 1 or 2: a lane walks down a strip of
+/// output columns of one channel.
+bool depthwiseColumnsTakes(const DepthwiseDesc &d, int inType, int outType);
+/// Strip (4 or 8 columns; 0: the faster) and band for d, and what they take.
+void chooseDepthwiseColumns(DepthwiseDesc &d, uint32_t strip);
+double depthwiseColumnsEstimateUs(const DepthwiseDesc &d);
+hipError_t launchDepthwiseColumns(const DepthwiseDesc &d, int inType,
+                                  int outType, const void *in,
+                                  const void *weightsPacked, const void *bias,
+                                  void *out, hipStream_t stream);
 /// True for the shapes launchDepthwise3x3 takes.
 bool depthwise3x3Takes(const DepthwiseDesc &d, int inType);
 hipError_t launchDepthwise3x3(const DepthwiseDesc &d, int inType,

@@ -206,6 +206,11 @@ void checkGfx950(const std::string &path, const Value &v, PlanConstraints &pc) {
       if (v > 1)
         throw invalid_option("'" + sub + "': Must be 0 or 1");
       pc.rowRing = int(v);
+    } else if (m.first == "columns") {
+      const unsigned v = requireUnsigned(sub, m.second);
+      if (v != 0 && v != 4 && v != 8)
+        throw invalid_option("'" + sub + "': Must be 0, 4 or 8");
+      pc.columns = int(v);
     } else if (m.first == "pointwise") {
       const unsigned v = requireUnsigned(sub, m.second);
       if (v > 1)

@@ -1940,6 +1940,25 @@ mxconv_plan makePlanWith(const ConvParams &params,
             "planConstraints gfx950 tileH x tileW: the input patch of such a "
             "tile does not fit 64 KB of LDS");
     }
+    // 5 x 5 and 7 x 7 taps: strips of columns, wherever no other kernel is
+    // named.  Against the two kernels above, at their choice: of 130 random
+    // layers one was 3 % slower and two level, the others 1.03 to 7 times as
+    // fast; small, large, strided and narrow ones alike, so there is no line
+    // to draw.
+    const bool columns =
+        pc.columns != 0 && !(pc.tileH || pc.tileW) && pc.rowRing != 1 &&
+        mxk::depthwiseColumnsTakes(d, dwType,
+                                   params.outputType == poplar::HALF
+                                       ? mxk::kHalf
+                                       : mxk::kFloat);
+    if (columns)
+      mxk::chooseDepthwiseColumns(d, pc.columns > 0 ? uint32_t(pc.columns) : 0);
+    else if (pc.columns > 0)
+      throw poplar::invalid_option(
+          "planConstraints gfx950 columns: that kernel takes fp16 inputs, 5x5 "
+          "or 7x7 taps at stride 1 or 2, without a tile or rowRing named");
+    if (d.columns)
+      d.dense3x3 = 0, d.stripPixels = 0;
     plan.weightPackedElems = plan.weightElems; // [kH*kW][C]
   } else {
     plan.weightPackedElems = plan.weightElems; // [G][K][Ci][Co]
@@ -1970,7 +1989,9 @@ std::string mxconv_plan::constraintsJson() const {
     os << "\"kernel\": \"depthwise\", \"rowRing\": "
        << (depthwise.dense3x3 == 2 ? 1 : 0);
     // (an explicit tile names the LDS-tiled kernel)
-    if (!depthwise.dense3x3 && depthwise.inDilH == 1 && depthwise.inDilW == 1)
+    if (depthwise.columns)
+      os << ", \"columns\": " << depthwise.columns;
+    else if (!depthwise.dense3x3 && depthwise.inDilH == 1 && depthwise.inDilW == 1)
       os << ", \"tileH\": " << depthwise.tileH << ", \"tileW\": "
          << depthwise.tileW;
     break;
@@ -2105,7 +2126,9 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
     return e;
   case Kernel::DEPTHWISE:
     e.computeUs = streamed(inputBytes() + outputBytes() + weightPackedBytes());
-    if (depthwise.dense3x3 == 2)
+    if (depthwise.columns)
+      e.computeUs = mxk::depthwiseColumnsEstimateUs(depthwise);
+    else if (depthwise.dense3x3 == 2)
       spread(e, mxk::depthwiseRowsLaunchShape(depthwise).workgroups, 1);
     break;
   case Kernel::IGEMM: {
@@ -2241,6 +2264,8 @@ std::string mxconv_plan::describe() const {
            : depthwise.inDilH != 1 || depthwise.inDilW != 1
                ? "depthwise direct (vector ALU, one thread per output "
                  "vector, dilated input)"
+           : depthwise.columns
+               ? "depthwise direct (vector ALU, strips of columns in registers)"
            : depthwise.dense3x3 == 2
                ? "depthwise direct (vector ALU, input rows streamed through "
                  "an LDS ring by persistent workgroups)"
@@ -2404,7 +2429,10 @@ std::string mxconv_plan::describe() const {
   } else if (kernel == Kernel::DEPTHWISE) {
     const auto &d = depthwise;
     os << "        channels                   " << d.channels << "\n";
-    if (!d.dense3x3)
+    if (d.columns)
+      os << "        output columns per lane    " << d.columns
+         << ", walked down in bands of " << d.columnRows << " rows\n";
+    else if (!d.dense3x3)
       os << "        output tile H x W          " << d.tileH << " x "
          << d.tileW
          << (d.stripPixels == 7
@@ -2493,21 +2521,26 @@ std::string mxconv_plan::describe() const {
        << (tiling.empty() ? "" : "; " + tiling) << "\n";
   }
   os << "        workspaceBytes             " << workspaceBytes << "\n";
-  if (kernel == Kernel::IGEMM &&
-      (igemm.small || (igemm.patch && igemm.splitK > 1))) {
-    // the plan without the small tiles, or without a resident patch and its
-    // parts of K, which they were weighed against
+  const bool columns = kernel == Kernel::DEPTHWISE && depthwise.columns;
+  if (columns || (kernel == Kernel::IGEMM &&
+                  (igemm.small || (igemm.patch && igemm.splitK > 1)))) {
+    // the plan without the small tiles, without a resident patch and its
+    // parts of K or without strips of columns, which they stand in for
     poplin::ConvOptions o = options;
     o.planConstraints = poplin::PlanConstraints{};
-    o.planConstraints.smallTile = 0;
-    if (!igemm.small)
+    if (columns)
+      o.planConstraints.columns = 0;
+    else
+      o.planConstraints.smallTile = 0;
+    if (!columns && !igemm.small)
       o.planConstraints.patch = 0;
     o.planConstraints.convGroupsPerGroup = convGroupsPerGroup;
     const mxconv_plan other = poplin::makePlan(params, o);
-    char line[96];
-    std::snprintf(line, sizeof line,
-                  "  Left aside for it (estimates: %.1f us, above %.1f us):\n",
-                  other.estimatedMicroseconds(), estimatedMicroseconds());
+    char line[96] = "  Left aside for it:\n";
+    if (!columns) // (the other depthwise estimates count bytes alone)
+      std::snprintf(line, sizeof line,
+                    "  Left aside for it (estimates: %.1f us, above %.1f us):\n",
+                    other.estimatedMicroseconds(), estimatedMicroseconds());
     // (without the heading, which names the chip again)
     const std::string text = other.describe();
     os << line << text.substr(text.find('\n') + 1);
