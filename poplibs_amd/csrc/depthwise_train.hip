@@ -380,23 +380,34 @@ __global__ __launch_bounds__(256) void depthwiseWeightDeltaKernel(
         float4{acc[i], acc[i + 1], acc[i + 2], acc[i + 3]};
 }
 
+// The sum has eight parts where the outputs (taps x channels) outnumber this.
+constexpr uint32_t kManyOutputs = 3500, kManyOutputsPerSlice = 25;
+
 /// out[c][tap] = sum over slices of partial[slice][tap][c], in a fixed order:
-/// a workgroup of 16 waves takes 16 outputs and cuts the slices into 64
-/// contiguous parts, a quarter of a wave (16 lanes, 64 contiguous bytes per
-/// slice) to each; a lane adds up its part with sixteen loads in flight, then
-/// one thread per output adds the 64 sums in order.  Few outputs per
-/// workgroup, because the outputs are few (taps x channels) and the walk over
-/// the slices is a chain of memory latencies: this way there are four times
-/// the workgroups and a quarter of the chain.
-template <class OutT>
-__global__ __launch_bounds__(1024) void depthwiseDeltaSumKernel(
+/// a workgroup takes COLUMNS outputs and cuts the slices into PARTS contiguous
+/// parts, COLUMNS lanes (contiguous in a slice) to each; a lane adds up its
+/// part with sixteen loads in flight, then the sums of an output meet in steps
+/// of eight, each in order (one thread adding all 64 is a chain of 64 LDS reads
+/// at the kernel's end).
+///
+/// The walk over the slices is a chain of memory latencies.  64 parts of 16
+/// outputs make it short, but launch a wave for every output: with many of
+/// those, eight parts of 32 take a quarter of the time (5 x 5 taps, 960
+/// channels, 16 slices: 8.0 -> 3.2 us).  Their chain is eight times as long,
+/// which shows right behind the kernel that writes the slices: of 70 passes the
+/// line below is where both are level (3 x 3, 128 channels, 80 slices 7.5 us
+/// with 64 parts, 8.4 with eight; 688, 256 slices 17.8 and 20.5; 920, 31
+/// slices 9.4 and 7.7; 5 x 5, 904, 93 slices 29.3 and 26.5).
+template <class OutT, int PARTS, int COLUMNS>
+__global__ __launch_bounds__(PARTS *COLUMNS) void depthwiseDeltaSumKernel(
     const float *__restrict__ partial, uint32_t slices, uint32_t taps,
     uint32_t channels, OutT *__restrict__ out) {
-  __shared__ float meet[64][16];
-  const uint32_t column = threadIdx.x % 16, part = threadIdx.x / 16;
+  static_assert(PARTS == 8 || PARTS == 64);
+  __shared__ float meet[PARTS][COLUMNS];
+  const uint32_t column = threadIdx.x % COLUMNS, part = threadIdx.x / COLUMNS;
   const uint32_t outputs = taps * channels;
-  const uint32_t i = blockIdx.x * 16 + column; // tap * C + c
-  const uint32_t per = (slices + 63) / 64;
+  const uint32_t i = blockIdx.x * COLUMNS + column; // tap * C + c
+  const uint32_t per = (slices + PARTS - 1) / PARTS;
   const uint32_t from = min(part * per, slices), to = min(from + per, slices);
   constexpr int kInFlight = 16;
   float sum[kInFlight] = {};
@@ -416,21 +427,21 @@ __global__ __launch_bounds__(1024) void depthwiseDeltaSumKernel(
 #pragma unroll
     for (int u = 0; u != width; ++u)
       sum[u] += sum[u + width];
-  // The 64 sums of an output meet in two steps of eight, each in order (one
-  // thread adding all 64 is a chain of 64 LDS reads at the kernel's end).
   meet[part][column] = sum[0];
   __syncthreads();
-  float eight = 0.0f;
-  if (part < 8) {
-    eight = meet[part * 8][column];
+  if constexpr (PARTS == 64) {
+    float eight = 0.0f;
+    if (part < 8) {
+      eight = meet[part * 8][column];
 #pragma unroll
-    for (int w = 1; w != 8; ++w)
-      eight += meet[part * 8 + w][column];
+      for (int w = 1; w != 8; ++w)
+        eight += meet[part * 8 + w][column];
+    }
+    __syncthreads();
+    if (part < 8)
+      meet[part][column] = eight;
+    __syncthreads();
   }
-  __syncthreads();
-  if (part < 8)
-    meet[part][column] = eight;
-  __syncthreads();
   if (part != 0 || i >= outputs)
     return;
   float total = meet[0][column];
@@ -439,6 +450,22 @@ __global__ __launch_bounds__(1024) void depthwiseDeltaSumKernel(
     total += meet[w][column];
   const uint32_t tap = i / channels, c = i - tap * channels;
   storeOut(out, size_t(c) * taps + tap, total);
+}
+
+template <class OutT>
+void launchDeltaSum(const float *partial, uint32_t slices, uint32_t taps,
+                    uint32_t channels, void *out, hipStream_t stream) {
+  const uint32_t outputs = taps * channels;
+  if (outputs < kManyOutputs + uint64_t(kManyOutputsPerSlice) * slices)
+    hipLaunchKernelGGL((depthwiseDeltaSumKernel<OutT, 64, 16>),
+                       dim3((outputs + 15) / 16), dim3(1024), 0, stream,
+                       partial, slices, taps, channels,
+                       static_cast<OutT *>(out));
+  else
+    hipLaunchKernelGGL((depthwiseDeltaSumKernel<OutT, 8, 32>),
+                       dim3((outputs + 31) / 32), dim3(256), 0, stream,
+                       partial, slices, taps, channels,
+                       static_cast<OutT *>(out));
 }
 
 /// Threads of a workgroup: itemsPerBlock items by `slots` parts of a slice.
@@ -589,17 +616,12 @@ hipError_t launchDepthwiseWeightDeltas(const DepthwiseDesc &d, int outType,
                          stream, a, static_cast<const __half *>(acts),
                          static_cast<const __half *>(deltas), partial);
   }
-  const uint32_t outputs = a.taps * d.channels;
-  const dim3 grid2{(outputs + 15) / 16};
-  const dim3 block2{1024};
   if (outType == kHalf)
-    hipLaunchKernelGGL(depthwiseDeltaSumKernel<__half>, grid2, block2, 0, stream,
-                       partial, a.slices, a.taps, d.channels,
-                       static_cast<__half *>(weightDeltas));
+    launchDeltaSum<__half>(partial, a.slices, a.taps, d.channels, weightDeltas,
+                           stream);
   else if (outType == kFloat)
-    hipLaunchKernelGGL(depthwiseDeltaSumKernel<float>, grid2, block2, 0, stream,
-                       partial, a.slices, a.taps, d.channels,
-                       static_cast<float *>(weightDeltas));
+    launchDeltaSum<float>(partial, a.slices, a.taps, d.channels, weightDeltas,
+                          stream);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
