@@ -1,36 +1,40 @@
 // Depthwise convolution with 5 x 5 or 7 x 7 taps at stride 1 or 2: a lane
-// walks down a strip of output columns of one channel.
+// walks down a strip of output columns of two neighbouring channels.
 //
 // Twenty-five or forty-nine multiply-adds per output and channel make the
 // vector ALU the bound, so the kernel is built around it: a lane holds its
-// channel's taps, the sums of the output rows under way (as many as a kernel
+// channels' taps, the sums of the output rows under way (as many as a kernel
 // meets an input row in) and one input row of its strip, and every input
 // element is read once per strip - not once per tap.  An input row of STRIP
-// outputs is S (STRIP - 1) + K columns, one load each, asked for a row ahead;
-// with unit stride and 7 x 7 taps it feeds 7 output rows of 8 columns x 7
-// taps, 392 multiply-adds for 14 loads.  Taps and columns go into the sums in
-// pairs (v_dot2_f32_f16: exact products, fp32 sums; 4.7 cycles a wave against
-// 2.3 to 2.9 for each of two fmac, so no faster in itself, but half the
-// registers of fp32 taps and no conversions: 7 to 14 % over the same kernel on
-// fp32 values); the odd last tap is a multiply-add on fp32 values, because a
-// pair filled with a zero tap would turn an infinity beside the window into a
-// NaN.  Against 64 bits the sums' error is 0.83 to 0.95 times a chain of fp32
-// multiply-adds (rms), and fp16 subnormals stay exact.
+// outputs is S (STRIP - 1) + K columns, one 4-byte load each, asked for a row
+// ahead; with unit stride and 7 x 7 taps it feeds 7 output rows of 4 columns x
+// 7 taps x 2 channels, 392 multiply-adds for 10 loads.  (A load instruction
+// holds the address unit for some eight cycles whatever its width: one channel
+// to a lane and strips twice as wide is 14 loads for them, and twice the
+// stores; 5 to 20 % slower with 5 x 5 taps.)
 //
-// Nothing goes through LDS.  Lanes are dealt (image, strip, channel), channel
-// fastest, so that a load is a run of neighbouring channels; a band of output
-// rows is a grid dimension.  Rows outside the input are left out, columns
-// outside it read as zeros (out-of-range buffer offsets).
+// Taps and columns go into the sums in pairs (v_dot2_f32_f16: exact products,
+// fp32 sums; 4.7 cycles a wave against 2.3 to 2.9 for each of two fmac, so no
+// faster in itself, but half the registers of fp32 taps and no conversions: 7
+// to 14 % over the same kernel on fp32 values); the odd last tap is a
+// multiply-add on fp32 values, because a pair filled with a zero tap would turn
+// an infinity beside the window into a NaN.  Against 64 bits the sums' error is
+// 0.83 to 0.95 times a chain of fp32 multiply-adds (rms), and fp16 subnormals
+// stay exact.
+//
+// Nothing goes through LDS.  Lanes are dealt (image, strip, channel pair),
+// channels fastest, so that a load is a run of neighbouring channels; a band of
+// output rows is a grid dimension.  Rows outside the input are left out,
+// columns outside it read as zeros (out-of-range buffer offsets).
 //
 // Measured (N x H x W, channels; us; the LDS-tiled or row-ring kernel before):
-// 7 x 7 taps 57 x 28 x 28, 240: 44.9 -> 20.7; 64 x 7 x 7, 768: 16.8 -> 9.5;
-// stride 2, 13 x 106 x 106, 304: 191 -> 34.8 (its tensors' bytes take 21);
-// 5 x 5 taps 32 x 28 x 28, 240: 15.8 -> 11.5; 8 x 90 x 90, 48: 13.2 -> 8.5;
-// stride 2, 32 x 28 x 28, 240: 10.1 -> 7.7; 32 x 112 x 112, 96: 25.2 -> 22.6.
-// Over 130 random layers 1.81 times as fast (geometric mean).  3 x 3 taps stay
-// with their own kernels, which are bound by the bytes: this one was within
-// 10 % of them either way for most layers and 1.3 to 1.5 us slower for small
-// ones.
+// 7 x 7 taps 57 x 28 x 28, 240: 44.9 -> 19.8; 64 x 7 x 7, 768: 16.8 -> 9.7;
+// stride 2, 13 x 106 x 106, 304: 191 -> 31.5 (its tensors' bytes take 21);
+// 5 x 5 taps 32 x 28 x 28, 240: 15.8 -> 10.4; 8 x 90 x 90, 48: 13.2 -> 7.6;
+// stride 2, 32 x 28 x 28, 240: 10.1 -> 6.5; 32 x 112 x 112, 96: 25.2 -> 20.4.
+// 3 x 3 taps stay with their own kernels, which are bound by the bytes: this
+// one (of one channel to a lane) was within 10 % of them either way for most
+// layers and 1.3 to 1.5 us slower for small ones.
 //
 // The reference's role: depthwise layers go through
 // lib/poplin/codelets/ConvPartialHorizontalMac.cpp there.
@@ -46,20 +50,30 @@ constexpr uint32_t kColInvalid = 0x40000000u;
 constexpr int kColThreads = 256;
 
 struct ColumnsArgs {
-  uint32_t items; // image x strip x channel
-  uint32_t channels, strips, bands, bandRows, outH, outW;
+  uint32_t items; // image x strip x pair of channels
+  uint32_t pairs, strips, bands, bandRows, outH, outW;
   int32_t padH, padW;
   uint32_t loH, hiH, loW, hiW;
   uint32_t pixelBytes, rowBytes, imageBytes, inBytes; // of the input
   uint32_t outPixelBytes, outRowBytes, outImageBytes, outBytes;
-  FastDiv divChannels, divStrips, divBands;
+  FastDiv divPairs, divStrips, divBands;
 };
 
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ half2v pairOf(uint16_t low, uint16_t high) {
-  return half2v{__builtin_bit_cast(_Float16, low),
-                __builtin_bit_cast(_Float16, high)};
+/// Channel CH of two elements of a channel pair.
+template <int CH>
+__device__ __forceinline__ half2v pairOf(uint32_t first, uint32_t second) {
+  return __builtin_bit_cast(
+      half2v, __builtin_amdgcn_perm(second, first,
+                                    CH == 0 ? 0x05040100u : 0x07060302u));
+}
+template <int CH> __device__ __forceinline__ float channelOf(uint32_t two) {
+  float v = float(__builtin_bit_cast(half2v, two)[CH]);
+  // (a float from here on: a multiply-add that converts runs at half the rate)
+  asm("" : "+v"(v));
+  return v;
 }
 
 /// Calls each with 0, 1, ... until one answers false.
@@ -73,7 +87,7 @@ __device__ __forceinline__ bool whileEach(std::integer_sequence<int, I...>,
 template <int K, int S, int STRIP, class OutT>
 __global__ __launch_bounds__(kColThreads) void depthwiseColumnsKernel(
     const ColumnsArgs a, const char *__restrict__ in,
-    const __half *__restrict__ weights, const OutT *__restrict__ bias,
+    const uint32_t *__restrict__ weights, const OutT *__restrict__ bias,
     char *__restrict__ out) {
   constexpr int NX = S * (STRIP - 1) + K;  // input columns of a strip
   constexpr int LIVE = (K + S - 1) / S;    // output rows under way
@@ -84,7 +98,7 @@ __global__ __launch_bounds__(kColThreads) void depthwiseColumnsKernel(
   const uint32_t item = itemBlock * kColThreads + threadIdx.x;
   const bool here = item < a.items;
   const uint32_t id = here ? item : 0;
-  const uint32_t over = a.divChannels(id), c = id - over * a.channels;
+  const uint32_t over = a.divPairs(id), c = id - over * a.pairs;
   const uint32_t b = a.divStrips(over), x0 = (over - b * a.strips) * STRIP;
   const uint32_t y0 = band * a.bandRows;
   const uint32_t rowsOut = a.outH - y0 < a.bandRows ? a.outH - y0 : a.bandRows;
@@ -95,7 +109,7 @@ __global__ __launch_bounds__(kColThreads) void depthwiseColumnsKernel(
   uint32_t offset[NX];
   {
     const uint32_t first = x0 * S - uint32_t(a.padW);
-    const uint32_t at = b * a.imageBytes + c * 2;
+    const uint32_t at = b * a.imageBytes + c * 4;
 #pragma unroll
     for (int i = 0; i != NX; ++i)
       offset[i] = here && first + i - a.loW < a.hiW - a.loW
@@ -109,40 +123,42 @@ __global__ __launch_bounds__(kColThreads) void depthwiseColumnsKernel(
   auto rowInside = [&](uint32_t r) {
     return uint32_t(firstRow + int(r)) - a.loH < a.hiH - a.loH;
   };
-  uint16_t raw[NX];
+  uint32_t raw[NX];
   auto load = [&](uint32_t r) {
     const uint32_t at =
         (rowInside(r) ? uint32_t(firstRow + int(r)) : a.loH) * a.rowBytes;
 #pragma unroll
     for (int i = 0; i != NX; ++i)
-      raw[i] = uint16_t(
-          __builtin_amdgcn_raw_buffer_load_b16(inBuf, offset[i], at, 0));
+      raw[i] = __builtin_amdgcn_raw_buffer_load_b32(inBuf, offset[i], at, 0);
   };
   load(0);
-  half2v pair[K][K / 2];
-  float last[K];
-  const __half *w = weights + c;
+  half2v pair[2][K][K / 2];
+  float last[2][K];
+  const uint32_t *w = weights + c;
 #pragma unroll
   for (int kh = 0; kh != K; ++kh) {
 #pragma unroll
-    for (int kw = 0; kw != K / 2; ++kw)
-      pair[kh][kw] = pairOf(
-          __half_as_ushort(w[(kh * K + 2 * kw) * a.channels]),
-          __half_as_ushort(w[(kh * K + 2 * kw + 1) * a.channels]));
-    last[kh] = __half2float(w[(kh * K + K - 1) * a.channels]);
-    // (a float from here on: a multiply-add that converts runs at half the
-    // rate)
-    asm("" : "+v"(last[kh]));
+    for (int kw = 0; kw != K / 2; ++kw) {
+      const uint32_t first = w[(kh * K + 2 * kw) * a.pairs],
+                     second = w[(kh * K + 2 * kw + 1) * a.pairs];
+      pair[0][kh][kw] = pairOf<0>(first, second);
+      pair[1][kh][kw] = pairOf<1>(first, second);
+    }
+    const uint32_t odd = w[(kh * K + K - 1) * a.pairs];
+    last[0][kh] = channelOf<0>(odd), last[1][kh] = channelOf<1>(odd);
   }
-  const float start = bias ? Load<OutT>::at(bias, c, 0) : 0.0f;
-  float sum[LIVE][STRIP];
+  const float start[2] = {bias ? Load<OutT>::at(bias, 2 * c, 0) : 0.0f,
+                          bias ? Load<OutT>::at(bias, 2 * c + 1, 0) : 0.0f};
+  float sum[2][LIVE][STRIP];
 #pragma unroll
-  for (int l = 0; l != LIVE; ++l)
+  for (int ch = 0; ch != 2; ++ch)
 #pragma unroll
-    for (int j = 0; j != STRIP; ++j)
-      sum[l][j] = 0.0f;
+    for (int l = 0; l != LIVE; ++l)
+#pragma unroll
+      for (int j = 0; j != STRIP; ++j)
+        sum[ch][l][j] = 0.0f;
   const uint32_t outAt =
-      b * a.outImageBytes + x0 * a.outPixelBytes + c * uint32_t(sizeof(OutT));
+      b * a.outImageBytes + x0 * a.outPixelBytes + c * 2 * uint32_t(sizeof(OutT));
 
   uint32_t base = 0;
   while (whileEach(std::make_integer_sequence<int, PERIOD>{}, [&](auto step) {
@@ -150,16 +166,16 @@ __global__ __launch_bounds__(kColThreads) void depthwiseColumnsKernel(
       const uint32_t r = base + R;
       if (r >= rowsIn)
         return false;
-      half2v x[NX]; // columns i and i + 1
-      float end[STRIP];
+      half2v x[2][NX]; // columns i and i + 1
+      float end[2][STRIP];
 #pragma unroll
       for (int i = 0; i < NX - 1; i += S)
-        x[i] = pairOf(raw[i], raw[i + 1]);
+        x[0][i] = pairOf<0>(raw[i], raw[i + 1]),
+        x[1][i] = pairOf<1>(raw[i], raw[i + 1]);
 #pragma unroll
-      for (int j = 0; j != STRIP; ++j) {
-        end[j] = __half2float(__ushort_as_half(raw[j * S + K - 1]));
-        asm("" : "+v"(end[j]));
-      }
+      for (int j = 0; j != STRIP; ++j)
+        end[0][j] = channelOf<0>(raw[j * S + K - 1]),
+        end[1][j] = channelOf<1>(raw[j * S + K - 1]);
       load(r + 1);
       auto add = [&](auto row) {
         constexpr int KH = decltype(row)::value;
@@ -169,11 +185,16 @@ __global__ __launch_bounds__(kColThreads) void depthwiseColumnsKernel(
           for (int kw = 0; kw != K / 2; ++kw)
 #pragma unroll
             for (int j = 0; j != STRIP; ++j)
-              sum[L][j] = __builtin_amdgcn_fdot2(
-                  pair[KH][kw], x[j * S + 2 * kw], sum[L][j], false);
+#pragma unroll
+              for (int ch = 0; ch != 2; ++ch)
+                sum[ch][L][j] = __builtin_amdgcn_fdot2(
+                    pair[ch][KH][kw], x[ch][j * S + 2 * kw], sum[ch][L][j],
+                    false);
 #pragma unroll
           for (int j = 0; j != STRIP; ++j)
-            sum[L][j] = fmaf(last[KH], end[j], sum[L][j]);
+#pragma unroll
+            for (int ch = 0; ch != 2; ++ch)
+              sum[ch][L][j] = fmaf(last[ch][KH], end[ch][j], sum[ch][L][j]);
         }
       };
       if (rowInside(r)) {
@@ -193,17 +214,22 @@ __global__ __launch_bounds__(kColThreads) void depthwiseColumnsKernel(
             const uint32_t at = here && x0 + j < a.outW
                                     ? outAt + j * a.outPixelBytes
                                     : kOutOfRange;
-            float v = sum[L][j] + start;
-            asm("" : "+v"(v)); // (rounded once, from the fp32 sum)
+            float v[2];
+#pragma unroll
+            for (int ch = 0; ch != 2; ++ch) {
+              v[ch] = sum[ch][L][j] + start[ch];
+              asm("" : "+v"(v[ch])); // (rounded once, from the fp32 sum)
+              sum[ch][L][j] = 0.0f;
+            }
             if constexpr (sizeof(OutT) == 2)
-              __builtin_amdgcn_raw_buffer_store_b16(
-                  short(__half_as_ushort(__float2half_rn(v))), outBuf, at,
-                  y * a.outRowBytes, 0);
-            else
               __builtin_amdgcn_raw_buffer_store_b32(
-                  __builtin_bit_cast(uint32_t, v), outBuf, at,
-                  y * a.outRowBytes, 0);
-            sum[L][j] = 0.0f;
+                  __builtin_bit_cast(uint32_t, __floats2half2_rn(v[0], v[1])),
+                  outBuf, at, y * a.outRowBytes, 0);
+            else
+              __builtin_amdgcn_raw_buffer_store_b64(
+                  u32x2{__builtin_bit_cast(uint32_t, v[0]),
+                        __builtin_bit_cast(uint32_t, v[1])},
+                  outBuf, at, y * a.outRowBytes, 0);
           }
         }
       }
@@ -214,7 +240,7 @@ __global__ __launch_bounds__(kColThreads) void depthwiseColumnsKernel(
 
 uint64_t columnItems(const DepthwiseDesc &d) {
   return uint64_t(d.batch) * ((d.outW + d.columns - 1) / d.columns) *
-         d.channels;
+         (d.channels / 2);
 }
 
 } // namespace
@@ -231,17 +257,16 @@ bool depthwiseColumnsTakes(const DepthwiseDesc &d, int inType, int outType) {
          d.strideH == d.strideW && (d.strideH == 1 || d.strideH == 2) &&
          d.dilH == 1 && d.dilW == 1 && d.inDilH == 1 && d.inDilW == 1 &&
          d.loH < d.hiH && d.hiH <= d.inH && d.loW < d.hiW && d.hiW <= d.inW &&
-         d.channels != 0 && d.batch != 0 && d.outH != 0 && d.outW != 0 &&
+         d.channels != 0 && d.channels % 2 == 0 && d.batch != 0 && d.outH != 0 && d.outW != 0 &&
          inImage < kColInvalid && outImage < kColInvalid && d.padH > -most &&
          d.padH < most && d.padW > -most && d.padW < most;
 }
 
-// What a strip and a band cost, fitted to 1800 timings of 130 random layers
-// (median error 5 %; the choice by it is within 2 % of the best on average):
-// a wave issues its multiply-adds and, for each input row, two instructions a
-// column and some twenty around them; the waves of a SIMD take turns, as if
-// there were half a one more (their waits); a round of waves begins with its
-// taps, and the tensors pass at 4.1 TB/s beside it.
+// What a strip and a band cost, fitted to 1700 timings of 130 random layers
+// (the choice by it is within 2 % of the best on average): a wave issues its
+// multiply-adds and, for each input row, three instructions a column and some
+// twenty around them; the waves of a SIMD take turns, as if there were two
+// thirds of one more (their waits), and the tensors pass at 5 TB/s beside it.
 double depthwiseColumnsEstimateUs(const DepthwiseDesc &d) {
   const uint32_t k = d.kH, s = d.strideH, strip = d.columns;
   const double rows = std::min(d.columnRows, d.outH);
@@ -250,27 +275,27 @@ double depthwiseColumnsEstimateUs(const DepthwiseDesc &d) {
       std::ceil(double(columnItems(d)) / kColThreads) * bands;
   const double rowsIn = (rows - 1) * s + k;
   const double columnsIn = s * (strip - 1) + k;
-  const double waveUs = (3.73 * rows * strip * k * (k / 2 + 1) +
-                         8.42 * rowsIn * (2 * columnsIn + 20)) *
+  const double waveUs = (4.34 * 2 * rows * strip * k * (k / 2 + 1) +
+                         5.88 * rowsIn * (3 * columnsIn + 20)) *
                         1e-3 / 2.4;
   // (waves a SIMD holds, by the kernels' registers)
-  const double resident = k == 5 ? (strip == 4 ? 6 : 4) : (strip == 4 ? 4 : 3);
+  const double resident =
+      k == 5 ? (strip == 2 ? (s == 1 ? 5 : 6) : 4) : (strip == 2 ? 4 : 3);
   const double perCu = blocks / 256;
   const double full = std::floor(perCu / resident);
   const double rest = std::ceil(perCu - full * resident);
-  const double us =
-      full * (resident + 0.53) * waveUs +
-      (rest > 0 ? (rest + 0.53) * waveUs + 0.051 * k : 0.0);
+  const double us = full * (resident + 0.68) * waveUs +
+                    (rest > 0 ? (rest + 0.68) * waveUs : 0.0);
   const double bytes = 2.0 * d.batch * d.channels *
                        (double(d.inH) * d.inW + double(d.outH) * d.outW);
-  return 3.5 + std::sqrt(std::hypot(us * us, std::pow(bytes / 4.1e6, 2)));
+  return 3.9 + std::sqrt(std::hypot(us * us, std::pow(bytes / 5.0e6, 2)));
 }
 
 void chooseDepthwiseColumns(DepthwiseDesc &d, uint32_t strip) {
   DepthwiseDesc t = d;
   double best = 0;
   d.columns = 0;
-  for (t.columns = 4; t.columns <= 8; t.columns += 4) {
+  for (t.columns = 2; t.columns <= 4; t.columns += 2) {
     if (strip != 0 && t.columns != strip)
       continue;
     for (uint32_t bands = 1; bands <= 32 && bands <= d.outH; ++bands) {
@@ -291,14 +316,14 @@ hipError_t launchColumns(const ColumnsArgs &a, uint32_t blocks, int outType,
     hipLaunchKernelGGL((depthwiseColumnsKernel<K, S, STRIP, __half>),
                        dim3(blocks), dim3(kColThreads), 0, stream, a,
                        static_cast<const char *>(in),
-                       static_cast<const __half *>(weights),
+                       static_cast<const uint32_t *>(weights),
                        static_cast<const __half *>(bias),
                        static_cast<char *>(out));
   else
     hipLaunchKernelGGL((depthwiseColumnsKernel<K, S, STRIP, float>),
                        dim3(blocks), dim3(kColThreads), 0, stream, a,
                        static_cast<const char *>(in),
-                       static_cast<const __half *>(weights),
+                       static_cast<const uint32_t *>(weights),
                        static_cast<const float *>(bias),
                        static_cast<char *>(out));
   return hipGetLastError();
@@ -310,11 +335,11 @@ hipError_t launchDepthwiseColumns(const DepthwiseDesc &d, int inType,
                                   const void *weightsPacked, const void *bias,
                                   void *out, hipStream_t stream) {
   if (!depthwiseColumnsTakes(d, inType, outType) ||
-      (d.columns != 4 && d.columns != 8) || d.columnRows == 0)
+      (d.columns != 2 && d.columns != 4) || d.columnRows == 0)
     return hipErrorInvalidValue;
   ColumnsArgs a{};
   a.items = uint32_t(columnItems(d));
-  a.channels = d.channels, a.strips = (d.outW + d.columns - 1) / d.columns;
+  a.pairs = d.channels / 2, a.strips = (d.outW + d.columns - 1) / d.columns;
   a.bandRows = std::min(d.columnRows, d.outH);
   a.bands = (d.outH + a.bandRows - 1) / a.bandRows;
   a.outH = d.outH, a.outW = d.outW;
@@ -327,7 +352,7 @@ hipError_t launchDepthwiseColumns(const DepthwiseDesc &d, int inType,
   a.outRowBytes = d.outW * a.outPixelBytes;
   a.outImageBytes = d.outH * a.outRowBytes;
   a.outBytes = d.batch * a.outImageBytes;
-  a.divChannels = makeFastDiv(a.channels), a.divStrips = makeFastDiv(a.strips);
+  a.divPairs = makeFastDiv(a.pairs), a.divStrips = makeFastDiv(a.strips);
   a.divBands = makeFastDiv(a.bands);
   const uint64_t blocks =
       (columnItems(d) + kColThreads - 1) / kColThreads * a.bands;
@@ -337,10 +362,10 @@ hipError_t launchDepthwiseColumns(const DepthwiseDesc &d, int inType,
     return hipErrorInvalidConfiguration;
   auto go = [&](auto k, auto s) {
     constexpr int K = decltype(k)::value, S = decltype(s)::value;
-    return d.columns == 4
-               ? launchColumns<K, S, 4>(a, uint32_t(blocks), outType, in, weightsPacked,
+    return d.columns == 2
+               ? launchColumns<K, S, 2>(a, uint32_t(blocks), outType, in, weightsPacked,
                                         bias, out, stream)
-               : launchColumns<K, S, 8>(a, uint32_t(blocks), outType, in, weightsPacked,
+               : launchColumns<K, S, 4>(a, uint32_t(blocks), outType, in, weightsPacked,
                                         bias, out, stream);
   };
   using One = std::integral_constant<int, 1>;

@@ -565,6 +565,9 @@ hipError_t launchDepthwiseDirect(const DepthwiseDesc &d, int inType,
 size_t depthwiseWeightDeltaWorkspaceBytes(const DepthwiseDesc &d) {
   if (d.dense3x3 == 2)
     return depthwiseRowsDeltaWorkspaceBytes(d);
+  if (d.columns)
+    return size_t(depthwiseColumnDeltasSlices(d)) * d.kH * d.kW * d.channels *
+           sizeof(float);
   return size_t(deltaSlices(d)) * d.kH * d.kW * d.channels * sizeof(float);
 }
 
@@ -594,6 +597,12 @@ hipError_t launchDepthwiseWeightDeltas(const DepthwiseDesc &d, int outType,
     // persistent workgroups with the rows in LDS rings: one tile each
     const hipError_t e = launchDepthwiseRowsDeltas(d, acts, deltas, partial,
                                                    &a.slices, stream);
+    if (e != hipSuccess)
+      return e;
+  } else if (d.columns) {
+    a.slices = depthwiseColumnDeltasSlices(d);
+    const hipError_t e =
+        launchDepthwiseColumnDeltas(d, acts, deltas, partial, stream);
     if (e != hipSuccess)
       return e;
   } else {

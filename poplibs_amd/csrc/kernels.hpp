@@ -409,9 +409,10 @@ struct DepthwiseDesc {
   // pixels of a row at once (7 x 7 taps, unit stride and dilation:
   // depthwiseStripTakes): 4 or 7; 0 = a pixel at a time.
   uint32_t stripPixels = 0;
-  // depthwiseColumnsKernel's output columns per lane (4 or 8; 0: it is not that
-  // kernel's) and output rows of a band
-  uint32_t columns = 0, columnRows = 0;
+  // depthwiseColumnsKernel's and depthwiseColumnDeltasKernel's output columns
+  // per lane (2 or 4; 0: another kernel's) and output rows of a band; strips
+  // that a lane of the latter walks down one after the other
+  uint32_t columns = 0, columnRows = 0, columnRounds = 0;
   // Bytes of an input element: 2 (fp16: every depthwise kernel), 4 (fp32) or
   // 1 (fp8) - those two by the LDS-tiled kernel only.
   uint32_t elemBytes = 2;
@@ -425,13 +426,22 @@ constexpr uint32_t kDepthwiseTileLdsMost = 80 * 1024;
 /// fp16, 5 x 5 or 7 x 7 taps, stride 1 or 2: a lane walks down a strip of
 /// output columns of one channel.
 bool depthwiseColumnsTakes(const DepthwiseDesc &d, int inType, int outType);
-/// Strip (4 or 8 columns; 0: the faster) and band for d, and what they take.
+/// Strip (2 or 4 columns; 0: the faster) and band for d, and what they take.
 void chooseDepthwiseColumns(DepthwiseDesc &d, uint32_t strip);
 double depthwiseColumnsEstimateUs(const DepthwiseDesc &d);
 hipError_t launchDepthwiseColumns(const DepthwiseDesc &d, int inType,
                                   int outType, const void *in,
                                   const void *weightsPacked, const void *bias,
                                   void *out, hipStream_t stream);
+/// The weight deltas of half layers of 3 x 3, 5 x 5 or 7 x 7 taps the same way:
+/// one fp32 tile [taps][C] per slice at partial[slice], to be added in order.
+bool depthwiseColumnDeltasTakes(const DepthwiseDesc &d);
+void chooseDepthwiseColumnDeltas(DepthwiseDesc &d, uint32_t strip);
+double depthwiseColumnDeltasEstimateUs(const DepthwiseDesc &d);
+uint32_t depthwiseColumnDeltasSlices(const DepthwiseDesc &d);
+hipError_t launchDepthwiseColumnDeltas(const DepthwiseDesc &d,
+                                       const void *acts, const void *deltas,
+                                       float *partial, hipStream_t stream);
 /// True for the shapes launchDepthwise3x3 takes.
 bool depthwise3x3Takes(const DepthwiseDesc &d, int inType);
 hipError_t launchDepthwise3x3(const DepthwiseDesc &d, int inType,

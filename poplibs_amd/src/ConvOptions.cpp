@@ -208,8 +208,8 @@ void checkGfx950(const std::string &path, const Value &v, PlanConstraints &pc) {
       pc.rowRing = int(v);
     } else if (m.first == "columns") {
       const unsigned v = requireUnsigned(sub, m.second);
-      if (v != 0 && v != 4 && v != 8)
-        throw invalid_option("'" + sub + "': Must be 0, 4 or 8");
+      if (v != 0 && v != 2 && v != 4)
+        throw invalid_option("'" + sub + "': Must be 0, 2 or 4");
       pc.columns = int(v);
     } else if (m.first == "pointwise") {
       const unsigned v = requireUnsigned(sub, m.second);

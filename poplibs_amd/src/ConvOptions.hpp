@@ -53,9 +53,10 @@ struct PlanConstraints {
   /// input rows in LDS: -1 planner's choice, 0 never, 1 whenever it can take
   /// the layer.
   int rowRing = -1;
-  /// The depthwise 5x5 and 7x7 kernel whose lanes walk down strips of output
-  /// columns: -1 planner's choice (never with a tile or rowRing 1), 0 never, 4
-  /// or 8 that strip (an error where it cannot take the layer).
+  /// The depthwise kernels whose lanes walk down strips of output columns
+  /// (forward: 5x5 and 7x7 taps; weight deltas: 3x3 too): -1 planner's choice
+  /// (never with a tile or rowRing 1), 0 never, 2 or 4 that strip (an error
+  /// where they cannot take the layer).
   int columns = -1;
   /// 64-channel tiles of the output per workgroup of the pointwise streaming
   /// kernel (1 to 4); 0 = planner's choice.

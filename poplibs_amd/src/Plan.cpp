@@ -852,6 +852,27 @@ mxconv_plan makePlanWith(const ConvParams &params,
            (l.workgroups * 2 >= gfx950::numCUs && l.rowsOut >= 4 &&
             (l.colsOut >= 4 || l.strips == 1))))
         f.dense3x3 = 2;
+      // Strips of columns for the others from some amount of work on: below,
+      // the kernel's longer program and the meeting of its sums cost 1 to 4 us
+      // more than they save (of 150 random layers, each above its line 1.02 to
+      // 5.5 times as fast, the ones below 0.6 to 1.2).
+      const double products =
+          double(f.batch) * f.outH * f.outW * f.channels * f.kH * f.kW;
+      const double enough = f.kH == 3 ? 8e6 : f.kH == 5 ? 20e6 : 43e6;
+      const int asked = options.planConstraints.columns;
+      const bool takes = params.inputType == poplar::HALF &&
+                         options.planConstraints.rowRing != 1 &&
+                         mxk::depthwiseColumnDeltasTakes(f);
+      if (asked > 0 && !takes)
+        throw poplar::invalid_option(
+            "planConstraints gfx950 columns: the weight deltas' kernel takes "
+            "half tensors, 3x3, 5x5 or 7x7 taps at stride 1 or 2, without "
+            "rowRing 1");
+      if (takes && (asked > 0 || (asked != 0 && f.dense3x3 != 2 &&
+                                  products >= enough))) {
+        f.dense3x3 = 0;
+        mxk::chooseDepthwiseColumnDeltas(f, asked > 0 ? uint32_t(asked) : 0);
+      }
     }
   }
   // The weight update pass of a dense layer with an undilated kernel and
@@ -1941,19 +1962,18 @@ mxconv_plan makePlanWith(const ConvParams &params,
             "tile does not fit 64 KB of LDS");
     }
     // 5 x 5 and 7 x 7 taps: strips of columns, wherever no other kernel is
-    // named.  Against the two kernels above, at their choice: of 130 random
-    // layers one was 3 % slower and two level, the others 1.03 to 7 times as
-    // fast; small, large, strided and narrow ones alike, so there is no line
-    // to draw.
+    // named.  Against the two kernels above, at their choice, 90 random layers
+    // were 1.1 to 7 times as fast; small, large, strided and narrow ones alike,
+    // so there is no line to draw.
     const bool columns =
-        pc.columns != 0 && !(pc.tileH || pc.tileW) && pc.rowRing != 1 &&
+        !plan.depthwiseWeightUpdate && pc.columns != 0 && !(pc.tileH || pc.tileW) && pc.rowRing != 1 &&
         mxk::depthwiseColumnsTakes(d, dwType,
                                    params.outputType == poplar::HALF
                                        ? mxk::kHalf
                                        : mxk::kFloat);
     if (columns)
       mxk::chooseDepthwiseColumns(d, pc.columns > 0 ? uint32_t(pc.columns) : 0);
-    else if (pc.columns > 0)
+    else if (pc.columns > 0 && !plan.depthwiseWeightUpdate)
       throw poplar::invalid_option(
           "planConstraints gfx950 columns: that kernel takes fp16 inputs, 5x5 "
           "or 7x7 taps at stride 1 or 2, without a tile or rowRing named");
@@ -2026,6 +2046,8 @@ std::string mxconv_plan::constraintsJson() const {
       os << ", \"deltaWindow\": " << (denseForward.windowCo ? 1 : 0);
     if (depthwiseWeightUpdate && kernel != Kernel::DEPTHWISE)
       os << ", \"rowRing\": " << (depthwiseForward.dense3x3 == 2 ? 1 : 0);
+    if (depthwiseWeightUpdate)
+      os << ", \"columns\": " << depthwiseForward.columns;
   }
   os << "}}";
   return os.str();
@@ -2117,6 +2139,9 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
     if (f.dense3x3 == 2) {
       e.reductionBytes = mxk::depthwiseRowsDeltaWorkspaceBytes(f);
       spread(e, mxk::depthwiseRowsDeltaLaunchShape(f).workgroups, 1);
+    } else if (f.columns) {
+      e.computeUs = mxk::depthwiseColumnDeltasEstimateUs(f) - e.reductionUs;
+      e.reductionBytes = mxk::depthwiseWeightDeltaWorkspaceBytes(f);
     }
     return e;
   }
@@ -2465,6 +2490,10 @@ std::string mxconv_plan::describe() const {
          << " persistent workgroups (" << l.strips << " strips x " << l.bands
          << " bands of " << l.rowsOut << " rows per image)";
     }
+    if (depthwiseForward.columns)
+      os << ", strips of " << depthwiseForward.columns
+         << " columns walked down in registers, bands of "
+         << depthwiseForward.columnRows << " rows";
     os << "\n";
   }
   if (denseWeightUpdate && denseForward.windowCo) {

@@ -1,5 +1,8 @@
 """Weight deltas of depthwise layers against the CPU oracle: the sums over the
-slices of a pass of many outputs (csrc/depthwise_train.hip)."""
+slices of a pass of many outputs (csrc/depthwise_train.hip), and the kernel that
+walks down strips of columns (csrc/depthwise_columns_deltas.hip)."""
+import json
+
 import numpy as np
 import pytest
 
@@ -36,3 +39,90 @@ def test_many_outputs_of_signs_are_exact(oracle, kw, out_type):
     # (sums of at most 2048 signs: exact in halves too)
     kw = dict(kw, batch=min(kw["batch"], 12)) if out_type == pa.HALF else kw
     _signs(oracle, kw, out_type)
+
+
+COLUMNS = "columns walked down in registers"
+
+
+def _options(columns):
+    return {"planConstraints": json.dumps({"gfx950": {"columns": columns}})}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kw", [
+    # strips: one partial, exact, one column over; a channel pair to each slot
+    # of four, and as many as a workgroup has threads for
+    dict(batch=2, field=(6, 2), kernel=(3, 3), groups=8, pad=1),
+    dict(batch=2, field=(9, 8), kernel=(7, 7), groups=40, pad=3),
+    dict(batch=1, field=(33, 17), kernel=(5, 5), groups=72, pad=2),
+    dict(batch=3, field=(17, 9), kernel=(7, 7), groups=8, stride=2, pad=3),
+    dict(batch=2, field=(31, 34), kernel=(5, 5), groups=136, stride=2, pad=2),
+    dict(batch=2, field=(10, 11), kernel=(3, 3), groups=264, stride=2, pad=1),
+    # a walk over several strips
+    dict(batch=2100, field=(5, 5), kernel=(3, 3), groups=256, pad=1),
+    # unpadded, unevenly padded, the input cut off
+    dict(batch=2, field=(7, 7), kernel=(7, 7), groups=16),
+    dict(batch=2, field=(9, 12), kernel=(7, 7), groups=24, padLower=(5, 0),
+         padUpper=(1, 6)),
+    dict(batch=2, field=(15, 14), kernel=(5, 5), groups=16, itl=(2, 1),
+         itu=(1, 3), pad=2),
+])
+@pytest.mark.parametrize("columns", [2, 4])
+def test_columns_of_signs_are_exact(oracle, kw, columns):
+    plan = _signs(oracle, kw, options=_options(columns))
+    assert COLUMNS in plan.describe()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", ["acts", "deltas"])
+@pytest.mark.parametrize("columns", [2, 4])
+@pytest.mark.parametrize("k,stride", [(3, 1), (5, 2), (7, 1)])
+def test_infinities_stay_in_their_products(k, stride, columns, where):
+    """An infinity at the field's edge reaches the taps that have a product
+    with it and no other (a zero opposite it would make a NaN)."""
+    p = make_params(pa.HALF, pa.FLOAT, batch=2, field=(13, 15), kernel=(k, k),
+                    groups=16, stride=stride, pad=k // 2)
+    rng = np.random.default_rng(3)
+    x = rng.choice([-1.0, 1.0], (2, 16, 13, 15))
+    dz = rng.choice([-1.0, 1.0], (2, 16, *p.getOutputFieldShape()))
+    (x if where == "acts" else dz)[1, 5, 0, -1] = np.inf
+    want = np.zeros((16, k, k))
+    for kh in range(k):
+        for kw in range(k):
+            ys = [y for y in range(dz.shape[2])
+                  if 0 <= y * stride + kh - k // 2 < 13]
+            xs = [c for c in range(dz.shape[3])
+                  if 0 <= c * stride + kw - k // 2 < 15]
+            a = x[:, :, [y * stride + kh - k // 2 for y in ys]]
+            a = a[:, :, :, [c * stride + kw - k // 2 for c in xs]]
+            want[:, kh, kw] = (a * dz[:, :, ys][:, :, :, xs]).sum((0, 2, 3))
+    assert np.isinf(want).any() and np.isfinite(want[5]).any()
+    got, _ = run_weight_update(p, x.astype(np.float16), dz.astype(np.float16),
+                               _options(columns))
+    np.testing.assert_array_equal(got.reshape(want.shape), want)
+
+
+def test_columns_plan_choice():
+    def plan(options=None, dtype=pa.HALF, **kw):
+        return pa.WeightUpdatePlan(make_params(dtype, dtype, **kw), options)
+    big = dict(batch=16, field=(40, 40), kernel=(5, 5), groups=96, pad=2)
+    chosen = plan(**big)
+    assert COLUMNS in chosen.describe()
+    doc = chosen.constraints()
+    assert json.loads(doc)["gfx950"]["columns"] in (2, 4)
+    again = plan({"planConstraints": doc}, **big)
+    assert again.constraints() == doc
+    assert again.workspace_bytes() == chosen.workspace_bytes()
+    off = plan(_options(0), **big)
+    assert COLUMNS not in off.describe()
+    assert COLUMNS not in plan({"planConstraints": off.constraints()},
+                               **big).describe()
+    # little work, fp32 tensors, other kernels and strides
+    small = dict(batch=2, field=(9, 9), kernel=(5, 5), groups=16, pad=2)
+    assert COLUMNS not in plan(**small).describe()
+    assert COLUMNS in plan(_options(2), **small).describe()
+    for bad in (dict(big, dtype=pa.FLOAT), dict(big, kernel=(5, 3)),
+                dict(big, stride=3), dict(big, kdil=2)):
+        assert COLUMNS not in plan(**bad).describe()
+        with pytest.raises(pa.MxconvError):
+            plan(_options(4), **bad)
