@@ -506,9 +506,12 @@ struct WuTapDesc {
   // the result's channels, where ci and co are those filled up to whole
   // vectors (0: the same)
   uint32_t resultCi = 0, resultCo = 0;
-  // wuWindowKernel's tile of output x input channels (32 or 64 each; 0: it is
-  // not that kernel's) and the k-steps of 32 columns a workgroup sums over
+  // wuWindowKernel's tile of output x input channels (32 or 64 each; fp32: 16,
+  // 32 or 48 both; 0: it is not that kernel's) and the k-steps of 32 columns a
+  // workgroup sums over
   uint32_t windowCo = 0, windowCi = 0, windowSteps = 0;
+  // of a channel: 2, or 4 (fp32: wuWindowFloatKernel only)
+  uint32_t elemBytes = 2;
 };
 bool wuTapTakes(const WuTapDesc &d);
 /// Pixels per workgroup that give about one workgroup per compute unit.
@@ -525,7 +528,8 @@ hipError_t launchWuTap(const WuTapDesc &d, int outType, const void *acts,
                        hipStream_t stream);
 
 /// The same by wuWindowKernel: kernels of one or three columns, strides of one
-/// or two along a row, channels in whole words of two, groups of any width.
+/// or two along a row, channels in whole words of two, groups of any width; fp32
+/// tensors too (d.elemBytes).
 bool wuWindowTakes(const WuTapDesc &d);
 /// Sets the tile and the chunks that are estimated to be the fastest (and
 /// flattens the field of a 1 x 1 kernel); the estimate in microseconds, or a

@@ -67,6 +67,106 @@ struct WuWindowArgs {
   FastDiv divCo;
 };
 
+struct WinPlace {
+  uint32_t chunk, g0, coTile, ciTile, kh;
+};
+
+/// Workgroup -> (chunk, groups, co tile, ci tile, kernel row), the row fastest;
+/// an XCD gets whole chunks.
+__device__ __forceinline__ WinPlace placeOfWorkgroup(const WuWindowArgs &a) {
+  WinPlace w;
+  const uint32_t block = xcdSwizzle(blockIdx.x, gridDim.x);
+  w.chunk = a.divTilesPerChunk(block);
+  uint32_t id = block - w.chunk * a.tilesPerChunk;
+  uint32_t over = a.divKH(id);
+  w.kh = id - over * a.d.kH;
+  id = over, over = a.divCiTiles(id);
+  w.ciTile = id - over * a.ciTiles;
+  id = over, over = a.divCoTiles(id);
+  w.coTile = id - over * a.coTiles;
+  w.g0 = over * a.perTile;
+  return w;
+}
+
+/// The waves' sums meet in LDS, a tap at a time, and leave.
+template <int JO, int JI, int KW, int NW, class OutT>
+__device__ __forceinline__ void
+storeWindow(const WuWindowArgs &a, const WinPlace &w,
+            const floatx4 (&acc)[KW][JO][JI], char *lds, OutT *out) {
+  const WuTapDesc &d = a.d;
+  const int t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint32_t q = (t & 63) >> 4, r = t & 15;
+  // Lane (q, r) holds output channels JO r + i and the 4 JI input channels from
+  // 4 JI q on (register n of block j is JI n + j of them): JI pieces of four,
+  // the output channel's pieces JI q and up.  A piece's place within its 16
+  // rotates, so that neither the writes nor the reads, which go along an output
+  // channel, meet in a bank.
+  constexpr int kPieces = 4 * JI; // of an output channel
+  auto placeOf = [](uint32_t i, uint32_t p, uint32_t rr) {
+    const uint32_t v = p % JI, qq = p / JI;
+    return (i * JI + v) * 64 + qq * 16 +
+           ((rr + p + (JI == 2 ? 8 * (i & 1) : 0)) & 15);
+  };
+  floatx4 *sums = reinterpret_cast<floatx4 *>(lds);
+  constexpr int kVectors = JO * JI * 64; // of the tile
+  const uint32_t tap0 = w.kh * KW;
+#pragma unroll
+  for (int k = 0; k != KW; ++k) {
+    if (k != 0)
+      __syncthreads();
+#pragma unroll
+    for (int i = 0; i != JO; ++i)
+#pragma unroll
+      for (int v = 0; v != JI; ++v) {
+        floatx4 x;
+#pragma unroll
+        for (int n = 0; n != 4; ++n)
+          x[n] = acc[k][i][(4 * v + n) % JI][(4 * v + n) / JI];
+        sums[wave * kVectors + placeOf(i, q * JI + v, r)] = x;
+      }
+    __syncthreads();
+    for (int e = t; e < kVectors; e += 64 * NW) {
+      const uint32_t co = e / kPieces, p = e % kPieces;
+      const uint32_t place = placeOf(co % JO, p, co / JO);
+      floatx4 total = sums[place];
+#pragma unroll
+      for (int other = 1; other != NW; ++other)
+        total += sums[other * kVectors + place];
+      const uint32_t ci = p * 4;
+      OutT *to = out + w.chunk * a.chunkElems + (tap0 + k) * a.strideTap;
+      if (a.perTile == 1) {
+        const uint32_t coIn = w.coTile * (16 * JO) + co,
+                       ciIn = w.ciTile * (16 * JI) + ci;
+        if (coIn >= a.resultCo || ciIn >= a.resultCi)
+          continue;
+        const size_t f =
+            (size_t(w.g0) * a.resultCo + coIn) * a.resultCi + ciIn;
+        if (a.strideF == 1 && a.resultCi % 4 == 0) {
+          const float v[4] = {total[0], total[1], total[2], total[3]};
+          storeOut4(to + f, v);
+        } else {
+#pragma unroll
+          for (uint32_t x = 0; x != 4; ++x)
+            if (ciIn + x < a.resultCi)
+              storeOut(to, (f + x) * a.strideF, total[x]);
+        }
+      } else {
+        const uint32_t gl = a.divCo(co), coIn = co - gl * d.co;
+        if (gl >= a.perTile || w.g0 + gl >= d.groups || coIn >= a.resultCo)
+          continue;
+        const size_t f = (size_t(w.g0 + gl) * a.resultCo + coIn) * a.resultCi;
+#pragma unroll
+        for (uint32_t x = 0; x != 4; ++x) {
+          const uint32_t ciIn = ci + x - gl * d.ci;
+          if (ciIn < a.resultCi)
+            storeOut(to, (f + ciIn) * a.strideF, total[x]);
+        }
+      }
+    }
+  }
+}
+
 template <int J> struct WinLoad;
 template <> struct WinLoad<2> {
   typedef uint32_t Words __attribute__((ext_vector_type(1)));
@@ -100,18 +200,8 @@ __global__ __launch_bounds__(64 * NW) void wuWindowKernel(
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const uint32_t q = lane >> 4, r = lane & 15;
 
-  // workgroup -> (chunk, groups, co tile, ci tile, kernel row), the row
-  // fastest; an XCD gets whole chunks
-  const uint32_t block = xcdSwizzle(blockIdx.x, gridDim.x);
-  const uint32_t chunk = a.divTilesPerChunk(block);
-  uint32_t id = block - chunk * a.tilesPerChunk;
-  uint32_t over = a.divKH(id);
-  const uint32_t kh = id - over * d.kH;
-  id = over, over = a.divCiTiles(id);
-  const uint32_t ciTile = id - over * a.ciTiles;
-  id = over, over = a.divCoTiles(id);
-  const uint32_t coTile = id - over * a.coTiles;
-  const uint32_t g0 = over * a.perTile;
+  const WinPlace place = placeOfWorkgroup(a);
+  const auto [chunk, g0, coTile, ciTile, kh] = place;
   const uint32_t u0 = chunk * a.unitsPerChunk;
   const uint32_t u1 =
       u0 + a.unitsPerChunk < a.units ? u0 + a.unitsPerChunk : a.units;
@@ -233,78 +323,150 @@ __global__ __launch_bounds__(64 * NW) void wuWindowKernel(
     at += 2 * kStride;
   }
 
-  // The waves' sums meet in LDS, a tap at a time.  Lane (q, r) holds output
-  // channels JO r + i and the input channels JI (4 q + v) + j: pieces of four
-  // input channels, JI of them, piece 4 q + v (JI = 4) or 2 q + v / 2 (JI = 2)
-  // of the output channel's.  A piece's place within its 16 rotates, so that
-  // neither the writes nor the reads, which go along an output channel, meet
-  // in a bank.
-  constexpr int kPieces = 4 * JI; // of an output channel
-  auto placeOf = [](uint32_t i, uint32_t p, uint32_t rr) {
-    const uint32_t v = p % JI, qq = p / JI;
-    return (i * JI + v) * 64 + qq * 16 +
-           ((rr + p + (JI == 2 ? 8 * (i & 1) : 0)) & 15);
-  };
-  floatx4 *sums = reinterpret_cast<floatx4 *>(lds);
-  constexpr int kVectors = JO * JI * 64; // of the tile
-  const uint32_t tap0 = kh * KW;
-#pragma unroll
-  for (int k = 0; k != KW; ++k) {
-    if (k != 0)
-      __syncthreads();
-#pragma unroll
-    for (int i = 0; i != JO; ++i)
-#pragma unroll
-      for (int v = 0; v != JI; ++v) {
-        floatx4 x;
-        if constexpr (JI == 4)
-          x = floatx4{acc[k][i][0][v], acc[k][i][1][v], acc[k][i][2][v],
-                      acc[k][i][3][v]};
-        else
-          x = floatx4{acc[k][i][0][2 * v], acc[k][i][1][2 * v],
-                      acc[k][i][0][2 * v + 1], acc[k][i][1][2 * v + 1]};
-        sums[wave * kVectors + placeOf(i, q * JI + v, r)] = x;
-      }
-    __syncthreads();
-    for (int e = t; e < kVectors; e += 64 * NW) {
-      const uint32_t co = e / kPieces, p = e % kPieces;
-      const uint32_t place = placeOf(co % JO, p, co / JO);
-      floatx4 total = sums[place];
-#pragma unroll
-      for (int w = 1; w != NW; ++w)
-        total += sums[w * kVectors + place];
-      const uint32_t ci = p * 4;
-      OutT *to = out + chunk * a.chunkElems + (tap0 + k) * a.strideTap;
-      if (a.perTile == 1) {
-        const uint32_t coIn = coTile * (16 * JO) + co,
-                       ciIn = ciTile * (16 * JI) + ci;
-        if (coIn >= a.resultCo || ciIn >= a.resultCi)
-          continue;
-        const size_t f =
-            (size_t(g0) * a.resultCo + coIn) * a.resultCi + ciIn;
-        if (a.strideF == 1 && a.resultCi % 4 == 0) {
-          const float v[4] = {total[0], total[1], total[2], total[3]};
-          storeOut4(to + f, v);
-        } else {
-#pragma unroll
-          for (uint32_t x = 0; x != 4; ++x)
-            if (ciIn + x < a.resultCi)
-              storeOut(to, (f + x) * a.strideF, total[x]);
-        }
-      } else {
-        const uint32_t gl = a.divCo(co), coIn = co - gl * d.co;
-        if (gl >= a.perTile || g0 + gl >= d.groups || coIn >= a.resultCo)
-          continue;
-        const size_t f = (size_t(g0 + gl) * a.resultCo + coIn) * a.resultCi;
-#pragma unroll
-        for (uint32_t x = 0; x != 4; ++x) {
-          const uint32_t ciIn = ci + x - gl * d.ci;
-          if (ciIn < a.resultCi)
-            storeOut(to, (f + ciIn) * a.strideF, total[x]);
-        }
-      }
-    }
+  storeWindow<JO, JI, KW, NW>(a, place, acc, lds, out);
+}
+
+template <int J> struct WinFloats;
+template <> struct WinFloats<1> {
+  typedef float Words __attribute__((ext_vector_type(1)));
+  static __device__ __forceinline__ Words at(__amdgpu_buffer_rsrc_t b,
+                                             uint32_t off) {
+    Words w;
+    w[0] = __builtin_bit_cast(
+        float, __builtin_amdgcn_raw_buffer_load_b32(b, off, 0, 0));
+    return w;
   }
+};
+template <> struct WinFloats<2> {
+  typedef float Words __attribute__((ext_vector_type(2)));
+  static __device__ __forceinline__ Words at(__amdgpu_buffer_rsrc_t b,
+                                             uint32_t off) {
+    return __builtin_bit_cast(
+        Words, __builtin_amdgcn_raw_buffer_load_b64(b, off, 0, 0));
+  }
+};
+template <> struct WinFloats<3> {
+  typedef float Words __attribute__((ext_vector_type(3)));
+  static __device__ __forceinline__ Words at(__amdgpu_buffer_rsrc_t b,
+                                             uint32_t off) {
+    return __builtin_bit_cast(
+        Words, __builtin_amdgcn_raw_buffer_load_b96(b, off, 0, 0));
+  }
+};
+
+/// The same for fp32 tensors, with an MFMA for each of a unit's pixels: lane
+/// (q, r) brings channels J r .. J r + J - 1 of pixel m of its unit, and k is
+/// the lane quarter, so the loads are the operands as they are.  Nothing is
+/// permuted; the matrix pipe (32 cycles for 16 x 16 x 4) is the bound, and
+/// tiles of J = 1, 2 or 3 blocks both ways leave little of it to padding.  The
+/// passes of these layers were convolutions of their own between two
+/// rearrangements, four launches and more; us before and after: 48 -> 43
+/// channels, 3 x 3, 15 x 9 x 9 28.8 -> 8.5; 312 -> 160, 1 x 1 stride 2, 10 x 15 x
+/// 15 34.7 -> 8; 32 groups of 16, 3 x 3, 64 x 16 x 16 224 -> 40; 128 -> 128, 3 x
+/// 3, 36 x 56 x 56 389 -> 275 (the matrix pipe's own time 222).  Over 340 random
+/// layers 4.6 times as fast (geometric mean, least 0.98).
+template <int J, int KW, int S, int NW, class OutT>
+__global__ __launch_bounds__(64 * NW) void wuWindowFloatKernel(
+    const WuWindowArgs a, const char *__restrict__ acts,
+    const char *__restrict__ deltas, OutT *__restrict__ out) {
+  constexpr int NX = S * 7 + KW; // columns a unit's taps read
+  extern __shared__ __align__(16) char lds[];
+  const WuTapDesc &d = a.d;
+  const int t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint32_t q = (t & 63) >> 4, r = t & 15;
+  const WinPlace place = placeOfWorkgroup(a);
+  const auto [chunk, g0, coTile, ciTile, kh] = place;
+  const uint32_t u0 = chunk * a.unitsPerChunk;
+  const uint32_t u1 =
+      u0 + a.unitsPerChunk < a.units ? u0 + a.unitsPerChunk : a.units;
+  const __amdgpu_buffer_rsrc_t actBuf = bufferOf(acts, a.actBytes);
+  const __amdgpu_buffer_rsrc_t deltaBuf = bufferOf(deltas, a.deltaBytes);
+  const uint32_t actLane = (g0 * d.ci + ciTile * (16 * J) + J * r) * 4;
+  const uint32_t deltaLane = (g0 * d.co + coTile * (16 * J) + J * r) * 4;
+  const uint32_t actFirst = actLane - uint32_t(d.padW) * a.actPixelBytes;
+
+  struct Raw {
+    typename WinFloats<J>::Words delta[8], act[NX];
+    uint32_t here; // pixels of the unit
+  };
+  auto load = [&](Raw &x, uint32_t first) {
+    const uint32_t u = first + q;
+    const uint32_t row = a.divSegs(u), seg = u - row * a.segs;
+    const uint32_t b = a.divOutH(row), y = row - b * d.outH;
+    const uint32_t x0 = seg * kWinUnit;
+    const bool valid = u < u1;
+    const uint32_t left = d.outW - x0;
+    x.here = valid ? (left < kWinUnit ? left : kWinUnit) : 0u;
+    uint32_t at = __umul24(__umul24(row, d.outW) + x0, a.deltaPixelBytes) +
+                  deltaLane;
+#pragma unroll
+    for (uint32_t i = 0; i != 8; ++i)
+      x.delta[i] = WinFloats<J>::at(
+          deltaBuf, i < x.here ? at + i * a.deltaPixelBytes : kWinInvalid);
+    const uint32_t iy = __umul24(y, d.strideH) + kh - uint32_t(d.padH);
+    const uint32_t ix = x0 * S - uint32_t(d.padW);
+    const bool rowIn = valid && iy - d.loH < d.hiH - d.loH;
+    at = __umul24(__umul24(b, d.inH) + iy, a.actRowBytes) +
+         __umul24(x0 * S, a.actPixelBytes) + actFirst;
+    const uint32_t span = rowIn ? d.hiW - d.loW : 0u;
+#pragma unroll
+    for (int i = 0; i != NX; ++i)
+      x.act[i] = WinFloats<J>::at(actBuf, ix + i - d.loW < span
+                                              ? at + i * a.actPixelBytes
+                                              : kWinInvalid);
+  };
+
+  floatx4 acc[KW][J][J];
+#pragma unroll
+  for (int k = 0; k != KW; ++k)
+#pragma unroll
+    for (int i = 0; i != J; ++i)
+#pragma unroll
+      for (int j = 0; j != J; ++j)
+        acc[k][i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  // (a partial unit's missing pixels are zero in both operands: an activation
+  // that another tap's product has, and that is infinite, would else meet a
+  // zero here)
+  auto multiply = [&](const Raw &x, auto partial) {
+#pragma unroll
+    for (int m = 0; m != 8; ++m)
+#pragma unroll
+      for (int k = 0; k != KW; ++k)
+#pragma unroll
+        for (int j = 0; j != J; ++j) {
+          float v = x.act[S * m + k][j];
+          if constexpr (decltype(partial)::value)
+            v = uint32_t(m) < x.here ? v : 0.0f;
+#pragma unroll
+          for (int i = 0; i != J; ++i)
+            acc[k][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                v, x.delta[m][i], acc[k][i][j], 0, 0, 0);
+        }
+  };
+  auto both = [&](const Raw &x) {
+    if (__any(x.here != 8 && x.here != 0))
+      multiply(x, std::true_type{});
+    else
+      multiply(x, std::false_type{});
+  };
+  constexpr uint32_t kStride = NW * kWinUnits;
+  uint32_t at = u0 + wave * kWinUnits;
+  Raw even, odd;
+  load(even, at);
+  while (at < u1) {
+    load(odd, at + kStride);
+    __builtin_amdgcn_sched_barrier(0);
+    both(even);
+    __builtin_amdgcn_sched_barrier(0);
+    load(even, at + 2 * kStride);
+    __builtin_amdgcn_sched_barrier(0);
+    both(odd);
+    __builtin_amdgcn_sched_barrier(0);
+    at += 2 * kStride;
+  }
+  storeWindow<J, J, KW, NW>(a, place, acc, lds, out);
 }
 
 /// out[f][tap] = sum over the chunks, in order, of partial[chunk][tap][f] for
@@ -398,25 +560,33 @@ bool wuWindowTakes(const WuTapDesc &d) {
   if ((d.kW != 1 && d.kW != 3) || d.strideH == 0 ||
       (d.strideW != 1 && d.strideW != 2))
     return false;
-  if (((d.windowCo != 32 || d.windowCi != 32) &&
+  const bool floats = d.elemBytes == 4;
+  if (d.elemBytes != 2 && !floats)
+    return false;
+  if (floats) {
+    if (d.windowCo != d.windowCi || (d.windowCo != 16 && d.windowCo != 32 &&
+                                     d.windowCo != 48))
+      return false;
+  } else if (((d.windowCo != 32 || d.windowCi != 32) &&
        (d.windowCo != 64 || d.windowCi != 32) &&
-       (d.windowCo != 32 || d.windowCi != 64)) ||
-      d.windowSteps == 0)
+       (d.windowCo != 32 || d.windowCi != 64)))
+    return false;
+  if (d.windowSteps == 0)
     return false;
   // words of two channels at multiples of four bytes
-  const uint64_t actPixel = uint64_t(d.groups) * d.ci * 2,
-                 deltaPixel = uint64_t(d.groups) * d.co * 2;
+  const uint64_t actPixel = uint64_t(d.groups) * d.ci * d.elemBytes,
+                 deltaPixel = uint64_t(d.groups) * d.co * d.elemBytes;
   if (actPixel % 4 != 0 || deltaPixel % 4 != 0)
     return false;
-  if (d.groups > 1 && (d.ci % 2 != 0 || d.co % 2 != 0))
+  if (!floats && d.groups > 1 && (d.ci % 2 != 0 || d.co % 2 != 0))
     return false;
   if (d.resultCi > d.ci || d.resultCo > d.co)
     return false;
   // (a unit's columns beyond a row's end are addressed too: they stay below
   // kWinInvalid twice over)
   if (uint64_t(d.batch) * d.inH * d.inW * actPixel +
-              64 * (actPixel + 128) >= kWinInvalid ||
-      M * deltaPixel + 64 * (deltaPixel + 128) >= kWinInvalid)
+              64 * (actPixel + 256) >= kWinInvalid ||
+      M * deltaPixel + 64 * (deltaPixel + 256) >= kWinInvalid)
     return false;
   // 24-bit products: rows, pixels, bytes of a pixel and of an input row
   const uint64_t k24 = 1u << 24;
@@ -473,14 +643,36 @@ constexpr WinFit kWinFits[3][2][2] = {
      {{6.11, 0.030, 0.109, 5.0, 0.122, 2.8, 0.44, 2.4},
       {6.59, 0.049, 0.153, 4.8, 0.191, 2.6, 0.46, 2.2}}}};
 
+/// fp32: tiles of 16, 32 and 48; one column, three (both strides).  Fitted to
+/// 6 200 measurements on 340 layers, within 8 to 10 %; the pick 2 % behind the
+/// best on average.
+constexpr WinFit kWinFloatFits[3][2] = {
+    {{4.63, 0.041, 0.077, 1.3, 0.113, 2.0, 3.15, 1.17},
+     {6.85, 0.011, 0.151, 4.2, 0.149, 2.5, 0.41, 0.78}},
+    {{4.99, 0.051, 0.178, 1.8, 0.186, 2.4, 0.85, 0.76},
+     {8.16, 0.018, 0.435, 6.5, 0.423, 3.3, 0.36, 1.48}},
+    {{5.72, 1.372, 0.311, 3.0, 0.340, 2.4, 0.54, 0.0},
+     {9.59, 3.941, 0.930, 10.5, 0.908, 4.1, 0.35, 1.29}}};
+
+uint32_t floatWaves(uint32_t tile) {
+  return tile == 16 ? 16 : tile == 32 ? 8 : 4;
+}
+
 double winEstimateUs(const WuTapDesc &d, const WinShape &s,
                      uint32_t computeUnits) {
-  const int tile = d.windowCo == 64 ? 1 : d.windowCi == 64 ? 2 : 0;
-  const WinFit &f = kWinFits[tile][d.kW == 1 ? 0 : 1][d.strideW - 1];
-  const uint32_t waves = tile == 0 ? 16 : 8;
+  const bool floats = d.elemBytes == 4;
+  const int tile = floats                ? int(d.windowCo / 16) - 1
+                   : d.windowCo == 64    ? 1
+                   : d.windowCi == 64    ? 2
+                                         : 0;
+  const WinFit &f = floats ? kWinFloatFits[tile][d.kW == 1 ? 0 : 1]
+                           : kWinFits[tile][d.kW == 1 ? 0 : 1][d.strideW - 1];
+  const uint32_t waves =
+      floats ? floatWaves(d.windowCo) : tile == 0 ? 16 : 8;
   const double steps = d.windowSteps;
-  // (a workgroup to a CU; two of eight waves where a kernel row is one column)
-  const double shared = tile != 0 && d.kW == 1 ? 2.0 : 1.0;
+  // (a workgroup to a CU; two of eight waves, or of fp32, where a kernel row is
+  // one column)
+  const double shared = (floats || tile != 0) && d.kW == 1 ? 2.0 : 1.0;
   const double perCU = std::max(
       1.0, std::ceil(shared * double(s.chunks * s.tiles) / computeUnits) /
                shared);
@@ -488,7 +680,7 @@ double winEstimateUs(const WuTapDesc &d, const WinShape &s,
   return f.call + std::max(f.wave * std::ceil(steps / waves), f.step * steps) +
          (perCU - 1) * (f.round + f.roundStep * steps) +
          (s.chunks > 1 ? f.second + f.partialMB * 4 * mb * s.chunks
-                       : f.resultMB * 2 * mb);
+                       : f.resultMB * d.elemBytes * mb);
 }
 } // namespace
 
@@ -509,9 +701,11 @@ double wuWindowChoose(WuTapDesc &d, uint32_t computeUnits) {
   for (uint32_t tile = 0; tile != 3; ++tile) {
     WuTapDesc t = d;
     t.windowCo = tile == 1 ? 64 : 32, t.windowCi = tile == 2 ? 64 : 32;
+    if (d.elemBytes == 4)
+      t.windowCo = t.windowCi = 16 * (tile + 1);
     t.windowSteps = 1;
     const WinShape one = winShape(t);
-    if (one.tiles == 0 || (tile != 0 && one.perTile > 1))
+    if (one.tiles == 0 || (d.elemBytes == 2 && tile != 0 && one.perTile > 1))
       continue;
     const uint32_t steps = one.chunks;
     // (four workgroups for every CU at most: more lose to their own start)
@@ -551,6 +745,37 @@ hipError_t launchWindow(const WuWindowArgs &a, uint32_t blocks, int outType,
   return hipGetLastError();
 }
 
+template <int J, int KW, int S>
+hipError_t launchWindowFloat(const WuWindowArgs &a, uint32_t blocks,
+                             int outType, const void *acts, const void *deltas,
+                             void *out, hipStream_t stream) {
+  constexpr int NW = J == 1 ? 16 : J == 2 ? 8 : 4; // (floatWaves)
+  constexpr int kLds = NW * J * J * 1024;
+  const dim3 grid(blocks), block(64 * NW);
+  const char *x = static_cast<const char *>(acts);
+  const char *dz = static_cast<const char *>(deltas);
+  if (outType == kHalf)
+    hipLaunchKernelGGL((wuWindowFloatKernel<J, KW, S, NW, __half>), grid, block,
+                       kLds, stream, a, x, dz, static_cast<__half *>(out));
+  else
+    hipLaunchKernelGGL((wuWindowFloatKernel<J, KW, S, NW, float>), grid, block,
+                       kLds, stream, a, x, dz, static_cast<float *>(out));
+  return hipGetLastError();
+}
+
+template <int J>
+hipError_t launchWindowFloats(const WuWindowArgs &a, uint32_t blocks,
+                              int outType, const void *acts,
+                              const void *deltas, void *out,
+                              hipStream_t stream) {
+  const auto go = a.d.kW == 1
+                      ? a.d.strideW == 1 ? &launchWindowFloat<J, 1, 1>
+                                         : &launchWindowFloat<J, 1, 2>
+                      : a.d.strideW == 1 ? &launchWindowFloat<J, 3, 1>
+                                         : &launchWindowFloat<J, 3, 2>;
+  return go(a, blocks, outType, acts, deltas, out, stream);
+}
+
 template <int JO, int JI, int NW>
 hipError_t launchWindowTaps(const WuWindowArgs &a, uint32_t blocks,
                             int outType, const void *acts, const void *deltas,
@@ -584,8 +809,8 @@ hipError_t launchWuWindow(const WuTapDesc &d, int outType, const void *acts,
   a.tilesPerChunk = uint32_t(s.tiles);
   a.resultCo = d.resultCo ? d.resultCo : d.co;
   a.resultCi = d.resultCi ? d.resultCi : d.ci;
-  a.actPixelBytes = d.groups * d.ci * 2;
-  a.deltaPixelBytes = d.groups * d.co * 2;
+  a.actPixelBytes = d.groups * d.ci * d.elemBytes;
+  a.deltaPixelBytes = d.groups * d.co * d.elemBytes;
   a.actRowBytes = d.inW * a.actPixelBytes;
   a.actBytes = d.batch * d.inH * a.actRowBytes;
   a.deltaBytes = d.batch * d.outH * d.outW * a.deltaPixelBytes;
@@ -600,7 +825,14 @@ hipError_t launchWuWindow(const WuTapDesc &d, int outType, const void *acts,
   void *to = direct ? out : workspace;
   const int toType = direct ? outType : int(kFloat);
   hipError_t e;
-  if (d.windowCo == 64)
+  if (d.elemBytes == 4)
+    e = d.windowCo == 16
+            ? launchWindowFloats<1>(a, blocks, toType, acts, deltas, to, stream)
+        : d.windowCo == 32
+            ? launchWindowFloats<2>(a, blocks, toType, acts, deltas, to, stream)
+            : launchWindowFloats<3>(a, blocks, toType, acts, deltas, to,
+                                    stream);
+  else if (d.windowCo == 64)
     e = launchWindowTaps<4, 2, 8>(a, blocks, toType, acts, deltas, to, stream);
   else if (d.windowCi == 64)
     e = launchWindowTaps<2, 4, 8>(a, blocks, toType, acts, deltas, to, stream);

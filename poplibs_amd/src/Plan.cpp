@@ -617,6 +617,15 @@ mxconv_plan makePlanWith(const ConvParams &params,
                          const ConvOptions &optionsIn,
                          unsigned convGroupsPerGroup);
 
+/// fp32 layers: wuWindowKernel's fp32 sibling wherever it takes the layer and
+/// nothing names a tile for the pass's own convolution (340 random layers 0.98
+/// to 100 times as fast as that, so there is no line to draw).
+bool floatWindowAsked(const PlanConstraints &pc) {
+  return pc.deltaWindow == 1 ||
+         (!pc.blockM && !pc.blockN && !pc.blockK && !pc.splitK && !pc.stages &&
+          pc.patch < 0 && pc.pointwise < 0 && pc.smallTile < 0);
+}
+
 /// The weight deltas of `layer` (channels of a group as the layer has them, in
 /// resultCi and resultCo) by wuWindowKernel, where that is named or estimated
 /// to be faster than what `plan` has; `fuse`: groups that plan takes as one.
@@ -636,6 +645,8 @@ void windowWeightDeltas(mxconv_plan &plan, const mxk::WuTapDesc &layer,
   w.chunkPixels = 64;
   w.ci = w.resultCi, w.co = w.resultCo;
   double us = mxk::wuWindowChoose(w, gfx950::numCUs);
+  if (!w.windowCo && w.elemBytes == 4)
+    return;
   if (!w.windowCo) {
     // (channels filled up to whole vectors, in copies, as wuTapKernel's are)
     w = layer;
@@ -691,7 +702,7 @@ void windowWeightDeltas(mxconv_plan &plan, const mxk::WuTapDesc &layer,
 void settleFewPixelWeightDeltas(mxconv_plan &plan) {
   const mxk::WuTapDesc &f = plan.denseForward;
   const std::size_t pixels = std::size_t(f.batch) * f.outH * f.outW;
-  if (!plan.denseWeightUpdate || pixels >= 1024 ||
+  if (!plan.denseWeightUpdate || pixels >= 1024 || f.elemBytes == 4 ||
       plan.options.planConstraints.weightDeltas == 1 ||
       plan.options.planConstraints.deltaWindow == 1)
     return;
@@ -887,11 +898,15 @@ mxconv_plan makePlanWith(const ConvParams &params,
         !w.hasDepth() && !w.outputPadded() && !w.kernelSelected &&
         !plan.zeroConv && !plan.depthwiseWeightUpdate && !w.inputDilated() &&
         w.batch == p.batchSize && w.strideH == 1 && w.strideW == 1 &&
-        params.inputType == poplar::HALF &&
+        (params.inputType == poplar::HALF ||
+         (params.inputType == poplar::FLOAT &&
+          floatWindowAsked(options.planConstraints))) &&
         (asked == 1 ||
          (options.planConstraints.kernel.empty() &&
           options.planConstraints.method == PlanConstraints::Method::ANY))) {
+      const bool half = params.inputType == poplar::HALF;
       mxk::WuTapDesc &f = plan.denseForward;
+      f.elemBytes = uint32_t(params.inputType.size());
       f.batch = uint32_t(p.inputChannelsPerConvGroup);
       f.inH = w.inH, f.inW = w.inW;
       f.outH = w.kH, f.outW = w.kW, f.kH = w.outH, f.kW = w.outW;
@@ -903,8 +918,9 @@ mxconv_plan makePlanWith(const ConvParams &params,
       // with theirs filled up)
       f.resultCi = uint32_t(p.batchSize);
       f.resultCo = uint32_t(p.outputChannelsPerConvGroup);
-      f.ci = (f.resultCi + 7) / 8 * 8;
-      f.co = (f.resultCo + 7) / 8 * 8;
+      const uint32_t vector = half ? 8 : 1;
+      f.ci = (f.resultCi + vector - 1) / vector * vector;
+      f.co = (f.resultCo + vector - 1) / vector * vector;
       f.chunkPixels = mxk::wuTapChunkPixels(f, gfx950::numCUs);
       plan.wuOwnTensors = true;
       plan.wuLayer = f;
@@ -924,7 +940,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
       // (settleFewPixelWeightDeltas).
       const bool worth = std::size_t(f.batch) * f.outH * f.outW < 1024 ||
                          (f.resultCi >= 16 && f.resultCo >= 16 && filled);
-      plan.denseWeightUpdate = (asked == 1 || worth) && mxk::wuTapTakes(f);
+      plan.denseWeightUpdate =
+          half && (asked == 1 || worth) && mxk::wuTapTakes(f);
       // ... or by the kernel that gathers pixels in registers
       windowWeightDeltas(plan, f, 1);
     }
@@ -939,7 +956,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
         !(plan.denseWeightUpdate && plan.denseForward.windowCo))
       throw poplar::invalid_option(
           "planConstraints gfx950 deltaWindow: that kernel takes weightDeltas "
-          "1 of half layers whose kernel has one or three columns and whose "
+          "1 of half and float layers whose kernel has one or three columns and whose "
           "stride along a row is one or two");
   }
   const auto &pc = options.planConstraints;
@@ -2504,7 +2521,9 @@ std::string mxconv_plan::describe() const {
                                             std::size_t((f.ci + 127) / 128) *
                                                 ((f.co + 127) / 128) * 16384;
     os << "        as a weight update pass    "
-       << (narrow ? "kernel of narrow groups" : "matrix-core weight-delta kernel")
+       << (narrow             ? "kernel of narrow groups"
+           : f.elemBytes == 4 ? "fp32 matrix-core kernel"
+                              : "matrix-core weight-delta kernel")
        << " on the layer's own tensors (pixels gathered in registers): tiles "
           "of "
        << f.windowCo << " output x " << f.windowCi
