@@ -364,7 +364,11 @@ struct ThinInputDesc {
   int32_t padH, padW; // as in IgemmDesc; padW >= 0
   uint32_t strideH, strideW;
   uint32_t loH, hiH, loW, hiW; // rows and columns outside read as zeros
+  // Output rows of a tile and workgroups to a compute unit (chooseThinInputTiles)
+  uint32_t tileRows = 1, perCU = 2;
 };
+/// Sets the tile and the workgroups that are estimated to be the fastest.
+void chooseThinInputTiles(ThinInputDesc &d, uint32_t cus);
 bool thinInputTakes(const ThinInputDesc &d, int inType, int outType);
 /// Elements of the packed weights ([16-channel block][k-step][lane][8]).
 uint64_t thinInputPackedElems(const ThinInputDesc &d);

@@ -387,7 +387,7 @@ struct ThinShape {
 
 uint32_t alignUp(uint32_t v, uint32_t to) { return (v + to - 1) / to * to; }
 
-ThinShape thinShape(const ThinInputDesc &d, uint32_t cus) {
+ThinShape thinShape(const ThinInputDesc &d) {
   ThinShape s{};
   s.kSteps = thinKSteps(d);
   const uint32_t pixelBytes = d.inChans * 2;
@@ -406,21 +406,10 @@ ThinShape thinShape(const ThinInputDesc &d, uint32_t cus) {
     return s;
   s.pitch = alignUp(uint32_t(extent), 16);
   const uint32_t weightBytes = (d.outChans / 16) * s.kSteps * 1024;
-  // the largest tile of 16, 8, ... output rows that fits 64 KB and leaves
-  // three tiles to two CUs; failing that the smallest
-  uint32_t chosen = 0;
-  for (uint32_t th = 16; th != 0; th /= 2) {
-    const uint32_t rows = (th - 1) * d.strideH + d.kH;
-    if (uint64_t(rows) * s.pitch > 64 * 1024)
-      continue;
-    chosen = th;
-    if (uint64_t(d.batch) * ((d.outH + th - 1) / th) * 2 >= 3ull * cus)
-      break;
-  }
-  if (!chosen)
-    return s;
-  s.tileRows = std::min(chosen, std::max(1u, d.outH));
+  s.tileRows = std::min(d.tileRows, std::max(1u, d.outH));
   s.ldsRows = (s.tileRows - 1) * d.strideH + d.kH;
+  if (uint64_t(s.ldsRows) * s.pitch > 64 * 1024)
+    return s;
   // (+ 256 bytes behind them for the bias, then the weights)
   s.ldsBytes = s.ldsRows * s.pitch + 256 + weightBytes;
   s.ok = true;
@@ -513,7 +502,7 @@ bool thinInputTakes(const ThinInputDesc &d, int inType, int outType) {
   if (uint64_t(d.batch) * d.outH * d.outW * d.outChans >= (1ull << 32) ||
       uint64_t(d.batch) * d.inH * d.inW * d.inChans >= (1ull << 32))
     return false;
-  return thinShape(d, 256).ok;
+  return thinShape(d).ok;
 }
 
 uint64_t thinInputPackedElems(const ThinInputDesc &d) {
@@ -523,17 +512,61 @@ uint64_t thinInputPackedElems(const ThinInputDesc &d) {
 uint32_t thinInputKSteps(const ThinInputDesc &d) { return thinKSteps(d); }
 
 ThinInputLaunch thinInputLaunchShape(const ThinInputDesc &d, uint32_t cus) {
-  const ThinShape s = thinShape(d, cus);
+  const ThinShape s = thinShape(d);
   ThinInputLaunch l{};
   l.tileRows = s.tileRows;
   l.ldsBytes = s.ldsBytes;
   const uint64_t tiles =
       uint64_t(d.batch) * ((d.outH + s.tileRows - 1) / std::max(1u, s.tileRows));
-  // (two workgroups to a CU: what the registers of the largest variant -
-  // 64 output channels, 7 kernel rows - allow)
-  l.workgroups = std::min<uint64_t>(tiles, uint64_t(cus) * 2);
+  l.workgroups = std::min<uint64_t>(tiles, uint64_t(cus) * d.perCU);
   l.tiles = tiles;
   return l;
+}
+
+// Tiles and workgroups so that the last round of tiles is a full one.  (Tiles
+// of 1, 2, 4, 8 or 16 rows, as many as made three to two CUs, left the two
+// workgroups of a CU 589 tiles for 512 places, say: 31 x 147 x 147, 7 x 7, 16
+// channels 23.6 -> 17.5 us with 1147 tiles of four rows for 768, whose registers
+// leave room for three; 33 x 138 x 138 21.6 -> 15.4; 32 x 224 x 224, 7 x 7
+// stride 2, 64 channels 20.4 -> 19.9 with 512 tiles of seven rows; N = 1 to 64,
+// 64 to 256 rows, 80 random layers 6 % at the geometric mean.)
+void chooseThinInputTiles(ThinInputDesc &d, uint32_t cus) {
+  ThinInputDesc t = d;
+  const uint32_t steps = thinKSteps(d), blocks = d.outChans / 16;
+  // registers: 97 for 16 output channels and one k-step
+  const uint32_t registers = alignUp(
+      97 + 4 * (blocks - 1) + (6 + 4 * blocks) * (steps - 1), 8);
+  double best = 0;
+  for (uint32_t rows = 1; rows <= std::min(32u, d.outH); ++rows) {
+    const uint32_t perImage = (d.outH + rows - 1) / rows;
+    t.tileRows = (d.outH + perImage - 1) / perImage;
+    if (t.tileRows != rows)
+      continue;
+    const ThinShape s = thinShape(t);
+    if (!s.ok)
+      break;
+    const uint64_t tiles = uint64_t(d.batch) * perImage;
+    const uint32_t most = std::max(
+        2u, std::min({4u, 512 / registers, 160 * 1024 / s.ldsBytes}));
+    for (t.perCU = 2; t.perCU <= most; ++t.perCU) {
+      // Microseconds, fitted to 1500 timings of those layers (5 %; the pick is
+      // within 1 % of the best on average): for a round of tiles on all
+      // workgroups, for each tile of the busiest CU, its blocks of 16 pixels
+      // and its input rows.
+      const uint64_t places = uint64_t(cus) * t.perCU;
+      const uint64_t full = tiles / places, rest = tiles - full * places;
+      const double rounds = double(full + (rest != 0));
+      const double perCU = double(full * t.perCU + (rest + cus - 1) / cus);
+      const double pixels = double(rows) * s.colBlocks;
+      const double us =
+          rounds * (0.345 + 0.0128 * pixels * steps) +
+          perCU * (0.189 + pixels * (0.0012 + 0.00055 * steps +
+                                     0.0064 * blocks) +
+                   0.049 * s.ldsRows * s.rowBytes / 1024.0);
+      if (best == 0 || us < best)
+        best = us, d.tileRows = rows, d.perCU = t.perCU;
+    }
+  }
 }
 
 hipError_t launchPackThinInputWeights(const ThinInputDesc &d, const void *src,
@@ -550,7 +583,7 @@ hipError_t launchThinInput(const ThinInputDesc &d, int inType, int outType,
                            const void *bias, void *out, hipStream_t stream) {
   if (!thinInputTakes(d, inType, outType))
     return hipErrorInvalidValue;
-  const ThinShape s = thinShape(d, 256);
+  const ThinShape s = thinShape(d);
   const ThinInputLaunch l = thinInputLaunchShape(d, 256);
   ThinArgs a{};
   a.d = d;

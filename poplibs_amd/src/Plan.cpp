@@ -1155,6 +1155,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
          (unconstrained &&
           (chosen == Kernel::IGEMM || igemmWhyNot == tooLittleWork)))) {
       plan.thinInputOn = true;
+      mxk::chooseThinInputTiles(t, gfx950::numCUs);
       reason = chosen != Kernel::IGEMM && pc.thinInput == 1
                    ? "forced by planConstraints"
                    : "few input channels: a kernel row's pixels as one k-step "
