@@ -1012,7 +1012,17 @@ mxconv_plan makePlanWith(const ConvParams &params,
     else if (ciPadded != ci && pc.kernel != "igemm" &&
              2.0 * double(s.batch) * s.outD * s.outH * s.outW * s.kD * s.kH *
                      s.kW * ci * co * p.numConvGroups <
-                 double(1u << 22))
+                 double(1u << 22) &&
+             // The generic kernel's time is its chain of products, of which a
+             // thread has all of an output's: 4 us and 0.09 a product in fp16,
+             // 0.075 in fp32, 0.36 in fp8; windows three to five times that.
+             // The matrix cores take 6 to 8 with the copy (fp32 8 to 14).  By
+             // the work alone, as before: fp16 1 x 1, 263 -> 440 channels, ten
+             // pixels 30.6 us, now 6; 5 x 5, 12 -> 6, 4 x 5 x 5 51 -> 8; fp8
+             // 1 x 1, 227 -> 6 73 -> 7; of 110 random layers below that line
+             // the 50 that leave it are 1.1 to 37 times as fast.
+             s.kD * s.kH * s.kW * ci <=
+                 (s.kD * s.kH * s.kW > 1 ? 36u : quarterIn ? 8u : 64u))
       igemmWhyNot = tooLittleWork;
     else if (std::size_t(s.outH) * s.strideH + std::size_t(s.kH) * s.dilH +
                      std::size_t(std::abs(s.padH)) >=
