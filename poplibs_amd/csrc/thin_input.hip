@@ -529,7 +529,7 @@ ThinInputLaunch thinInputLaunchShape(const ThinInputDesc &d, uint32_t cus) {
 // channels 23.6 -> 17.5 us with 1147 tiles of four rows for 768, whose registers
 // leave room for three; 33 x 138 x 138 21.6 -> 15.4; 32 x 224 x 224, 7 x 7
 // stride 2, 64 channels 20.4 -> 19.9 with 512 tiles of seven rows; N = 1 to 64,
-// 64 to 256 rows, 80 random layers 6 % at the geometric mean.)
+// 64 to 256 rows, 136 random layers 8 % at the geometric mean.)
 void chooseThinInputTiles(ThinInputDesc &d, uint32_t cus) {
   ThinInputDesc t = d;
   const uint32_t steps = thinKSteps(d), blocks = d.outChans / 16;
@@ -549,11 +549,18 @@ void chooseThinInputTiles(ThinInputDesc &d, uint32_t cus) {
     const uint32_t most = std::max(
         2u, std::min({4u, 512 / registers, 160 * 1024 / s.ldsBytes}));
     for (t.perCU = 2; t.perCU <= most; ++t.perCU) {
-      // Microseconds, fitted to 1500 timings of those layers (5 %; the pick is
-      // within 1 % of the best on average): for a round of tiles on all
+      // Microseconds, fitted to 1500 timings of 80 layers (5 %; the pick is within
+      // 1 % of the best on average): for a round of tiles on all
       // workgroups, for each tile of the busiest CU, its blocks of 16 pixels
       // and its input rows.
       const uint64_t places = uint64_t(cus) * t.perCU;
+      // (more than two to a CU, all in different parts of a large output, lose
+      // what they gain to its stores: 32 x 224 x 224, 3 x 3, 32 channels 25.9
+      // us with two workgroups of seven rows, 31.4 with four, 24.8 with four
+      // of two rows)
+      if (t.perCU > 2 && std::min(places, tiles) * rows * d.outW *
+                                 d.outChans * 2 > 48000000)
+        break;
       const uint64_t full = tiles / places, rest = tiles - full * places;
       const double rounds = double(full + (rest != 0));
       const double perCU = double(full * t.perCU + (rest + cus - 1) / cus);

@@ -1020,7 +1020,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
              // the work alone, as before: fp16 1 x 1, 263 -> 440 channels, ten
              // pixels 30.6 us, now 6; 5 x 5, 12 -> 6, 4 x 5 x 5 51 -> 8; fp8
              // 1 x 1, 227 -> 6 73 -> 7; of 110 random layers below that line
-             // the 50 that leave it are 1.1 to 37 times as fast.
+             // the 61 that leave it are 0.98 to 37 times as fast (3.6 at the
+             // geometric mean).
              s.kD * s.kH * s.kW * ci <=
                  (s.kD * s.kH * s.kW > 1 ? 36u : quarterIn ? 8u : 64u))
       igemmWhyNot = tooLittleWork;
