@@ -503,8 +503,9 @@ hipError_t launchDepthwise(const DepthwiseDesc &d, int inType, int outType,
                            const void *bias, void *out, const QuarterInfo &q,
                            hipStream_t stream) {
   // The kernels address a launch's tensors with 32-bit offsets.  Images are
-  // independent: a batch whose input or output exceeds that goes out as
-  // several launches of as many images as fit.
+  // independent: a batch whose input or output reaches the limit goes out as
+  // several launches of as many images as stay below it (a part that is
+  // itself at the limit would come back here for ever).
   {
     const uint64_t outBytes = outType == kHalf ? 2 : 4;
     const uint64_t inImage = uint64_t(d.inH) * d.inW * d.channels * d.elemBytes;
@@ -512,7 +513,7 @@ hipError_t launchDepthwise(const DepthwiseDesc &d, int inType, int outType,
     const uint64_t limit = kOutOfRange / 2;
     const uint64_t image = inImage > outImage ? inImage : outImage;
     if (image != 0 && image < limit && uint64_t(d.batch) * image >= limit) {
-      const uint32_t perLaunch = uint32_t(limit / image);
+      const uint32_t perLaunch = uint32_t((limit - 1) / image);
       for (uint32_t first = 0; first < d.batch; first += perLaunch) {
         DepthwiseDesc part = d;
         part.batch = d.batch - first < perLaunch ? d.batch - first : perLaunch;
