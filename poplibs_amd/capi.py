@@ -74,26 +74,19 @@ class CParams(Structure):
                 ("output_transform", _COutputTransform)]
 
 
-# CParams as one record: native types and alignment, closed by that of a
-# 64-bit field.
-_PARAMS_RECORD = struct.Struct(
-    "@iiIIQ{m}Q{m}QQQQ{i}{i}{o}0Q".format(
-        m=MAX_FIELD_DIMS, i=f"{5 * MAX_FIELD_DIMS}I{MAX_FIELD_DIMS}B",
-        o=f"{5 * MAX_FIELD_DIMS}I"))
-assert _PARAMS_RECORD.size == ctypes.sizeof(CParams)
-
-
-def _plane_record():
-    """... of two field dimensions, what the others take left out."""
-    r = MAX_FIELD_DIMS - 2
-    words = f"2I{4 * r}x" * 5
-    record = struct.Struct("@iiIIQ2Q{q}x2Q{q}xQQQ{i}{i}{w}0Q".format(
-        q=8 * r, i=f"{words}2B{r}x", w=words))
+def _record(n):
+    """CParams of n field dimensions as one record: native types and
+    alignment, the other dimensions' room left out (zeros), closed by the
+    alignment of a 64-bit field."""
+    r = MAX_FIELD_DIMS - n
+    words = f"{n}I{4 * r}x" * 5
+    record = struct.Struct("@iiIIQ{n}Q{q}x{n}Q{q}xQQQ{i}{i}{w}0Q".format(
+        n=n, q=8 * r, i=f"{words}{n}B{r}x", w=words))
     assert record.size == ctypes.sizeof(CParams)
     return record
 
 
-_PLANE_RECORD = _plane_record()
+_RECORDS = [_record(n) for n in range(MAX_FIELD_DIMS + 1)]
 
 
 class _CPhaseCost(Structure):
@@ -336,12 +329,13 @@ class ConvParams:
 
     # -- marshalling ------------------------------------------------------
     def to_c(self):
+        # One record packed at once, lists and all (a training step makes this
+        # call: field by field it was a tenth of a small layer's step).
         n = len(self.inputFieldShape)
-        # Two dimensions at once, where every list has two entries (a training
-        # step makes this call; 1.9 us, 1.1 this way).
         t, k, o = self.inputTransform, self.kernelTransform, \
             self.outputTransform
-        if (n == 2 == len(self.kernelShape) == len(t.truncationLower)
+        if n > MAX_FIELD_DIMS or not (
+                n == len(self.kernelShape) == len(t.truncationLower)
                 == len(t.truncationUpper) == len(t.dilation)
                 == len(t.paddingLower) == len(t.paddingUpper) == len(t.flip)
                 == len(k.truncationLower) == len(k.truncationUpper)
@@ -350,20 +344,25 @@ class ConvParams:
                 == len(o.truncationLower) == len(o.truncationUpper)
                 == len(o.stride) == len(o.paddingLower)
                 == len(o.paddingUpper)):
-            try:
-                return CParams.from_buffer_copy(_PLANE_RECORD.pack(
-                    self.inputType, self.outputType, 2, 0, self.batchSize,
-                    *self.inputFieldShape, *self.kernelShape,
-                    self.inputChannelsPerConvGroup,
-                    self.outputChannelsPerConvGroup, self.numConvGroups,
-                    *t.truncationLower, *t.truncationUpper, *t.dilation,
-                    *t.paddingLower, *t.paddingUpper, *t.flip,
-                    *k.truncationLower, *k.truncationUpper, *k.dilation,
-                    *k.paddingLower, *k.paddingUpper, *k.flip,
-                    *o.truncationLower, *o.truncationUpper, *o.stride,
-                    *o.paddingLower, *o.paddingUpper))
-            except struct.error:
-                return self._to_c_by_field(n)
+            self._refuse_dims(n)
+        try:
+            return CParams.from_buffer_copy(_RECORDS[n].pack(
+                self.inputType, self.outputType, n, 0, self.batchSize,
+                *self.inputFieldShape, *self.kernelShape,
+                self.inputChannelsPerConvGroup,
+                self.outputChannelsPerConvGroup, self.numConvGroups,
+                *t.truncationLower, *t.truncationUpper, *t.dilation,
+                *t.paddingLower, *t.paddingUpper, *t.flip,
+                *k.truncationLower, *k.truncationUpper, *k.dilation,
+                *k.paddingLower, *k.paddingUpper, *k.flip,
+                *o.truncationLower, *o.truncationUpper, *o.stride,
+                *o.paddingLower, *o.paddingUpper))
+        except struct.error:
+            # (values a field takes modulo its size, or that int() takes)
+            return self._to_c_by_field(n)
+
+    def _refuse_dims(self, n):
+        """Raises for what does not have n dimensions, or for n itself."""
         if n > MAX_FIELD_DIMS:
             raise MxconvError(Status.INVALID_PARAMS,
                               "too many field dimensions")
@@ -372,40 +371,20 @@ class ConvParams:
                 Status.INVALID_PARAMS,
                 "Number of kernel field dimensions does not match the number "
                 "of input field dimensions")
-        # One record packed at once (a training step makes this call: field
-        # by field it was a tenth of a small layer's step).
-        rest = [0] * (MAX_FIELD_DIMS - n)
-        values = [self.inputType, self.outputType, n, 0, self.batchSize,
-                  *self.inputFieldShape, *rest, *self.kernelShape, *rest,
-                  self.inputChannelsPerConvGroup,
-                  self.outputChannelsPerConvGroup, self.numConvGroups]
-        for src, what in (
-                (t.truncationLower, "input truncation"),
-                (t.truncationUpper, "input truncation"),
-                (t.dilation, "input dilation"),
-                (t.paddingLower, "input padding"),
-                (t.paddingUpper, "input padding"), (t.flip, "input flip"),
-                (k.truncationLower, "kernel truncation"),
-                (k.truncationUpper, "kernel truncation"),
-                (k.dilation, "kernel dilation"),
-                (k.paddingLower, "kernel padding"),
-                (k.paddingUpper, "kernel padding"), (k.flip, "kernel flip"),
-                (o.truncationLower, "output truncation"),
-                (o.truncationUpper, "output truncation"),
-                (o.stride, "stride"), (o.paddingLower, "output padding"),
-                (o.paddingUpper, "output padding")):
-            if len(src) != n:
+        each = ("truncation", "truncation", "dilation", "padding", "padding",
+                "flip")
+        names = ([f"input {what}" for what in each]
+                 + [f"kernel {what}" for what in each]
+                 + ["output truncation", "output truncation", "stride",
+                    "output padding", "output padding"])
+        for what, values in zip(names, (*self.inputTransform._fields(),
+                                        *self.kernelTransform._fields(),
+                                        *self.outputTransform._fields())):
+            if len(values) != n:
                 raise MxconvError(
                     Status.INVALID_PARAMS,
-                    f"Number of {what} dimensions ({len(src)}) does not match "
-                    f"the number of field dimensions ({n})")
-            values += src
-            values += rest
-        try:
-            return CParams.from_buffer_copy(_PARAMS_RECORD.pack(*values))
-        except struct.error:
-            # (values a field takes modulo its size, or that int() takes)
-            return self._to_c_by_field(n)
+                    f"Number of {what} dimensions ({len(values)}) does not "
+                    f"match the number of field dimensions ({n})")
 
     def _to_c_by_field(self, n):
         c = CParams()

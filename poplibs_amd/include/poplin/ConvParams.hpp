@@ -119,6 +119,8 @@ struct ConvParams {
 
   /// Throws poputil::poplibs_error when the descriptor is inconsistent.
   void validate() const;
+  /// The same rules on the C interface's parameters, as they are.
+  static void validate(const mxconv_params &params);
   /// Normal form that computes the same result: unused padding / truncation
   /// stripped, stride 1 where one output remains, no flip or dilation on
   /// single-element dimensions; all-zero results map to one "zero conv".

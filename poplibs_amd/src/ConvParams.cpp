@@ -136,10 +136,12 @@ bool operator==(const ConvParams &a, const ConvParams &b) {
 
 // ---- size arithmetic (lib/poplin/ConvParams.cpp:631-698) ------------------
 
-static unsigned transformedSize(const std::vector<std::size_t> &shape,
-                                const InputTransform &t, unsigned dim) {
+/// Of a field or kernel dimension of `size`; T: InputTransform, or the same
+/// members as arrays.
+template <class T>
+static unsigned transformedSize(std::size_t size, const T &t, unsigned dim) {
   const unsigned truncated =
-      unsigned(shape[dim]) - (t.truncationLower[dim] + t.truncationUpper[dim]);
+      unsigned(size) - (t.truncationLower[dim] + t.truncationUpper[dim]);
   return t.paddingLower[dim] + getDilatedSize(truncated, t.dilation[dim]) +
          t.paddingUpper[dim];
 }
@@ -153,10 +155,10 @@ unsigned ConvParams::getTruncatedKernelSize(unsigned dim) const {
                                        kernelTransform.truncationUpper[dim]);
 }
 unsigned ConvParams::getTransformedInputSize(unsigned dim) const {
-  return transformedSize(inputFieldShape, inputTransform, dim);
+  return transformedSize(inputFieldShape[dim], inputTransform, dim);
 }
 unsigned ConvParams::getTransformedKernelSize(unsigned dim) const {
-  return transformedSize(kernelShape, kernelTransform, dim);
+  return transformedSize(kernelShape[dim], kernelTransform, dim);
 }
 std::size_t ConvParams::getUntransformedOutputSize(unsigned dim) const {
   return std::size_t(getTransformedInputSize(dim)) + 1 -
@@ -181,6 +183,103 @@ std::vector<std::size_t> ConvParams::getOutputFieldShape() const {
 
 static std::string num(std::size_t v) { return std::to_string(v); }
 
+namespace {
+/// The field dimensions of a layer's parameters, wherever they are held.
+struct FieldDims {
+  struct Input {
+    const unsigned *truncationLower, *truncationUpper, *dilation,
+        *paddingLower, *paddingUpper;
+    Input(const InputTransform &t)
+        : truncationLower(t.truncationLower.data()),
+          truncationUpper(t.truncationUpper.data()),
+          dilation(t.dilation.data()), paddingLower(t.paddingLower.data()),
+          paddingUpper(t.paddingUpper.data()) {}
+    Input(const mxconv_input_transform &t)
+        : truncationLower(t.truncation_lower),
+          truncationUpper(t.truncation_upper), dilation(t.dilation),
+          paddingLower(t.padding_lower), paddingUpper(t.padding_upper) {}
+  };
+  unsigned count;
+  const std::size_t *inputField, *kernel;
+  Input input, kernelTransform;
+  const unsigned *outTruncationLower, *outTruncationUpper, *stride;
+
+  FieldDims(const ConvParams &p)
+      : count(unsigned(p.inputFieldShape.size())),
+        inputField(p.inputFieldShape.data()), kernel(p.kernelShape.data()),
+        input(p.inputTransform), kernelTransform(p.kernelTransform),
+        outTruncationLower(p.outputTransform.truncationLower.data()),
+        outTruncationUpper(p.outputTransform.truncationUpper.data()),
+        stride(p.outputTransform.stride.data()) {}
+  FieldDims(const mxconv_params &p)
+      : count(p.num_field_dims), inputField(p.input_field_shape),
+        kernel(p.kernel_shape), input(p.input_transform),
+        kernelTransform(p.kernel_transform),
+        outTruncationLower(p.output_transform.truncation_lower),
+        outTruncationUpper(p.output_transform.truncation_upper),
+        stride(p.output_transform.stride) {}
+};
+
+void validateFieldDims(const FieldDims &f) {
+  for (unsigned dim = 0; dim != f.count; ++dim)
+    if (f.stride[dim] == 0)
+      throw poplibs_error("Stride must be non zero");
+  for (unsigned dim = 0; dim != f.count; ++dim)
+    if (f.input.dilation[dim] == 0)
+      throw poplibs_error("Input dilation must be non zero."
+                          " Dilation = 1 results in no dilation");
+  for (unsigned dim = 0; dim != f.count; ++dim)
+    if (f.kernelTransform.dilation[dim] == 0)
+      throw poplibs_error("Kernel dilation must be non zero."
+                          " Dilation = 1 results in no dilation");
+  for (unsigned dim = 0; dim != f.count; ++dim) {
+    const auto inTrunc = std::size_t(f.input.truncationLower[dim]) +
+                         f.input.truncationUpper[dim];
+    if (inTrunc > f.inputField[dim])
+      throw poplibs_error("Truncation for dimension " + num(dim) + " (" +
+                          num(inTrunc) +
+                          ") truncates by more than the size of the field (" +
+                          num(f.inputField[dim]) + ")");
+    const auto kTrunc = std::size_t(f.kernelTransform.truncationLower[dim]) +
+                        f.kernelTransform.truncationUpper[dim];
+    if (kTrunc > f.kernel[dim])
+      throw poplibs_error("Truncation for dimension " + num(dim) + " (" +
+                          num(kTrunc) +
+                          ") truncates by more than the size of the kernel (" +
+                          num(f.kernel[dim]) + ")");
+    const auto tin = transformedSize(f.inputField[dim], f.input, dim);
+    const auto tk = transformedSize(f.kernel[dim], f.kernelTransform, dim);
+    if (tk == 0)
+      throw poplibs_error("Transformed kernel for dimension " + num(dim) +
+                          " has zero size");
+    if (tin < tk)
+      throw poplibs_error("Transformed input size for dimension " + num(dim) +
+                          " (" + num(tin) +
+                          ") is less than the transformed kernel size (" +
+                          num(tk) + ")");
+    const auto convOut = std::size_t(tin) + 1 - tk;
+    const auto outTrunc =
+        std::size_t(f.outTruncationLower[dim]) + f.outTruncationUpper[dim];
+    if (outTrunc > convOut)
+      throw poplibs_error("Output truncation for dimension " + num(dim) +
+                          " (" + num(outTrunc) +
+                          ") truncates by more than the size of the "
+                          "convolution output (" +
+                          num(convOut) + ")");
+  }
+}
+
+/// What of the C interface's parameters the class cannot hold.
+void validateIds(const mxconv_params &c) {
+  if (c.num_field_dims > MXCONV_MAX_FIELD_DIMS)
+    throw poplibs_error("num_field_dims (" + num(c.num_field_dims) +
+                        ") exceeds MXCONV_MAX_FIELD_DIMS");
+  if (c.input_type < 0 || c.input_type > 2 || c.output_type < 0 ||
+      c.output_type > 2)
+    throw poplibs_error("Unknown element type id");
+}
+} // namespace
+
 void ConvParams::validate() const {
   const auto numFieldDims = inputFieldShape.size();
   if (kernelShape.size() != numFieldDims)
@@ -189,17 +288,6 @@ void ConvParams::validate() const {
                         ") does not match the number of input field "
                         "dimensions (" +
                         num(numFieldDims) + ")");
-  for (auto s : outputTransform.stride)
-    if (s == 0)
-      throw poplibs_error("Stride must be non zero");
-  for (auto d : inputTransform.dilation)
-    if (d == 0)
-      throw poplibs_error("Input dilation must be non zero."
-                          " Dilation = 1 results in no dilation");
-  for (auto d : kernelTransform.dilation)
-    if (d == 0)
-      throw poplibs_error("Kernel dilation must be non zero."
-                          " Dilation = 1 results in no dilation");
   const std::pair<std::size_t, const char *> ranks[] = {
       {inputTransform.truncationLower.size(), "input truncation (lower)"},
       {inputTransform.truncationUpper.size(), "input truncation (upper)"},
@@ -225,41 +313,12 @@ void ConvParams::validate() const {
                           " dimensions (" + num(r.first) +
                           ") does not match the number of field dimensions (" +
                           num(numFieldDims) + ")");
-  for (unsigned dim = 0; dim != numFieldDims; ++dim) {
-    const auto inTrunc = std::size_t(inputTransform.truncationLower[dim]) +
-                         inputTransform.truncationUpper[dim];
-    if (inTrunc > inputFieldShape[dim])
-      throw poplibs_error("Truncation for dimension " + num(dim) + " (" +
-                          num(inTrunc) +
-                          ") truncates by more than the size of the field (" +
-                          num(inputFieldShape[dim]) + ")");
-    const auto kTrunc = std::size_t(kernelTransform.truncationLower[dim]) +
-                        kernelTransform.truncationUpper[dim];
-    if (kTrunc > kernelShape[dim])
-      throw poplibs_error("Truncation for dimension " + num(dim) + " (" +
-                          num(kTrunc) +
-                          ") truncates by more than the size of the kernel (" +
-                          num(kernelShape[dim]) + ")");
-    const auto tin = getTransformedInputSize(dim);
-    const auto tk = getTransformedKernelSize(dim);
-    if (tk == 0)
-      throw poplibs_error("Transformed kernel for dimension " + num(dim) +
-                          " has zero size");
-    if (tin < tk)
-      throw poplibs_error("Transformed input size for dimension " + num(dim) +
-                          " (" + num(tin) +
-                          ") is less than the transformed kernel size (" +
-                          num(tk) + ")");
-    const auto convOut = getUntransformedOutputSize(dim);
-    const auto outTrunc = std::size_t(outputTransform.truncationLower[dim]) +
-                          outputTransform.truncationUpper[dim];
-    if (outTrunc > convOut)
-      throw poplibs_error("Output truncation for dimension " + num(dim) +
-                          " (" + num(outTrunc) +
-                          ") truncates by more than the size of the "
-                          "convolution output (" +
-                          num(convOut) + ")");
-  }
+  validateFieldDims(*this);
+}
+
+void ConvParams::validate(const mxconv_params &c) {
+  validateIds(c);
+  validateFieldDims(c);
 }
 
 // ---- normal form (lib/poplin/ConvParams.cpp:468-629) ----------------------
@@ -611,12 +670,7 @@ void ConvParams::toC(mxconv_params &c) const {
 }
 
 ConvParams ConvParams::fromC(const mxconv_params &c) {
-  if (c.num_field_dims > MXCONV_MAX_FIELD_DIMS)
-    throw poplibs_error("num_field_dims (" + num(c.num_field_dims) +
-                        ") exceeds MXCONV_MAX_FIELD_DIMS");
-  if (c.input_type < 0 || c.input_type > 2 || c.output_type < 0 ||
-      c.output_type > 2)
-    throw poplibs_error("Unknown element type id");
+  validateIds(c);
   const unsigned n = c.num_field_dims;
   ConvParams p;
   p.inputType = poplar::Type(c.input_type);
