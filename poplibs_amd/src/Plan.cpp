@@ -772,6 +772,75 @@ mxconv_plan makePlan(const ConvParams &params, const ConvOptions &optionsIn) {
 
 namespace {
 
+/// The kernels of LDS halo tiles and of rings of rows (3 x 3 taps, input
+/// dilations, other element types; 5 x 5 and 7 x 7 halves where a plan names one
+/// of them or `columns` 0).
+void chooseDepthwiseTileOrRing(mxk::DepthwiseDesc &d, const PlanConstraints &pc,
+                               bool inputDilated, int dwType) {
+  // 7 x 7 taps at unit stride: a thread forms a strip of neighbouring
+  // pixels, and the tile is chosen to fill the workgroup's 256 threads.
+  if (mxk::depthwiseStripTakes(d) && !(pc.tileH || pc.tileW))
+    chooseDepthwiseStripTile(d);
+  // An explicit tile asks for the LDS-tiled kernel.
+  d.dense3x3 = !inputDilated && !(pc.tileH || pc.tileW) &&
+               mxk::depthwise3x3Takes(d, dwType);
+  // Layers that give every CU a band of at least four output rows go to
+  // the persistent kernel with a ring of input rows in LDS: its start-up
+  // (seven rows before the first output; 3.5 us for the smallest layer
+  // against 2.9 us) wants rows to spread over.  Layers of more channels
+  // than the small-workgroup kernel takes (224) always do: the kernel of
+  // LDS halo tiles needs 5 to 8 us for the smallest of them.
+  if (!inputDilated && !(pc.tileH || pc.tileW) && pc.rowRing != 0) {
+    d.cus = gfx950::numCUs;
+    const mxk::DepthwiseRowsLaunch l = mxk::depthwiseRowsLaunchShape(d);
+    const bool takes = mxk::depthwiseRowsTakes(d, dwType);
+    if (pc.rowRing == 1 && !takes)
+      throw poplar::invalid_option(
+          "planConstraints gfx950 rowRing: that kernel takes 3x3 or 5x5 "
+          "taps, stride 1 or 2, channels in vectors of 8, at most 2048 "
+          "(5x5: 1224) to a pixel");
+    // 5 x 5 taps (25 multiply-adds per output and channel: the vector ALU
+    // shares the bound): strips of four columns or more, and at stride 2
+    // bands of six rows or more - N = 32, 56 x 56, 144 channels, stride 2
+    // 26.0 -> 13.1 us and 14 x 14, 480 channels 14.7 -> 9.3, but 28 x 28,
+    // 240 channels, stride 2 8.1 -> 9.3 and 7 x 7, 1152 channels (strips of
+    // one column) 10.6 -> 12.6.
+    const bool five = d.kH == 5;
+    // Layers of less than 6 MB take it with strips of two columns and any
+    // band: a tile's patch and its rounds of pixels are a longer chain than
+    // the ring's first rows (of 48 such layers, stride 2 but one, all were
+    // faster, by 23 % at the median: N = 10, 29 x 29, 40 channels 8.8 ->
+    // 5.1, N = 3, 23 x 23, 416 8.1 -> 5.0, N = 37, 9 x 9, 640 7.7 -> 6.4).
+    const double bytes = 2.0 * d.batch * d.channels *
+                         (double(d.inH) * d.inW + double(d.outH) * d.outW);
+    const bool fiveWorth =
+        ((l.colsOut >= 4 || l.strips == 1) &&
+         (d.strideH == 1 || l.rowsOut >= 6)) ||
+        (l.colsOut >= 2 && bytes < 6e6);
+    if (takes &&
+        (pc.rowRing == 1 ||
+         (five ? fiveWorth
+               : !d.dense3x3 || (l.workgroups * 2 >= gfx950::numCUs &&
+                                 l.rowsOut >= 4))))
+      d.dense3x3 = 2;
+  } else if (pc.rowRing == 1) {
+    throw poplar::invalid_option(
+        "planConstraints gfx950 rowRing: the layer is not one the "
+        "depthwise 3x3 kernels take");
+  }
+  if (!inputDilated && (pc.tileH || pc.tileW)) {
+    d.tileH = pc.tileH ? pc.tileH : d.tileH;
+    d.tileW = pc.tileW ? pc.tileW : d.tileW;
+    if (mxk::depthwiseStripTakes(d))
+      d.stripPixels = stripPixelsFor(d, d.tileH, d.tileW);
+    if (mxk::depthwiseTileLdsBytes(d) >
+        (d.stripPixels ? mxk::kDepthwiseTileLdsMost : 64 * 1024))
+      throw poplar::invalid_option(
+          "planConstraints gfx950 tileH x tileW: the input patch of such a "
+          "tile does not fit 64 KB of LDS");
+  }
+}
+
 mxconv_plan makePlanWith(const ConvParams &params,
                          const ConvOptions &optionsIn,
                          unsigned convGroupsPerGroup) {
@@ -1928,74 +1997,13 @@ mxconv_plan makePlanWith(const ConvParams &params,
     const int dwType = halfIn ? mxk::kHalf
                        : floatIn ? mxk::kFloat
                                  : mxk::kQuarter;
-    // 7 x 7 taps at unit stride: a thread forms a strip of neighbouring
-    // pixels, and the tile is chosen to fill the workgroup's 256 threads.
-    if (mxk::depthwiseStripTakes(d) && !(pc.tileH || pc.tileW))
-      chooseDepthwiseStripTile(d);
-    // An explicit tile asks for the LDS-tiled kernel.
-    d.dense3x3 = !s.inputDilated() && !(pc.tileH || pc.tileW) &&
-                 mxk::depthwise3x3Takes(d, dwType);
-    // Layers that give every CU a band of at least four output rows go to
-    // the persistent kernel with a ring of input rows in LDS: its start-up
-    // (seven rows before the first output; 3.5 us for the smallest layer
-    // against 2.9 us) wants rows to spread over.  Layers of more channels
-    // than the small-workgroup kernel takes (224) always do: the kernel of
-    // LDS halo tiles needs 5 to 8 us for the smallest of them.
-    if (!s.inputDilated() && !(pc.tileH || pc.tileW) && pc.rowRing != 0) {
-      d.cus = gfx950::numCUs;
-      const mxk::DepthwiseRowsLaunch l = mxk::depthwiseRowsLaunchShape(d);
-      const bool takes = mxk::depthwiseRowsTakes(d, dwType);
-      if (pc.rowRing == 1 && !takes)
-        throw poplar::invalid_option(
-            "planConstraints gfx950 rowRing: that kernel takes 3x3 or 5x5 "
-            "taps, stride 1 or 2, channels in vectors of 8, at most 2048 "
-            "(5x5: 1224) to a pixel");
-      // 5 x 5 taps (25 multiply-adds per output and channel: the vector ALU
-      // shares the bound): strips of four columns or more, and at stride 2
-      // bands of six rows or more - N = 32, 56 x 56, 144 channels, stride 2
-      // 26.0 -> 13.1 us and 14 x 14, 480 channels 14.7 -> 9.3, but 28 x 28,
-      // 240 channels, stride 2 8.1 -> 9.3 and 7 x 7, 1152 channels (strips of
-      // one column) 10.6 -> 12.6.
-      const bool five = d.kH == 5;
-      // Layers of less than 6 MB take it with strips of two columns and any
-      // band: a tile's patch and its rounds of pixels are a longer chain than
-      // the ring's first rows (of 48 such layers, stride 2 but one, all were
-      // faster, by 23 % at the median: N = 10, 29 x 29, 40 channels 8.8 ->
-      // 5.1, N = 3, 23 x 23, 416 8.1 -> 5.0, N = 37, 9 x 9, 640 7.7 -> 6.4).
-      const double bytes = 2.0 * d.batch * d.channels *
-                           (double(d.inH) * d.inW + double(d.outH) * d.outW);
-      const bool fiveWorth =
-          ((l.colsOut >= 4 || l.strips == 1) &&
-           (d.strideH == 1 || l.rowsOut >= 6)) ||
-          (l.colsOut >= 2 && bytes < 6e6);
-      if (takes &&
-          (pc.rowRing == 1 ||
-           (five ? fiveWorth
-                 : !d.dense3x3 || (l.workgroups * 2 >= gfx950::numCUs &&
-                                   l.rowsOut >= 4))))
-        d.dense3x3 = 2;
-    } else if (pc.rowRing == 1) {
-      throw poplar::invalid_option(
-          "planConstraints gfx950 rowRing: the layer is not one the "
-          "depthwise 3x3 kernels take");
-    }
-    if (!s.inputDilated() && (pc.tileH || pc.tileW)) {
-      d.tileH = pc.tileH ? pc.tileH : d.tileH;
-      d.tileW = pc.tileW ? pc.tileW : d.tileW;
-      if (mxk::depthwiseStripTakes(d))
-        d.stripPixels = stripPixelsFor(d, d.tileH, d.tileW);
-      if (mxk::depthwiseTileLdsBytes(d) >
-          (d.stripPixels ? mxk::kDepthwiseTileLdsMost : 64 * 1024))
-        throw poplar::invalid_option(
-            "planConstraints gfx950 tileH x tileW: the input patch of such a "
-            "tile does not fit 64 KB of LDS");
-    }
     // 5 x 5 and 7 x 7 taps: strips of columns, wherever no other kernel is
-    // named.  Against the two kernels above, at their choice, 90 random layers
-    // were 1.1 to 7 times as fast; small, large, strided and narrow ones alike,
-    // so there is no line to draw.
+    // named.  Against the kernels below, at their choice, 90 random layers were
+    // 1.1 to 7 times as fast; small, large, strided and narrow ones alike, so
+    // there is no line to draw.
     const bool columns =
-        !plan.depthwiseWeightUpdate && pc.columns != 0 && !(pc.tileH || pc.tileW) && pc.rowRing != 1 &&
+        !plan.depthwiseWeightUpdate && pc.columns != 0 &&
+        !(pc.tileH || pc.tileW) && pc.rowRing != 1 &&
         mxk::depthwiseColumnsTakes(d, dwType,
                                    params.outputType == poplar::HALF
                                        ? mxk::kHalf
@@ -2006,8 +2014,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
       throw poplar::invalid_option(
           "planConstraints gfx950 columns: that kernel takes fp16 inputs, 5x5 "
           "or 7x7 taps at stride 1 or 2, without a tile or rowRing named");
-    if (d.columns)
-      d.dense3x3 = 0, d.stripPixels = 0;
+    else
+      chooseDepthwiseTileOrRing(d, pc, s.inputDilated(), dwType);
     plan.weightPackedElems = plan.weightElems; // [kH*kW][C]
   } else {
     plan.weightPackedElems = plan.weightElems; // [G][K][Ci][Co]
