@@ -38,7 +38,7 @@
 //
 // The reference's role: depthwise layers go through
 // lib/poplin/codelets/ConvPartialHorizontalMac.cpp there.
-#include "igemm_common.hpp"
+#include "depthwise_columns.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -47,7 +47,6 @@ namespace mxk {
 namespace {
 
 constexpr uint32_t kColInvalid = 0x40000000u;
-constexpr int kColThreads = 256;
 
 struct ColumnsArgs {
   uint32_t items; // image x strip x pair of channels
@@ -60,27 +59,12 @@ struct ColumnsArgs {
 };
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
-/// Channel CH of two elements of a channel pair.
-template <int CH>
-__device__ __forceinline__ half2v pairOf(uint32_t first, uint32_t second) {
-  return __builtin_bit_cast(
-      half2v, __builtin_amdgcn_perm(second, first,
-                                    CH == 0 ? 0x05040100u : 0x07060302u));
-}
 template <int CH> __device__ __forceinline__ float channelOf(uint32_t two) {
   float v = float(__builtin_bit_cast(half2v, two)[CH]);
   // (a float from here on: a multiply-add that converts runs at half the rate)
   asm("" : "+v"(v));
   return v;
-}
-
-/// Calls each with 0, 1, ... until one answers false.
-template <int... I, class F>
-__device__ __forceinline__ bool whileEach(std::integer_sequence<int, I...>,
-                                          F &&each) {
-  return (each(std::integral_constant<int, I>{}) && ...);
 }
 
 /// K x K taps, stride S; STRIP output columns per lane.
@@ -89,9 +73,8 @@ __global__ __launch_bounds__(kColThreads) void depthwiseColumnsKernel(
     const ColumnsArgs a, const char *__restrict__ in,
     const uint32_t *__restrict__ weights, const OutT *__restrict__ bias,
     char *__restrict__ out) {
-  constexpr int NX = S * (STRIP - 1) + K;  // input columns of a strip
-  constexpr int LIVE = (K + S - 1) / S;    // output rows under way
-  constexpr int PERIOD = LIVE * S;         // input rows until they come round
+  using Walk = ColumnWalk<K, S, STRIP>;
+  constexpr int NX = Walk::kColumns, LIVE = Walk::kLive, PERIOD = Walk::kPeriod;
   const uint32_t block = xcdSwizzle(blockIdx.x, gridDim.x);
   const uint32_t itemBlock = a.divBands(block);
   const uint32_t band = block - itemBlock * a.bands;
@@ -121,7 +104,7 @@ __global__ __launch_bounds__(kColThreads) void depthwiseColumnsKernel(
   // out of the sums, so that every load is unconditional.)
   const int firstRow = int(y0 * S) - a.padH;
   auto rowInside = [&](uint32_t r) {
-    return uint32_t(firstRow + int(r)) - a.loH < a.hiH - a.loH;
+    return rowIsRead(firstRow + int(r), a.loH, a.hiH);
   };
   uint32_t raw[NX];
   auto load = [&](uint32_t r) {

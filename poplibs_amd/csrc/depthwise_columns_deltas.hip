@@ -29,16 +29,13 @@
 //
 // The reference's role: the weight update passes of depthwise layers go
 // through lib/poplin/codelets/ConvPartialHorizontalMac.cpp there.
-#include "igemm_common.hpp"
+#include "depthwise_columns.hpp"
 
 #include <algorithm>
 #include <cmath>
 
 namespace mxk {
 namespace {
-
-constexpr int kColThreads = 256;
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
 struct ColumnDeltasArgs {
   uint32_t pairs, perBlock, blocksC, slots; // (of channel pairs)
@@ -51,28 +48,12 @@ struct ColumnDeltasArgs {
   FastDiv divPerBlock, divStrips, divBlocksC, divBands;
 };
 
-/// Channel CH of two elements of a channel pair.
-template <int CH>
-__device__ __forceinline__ half2v pairOf(uint32_t first, uint32_t second) {
-  return __builtin_bit_cast(
-      half2v, __builtin_amdgcn_perm(second, first,
-                                    CH == 0 ? 0x05040100u : 0x07060302u));
-}
-
-/// Calls each with 0, 1, ... until one answers false.
-template <int... I, class F>
-__device__ __forceinline__ bool whileEach(std::integer_sequence<int, I...>,
-                                          F &&each) {
-  return (each(std::integral_constant<int, I>{}) && ...);
-}
-
 template <int K, int S, int STRIP>
 __global__ __launch_bounds__(kColThreads) void depthwiseColumnDeltasKernel(
     const ColumnDeltasArgs a, const char *__restrict__ acts,
     const char *__restrict__ deltas, float *__restrict__ partial) {
-  constexpr int NX = S * (STRIP - 1) + K; // input columns of a strip
-  constexpr int LIVE = (K + S - 1) / S;   // rows of deltas under way
-  constexpr int PERIOD = LIVE * S;        // input rows until they come round
+  using Walk = ColumnWalk<K, S, STRIP>;
+  constexpr int NX = Walk::kColumns, LIVE = Walk::kLive, PERIOD = Walk::kPeriod;
   __shared__ float meet[K * K][kColThreads];
   const uint32_t block = xcdSwizzle(blockIdx.x, gridDim.x);
   const uint32_t rest = a.divBlocksC(block);
@@ -88,7 +69,7 @@ __global__ __launch_bounds__(kColThreads) void depthwiseColumnDeltasKernel(
   const __amdgpu_buffer_rsrc_t inBuf = bufferOf(acts, a.inBytes);
   const __amdgpu_buffer_rsrc_t outBuf = bufferOf(deltas, a.outBytes);
   auto rowInside = [&](uint32_t r) {
-    return uint32_t(firstRow + int(r)) - a.loH < a.hiH - a.loH;
+    return rowIsRead(firstRow + int(r), a.loH, a.hiH);
   };
 
   float sum[2][K][K];
