@@ -95,6 +95,33 @@ def test_infinities_stay_in_their_windows(oracle, k, stride, columns):
     np.testing.assert_array_equal(got[~inside], finite[~inside])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["acts", "weights", "both"])
+@pytest.mark.parametrize("columns", [2, 4])
+@pytest.mark.parametrize("k,stride", [(5, 2), (7, 1)])
+def test_subnormal_halves_are_exact(oracle, k, stride, columns, which):
+    """Subnormals (multiples of 2^-24 below 2^-14) against signs, and against
+    each other: the sums are below 2^24 of their unit, which fp32 holds."""
+    from gpu_helpers import run_conv
+    p = make_params(pa.HALF, pa.FLOAT, batch=2, field=(17, 13), kernel=(k, k),
+                    groups=24, stride=stride, pad=k // 2)
+    print("case", k, stride, columns, which, flush=True)
+    acts, weights, _ = random_data(p, 23, "pm1")
+    rng = np.random.default_rng(23)
+
+    def small(like):
+        return like * rng.integers(1, 256, like.shape) * 2.0 ** -24
+
+    if which != "weights":
+        acts = small(acts)
+    if which != "acts":
+        weights = small(weights)
+    got = run_conv(p, acts.astype(np.float16), weights.astype(np.float16),
+                   None, _options(columns))
+    want = oracle.convolution(p, acts, weights, threads=8)
+    np.testing.assert_array_equal(got, want)
+
+
 def test_columns_plan_choice():
     kw = dict(batch=4, field=(30, 30), kernel=(7, 7), groups=48, pad=3)
     plan = pa.Plan(make_params(pa.HALF, **kw))

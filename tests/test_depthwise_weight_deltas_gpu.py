@@ -74,6 +74,32 @@ def test_columns_of_signs_are_exact(oracle, kw, columns):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("which", ["acts", "deltas", "both"])
+@pytest.mark.parametrize("columns", [2, 4])
+@pytest.mark.parametrize("k,stride", [(3, 1), (5, 2), (7, 1)])
+def test_subnormal_halves_are_exact(oracle, k, stride, columns, which):
+    """Multiples of 2^-24 below 2^-14 against signs, and against each other:
+    sums of 234 products of at most 2^16 units, which fp32 holds."""
+    p = make_params(pa.HALF, pa.FLOAT, batch=2, field=(13, 9), kernel=(k, k),
+                    groups=16, stride=stride, pad=k // 2)
+    print("case", k, stride, columns, which, flush=True)
+    rng = np.random.default_rng(29)
+
+    def data(shape, small):
+        signs = rng.choice([-1.0, 1.0], shape)
+        return signs * rng.integers(1, 256, shape) * 2.0 ** -24 if small \
+            else signs
+
+    x = data((2, 16, 13, 9), which != "deltas")
+    dz = data((2, 16, *p.getOutputFieldShape()), which != "acts")
+    got, plan = run_weight_update(p, x.astype(np.float16),
+                                  dz.astype(np.float16), _options(columns))
+    assert COLUMNS in plan.describe()
+    np.testing.assert_array_equal(got, oracle.weight_deltas(p, x, dz,
+                                                            threads=8))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("where", ["acts", "deltas"])
 @pytest.mark.parametrize("columns", [2, 4])
 @pytest.mark.parametrize("k,stride", [(3, 1), (5, 2), (7, 1)])

@@ -75,6 +75,35 @@ def test_window_weight_deltas_of_signs_are_exact(oracle, kw):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kw", [
+    # odd channels in groups: copies filled up to whole vectors, of both
+    # tensors or of one; groups that stay by themselves, that run as one, a
+    # last tile with fewer; one chunk and many
+    dict(batch=3, field=(10, 9), kernel=(3, 3), ci=5, co=7, groups=4, pad=1),
+    dict(batch=3, field=(10, 9), kernel=(3, 3), ci=5, co=7, groups=8, pad=1),
+    dict(batch=3, field=(10, 9), kernel=(3, 3), ci=9, co=16, groups=3, pad=1),
+    dict(batch=3, field=(10, 9), kernel=(1, 1), ci=8, co=3, groups=16,
+         stride=2),
+    dict(batch=2, field=(9, 11), kernel=(3, 3), ci=33, co=17, groups=2, pad=1),
+    dict(batch=20, field=(23, 25), kernel=(3, 3), ci=3, co=3, groups=16,
+         pad=1),
+])
+@pytest.mark.parametrize("out_type", [pa.HALF, pa.FLOAT])
+def test_odd_channels_in_groups_are_exact(oracle, kw, out_type):
+    from test_weight_update import run_weight_update
+    p = make_params(pa.HALF, out_type, **kw)
+    print("case", p, flush=True)
+    x, dz = _signs(p, 74)
+    got, plan = run_weight_update(p, x.astype(np.float16),
+                                  dz.astype(np.float16), BY_NAME)
+    assert WINDOW in plan.describe(), plan.describe()
+    want = oracle.weight_deltas(p, x, dz, threads=8)
+    np.testing.assert_array_equal(
+        got, want if out_type == pa.FLOAT else
+        want.astype(np.float16).astype(np.float64))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kw", [CASES[3], CASES[5], CASES[9], CASES[16],
                                 CASES[-4], CASES[-1]])
 def test_window_weight_deltas_to_half(oracle, kw):
