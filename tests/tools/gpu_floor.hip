@@ -26,9 +26,20 @@
 //       Cache), 200 launches in a replayed HIP graph as bench.py issues its
 //       steps.  Variants: U outputs per thread, plain or non-temporal loads
 //       and stores, the four loads of an output far apart or adjacent.
+//
+//   gpu_floor call libmxconv.so
+//       the host's time for one call, when the stream has room (64 calls
+//       behind an empty queue, best of 30) and among thousands: an empty
+//       kernel with 256 bytes of arguments launched bare, and mxconv_fwd of
+//       the smallest layer that perf/cases.py lists (one 32 x 32 image, 3 x 3,
+//       16 -> 16, fp32; one launch) from the library named.
+#include <dlfcn.h>
 #include <hip/hip_runtime.h>
 
+#include "mxconv.h"
+
 #include <algorithm>
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -270,11 +281,104 @@ void clockUnderLoad(int workgroups) {
   CHECK(hipFree(sink));
 }
 
+struct CallArgs {
+  uint32_t words[62];
+  int *never;
+};
+__global__ void emptyCall(CallArgs a) {
+  if (a.never && threadIdx.x == 0x7fffffff)
+    *a.never = int(a.words[3]);
+}
+
+/// Prints the host's microseconds per call of `call`.
+template <class F> void callTime(const char *what, F &&call) {
+  auto timed = [&](int calls, int passes, bool drained) {
+    double best = 1e30;
+    for (int p = 0; p != passes; ++p) {
+      CHECK(hipDeviceSynchronize());
+      const auto start = std::chrono::steady_clock::now();
+      for (int i = 0; i != calls; ++i)
+        call();
+      if (drained)
+        CHECK(hipDeviceSynchronize());
+      const std::chrono::duration<double, std::micro> us =
+          std::chrono::steady_clock::now() - start;
+      best = std::min(best, us.count() / calls);
+    }
+    CHECK(hipDeviceSynchronize());
+    return best;
+  };
+  const double alone = timed(64, 30, false);
+  std::printf("| %s | %.2f | %.2f |\n", what, alone, timed(5000, 5, true));
+}
+
+void callCosts(const char *library) {
+  void *lib = dlopen(library, RTLD_NOW);
+  if (!lib) {
+    std::fprintf(stderr, "%s\n", dlerror());
+    std::exit(1);
+  }
+  auto symbol = [&](auto *type, const char *name) {
+    void *at = dlsym(lib, name);
+    if (!at) {
+      std::fprintf(stderr, "%s: no %s\n", library, name);
+      std::exit(1);
+    }
+    return reinterpret_cast<decltype(type)>(at);
+  };
+  const auto ok = [](mxconv_status status) {
+    if (status != MXCONV_OK) {
+      std::fprintf(stderr, "mxconv status %d\n", int(status));
+      std::exit(1);
+    }
+  };
+  mxconv_params params;
+  const uint64_t field[2] = {32, 32}, kernel[2] = {3, 3};
+  ok(symbol(&mxconv_params_init, "mxconv_params_init")(
+      &params, MXCONV_FLOAT, MXCONV_FLOAT, 1, 2, field, kernel, 16, 16, 1));
+  for (int d = 0; d != 2; ++d)
+    params.input_transform.padding_lower[d] =
+        params.input_transform.padding_upper[d] = 1;
+  mxconv_plan *plan = nullptr;
+  ok(symbol(&mxconv_plan_create, "mxconv_plan_create")(&params, nullptr,
+                                                       nullptr, 0, &plan));
+  void *buffers[5];
+  size_t bytes[5];
+  for (int b = 0; b != 5; ++b) {
+    ok(symbol(&mxconv_plan_buffer_bytes, "mxconv_plan_buffer_bytes")(plan, b,
+                                                                     &bytes[b]));
+    CHECK(hipMalloc(&buffers[b], bytes[b] + 256));
+    CHECK(hipMemset(buffers[b], 0, bytes[b] + 256));
+  }
+  const auto fwd = symbol(&mxconv_fwd, "mxconv_fwd");
+  hipStream_t stream;
+  CHECK(hipStreamCreate(&stream));
+  int version = 0;
+  CHECK(hipRuntimeGetVersion(&version));
+  std::printf("HIP runtime %d\n\n| call | us, the queue empty | us, among "
+              "5000 |\n|---|---|---|\n", version);
+  callTime("empty kernel, 64 workgroups of 256, 256 bytes of arguments", [&] {
+    hipLaunchKernelGGL(emptyCall, dim3(64), dim3(256), 0, stream, CallArgs{});
+  });
+  callTime("mxconv_fwd, one 32 x 32 image, 3 x 3, 16 -> 16, fp32", [&] {
+    ok(fwd(plan, buffers[MXCONV_BUFFER_INPUT],
+           buffers[MXCONV_BUFFER_WEIGHTS_PACKED], nullptr,
+           buffers[MXCONV_BUFFER_OUTPUT], buffers[MXCONV_BUFFER_WORKSPACE],
+           bytes[MXCONV_BUFFER_WORKSPACE],
+           reinterpret_cast<mxconv_stream>(stream)));
+  });
+}
+
 int main(int argc, char **argv) {
+  if (argc == 3 && !std::strcmp(argv[1], "call")) {
+    callCosts(argv[2]);
+    return 0;
+  }
   if (argc < 2 || (std::strcmp(argv[1], "launch") && std::strcmp(argv[1], "clock") &&
                    std::strcmp(argv[1], "stream"))) {
     std::fprintf(stderr, "usage: gpu_floor launch | gpu_floor clock "
-                         "[workgroups ...] | gpu_floor stream\n");
+                         "[workgroups ...] | gpu_floor stream | gpu_floor "
+                         "call libmxconv.so\n");
     return 2;
   }
   hipDeviceProp_t prop;
