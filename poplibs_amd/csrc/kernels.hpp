@@ -428,7 +428,7 @@ bool depthwiseStripTakes(const DepthwiseDesc &d);
 uint64_t depthwiseTileLdsBytes(const DepthwiseDesc &d);
 constexpr uint32_t kDepthwiseTileLdsMost = 80 * 1024;
 /// fp16, 5 x 5 or 7 x 7 taps, stride 1 or 2: a lane walks down a strip of
-/// output columns of one channel.
+/// output columns of two neighbouring channels.
 bool depthwiseColumnsTakes(const DepthwiseDesc &d, int inType, int outType);
 /// Strip (2 or 4 columns; 0: the faster) and band for d, and what they take.
 void chooseDepthwiseColumns(DepthwiseDesc &d, uint32_t strip);

@@ -360,11 +360,14 @@ template <> struct WinFloats<3> {
 /// permuted; the matrix pipe (32 cycles for 16 x 16 x 4) is the bound, and
 /// tiles of J = 1, 2 or 3 blocks both ways leave little of it to padding.  The
 /// passes of these layers were convolutions of their own between two
-/// rearrangements, four launches and more; us before and after: 48 -> 43
-/// channels, 3 x 3, 15 x 9 x 9 28.8 -> 8.5; 312 -> 160, 1 x 1 stride 2, 10 x 15 x
-/// 15 34.7 -> 8; 32 groups of 16, 3 x 3, 64 x 16 x 16 224 -> 40; 128 -> 128, 3 x
-/// 3, 36 x 56 x 56 389 -> 275 (the matrix pipe's own time 222).  Over 340 random
-/// layers 4.6 times as fast (geometric mean, least 0.98).
+/// rearrangements, four launches and more; us before and after, a pass in a
+/// replayed graph: 48 -> 43 channels, 3 x 3, 15 x 9 x 9 28.2 -> 9.6; 312 -> 160,
+/// 1 x 1 stride 2, 10 x 15 x 15 34.7 -> 5.8; 32 groups of 16, 3 x 3, 64 x 16 x 16
+/// 224 -> 40; 128 -> 128, 3 x 3, 36 x 56 x 56 346 -> 275 (the matrix pipe's own
+/// time 222).  Over 14 150 random layers of up to 512 channels and 10 GFLOP 3.8
+/// times as fast (geometric mean).  Rows of few columns leave a unit of eight
+/// half empty: wide layers of them are where it loses (floatWindowAsked in
+/// Plan.cpp).
 template <int J, int KW, int S, int NW, class OutT>
 __global__ __launch_bounds__(64 * NW) void wuWindowFloatKernel(
     const WuWindowArgs a, const char *__restrict__ acts,

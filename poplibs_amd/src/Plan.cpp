@@ -618,8 +618,17 @@ mxconv_plan makePlanWith(const ConvParams &params,
                          unsigned convGroupsPerGroup);
 
 /// fp32 layers: wuWindowKernel's fp32 sibling wherever it takes the layer and
-/// nothing names a tile for the pass's own convolution (340 random layers 0.98
-/// to 100 times as fast as that, so there is no line to draw).
+/// nothing names a tile for the pass's own convolution.  Over 14 150 random
+/// layers (1 to 64 images of 5 to 64 squared, up to 512 channels and 10 GFLOP)
+/// it is 3.8 times as fast (geometric mean), slower for 24 of them.  Those, and
+/// 498 of 6 350 of up to 1024 channels and 60 GFLOP, are 3 x 3 layers, all but
+/// three of more than 200 channels, most with rows that fill the kernel's units
+/// of eight columns to 75 % or less (61 images of 7 x 7 at stride 2, 389 -> 442
+/// 108.7 us, the convolution 67.7; 36 of 9 x 9, 699 -> 619 475 against 236).  They
+/// stay with the kernel all the same: the convolution adds its pixels in one
+/// chain, or a few, and its error against 64 bits was 1.7 to 3.4 times the
+/// kernel's for six of them (those two 4.7e-7 against 1.8e-7 and 9.0e-7 against
+/// 3.2e-7).
 bool floatWindowAsked(const PlanConstraints &pc) {
   return pc.deltaWindow == 1 ||
          (!pc.blockM && !pc.blockN && !pc.blockK && !pc.splitK && !pc.stages &&
@@ -629,11 +638,12 @@ bool floatWindowAsked(const PlanConstraints &pc) {
 /// The weight deltas of `layer` (channels of a group as the layer has them, in
 /// resultCi and resultCo) by wuWindowKernel, where that is named or estimated
 /// to be faster than what `plan` has; `fuse`: groups that plan takes as one.
-/// Of 4 500 random layers that both kernels take, the estimates' choice was
-/// 0.6 % slower than the faster of the two on average and 20 % faster than
-/// wuTapKernel for all.  The line at 0.93: wide layers (128 -> 128 channels, 28 x
-/// 28, 3 x 3, 32 images: 20.5 us by taps, 21.3 by windows) are estimated that
-/// much too slow by taps.
+/// The line at 0.93: of 12 950 random layers that both kernels take (1 to 64
+/// images of 5 to 64 squared, 16 to 768 channels, 1 x 1 and 3 x 3, up to 25
+/// GFLOP) the choice is on average 0.6 % slower than the faster of the two, 0.7 %
+/// in total time; at 0.85 2.2 and 2.0 %, at 0.9 1.0 and 1.0, at 0.96 0.4 and 0.7,
+/// at 1 0.6 and 0.9, at 1.05 0.9 and 1.4 (wuTapKernel for all 24 %, this one for
+/// all 2.5 %).
 void windowWeightDeltas(mxconv_plan &plan, const mxk::WuTapDesc &layer,
                         unsigned fuse) {
   const auto &pc = plan.options.planConstraints;
@@ -1000,7 +1010,11 @@ mxconv_plan makePlanWith(const ConvParams &params,
       // 117 us, 8 groups of 32 -> 32 78 against 49, 2 groups of 64 -> 64 26
       // against 26.5, 4 groups of 64 -> 64 41 against 34 and 2 such groups on
       // 56 x 56 70 against 52; without groups 16 -> 16 on 56 x 56 ties at
-      // 39 us and 32 -> 64 wins with 18 against 25).
+      // 39 us and 32 -> 64 wins with 18 against 25).  What is refused here goes
+      // to wuWindowKernel where that takes it, without a comparison: of 12 640
+      // random half layers of that kind (2 to 64 groups, or fewer than 16
+      // channels on a side) the plan took 0.31 of the convolution's time, and
+      // 0.86 at most.
       const std::size_t tileArea = std::size_t((f.ci + 127) / 128 * 128) *
                                    ((f.co + 127) / 128 * 128);
       const bool filled =
