@@ -39,6 +39,7 @@
 #include "igemm_common.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace mxk {
@@ -447,14 +448,11 @@ bool wuTapTakes(const WuTapDesc &d) {
 
 uint32_t wuTapChunkPixels(const WuTapDesc &d, uint32_t computeUnits) {
   // One workgroup to a CU at a time: as many chunks of whole super-steps of 64
-  // pixels as make the rounds of workgroups shortest, each with its start-up
-  // and the tile's way out (4 us), a super-step 0.7 us, and the partial tiles
-  // written and read at 5 TB/s.  A layer whose tiles do not go into the CUs
-  // evenly takes several rounds of short chunks (N = 32, 14 x 14, 3 x 3, 512
-  // -> 512, 144 tiles: one chunk 67 us with the sum, three 58).
+  // pixels as the estimate finds the fastest, which are about one workgroup for
+  // every CU or some whole rounds of them (N = 32, 14 x 14, 3 x 3, 512 -> 512, 144
+  // tiles: one chunk 67 us with the sum, three 58).
   const uint64_t M = uint64_t(d.batch) * d.outH * d.outW;
   const uint64_t tiles = std::max<uint64_t>(1, tilesOf(d));
-  const double tileUs = 2 * 65536.0 / 5e6;
   uint64_t best = 0;
   double bestUs = 0;
   for (uint64_t n = 1; n <= 8 || n * tiles <= computeUnits; ++n) {
@@ -464,15 +462,15 @@ uint32_t wuTapChunkPixels(const WuTapDesc &d, uint32_t computeUnits) {
     // (no more than the workspace may hold: wuTapTakes)
     if (best && chunks * tiles * 65536 > (1ull << 31))
       break;
-    const uint64_t rounds = (chunks * tiles + computeUnits - 1) / computeUnits;
-    const double us = double(rounds) * (4.0 + 0.7 * double(pixels / 64)) +
-                      double(chunks * tiles) * tileUs;
+    WuTapDesc t = d;
+    t.chunkPixels = uint32_t(std::min<uint64_t>(pixels, 1u << 30));
+    const double us = wuTapEstimateUs(t, computeUnits);
     if (!best || us < bestUs)
-      best = pixels, bestUs = us;
+      best = t.chunkPixels, bestUs = us;
     if (pixels == 256)
       break;
   }
-  return uint32_t(std::min<uint64_t>(best, 1u << 30));
+  return uint32_t(best);
 }
 
 uint64_t wuTapWorkspaceBytes(const WuTapDesc &d) {
@@ -484,21 +482,25 @@ uint64_t wuTapWorkspaceBytes(const WuTapDesc &d) {
 }
 
 double wuTapEstimateUs(const WuTapDesc &d, uint32_t computeUnits) {
-  // Fitted to 4 500 random layers with the chunks chosen above, within 6 %.
+  // Fitted to 3 070 measurements on 379 random layers (4 to 64 images of 7 to 64
+  // squared, 24 to 512 channels, 1 x 1 to 5 x 5, up to ten counts of chunks each),
+  // within 5 %; the count picked by it is on average 1 % behind the best.
   const uint64_t M = uint64_t(d.batch) * d.outH * d.outW;
   const double steps =
       double((std::min<uint64_t>(d.chunkPixels, M) + 63) / 64);
   const double chunks = double((M + d.chunkPixels - 1) / d.chunkPixels);
-  const double rounds =
-      std::max(1.0, chunks * double(tilesOf(d)) / computeUnits);
+  const double perCU = chunks * double(tilesOf(d)) / double(computeUnits);
+  const double rounds = std::max(1.0, std::ceil(perCU));
   const double deltasMB =
       double(d.groups) * d.ci * d.co * d.kH * d.kW * 1e-6;
   const double partialMB = 4.0 * deltasMB * chunks;
-  return 6.8 + 0.56 * steps + (rounds - 1) * (4.0 + 0.75 * steps) +
-         0.48 * std::min(partialMB, 8.0) +
-         0.35 * std::min(std::max(partialMB - 8.0, 0.0), 9.0) +
-         1.5 * std::max(partialMB - 17.0, 0.0) + 2.0 * deltasMB +
-         0.011 * std::min(chunks, 32.0);
+  // (pixels of whole 128-byte lines on both sides come, and go, faster)
+  const bool lines = d.ci % 64 == 0 && d.co % 64 == 0;
+  return 7.3 + (0.418 + 0.045 * std::min(perCU, 1.0) - (lines ? 0.026 : 0.0)) *
+                   steps +
+         (rounds - 1) * (3.5 + 0.4 * steps) +
+         (lines ? 0.48 : 0.51) * std::min(partialMB, 14.4) +
+         0.23 * std::max(partialMB - 14.4, 0.0) + 1.33 * deltasMB;
 }
 
 hipError_t launchWuTap(const WuTapDesc &d, int outType, const void *acts,
