@@ -394,9 +394,9 @@ template <int BN, class OutT> constexpr int epilogueLdsBytes() {
   return kBlockM * (BN * int(sizeof(OutT)) + 16);
 }
 
-/// LDS of a workgroup: the stages and the row table - or the output tile, if
-/// that is larger (two stages and fp32 outputs).
-template <int BN, int NS, class OutT> constexpr int igemmLdsBytes() {
+/// Where the tile's bias lies in LDS, as fp32: behind the stages and the row
+/// table - or the output tile, if that is larger (two stages and fp32 outputs).
+template <int BN, int NS, class OutT> constexpr int igemmBiasByte() {
   constexpr int loop =
       NS * (kBlockM + BN) * kRowBytes +
       kBlockM * int(sizeof(uint2) + sizeof(uint32_t));
@@ -404,14 +404,19 @@ template <int BN, int NS, class OutT> constexpr int igemmLdsBytes() {
                                              : epilogueLdsBytes<BN, OutT>();
 }
 
+/// LDS of a workgroup.
+template <int BN, int NS, class OutT> constexpr int igemmLdsBytes() {
+  return igemmBiasByte<BN, NS, OutT>() + BN * int(sizeof(float));
+}
+
 /// Writes the workgroup's finished 128 x BN tile.  Call with every wave past
 /// its last use of LDS (a workgroup barrier behind it): LDS is reused from
-/// offset 0.
+/// offset 0.  biasLds: the tile's bias as fp32 (zeros without one).
 template <int BN, class OutT>
 __device__ __forceinline__ void
 igemmEpilogue(char *lds, const IgemmArgs &a, floatx16 (&acc)[2][BN / 64],
               bool producer, int t, int lane, int wm, int wn, uint32_t mTile,
-              uint32_t nTile, uint32_t g, const OutT *__restrict__ bias,
+              uint32_t nTile, uint32_t g, const float *biasLds,
               OutT *__restrict__ out, float scale) {
   constexpr int TN = BN / 64;
   const IgemmDesc &d = a.d;
@@ -431,14 +436,7 @@ igemmEpilogue(char *lds, const IgemmArgs &a, floatx16 (&acc)[2][BN / 64],
 #pragma unroll
       for (int q = 0; q != 4; ++q) {
         const uint32_t nLocal = wn * (BN / 2) + j * 32 + 8 * q + nOff4;
-        float bv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (bias) {
-          const uint32_t n = nTile * BN + nLocal;
-#pragma unroll
-          for (int e = 0; e != 4; ++e)
-            if (n + e < d.outChansPerGroup)
-              bv[e] = Load<OutT>::at(bias, g * d.outChansPerGroup + n + e, 0);
-        }
+        const floatx4 bv = *reinterpret_cast<const floatx4 *>(biasLds + nLocal);
 #pragma unroll
         for (int i = 0; i != 2; ++i) {
           const uint32_t mLocal = wm * 64 + i * 32 + mRow;
