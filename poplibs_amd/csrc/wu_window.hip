@@ -37,6 +37,13 @@
 // 52 -> 15; 72 -> 72, 1 x 1, 21 x 9 x 9 8.9 -> 6.3; 256 -> 64, 1 x 1, 32 x 56 x 56
 // 20 -> 17; over 3 500 random layers it halves the pass (geometric mean).
 //
+// Eight waves: their sums pass through LDS twice, 192 KB for a tile of 32 x 32 and
+// three taps, which with sixteen was 1.5 us of a small layer's pass (7 x 15 x 15,
+// 3 x 3 stride 2, 208 -> 64 9.7 -> 6.5 us; 21 x 39 x 39 stride 2, 32 groups of 16
+// 22.4 -> 18.7; 8 x 54 x 54, 32 -> 64 13.2 -> 11.3; tiles and chunks fitted anew).
+// Four are faster only where the tile is 32 x 32 and the chunk short (0.3 % over
+// 330 layers), a quarter slower on long ones.
+//
 // With one chunk the deltas leave in weight order, one launch in all; with
 // several, fp32 sums go to the workspace as [chunk][tap][g][co][ci] and
 // wuWindowSumKernel adds them in order.
@@ -621,41 +628,41 @@ namespace {
 /// The pass's time by tile, kernel columns and stride along a row: `call`, a
 /// workgroup's k-steps at the pace of a wave (`wave` each of its own) or of the
 /// CU (`step`), `round` + `roundStep` per k-step for what does not go side by
-/// side on 256 CUs, and the second launch with its partial sums or the one
-/// launch's scattered results.  Fitted to 45 000 measurements on 5 900 random
-/// layers (1 to 64 images, fields of 5 to 64, 4 to 512 channels, up to 32
-/// groups), within 7 to 10 %; the tile and chunks picked by it are on average
-/// 3 % behind the best of those measured.
+/// side on 256 CUs that take `places` workgroups each, and the second launch with
+/// its partial sums or the one launch's scattered results.  Fitted to 7 000
+/// measurements on 330 layers (4 to 64 images, fields of 7 to 64, 4 to 512
+/// channels, up to 32 groups), within 5 to 9 %; the tile and chunks picked by it
+/// are on average 1.8 % behind the best of those measured.
 struct WinFit {
-  double call, wave, step, round, roundStep, second, partialMB, resultMB;
+  double call, wave, step, round, roundStep, second, partialMB, resultMB, places;
 };
 constexpr WinFit kWinFits[3][2][2] = {
     // 32 x 32: one column, three; stride 1, 2
-    {{{3.53, 0.041, 0.063, 1.3, 0.142, 2.7, 0.56, 4.6},
-      {3.67, 0.006, 0.059, 1.2, 0.160, 2.5, 0.53, 2.3}},
-     {{6.20, 0.027, 0.076, 4.9, 0.097, 2.8, 0.43, 1.5},
-      {6.43, 0.080, 0.120, 4.7, 0.192, 2.9, 0.55, 1.9}}},
+    {{{3.00, 0.505, 0.080, 0.6, 0.090, 2.8, 0.66, 3.05, 1},
+      {3.69, 0.372, 0.066, 1.0, 0.078, 2.5, 0.44, 1.45, 3}},
+     {{5.29, 0.025, 0.088, 2.0, 0.071, 3.0, 0.40, 2.00, 1},
+      {5.64, 0.593, 0.102, 3.4, 0.133, 2.8, 0.34, 1.29, 1}}},
     // 64 output x 32 input channels
-    {{{3.54, 0.029, 0.092, 0.8, 0.159, 2.7, 0.53, 4.1},
-      {3.61, 0.011, 0.087, 0.6, 0.189, 2.5, 0.50, 1.7}},
-     {{5.85, 0.079, 0.109, 5.0, 0.114, 2.9, 0.46, 2.5},
-      {6.27, 0.113, 0.129, 4.7, 0.148, 2.7, 0.48, 2.3}}},
+    {{{3.51, 0.055, 0.105, 0.9, 0.125, 2.9, 0.55, 2.25, 1},
+      {4.22, 0.153, 0.091, 1.1, 0.135, 2.4, 0.52, 0.58, 3}},
+     {{6.48, 0.213, 0.110, 4.8, 0.107, 2.9, 0.47, 2.37, 1},
+      {7.10, 0.233, 0.128, 4.8, 0.147, 2.5, 0.46, 2.28, 1}}},
     // 32 x 64
-    {{{3.51, 0.055, 0.084, 0.8, 0.156, 2.7, 0.51, 4.0},
-      {3.58, 0.025, 0.081, 0.8, 0.170, 2.5, 0.48, 1.7}},
-     {{6.11, 0.030, 0.109, 5.0, 0.122, 2.8, 0.44, 2.4},
-      {6.59, 0.049, 0.153, 4.8, 0.191, 2.6, 0.46, 2.2}}}};
+    {{{3.46, 0.143, 0.099, 0.9, 0.122, 2.9, 0.55, 0.60, 1},
+      {4.12, 0.170, 0.085, 1.1, 0.143, 2.5, 0.49, 0.54, 3}},
+     {{6.96, 0.099, 0.113, 5.0, 0.115, 2.8, 0.43, 2.12, 1},
+      {7.76, 0.011, 0.154, 5.2, 0.174, 2.3, 0.44, 1.97, 1}}}};
 
 /// fp32: tiles of 16, 32 and 48; one column, three (both strides).  Fitted to
 /// 6 200 measurements on 340 layers, within 8 to 10 %; the pick 2 % behind the
 /// best on average.
 constexpr WinFit kWinFloatFits[3][2] = {
-    {{4.63, 0.041, 0.077, 1.3, 0.113, 2.0, 3.15, 1.17},
-     {6.85, 0.011, 0.151, 4.2, 0.149, 2.5, 0.41, 0.78}},
-    {{4.99, 0.051, 0.178, 1.8, 0.186, 2.4, 0.85, 0.76},
-     {8.16, 0.018, 0.435, 6.5, 0.423, 3.3, 0.36, 1.48}},
-    {{5.72, 1.372, 0.311, 3.0, 0.340, 2.4, 0.54, 0.0},
-     {9.59, 3.941, 0.930, 10.5, 0.908, 4.1, 0.35, 1.29}}};
+    {{4.63, 0.041, 0.077, 1.3, 0.113, 2.0, 3.15, 1.17, 2},
+     {6.85, 0.011, 0.151, 4.2, 0.149, 2.5, 0.41, 0.78, 1}},
+    {{4.99, 0.051, 0.178, 1.8, 0.186, 2.4, 0.85, 0.76, 2},
+     {8.16, 0.018, 0.435, 6.5, 0.423, 3.3, 0.36, 1.48, 1}},
+    {{5.72, 1.372, 0.311, 3.0, 0.340, 2.4, 0.54, 0.0, 2},
+     {9.59, 3.941, 0.930, 10.5, 0.908, 4.1, 0.35, 1.29, 1}}};
 
 uint32_t floatWaves(uint32_t tile) {
   return tile == 16 ? 16 : tile == 32 ? 8 : 4;
@@ -670,15 +677,11 @@ double winEstimateUs(const WuTapDesc &d, const WinShape &s,
                                          : 0;
   const WinFit &f = floats ? kWinFloatFits[tile][d.kW == 1 ? 0 : 1]
                            : kWinFits[tile][d.kW == 1 ? 0 : 1][d.strideW - 1];
-  const uint32_t waves =
-      floats ? floatWaves(d.windowCo) : tile == 0 ? 16 : 8;
+  const uint32_t waves = floats ? floatWaves(d.windowCo) : 8;
   const double steps = d.windowSteps;
-  // (a workgroup to a CU; two of eight waves, or of fp32, where a kernel row is
-  // one column)
-  const double shared = (floats || tile != 0) && d.kW == 1 ? 2.0 : 1.0;
   const double perCU = std::max(
-      1.0, std::ceil(shared * double(s.chunks * s.tiles) / computeUnits) /
-               shared);
+      1.0, std::ceil(f.places * double(s.chunks * s.tiles) / computeUnits) /
+               f.places);
   const double mb = double(s.elems) * 1e-6;
   return f.call + std::max(f.wave * std::ceil(steps / waves), f.step * steps) +
          (perCU - 1) * (f.round + f.roundStep * steps) +
@@ -729,11 +732,11 @@ double wuWindowChoose(WuTapDesc &d, uint32_t computeUnits) {
 }
 
 namespace {
-template <int JO, int JI, int KW, int S, int NW>
+template <int JO, int JI, int KW, int S>
 hipError_t launchWindow(const WuWindowArgs &a, uint32_t blocks, int outType,
                         const void *acts, const void *deltas, void *out,
                         hipStream_t stream) {
-  constexpr int kLds = NW * JO * JI * 1024;
+  constexpr int NW = 8, kLds = NW * JO * JI * 1024;
   static_assert(kLds <= 64 * 1024, "within the LDS of any launch");
   const dim3 grid(blocks), block(64 * NW);
   const char *x = static_cast<const char *>(acts);
@@ -779,21 +782,15 @@ hipError_t launchWindowFloats(const WuWindowArgs &a, uint32_t blocks,
   return go(a, blocks, outType, acts, deltas, out, stream);
 }
 
-template <int JO, int JI, int NW>
+template <int JO, int JI>
 hipError_t launchWindowTaps(const WuWindowArgs &a, uint32_t blocks,
                             int outType, const void *acts, const void *deltas,
                             void *out, hipStream_t stream) {
-  if (a.d.kW == 1)
-    return a.d.strideW == 1
-               ? launchWindow<JO, JI, 1, 1, NW>(a, blocks, outType, acts,
-                                                deltas, out, stream)
-               : launchWindow<JO, JI, 1, 2, NW>(a, blocks, outType, acts,
-                                                deltas, out, stream);
-  return a.d.strideW == 1
-             ? launchWindow<JO, JI, 3, 1, NW>(a, blocks, outType, acts, deltas,
-                                              out, stream)
-             : launchWindow<JO, JI, 3, 2, NW>(a, blocks, outType, acts, deltas,
-                                              out, stream);
+  const auto go = a.d.kW == 1 ? a.d.strideW == 1 ? &launchWindow<JO, JI, 1, 1>
+                                                 : &launchWindow<JO, JI, 1, 2>
+                  : a.d.strideW == 1 ? &launchWindow<JO, JI, 3, 1>
+                                     : &launchWindow<JO, JI, 3, 2>;
+  return go(a, blocks, outType, acts, deltas, out, stream);
 }
 } // namespace
 
@@ -836,12 +833,11 @@ hipError_t launchWuWindow(const WuTapDesc &d, int outType, const void *acts,
             : launchWindowFloats<3>(a, blocks, toType, acts, deltas, to,
                                     stream);
   else if (d.windowCo == 64)
-    e = launchWindowTaps<4, 2, 8>(a, blocks, toType, acts, deltas, to, stream);
+    e = launchWindowTaps<4, 2>(a, blocks, toType, acts, deltas, to, stream);
   else if (d.windowCi == 64)
-    e = launchWindowTaps<2, 4, 8>(a, blocks, toType, acts, deltas, to, stream);
+    e = launchWindowTaps<2, 4>(a, blocks, toType, acts, deltas, to, stream);
   else
-    e = launchWindowTaps<2, 2, 16>(a, blocks, toType, acts, deltas, to,
-                                   stream);
+    e = launchWindowTaps<2, 2>(a, blocks, toType, acts, deltas, to, stream);
   if (e != hipSuccess || direct)
     return e;
   const uint32_t F = uint32_t(s.elems / taps);

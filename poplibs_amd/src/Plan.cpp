@@ -638,12 +638,12 @@ bool floatWindowAsked(const PlanConstraints &pc) {
 /// The weight deltas of `layer` (channels of a group as the layer has them, in
 /// resultCi and resultCo) by wuWindowKernel, where that is named or estimated
 /// to be faster than what `plan` has; `fuse`: groups that plan takes as one.
-/// The line at 0.93: of 320 random layers that both kernels take (4 to 64 images
-/// of 7 to 64 squared, 24 to 512 channels, 1 x 1 and 3 x 3, up to 40 GFLOP) the
-/// choice is on average 0.6 % slower than the faster of the two, 0.6 % in total
-/// time; at 0.85 1.2 and 1.1 %, at 0.9 0.8 and 0.8, at 0.96 0.5 and 0.6, at 1 1.0
-/// and 1.0, at 1.04 1.7 and 1.8 (wuTapKernel for all 9.2 %, this one for all 6.8
-/// %).
+/// Both estimates as they are: of 187 random layers that both kernels take (4 to
+/// 64 images of 7 to 64 squared, 24 to 512 channels, 1 x 1 and 3 x 3, up to 40
+/// GFLOP) the choice is on average 0.4 % slower than the faster of the two, 0.6 %
+/// in total time; this one's times 1.08 1.3 and 1.5 %, 1.04 0.7 and 0.8, 0.96 0.8
+/// and 1.4, 0.93 1.2 and 2.1 (over 300 layers wuTapKernel for all 55 %, this one
+/// for all 1.8 %).
 void windowWeightDeltas(mxconv_plan &plan, const mxk::WuTapDesc &layer,
                         unsigned fuse) {
   const auto &pc = plan.options.planConstraints;
@@ -686,7 +686,7 @@ void windowWeightDeltas(mxconv_plan &plan, const mxk::WuTapDesc &layer,
     // (the diagonal blocks of groups taken as one are a launch of their own)
     if (fuse > 1)
       otherUs += 2.2;
-    if (us >= 0.93 * otherUs)
+    if (us >= otherUs)
       return;
   }
   plan.denseWeightUpdate = true;
