@@ -292,32 +292,50 @@ uint32_t depthwiseColumnDeltasSlices(const DepthwiseDesc &d) {
   return h.bands * h.chunks;
 }
 
-// The pass (both kernels), fitted to 3000 timings of 150 random layers (the
-// choice by it is within 2 % of the best on average); as
-// depthwiseColumnsEstimateUs.
+// The pass (both kernels), by taps and stride fitted to 5 400 timings of 420 random
+// layers over several sets of buffers (4 to 64 images of 7 to 112 squared, 32 to
+// 960 channels), within 5 to 7 % (3 x 3 at stride 2 10 %); the choice by it is 0.8
+// to 1.5 % behind the best on average.  A walk's instructions, as in
+// depthwiseColumnsEstimateUs, by the workgroups that a CU holds (by strips of two
+// and four) and their start (`start` walks), against the bytes; then the slices'
+// sum and the slots' meeting.
 double depthwiseColumnDeltasEstimateUs(const DepthwiseDesc &d) {
+  struct Fit {
+    double product, row, perRow, taps, start, call, rate, partial, slice, slot;
+    int resident[2];
+  };
+  constexpr Fit fits[3][2] = {
+      {{0.0, 4.96, 20.5, 0.0126, 2.12, 5.60, 5.94e6, 1.08e-6, 0.0037, 0.106, {8, 7}},
+       {0.0, 6.03, 22.2, 0.0007, 1.48, 5.83, 6.60e6, 1.21e-6, 0.0037, 0.075, {8, 6}}},
+      {{1.54, 5.12, 19.6, 0.0, 1.19, 7.89, 5.14e6, 0.86e-6, 0.0035, 0.012, {4, 4}},
+       {0.10, 5.84, 19.9, 0.0, 1.40, 7.16, 5.34e6, 1.12e-6, 0.0023, 0.001, {4, 4}}},
+      {{2.51, 5.14, 19.6, 0.0, 0.65, 10.18, 4.14e6, 0.73e-6, 0.0047, 0.0, {3, 2}},
+       {0.0, 6.10, 19.9, 0.0057, 1.44, 8.08, 3.82e6, 0.66e-6, 0.0028, 0.0, {3, 2}}}};
   const ColumnDeltasShape h = shapeOf(d);
   const uint32_t k = d.kH, s = d.strideH, strip = d.columns;
+  const Fit &f = fits[k / 2 - 1][s - 1];
   const double rowsIn = (h.bandRows - 1.0) * s + k;
   const double columnsIn = s * (strip - 1) + k;
   const double perRow = double(h.bandRows) * strip;
   const double waveUs =
       h.rounds *
-          (1.79 * perRow * k * k +
-           6.98 * (rowsIn * (3 * columnsIn + 20) + 3 * perRow)) *
+          (f.product * perRow * k * k +
+           f.row * (rowsIn * (3 * columnsIn + f.perRow) + 3 * perRow)) *
           1e-3 / 2.4 +
-      0.0238 * k * k;
-  const double resident = k == 3 ? (strip == 2 ? 8 : 6) : k == 5 ? 4 : 2;
+      f.taps * k * k;
+  const double resident = f.resident[strip / 2 - 1];
   const double slices = double(h.bands) * h.chunks;
   const double perCu = slices * h.blocksC / 256;
   const double full = std::floor(perCu / resident);
   const double rest = std::ceil(perCu - full * resident);
-  const double us = full * (resident + 0.78) * waveUs +
-                    (rest > 0 ? (rest + 0.78) * waveUs : 0.0);
+  const double us = full * (resident + f.start) * waveUs +
+                    (rest > 0 ? (rest + f.start) * waveUs : 0.0);
   const double bytes = 2.0 * d.batch * d.channels *
                        (double(d.inH) * d.inW + double(d.outH) * d.outW);
-  return 7.7 + std::sqrt(std::hypot(us * us, std::pow(bytes / 4.3e6, 2))) +
-         0.44e-6 * slices * k * k * d.channels * 4;
+  return f.call +
+         std::sqrt(std::hypot(us * us, std::pow(bytes / f.rate, 2))) +
+         f.partial * slices * k * k * d.channels * 4 + f.slice * slices +
+         f.slot * h.slots;
 }
 
 void chooseDepthwiseColumnDeltas(DepthwiseDesc &d, uint32_t strip) {

@@ -472,6 +472,8 @@ hipError_t launchDepthwiseRows(const DepthwiseDesc &d, int inType, int outType,
 bool depthwiseRowsDeltaTakes(const DepthwiseDesc &d);
 DepthwiseRowsLaunch depthwiseRowsDeltaLaunchShape(const DepthwiseDesc &d);
 size_t depthwiseRowsDeltaWorkspaceBytes(const DepthwiseDesc &d);
+/// Estimated microseconds of the pass, both launches.
+double depthwiseRowsDeltaEstimateUs(const DepthwiseDesc &d);
 hipError_t launchDepthwiseRowsDeltas(const DepthwiseDesc &d, const void *acts,
                                      const void *deltas, void *partial,
                                      uint32_t *walkers, hipStream_t stream);

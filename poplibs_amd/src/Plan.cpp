@@ -929,7 +929,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
       f.dilH = w.strideH, f.dilW = w.strideW;
       f.loH = w.loH, f.hiH = w.hiH, f.loW = w.loW, f.hiW = w.hiW;
       // 3x3 layers that give every CU a band of rows: the persistent kernel
-      // with the rows of both tensors in LDS rings (as for the forward pass)
+      // with the rows of both tensors in LDS rings (as for the forward pass),
+      // where strips of columns are not estimated to be faster
       f.cus = gfx950::numCUs;
       const mxk::DepthwiseRowsLaunch l =
           mxk::depthwiseRowsDeltaLaunchShape(f);
@@ -942,13 +943,19 @@ mxconv_plan makePlanWith(const ConvParams &params,
            (l.workgroups * 2 >= gfx950::numCUs && l.rowsOut >= 4 &&
             (l.colsOut >= 4 || l.strips == 1))))
         f.dense3x3 = 2;
-      // Strips of columns for the others from some amount of work on: below,
-      // the kernel's longer program and the meeting of its sums cost 1 to 4 us
-      // more than they save (of 150 random layers, each above its line 1.02 to
-      // 5.5 times as fast, the ones below 0.6 to 1.2).
+      // Strips of columns for the others from some amount of work on, for 3 x 3
+      // taps more of it where channels are few and many slots' sums meet: below,
+      // the kernel's longer program and the meeting cost up to 1.5 us more than
+      // they save.  Of 420 layers (4 to 64 images of 7 to 112 squared, 32 to 960
+      // channels) the choice is 0.8, 1.0 and 0.8 % behind the faster of the two
+      // for 3, 5 and 7 taps a side, with lines at 8e6, 20e6 and 43e6 products
+      // 3.2, 2.2 and 2.7 %.
       const double products =
           double(f.batch) * f.outH * f.outW * f.channels * f.kH * f.kW;
-      const double enough = f.kH == 3 ? 8e6 : f.kH == 5 ? 20e6 : 43e6;
+      const double enough =
+          f.kH == 3   ? 1e6 * std::max(1.0, 192.0 / f.channels)
+          : f.kH == 5 ? 8e6
+                      : 14e6;
       const int asked = options.planConstraints.columns;
       const bool takes = params.inputType == poplar::HALF &&
                          options.planConstraints.rowRing != 1 &&
@@ -958,10 +965,24 @@ mxconv_plan makePlanWith(const ConvParams &params,
             "planConstraints gfx950 columns: the weight deltas' kernel takes "
             "half tensors, 3x3, 5x5 or 7x7 taps at stride 1 or 2, without "
             "rowRing 1");
-      if (takes && (asked > 0 || (asked != 0 && f.dense3x3 != 2 &&
-                                  products >= enough))) {
-        f.dense3x3 = 0;
-        mxk::chooseDepthwiseColumnDeltas(f, asked > 0 ? uint32_t(asked) : 0);
+      if (takes && (asked > 0 || (asked != 0 && products >= enough))) {
+        // The rings win where a few channels make long strips and the tensors
+        // come from HBM (32 x 112 x 112 stride 2, 96 channels 24.2 us against
+        // 28.1; 32 x 56 x 56, 144 19.1 against 19.8): every workgroup leaves a
+        // tile of all channels, whose sums their columns meet for in LDS (9 x 17
+        // x 17, 856 channels 19.8 us, 10.4 in strips; 32 x 14 x 14, 504 16.8 and
+        // 10.0; 11 x 56 x 56, 320 18.4 and 14.4).  Of 80 layers that the rings
+        // take the choice is 1.0 % behind the best.
+        const double ringUs = f.dense3x3 == 2
+                                  ? mxk::depthwiseRowsDeltaEstimateUs(f)
+                                  : 0.0;
+        mxk::DepthwiseDesc c = f;
+        mxk::chooseDepthwiseColumnDeltas(c, asked > 0 ? uint32_t(asked) : 0);
+        if (asked > 0 || f.dense3x3 != 2 ||
+            mxk::depthwiseColumnDeltasEstimateUs(c) <= ringUs) {
+          f = c;
+          f.dense3x3 = 0;
+        }
       }
     }
   }

@@ -683,6 +683,23 @@ def test_depthwise_weight_update_row_rings_plan_choice():
     assert RING_WU not in pa.WeightUpdatePlan(five, ROW_RING).describe()
 
 
+@pytest.mark.parametrize("kw,ring", [
+    # rings where a few channels make long strips, strips of columns where a
+    # workgroup's tile of all channels costs more than its walk, and the
+    # slices' walk for little work
+    (dict(batch=64, field=(112, 112), kernel=(3, 3), groups=64, stride=2,
+          pad=1), True),
+    (dict(batch=32, field=(112, 112), kernel=(3, 3), groups=32, pad=1), True),
+    (dict(batch=32, field=(14, 14), kernel=(3, 3), groups=504, pad=1), False),
+    (dict(batch=11, field=(56, 56), kernel=(3, 3), groups=320, pad=1), False),
+    (dict(batch=9, field=(17, 17), kernel=(3, 3), groups=856, pad=1), False),
+    (dict(batch=4, field=(8, 8), kernel=(3, 3), groups=32, pad=1), None)])
+def test_depthwise_weight_deltas_by_rings_or_columns(kw, ring):
+    text = pa.WeightUpdatePlan(make_params(pa.HALF, **kw)).describe()
+    assert (RING_WU in text) == (ring is True), text
+    assert ("columns walked down in registers" in text) == (ring is False), text
+
+
 @pytest.mark.gpu
 def test_weight_update_applies_scaled_deltas(oracle):
     from gpu_helpers import quantize
