@@ -453,7 +453,8 @@ __global__ __launch_bounds__(256) void channelSumKernel(
     uint32_t r = rowLane; // within the split
     const T *at = z + (first + r) * channels + c;
     const uint64_t step = uint64_t(rowLanes) * channels;
-    // (whole groups first; what is left of the rows one at a time)
+    // (whole groups first; then what is left of the rows, at once, those beyond
+    // the last the last again and not added)
     for (; r + (kReduceUnroll - 1) * rowLanes < last;
          r += kReduceUnroll * rowLanes) {
       Vec v[kReduceUnroll];
@@ -466,11 +467,19 @@ __global__ __launch_bounds__(256) void channelSumKernel(
         for (int e = 0; e != VEC; ++e)
           sum[e] += Load<T>::at(v[u].e, e, 0);
     }
-    for (; r < last; r += rowLanes, at += step) {
-      const Vec v = *reinterpret_cast<const Vec *>(at);
+    if (r < last) {
+      Vec v[kReduceUnroll];
 #pragma unroll
-      for (int e = 0; e != VEC; ++e)
-        sum[e] += Load<T>::at(v.e, e, 0);
+      for (uint32_t u = 0; u != kReduceUnroll; ++u) {
+        v[u] = *reinterpret_cast<const Vec *>(at);
+        at += r + (u + 1) * rowLanes < last ? step : 0;
+      }
+#pragma unroll
+      for (uint32_t u = 0; u != kReduceUnroll; ++u)
+        if (r + u * rowLanes < last)
+#pragma unroll
+          for (int e = 0; e != VEC; ++e)
+            sum[e] += Load<T>::at(v[u].e, e, 0);
     }
   }
 #pragma unroll
@@ -484,6 +493,7 @@ __global__ __launch_bounds__(256) void channelSumKernel(
     if (ch >= channels)
       break;
     float total = lanes[i];
+#pragma unroll 8
     for (uint32_t l = 1; l != rowLanes; ++l)
       total += lanes[l * own + i];
     partial[uint64_t(blockIdx.y) * channels + ch] = total;
