@@ -331,23 +331,32 @@ wideTile(const IgemmArgs &a, const char *__restrict__ in,
         }
     }
     __syncthreads();
-    for (int idx = t; idx < 128 * kVecsPerRow; idx += kThreads) {
-      const uint32_t mLocal = idx / kVecsPerRow, vec = idx % kVecsPerRow;
-      const uint32_t m = mTile * kWideM + pass * 128 + mLocal;
-      const uint32_t n = nTile * BN + vec * kVecElems;
-      if (m >= a.M || n >= d.outChansPerGroup)
-        continue;
-      const char *src = lds + mLocal * kOutRow + vec * 16;
-      OutT *dst = out + outPixel(a, m) * outChans + g * d.outChansPerGroup + n;
-      if (n + kVecElems <= d.outChansPerGroup) {
-        const uintx4 whole = *reinterpret_cast<const uintx4 *>(src);
-        *reinterpret_cast<AnyWords *>(dst) = whole;
-      } else {
-        const OutT *e = reinterpret_cast<const OutT *>(src);
-        for (int k = 0; k != kVecElems && n + k < d.outChansPerGroup; ++k)
-          dst[k] = e[k];
+    auto copyOut = [&](auto through) {
+      for (int idx = t; idx < 128 * kVecsPerRow; idx += kThreads) {
+        const uint32_t mLocal = idx / kVecsPerRow, vec = idx % kVecsPerRow;
+        const uint32_t m = mTile * kWideM + pass * 128 + mLocal;
+        const uint32_t n = nTile * BN + vec * kVecElems;
+        if (m >= a.M || n >= d.outChansPerGroup)
+          continue;
+        const char *src = lds + mLocal * kOutRow + vec * 16;
+        OutT *dst =
+            out + outPixel(a, m) * outChans + g * d.outChansPerGroup + n;
+        if constexpr (decltype(through)::value) {
+          storeThrough(dst, *reinterpret_cast<const uintx4 *>(src));
+        } else if (n + kVecElems <= d.outChansPerGroup) {
+          const uintx4 whole = *reinterpret_cast<const uintx4 *>(src);
+          *reinterpret_cast<AnyWords *>(dst) = whole;
+        } else {
+          const OutT *e = reinterpret_cast<const OutT *>(src);
+          for (int k = 0; k != kVecElems && n + k < d.outChansPerGroup; ++k)
+            dst[k] = e[k];
+        }
       }
-    }
+    };
+    if (a.outThrough)
+      copyOut(std::true_type{});
+    else
+      copyOut(std::false_type{});
   }
 }
 

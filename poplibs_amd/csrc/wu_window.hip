@@ -151,7 +151,7 @@ storeWindow(const WuWindowArgs &a, const WinPlace &w,
             (size_t(w.g0) * a.resultCo + coIn) * a.resultCi + ciIn;
         if (a.strideF == 1 && a.resultCi % 4 == 0) {
           const float v[4] = {total[0], total[1], total[2], total[3]};
-          storeOut4(to + f, v);
+          storeOut4Through(to + f, v);
         } else {
 #pragma unroll
           for (uint32_t x = 0; x != 4; ++x)
