@@ -62,13 +62,16 @@ struct Dw3x3Args {
 };
 
 template <class OutT> struct StoreVec;
+// (Through the L2: its layers are small, and the L2s have nothing to write back
+// when the kernel ends; 16 x 76 x 76 stride 2, 40 channels 4.7 -> 3.7 us
+// non-temporal before.)
 template <> struct StoreVec<__half> {
   static __device__ __forceinline__ void put(__half *p, const float (&v)[8]) {
     Vec8 o;
 #pragma unroll
     for (int i = 0; i != 4; ++i)
       o.h2[i] = roundPairToHalf(v[2 * i], v[2 * i + 1]);
-    __builtin_nontemporal_store(o.raw, reinterpret_cast<uintx4 *>(p));
+    storeThrough(p, o.raw);
   }
 };
 template <> struct StoreVec<float> {

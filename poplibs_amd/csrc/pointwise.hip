@@ -69,6 +69,7 @@ struct PwArgs {
   // fp8: 2^(scaleIn + scaleWeights), applied to the sums on their way out,
   // and its inverse, by which the bias enters them
   float scale, invScale;
+  uint32_t through; // outputs are stored through the L2
 };
 
 /// One 32-byte k-slice of a 32 x 32 block: `w` and `x` are a lane's 16 bytes
@@ -341,11 +342,15 @@ __global__ __launch_bounds__(TM * 4 + 64 * LW) void pointwiseKernel(
                 nTile * NT * kPwChans + (nb * NT + 2 * np) * 32 + vec * 8;
             const uintx4 data = *reinterpret_cast<const uintx4 *>(
                 stage + r * kPwPairRow + vec * 16);
-            if (m < a.M && n < d.outChansPerGroup)
-              __builtin_nontemporal_store(
-                  data, reinterpret_cast<uintx4 *>(
-                            out + size_t(m) * outChans +
-                            g * d.outChansPerGroup + n));
+            if (m < a.M && n < d.outChansPerGroup) {
+              OutT *dst =
+                  out + size_t(m) * outChans + g * d.outChansPerGroup + n;
+              if (a.through)
+                storeThrough(dst, data);
+              else
+                __builtin_nontemporal_store(data,
+                                            reinterpret_cast<uintx4 *>(dst));
+            }
           }
           MXK_WAIT_LGKMCNT0(); // read before the next pixels overwrite it
         }
@@ -412,7 +417,10 @@ __global__ __launch_bounds__(TM * 4 + 64 * LW) void pointwiseKernel(
             // streaming store (the output is not read again here): 15.2 ->
             // 12.4 us on the 56 x 56, 256 -> 64 layer.  The same hint on the
             // loads loses a microsecond of that.
-            __builtin_nontemporal_store(data, dst);
+            if (a.through)
+              storeThrough(dst, data);
+            else
+              __builtin_nontemporal_store(data, dst);
           }
         }
         MXK_WAIT_LGKMCNT0(); // staging is read before the next pass rewrites it
@@ -673,6 +681,22 @@ hipError_t launchPointwise(const PointwiseDesc &d, int inType, int outType,
   PwArgs a;
   a.d = d;
   a.M = uint32_t(uint64_t(d.batch) * d.pixels);
+  // Rows that are no whole 64-byte pieces: through the L2 where the output is
+  // small (1.03 times as fast on average up to 6 MB), or larger than the L2s and
+  // most of what is moved - a piece stored non-temporal without its neighbours is
+  // a write of its own, 98 x 21 x 21, 32 -> 712 37.4 us, 16.2 through; fp8 32 x 33 x
+  // 33, 48 -> 720 25.5 and 14.1.  Where the loads are the larger part it is the
+  // other way round, 86 x 28 x 28, 480 -> 336 35.6 and 59.6, 64 x 56 x 56, 96 -> 496
+  // 51.7 and 87.6, and so it is with 9 MB, 32 x 28 x 28, 64 -> 184 6.6 and 7.4, or
+  // 250, 64 x 56 x 56, 40 -> 624 100 and 113.
+  const uint32_t inPixel = d.groups * d.inChansPerGroup * d.elemBytes;
+  const uint32_t outPixel =
+      d.groups * d.outChansPerGroup * (outType == kFloat ? 4 : 2);
+  const uint64_t outBytes = uint64_t(a.M) * outPixel;
+  a.through = outPixel % 64 != 0 &&
+              (outBytes <= 6000000 ||
+               (outBytes >= 12000000 && outBytes <= 150000000 &&
+                inPixel <= 128 && outPixel * 2 >= inPixel * 5));
   a.mTiles = 0; // set for the tile height of the kernel that runs
   a.nTiles = (d.outChansPerGroup + kPwChans - 1) / kPwChans;
   a.nBlocks = a.nTiles * 2;

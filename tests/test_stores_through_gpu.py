@@ -30,6 +30,10 @@ CASES = [
        dict(blockM=256, blockN=bn)) for co, bn in ((200, 192), (264, 256))],
     *[(dict(batch=1, field=(9, 8), kernel=(3, 3), ci=40, co=co, pad=1),
        dict(smallTile=2)) for co in (4, 36)],
+    # pointwise rows that are no whole 64-byte pieces: few bytes of them, and
+    # more than 12 MB (a pair of channel blocks to a store)
+    *[(dict(batch=b, field=(31, 33), kernel=(1, 1), ci=32, co=co),
+       dict(pointwise=1)) for b, co in ((2, 40), (40, 168))],
 ]
 
 
