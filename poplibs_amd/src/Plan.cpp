@@ -1634,8 +1634,20 @@ mxconv_plan makePlanWith(const ConvParams &params,
     // 256 -> 64: 8.4 against 11.0, 112 x 112, 32 -> 64: 14.6 against 24.1)
     const bool deepQuarter =
         quarterIn && ci >= 512 && pc.pointwise != 1;
+    // (A large output in rows of no whole 64-byte pieces, most of what is moved:
+    // its pieces are written one by one, whole rows of tiles at a time by the
+    // others.  Of 420 layers of such rows those of 150 MB and more took 1.04 to
+    // 2.4 times as long here, fp8 81 x 61 x 61, 112 -> 400 167 us, 93 in tiles of
+    // 128; smaller ones 0.6 to 1.5 times, 0.85 on average.)
+    const std::size_t inPixel = ci * p.numConvGroups * params.inputType.size();
+    const std::size_t outPixel = co * p.numConvGroups * params.outputType.size();
+    const bool largeOddRows =
+        outPixel % 64 != 0 && inPixel <= 256 && outPixel * 2 >= inPixel * 5 &&
+        std::size_t(pw.batch) * pw.pixels * outPixel > 150000000 &&
+        pc.pointwise != 1;
     plan.pointwiseOn =
         unitWindow && ciPadded == ci && !paddedSmall && !deepQuarter &&
+        !largeOddRows &&
         (pc.kernel != "igemm" || pc.pointwise == 1) && pc.pointwise != 0 &&
         pc.patch < 1 && !pc.blockM &&
         !pc.blockN && !pc.blockK &&

@@ -72,3 +72,16 @@ def test_a_short_sum_keeps_narrow_tiles(kw):
 def test_products_that_fill_the_chip_keep_it():
     plan = pa.MatMulPlan(H, H, 1, 4096, 4096, 4096)
     assert _tile(plan) == "256 x 256 x 64"
+
+
+@pytest.mark.parametrize("co,batch,pointwise", [
+    # 155 MB of output in rows of 1232 bytes, of whole 64-byte pieces, and less
+    (616, 40, False), (608, 40, True), (616, 32, True)])
+def test_large_outputs_in_odd_rows_leave_the_pointwise_kernel(co, batch,
+                                                              pointwise):
+    p = make_params(H, batch=batch, field=(56, 56), kernel=(1, 1), ci=40,
+                    co=co)
+    text = pa.Plan(p).describe()
+    assert ("pointwise streaming" in text) == pointwise, text
+    asked = {"planConstraints": '{"gfx950": {"pointwise": 1}}'}
+    assert "pointwise streaming" in pa.Plan(p, asked).describe()
