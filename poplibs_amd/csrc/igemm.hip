@@ -420,11 +420,13 @@ __device__ __forceinline__ void igemmTile(
   } else {
     // While the producers start the weight loads, the first 128 consumer
     // threads work out the row table, one tile row each.  The bias is asked for
-    // first, a channel each, and put into LDS behind the loop: its trip to memory
-    // runs under all of that.  (Read where it is added, channel by channel in
-    // front of the stores, it kept every tile waiting: with and without a bias
-    // 17.8 and 15.0 us for 25 x 57 x 57, 3 x 3 stride 2, 72 -> 200, 117.7 and
-    // 92.6 for 96 x 39 x 39, 3 x 3, fp8, 96 -> 480, now 15.4 and 94.2 with one.)
+    // first, a channel each, and put into LDS when the first stage is there, which
+    // was asked for later: its trip to memory runs under all of that.  (Read where
+    // it is added, channel by channel in front of the stores, it kept every tile
+    // waiting: with and without a bias 17.8 and 15.0 us for 25 x 57 x 57, 3 x 3
+    // stride 2, 72 -> 200, 117.7 and 92.6 for 96 x 39 x 39, 3 x 3, fp8, 96 -> 480,
+    // now 15.4 and 94.2 with one.  Kept in a register through the loop it made long
+    // ones of fp32 3 to 7 % slower: 6 x 21 x 21, 5 x 5, 238 -> 168 67.4 us, 62.2 so.)
     float biasHere = 0.0f;
     if (bias && t < BN && nTile * BN + t < d.outChansPerGroup)
       biasHere = Load<OutT>::at(
@@ -529,6 +531,8 @@ __device__ __forceinline__ void igemmTile(
     // returned by then (the producers may refill it), the next stage has
     // landed, and its first reads go out under the last sub-step's MFMAs.
     stepBarrier(); // barrier 0
+    if (t < BN)
+      biasLds[t] = biasHere;
     if (a.kSteps != 0)
       staticFor<0, P>([&](auto sub) { fetch(0, sub); });
     pin();
@@ -550,8 +554,6 @@ __device__ __forceinline__ void igemmTile(
       });
       pin();
     }
-    if (t < BN)
-      biasLds[t] = biasHere;
   }
   // One more meeting point: the producers' trailing loads have landed, so
   // LDS can be reused for the output tile.
@@ -844,8 +846,6 @@ size_t igemmWorkspaceBytes(const IgemmDesc &d) {
 
 namespace {
 
-/// Checks `d` against what the kernels are compiled for (the planner only
-/// produces such shapes) and fills in the kernel's arguments.
 /// Whether a launch stores its output through the L2: rows of whole vectors at a
 /// multiple of their size, and in tiles of 128 pixels no more of them than
 /// kMostThrough (of 256 pixels a CU has one tile at a time, whose outputs all
@@ -863,6 +863,8 @@ bool storesThrough(const IgemmArgs &a, int outType, const void *out) {
          (a.d.blockM == 256 || bytes <= kMostThrough);
 }
 
+/// Checks `d` against what the kernels are compiled for (the planner only
+/// produces such shapes) and fills in the kernel's arguments.
 hipError_t prepare(const IgemmDesc &d, int inType, bool haveWorkspace,
                    IgemmArgs &a) {
   const uint32_t eb = inType == kFloat ? 4 : inType == kHalf ? 2 : 1;
