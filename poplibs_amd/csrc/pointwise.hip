@@ -66,10 +66,10 @@ struct PwArgs {
   uint32_t nBlocks;    // 32-channel blocks per group in the packed weights
   uint32_t walkers;    // workgroups sharing the pixel tiles of one (g, nTile)
   uint32_t inBytes, wBytes;
+  uint32_t outBytes; // of an output that is stored through the L2
   // fp8: 2^(scaleIn + scaleWeights), applied to the sums on their way out,
   // and its inverse, by which the bias enters them
   float scale, invScale;
-  uint32_t through; // outputs are stored through the L2
 };
 
 /// One 32-byte k-slice of a 32 x 32 block: `w` and `x` are a lane's 16 bytes
@@ -107,6 +107,14 @@ __device__ __forceinline__ floatx16 pwMma(const uintx4 &w, const uintx4 &x,
   }
 }
 
+/// Waves of a SIMD that the registers have to leave room for: two workgroups of
+/// ten where the LDS takes two (walkersFor), which is 96 registers at most.  The
+/// compiler is told only where it would use more; the others use no more, and the
+/// schedules that it picks for them when told are 1 to 3 % slower.
+constexpr int pwWavesPerSimd(int ks, int nt, bool through) {
+  return ks == 4 && nt <= 3 && through ? 5 : 1;
+}
+
 /// KS: k-slices of 16 channels (Ci / 16).  TM: pixels per tile (32, 64, 128);
 /// the workgroup has TM / 16 compute waves and LW loader waves, which take
 /// the loads of a tile in turn.  NB: tile buffers in LDS; NB - 1 tiles are in
@@ -116,9 +124,15 @@ __device__ __forceinline__ floatx16 pwMma(const uintx4 &w, const uintx4 &x,
 /// less - 64 -> 256 channels on N = 32, 56 x 56: four shares of 64 re-read
 /// 13 MB four times beside 51 MB of output.
 /// F: the operands' type, see pwMma (a k-slice is 32 bytes of a row: 16 fp16
-/// channels or 32 fp8 ones).
-template <int KS, int TM, int NB, int LW, int NT, class OutT, int F = 0>
-__global__ __launch_bounds__(TM * 4 + 64 * LW) void pointwiseKernel(
+/// channels or 32 fp8 ones).  THROUGH: outputs are stored through the L2.  (Not an
+/// argument: with both ways to store the fp8 kernel of 128 channels and two tiles
+/// had 98 registers, and a CU one workgroup instead of two: N = 32, 56 x 56, 96 ->
+/// 128 11.0 us, 10.5 so.)
+template <int KS, int TM, int NB, int LW, int NT, class OutT, int F,
+          bool THROUGH>
+__global__
+__launch_bounds__(TM * 4 + 64 * LW,
+                  pwWavesPerSimd(KS, NT, THROUGH)) void pointwiseKernel(
     PwArgs a, const char *__restrict__ in, const char *__restrict__ w,
     const OutT *__restrict__ bias, OutT *__restrict__ out) {
   constexpr int kRow = KS * 32;                 // bytes of one activation row
@@ -267,6 +281,24 @@ __global__ __launch_bounds__(TM * 4 + 64 * LW) void pointwiseKernel(
   constexpr int kPassChans = 64 / int(sizeof(OutT));
   constexpr int kVecElems = 16 / int(sizeof(OutT));
 
+  auto store = [&](uintx4 data, uint32_t m, uint32_t n) {
+    if constexpr (THROUGH) {
+#if defined(__HIP_DEVICE_COMPILE__)
+      __builtin_amdgcn_raw_buffer_store_b128(
+          data, bufferOf(out, a.outBytes),
+          (m * outChans + g * d.outChansPerGroup + n) * uint32_t(sizeof(OutT)),
+          0, kWriteThroughStore);
+#endif
+    } else {
+      // streaming (the output is not read again here): 15.2 -> 12.4 us on the
+      // 56 x 56, 256 -> 64 layer.  The same hint on the loads loses a
+      // microsecond of that.
+      __builtin_nontemporal_store(
+          data, reinterpret_cast<uintx4 *>(out + size_t(m) * outChans +
+                                           g * d.outChansPerGroup + n));
+    }
+  };
+
   uint32_t buffer = 0;
   for (uint32_t mTile = walker; mTile < a.mTiles; mTile += a.walkers) {
     stepBarrier(); // tile i has landed
@@ -342,15 +374,8 @@ __global__ __launch_bounds__(TM * 4 + 64 * LW) void pointwiseKernel(
                 nTile * NT * kPwChans + (nb * NT + 2 * np) * 32 + vec * 8;
             const uintx4 data = *reinterpret_cast<const uintx4 *>(
                 stage + r * kPwPairRow + vec * 16);
-            if (m < a.M && n < d.outChansPerGroup) {
-              OutT *dst =
-                  out + size_t(m) * outChans + g * d.outChansPerGroup + n;
-              if (a.through)
-                storeThrough(dst, data);
-              else
-                __builtin_nontemporal_store(data,
-                                            reinterpret_cast<uintx4 *>(dst));
-            }
+            if (m < a.M && n < d.outChansPerGroup)
+              store(data, m, n);
           }
           MXK_WAIT_LGKMCNT0(); // read before the next pixels overwrite it
         }
@@ -411,17 +436,8 @@ __global__ __launch_bounds__(TM * 4 + 64 * LW) void pointwiseKernel(
           const uint32_t m = mTile * TM + mb * 32 + r;
           const uintx4 data = *reinterpret_cast<const uintx4 *>(
               stage + r * kPwStageRow + vec * 16);
-          if (m < a.M && n < d.outChansPerGroup) {
-            uintx4 *dst = reinterpret_cast<uintx4 *>(
-                out + size_t(m) * outChans + g * d.outChansPerGroup + n);
-            // streaming store (the output is not read again here): 15.2 ->
-            // 12.4 us on the 56 x 56, 256 -> 64 layer.  The same hint on the
-            // loads loses a microsecond of that.
-            if (a.through)
-              storeThrough(dst, data);
-            else
-              __builtin_nontemporal_store(data, dst);
-          }
+          if (m < a.M && n < d.outChansPerGroup)
+            store(data, m, n);
         }
         MXK_WAIT_LGKMCNT0(); // staging is read before the next pass rewrites it
       }
@@ -433,7 +449,9 @@ __global__ __launch_bounds__(TM * 4 + 64 * LW) void pointwiseKernel(
 /// as many workgroups as fit the chip at once (LDS allows 160 KB / ldsBytes
 /// per CU), shared out over the pairs - and no more than give every walker
 /// the same number of tiles (to within one): 3.1 tiles per walker would mean
-/// a fourth round at a quarter of the chip.
+/// a fourth round at a quarter of the chip.  (Registers: with 64 input channels
+/// of fp16, or 128 of fp8, and up to three channel tiles, where LDS has room for
+/// two workgroups of ten waves, the kernels keep to the 96 that they take then.)
 uint64_t walkersFor(uint64_t mTiles, uint64_t pairs, uint32_t ldsBytes,
                     uint32_t cus) {
   const uint64_t resident = uint64_t(cus) * ((160 * 1024) / ldsBytes);
@@ -516,13 +534,14 @@ int deviceCUs() {
   return cus;
 }
 
-template <int KS, int TM, int NB, int LW, int NT, class OutT, int F>
+template <int KS, int TM, int NB, int LW, int NT, class OutT, int F,
+          bool THROUGH>
 hipError_t run(PwArgs a, const void *in, const void *w, const void *bias,
                void *out, hipStream_t stream) {
   constexpr int ldsBytes = ldsBytesOf(PwShape{TM, NB, LW}, KS * 16, NT);
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void *>(
-          &pointwiseKernel<KS, TM, NB, LW, NT, OutT, F>),
+          &pointwiseKernel<KS, TM, NB, LW, NT, OutT, F, THROUGH>),
       hipFuncAttributeMaxDynamicSharedMemorySize, ldsBytes);
   if (attr != hipSuccess)
     return attr;
@@ -539,7 +558,7 @@ hipError_t run(PwArgs a, const void *in, const void *w, const void *bias,
   if (blocks > 0x7fffffffull ||
       uint64_t(a.mTiles) + uint64_t(NB) * walkers > 0x7fffffffull / TM)
     return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((pointwiseKernel<KS, TM, NB, LW, NT, OutT, F>),
+  hipLaunchKernelGGL((pointwiseKernel<KS, TM, NB, LW, NT, OutT, F, THROUGH>),
                      dim3(uint32_t(blocks)), dim3(TM * 4 + 64 * LW), ldsBytes,
                      stream, a, static_cast<const char *>(in),
                      static_cast<const char *>(w),
@@ -547,61 +566,61 @@ hipError_t run(PwArgs a, const void *in, const void *w, const void *bias,
   return hipGetLastError();
 }
 
-template <class OutT, int F>
+template <class OutT, int F, bool THROUGH>
 hipError_t runSlices(const PwArgs &a, const void *in, const void *w,
                      const void *bias, void *out, hipStream_t stream) {
   const uint32_t nt = chanTilesFor(a.d, uint32_t(deviceCUs()));
   switch (pwPaddedChans(pwRowChans(a.d))) {
   case 16:
     if (nt == 4)
-      return run<1, kShape64.tm, kShape64.nb, kShape64.lw, 4, OutT, F>(
+      return run<1, kShape64.tm, kShape64.nb, kShape64.lw, 4, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
     if (nt == 3)
-      return run<1, kShape64.tm, kShape64.nb, kShape64.lw, 3, OutT, F>(
+      return run<1, kShape64.tm, kShape64.nb, kShape64.lw, 3, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
     if (nt == 2)
-      return run<1, kShape64.tm, kShape64.nb, kShape64.lw, 2, OutT, F>(
+      return run<1, kShape64.tm, kShape64.nb, kShape64.lw, 2, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
-    return run<1, kShape64.tm, kShape64.nb, kShape64.lw, 1, OutT, F>(
+    return run<1, kShape64.tm, kShape64.nb, kShape64.lw, 1, OutT, F, THROUGH>(
         a, in, w, bias, out, stream);
   case 32:
     if (nt == 4)
-      return run<2, kShape64.tm, kShape64.nb, kShape64.lw, 4, OutT, F>(
+      return run<2, kShape64.tm, kShape64.nb, kShape64.lw, 4, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
     if (nt == 3)
-      return run<2, kShape64.tm, kShape64.nb, kShape64.lw, 3, OutT, F>(
+      return run<2, kShape64.tm, kShape64.nb, kShape64.lw, 3, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
     if (nt == 2)
-      return run<2, kShape64.tm, kShape64.nb, kShape64.lw, 2, OutT, F>(
+      return run<2, kShape64.tm, kShape64.nb, kShape64.lw, 2, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
-    return run<2, kShape64.tm, kShape64.nb, kShape64.lw, 1, OutT, F>(
+    return run<2, kShape64.tm, kShape64.nb, kShape64.lw, 1, OutT, F, THROUGH>(
         a, in, w, bias, out, stream);
   case 64:
     if (nt == 4)
-      return run<4, kShape64.tm, kShape64.nb, kShape64.lw, 4, OutT, F>(
+      return run<4, kShape64.tm, kShape64.nb, kShape64.lw, 4, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
     if (nt == 3)
-      return run<4, kShape64.tm, kShape64.nb, kShape64.lw, 3, OutT, F>(
+      return run<4, kShape64.tm, kShape64.nb, kShape64.lw, 3, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
     if (nt == 2)
-      return run<4, kShape64.tm, kShape64.nb, kShape64.lw, 2, OutT, F>(
+      return run<4, kShape64.tm, kShape64.nb, kShape64.lw, 2, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
-    return run<4, kShape64.tm, kShape64.nb, kShape64.lw, 1, OutT, F>(
+    return run<4, kShape64.tm, kShape64.nb, kShape64.lw, 1, OutT, F, THROUGH>(
         a, in, w, bias, out, stream);
   case 128:
     if (nt == 2)
-      return run<8, kShape128.tm, kShape128.nb, kShape128.lw, 2, OutT, F>(
+      return run<8, kShape128.tm, kShape128.nb, kShape128.lw, 2, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
-    return run<8, kShape128.tm, kShape128.nb, kShape128.lw, 1, OutT, F>(
+    return run<8, kShape128.tm, kShape128.nb, kShape128.lw, 1, OutT, F, THROUGH>(
         a, in, w, bias, out, stream);
   case 256:
     if (nt == 2)
-      return run<16, kShape256.tm, kShape256.nb, kShape256.lw, 2, OutT, F>(
+      return run<16, kShape256.tm, kShape256.nb, kShape256.lw, 2, OutT, F, THROUGH>(
           a, in, w, bias, out, stream);
-    return run<16, kShape256.tm, kShape256.nb, kShape256.lw, 1, OutT, F>(
+    return run<16, kShape256.tm, kShape256.nb, kShape256.lw, 1, OutT, F, THROUGH>(
         a, in, w, bias, out, stream);
   case 512:
-    return run<32, kShape512.tm, kShape512.nb, kShape512.lw, 1, OutT, F>(
+    return run<32, kShape512.tm, kShape512.nb, kShape512.lw, 1, OutT, F, THROUGH>(
         a, in, w, bias, out, stream);
   }
   return hipErrorInvalidValue;
@@ -693,10 +712,11 @@ hipError_t launchPointwise(const PointwiseDesc &d, int inType, int outType,
   const uint32_t outPixel =
       d.groups * d.outChansPerGroup * (outType == kFloat ? 4 : 2);
   const uint64_t outBytes = uint64_t(a.M) * outPixel;
-  a.through = outPixel % 64 != 0 &&
-              (outBytes <= 6000000 ||
-               (outBytes >= 12000000 && outBytes <= 150000000 &&
-                inPixel <= 128 && outPixel * 2 >= inPixel * 5));
+  const bool through = outPixel % 64 != 0 &&
+                       (outBytes <= 6000000 ||
+                        (outBytes >= 12000000 && outBytes <= 150000000 &&
+                         inPixel <= 128 && outPixel * 2 >= inPixel * 5));
+  a.outBytes = through ? uint32_t(outBytes) : 0;
   a.mTiles = 0; // set for the tile height of the kernel that runs
   a.nTiles = (d.outChansPerGroup + kPwChans - 1) / kPwChans;
   a.nBlocks = a.nTiles * 2;
@@ -705,19 +725,25 @@ hipError_t launchPointwise(const PointwiseDesc &d, int inType, int outType,
   a.wBytes = uint32_t(pointwisePackedElems(d) * d.elemBytes);
   a.scale = inType == kQuarter ? q.scale : 1.0f;
   a.invScale = 1.0f / a.scale;
-  if (inType == kQuarter) {
+  auto go = [&](auto storesThrough) {
+    constexpr bool THROUGH = decltype(storesThrough)::value;
+    if (inType != kQuarter)
+      return outType == kHalf ? runSlices<__half, 0, THROUGH>(
+                                    a, in, weightsPacked, bias, out, stream)
+                              : runSlices<float, 0, THROUGH>(
+                                    a, in, weightsPacked, bias, out, stream);
     const bool actsE5M2 = q.inFormat != kE4M3, wE5M2 = q.weightFormat != kE4M3;
-    if (!actsE5M2 && !wE5M2)
-      return runSlices<__half, 1>(a, in, weightsPacked, bias, out, stream);
-    if (actsE5M2 && !wE5M2)
-      return runSlices<__half, 2>(a, in, weightsPacked, bias, out, stream);
-    if (!actsE5M2 && wE5M2)
-      return runSlices<__half, 3>(a, in, weightsPacked, bias, out, stream);
-    return runSlices<__half, 4>(a, in, weightsPacked, bias, out, stream);
-  }
-  if (outType == kHalf)
-    return runSlices<__half, 0>(a, in, weightsPacked, bias, out, stream);
-  return runSlices<float, 0>(a, in, weightsPacked, bias, out, stream);
+    if (!wE5M2)
+      return actsE5M2 ? runSlices<__half, 2, THROUGH>(a, in, weightsPacked,
+                                                      bias, out, stream)
+                      : runSlices<__half, 1, THROUGH>(a, in, weightsPacked,
+                                                      bias, out, stream);
+    return actsE5M2 ? runSlices<__half, 4, THROUGH>(a, in, weightsPacked, bias,
+                                                    out, stream)
+                    : runSlices<__half, 3, THROUGH>(a, in, weightsPacked, bias,
+                                                    out, stream);
+  };
+  return through ? go(std::true_type{}) : go(std::false_type{});
 }
 
 } // namespace mxk
