@@ -105,7 +105,7 @@ struct RowsArgs {
   uint32_t colsIn;            // input columns of a strip: (colsOut-1)*S + 3
   uint32_t inBytes;
   FastDiv divVecs, divStrips, divBands;
-  uint32_t through; // outputs are stored through the L2
+  uint32_t outThrough; // bytes of the output if it is stored through the L2, else 0
 };
 
 union Vec8 {
@@ -115,21 +115,23 @@ union Vec8 {
 
 template <class OutT> struct PutVec;
 template <> struct PutVec<__half> {
-  static __device__ __forceinline__ void put(__half *p, const float (&v)[8],
-                                             bool through) {
+  static __device__ __forceinline__ void put(__half *out, size_t i,
+                                             const float (&v)[8],
+                                             uint32_t through) {
     Vec8 o;
 #pragma unroll
     for (int i = 0; i != 4; ++i)
       o.h2[i] = roundPairToHalf(v[2 * i], v[2 * i + 1]);
     if (through)
-      storeThrough(p, o.raw);
+      storeThrough(bufferOf(out, through), uint32_t(i) * 2, o.raw);
     else
-      __builtin_nontemporal_store(o.raw, reinterpret_cast<uintx4 *>(p));
+      __builtin_nontemporal_store(o.raw, reinterpret_cast<uintx4 *>(out + i));
   }
 };
 template <> struct PutVec<float> {
-  static __device__ __forceinline__ void put(float *p, const float (&v)[8],
-                                             bool) {
+  static __device__ __forceinline__ void put(float *out, size_t i,
+                                             const float (&v)[8], uint32_t) {
+    float *p = out + i;
     __builtin_nontemporal_store(floatx4{v[0], v[1], v[2], v[3]},
                                 reinterpret_cast<floatx4 *>(p));
     __builtin_nontemporal_store(floatx4{v[4], v[5], v[6], v[7]},
@@ -271,7 +273,7 @@ __global__ __launch_bounds__((Ring<S, K>::kThreads)) void depthwiseRowsKernel(
     biasV[e] = biasRaw.at(e);
   // the thread's window in a row slot: columns col * S .. + 2
   const uint32_t windowByte = ((active ? col : 0) * S * a.vecs + v) * 16;
-  OutT *dst = out + ((size_t(b) * d.outH + oh0) * d.outW + ow) * d.channels + c;
+  size_t dst = ((size_t(b) * d.outH + oh0) * d.outW + ow) * d.channels + c;
   const size_t outRow = size_t(d.outW) * d.channels;
   auto rowOf = [&](uint32_t slot) {
     return lds + slot * kSlotBytes + windowByte;
@@ -306,7 +308,7 @@ __global__ __launch_bounds__((Ring<S, K>::kThreads)) void depthwiseRowsKernel(
         }
       }
     if (active)
-      PutVec<OutT>::put(dst, acc, a.through);
+      PutVec<OutT>::put(out, dst, acc, a.outThrough);
     dst += outRow;
   };
   auto next = [&](uint32_t slot) {
@@ -364,7 +366,7 @@ __global__ __launch_bounds__((Ring<S, K>::kThreads)) void depthwiseRowsKernel(
           }
         }
         if (active)
-          PutVec<OutT>::put(dst, acc, a.through);
+          PutVec<OutT>::put(out, dst, acc, a.outThrough);
         dst += outRow;
       }
       slot += S;
@@ -707,8 +709,9 @@ hipError_t launchDepthwiseRows(const DepthwiseDesc &d, int inType, int outType,
   a.divVecs = makeFastDiv(a.vecs);
   a.divStrips = makeFastDiv(a.strips);
   a.divBands = makeFastDiv(a.bands);
-  a.through =
-      uint64_t(d.batch) * d.outH * d.outW * d.channels * 2 <= kRowsThrough;
+  const uint64_t outBytes =
+      uint64_t(d.batch) * d.outH * d.outW * d.channels * 2;
+  a.outThrough = outBytes <= kRowsThrough ? reachableBytes(outBytes) : 0;
   const bool s1 = d.strideH == 1, k3 = d.kH == 3;
   if (outType == kHalf)
     return s1 ? (k3 ? run<1, 3, __half>(a, in, weightsPacked, bias, out, stream)

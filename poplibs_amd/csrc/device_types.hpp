@@ -154,41 +154,55 @@ __device__ __forceinline__ void storeOut4(__half *p, const float (&v)[4]) {
   *reinterpret_cast<uint2 *>(p) = pack.u;
 }
 
-/// The same, and 16 bytes, through the L2 to memory at once (device scope): what a
-/// kernel leaves dirty in the eight L2s is written back when it ends, before the
-/// next one starts, and a kernel whose workgroups all store at their end leaves
-/// its whole output.  For whole vectors at addresses that are multiples of their
-/// size: 22 MB in rows of 548 bytes took 19.1 us, 12.8 by way of the L2.
-/// (A store of more than 8 bytes reads its registers a cycle late: nothing may
-/// write them in the next one, which the compiler does not see to here.)
+/// Cache policy of a store that goes through the L2 to memory at once
+/// (device scope) instead of leaving a dirty line there.  What a kernel leaves
+/// dirty in the eight L2s is written back when it ends, before the next kernel
+/// of the stream starts; for a kernel of a few microseconds whose output comes
+/// all at its end that write-back is a measurable part (3x3 on 28x28, 128
+/// channels: 9.1 -> 8.9 us).  Kernels that stream their output while they run
+/// lose by it (1x1 on 56x56: 12.3 -> 15.5 us).
+constexpr int kWriteThroughStore = 16;
+
 typedef unsigned int ThroughWords4 __attribute__((ext_vector_type(4)));
 typedef unsigned int ThroughWords2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void storeThrough(void *p, ThroughWords4 v) {
+/// 16 or 8 bytes into a buffer by that policy, at a multiple of their size (another
+/// address gives the same bytes, more slowly: 22 MB in rows of 548 bytes took
+/// 19.1 us, 12.8 by way of the L2).  A buffer store and no assembly: the compiler
+/// has to see it, because a vector instruction may rewrite the registers of a
+/// store of more than 8 bytes only after two wait states, and a store may read
+/// an MFMA's result only after more, which it sees to.
+__device__ __forceinline__ void storeThrough(__amdgpu_buffer_rsrc_t to,
+                                             uint32_t byte, ThroughWords4 v) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p),
-               "v"(v)
-               : "memory");
+  __builtin_amdgcn_raw_buffer_store_b128(v, to, byte, 0, kWriteThroughStore);
 #endif
 }
-__device__ __forceinline__ void storeThrough(void *p, ThroughWords2 v) {
+__device__ __forceinline__ void storeThrough(__amdgpu_buffer_rsrc_t to,
+                                             uint32_t byte, ThroughWords2 v) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("global_store_dwordx2 %0, %1, off sc1\n\ts_nop 0" ::"v"(p),
-               "v"(v)
-               : "memory");
+  __builtin_amdgcn_raw_buffer_store_b64(v, to, byte, 0, kWriteThroughStore);
 #endif
 }
-__device__ __forceinline__ void storeOut4Through(float *p,
+/// Four consecutive outputs, the first of them element i of the buffer.
+__device__ __forceinline__ void storeOut4Through(__amdgpu_buffer_rsrc_t to,
+                                                 uint32_t i, const float *,
                                                  const float (&v)[4]) {
-  storeThrough(p, __builtin_bit_cast(ThroughWords4,
-                                     float4{v[0], v[1], v[2], v[3]}));
+  storeThrough(to, i * 4,
+               __builtin_bit_cast(ThroughWords4, float4{v[0], v[1], v[2], v[3]}));
 }
-__device__ __forceinline__ void storeOut4Through(__half *p,
+__device__ __forceinline__ void storeOut4Through(__amdgpu_buffer_rsrc_t to,
+                                                 uint32_t i, const __half *,
                                                  const float (&v)[4]) {
   const __half2 h[2] = {roundPairToHalf(v[0], v[1]),
                         roundPairToHalf(v[2], v[3])};
   ThroughWords2 u;
   __builtin_memcpy(&u, h, 8);
-  storeThrough(p, u);
+  storeThrough(to, i * 2, u);
+}
+/// What such a kernel is told of an output: its bytes, for the buffer's range, or 0
+/// where they are more than a buffer's offset reaches.
+constexpr uint32_t reachableBytes(uint64_t bytes) {
+  return bytes < 0x80000000u ? uint32_t(bytes) : 0;
 }
 
 } // namespace mxk

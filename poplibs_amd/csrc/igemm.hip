@@ -786,7 +786,9 @@ __global__ __launch_bounds__(64) void splitKReduceKernel(
     return;
   }
   if constexpr (V == 4)
-    storeOut4Through(out + i, v);
+    storeOut4Through(bufferOf(out + uint64_t(blockIdx.x) * blockDim.x * V,
+                              64 * V * sizeof(OutT)),
+                     threadIdx.x * V, out, v);
   else
     storeOut(out, i, v[0]);
 }
@@ -846,7 +848,7 @@ size_t igemmWorkspaceBytes(const IgemmDesc &d) {
 
 namespace {
 
-/// Whether a launch stores its output through the L2: rows of whole vectors at a
+/// The bytes of an output that a launch stores through the L2, else 0: rows of whole vectors at a
 /// multiple of their size, and in tiles of 128 pixels no more of them than
 /// kMostThrough (of 256 pixels a CU has one tile at a time, whose outputs all
 /// leave at its end: 1.02 to 1.14 times as fast from 10 to 250 MB).  Of 290 layers
@@ -855,12 +857,19 @@ namespace {
 /// us, by way of the L2 and through it: 50 x 37 x 37, 1 x 1 stride 2, 272 -> 368
 /// 11.1 -> 9.5; fp8 119 x 13 x 13, 3 x 3, 176 -> 288 16.5 -> 14.9; product 3698 x
 /// 648 x 2000 17.8 -> 16.0; fp32 8 x 52 x 52, 1 x 1, 48 -> 192 11.5 -> 9.7.
-bool storesThrough(const IgemmArgs &a, int outType, const void *out) {
-  const uint64_t bytes = uint64_t(a.M) * a.d.groups * a.d.outChansPerGroup *
+uint32_t throughBytes(const IgemmArgs &a, int outType, const void *out) {
+  const IgemmDesc &d = a.d;
+  const uint64_t pixel = uint64_t(d.groups) * d.outChansPerGroup *
                          (outType == kFloat ? 4 : 2);
-  return a.d.outChansPerGroup % 8 == 0 && !a.outTransposed &&
-         reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-         (a.d.blockM == 256 || bytes <= kMostThrough);
+  const bool through = d.outChansPerGroup % 8 == 0 && !a.outTransposed &&
+                       reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
+                       (d.blockM == 256 || a.M * pixel <= kMostThrough);
+  if (!through)
+    return 0;
+  const uint64_t pixels = a.outMapped ? uint64_t(d.batch) * d.outFullD *
+                                            d.outFullH * d.outFullW
+                                      : a.M;
+  return reachableBytes(pixels * pixel);
 }
 
 /// Checks `d` against what the kernels are compiled for (the planner only
@@ -981,7 +990,7 @@ hipError_t launchIgemm(const IgemmDesc &d, int inType, int outType,
   if (e != hipSuccess)
     return e;
   const bool split = d.blockM != 256 && d.splitK != 1;
-  a.outThrough = storesThrough(a, split ? int(kFloat) : outType,
+  a.outThrough = throughBytes(a, split ? int(kFloat) : outType,
                                split ? workspace : out);
   if (d.blockM == 256)
     return launchIgemmWide(a, inType, outType, in, weightsPacked, bias, out, q,
@@ -1058,7 +1067,7 @@ hipError_t launchIgemmFused(const IgemmFusedItem *items, size_t count,
     const hipError_t e = prepare(*x.d, x.inType, false, m.a[i]);
     if (e != hipSuccess)
       return e;
-    m.a[i].outThrough = storesThrough(m.a[i], x.outType, x.out);
+    m.a[i].outThrough = throughBytes(m.a[i], x.outType, x.out);
     m.firstBlock[i] = uint32_t(blocks);
     blocks += uint64_t(m.a[i].mTiles) * m.a[i].nTiles * x.d->groups;
     if (blocks > 0x7fffffffull)

@@ -21,7 +21,9 @@ struct IgemmArgs {
   uint32_t tapPlaneStarts; // ... and bit kd * kH * kW for every kernel plane
   uint32_t outMapped; // outputs go to every outStep-th pixel of a larger field
   uint32_t outTransposed; // the final result as [channel][pixel]
-  uint32_t outThrough;    // whole vectors, stored through the L2 (storesThrough)
+  // bytes of the output where it is stored through the L2 as whole vectors
+  // (throughBytes), else 0
+  uint32_t outThrough;
   uint32_t mode;     // kMaskTaps, kRangeTaps or kDilatedTaps
   uint32_t M;        // batch * outH * outW
   uint32_t mTiles, nTiles;
@@ -113,14 +115,6 @@ using LdsPtr = __attribute__((address_space(3))) void *;
 /// POLICY: the load's cache policy bits - 0, or kStreamingLoad for data that
 /// is read once.
 constexpr int kStreamingLoad = 2;
-/// Cache policy of a store that goes through the L2 to memory at once
-/// (device scope) instead of leaving a dirty line there.  What a kernel leaves
-/// dirty in the eight L2s is written back when it ends, before the next kernel
-/// of the stream starts; for a kernel of a few microseconds whose output comes
-/// all at its end that write-back is a measurable part (3x3 on 28x28, 128
-/// channels: 9.1 -> 8.9 us).  Kernels that stream their output while they run
-/// lose by it (1x1 on 56x56: 12.3 -> 15.5 us).
-constexpr int kWriteThroughStore = 16;
 /// Outputs of more bytes than this are on their way while a kernel of small tiles
 /// runs, which is 0.5 to 3 % faster by leaving them to the L2 (32 x 64 x 64,
 /// 3 x 3, 80 -> 632, 166 MB 146 us, 151 through it).
@@ -459,6 +453,7 @@ igemmEpilogue(char *lds, const IgemmArgs &a, floatx16 (&acc)[2][BN / 64],
   constexpr int kVecsPerRow = BN / kVecElems;
   // (16-byte stores whatever the rows start at; the channels beyond the last
   // whole vector one by one)
+  const __amdgpu_buffer_rsrc_t outBuf = bufferOf(out, a.outThrough);
   auto copyOut = [&](auto through) {
     for (int idx = t; idx < kBlockM * kVecsPerRow; idx += kThreads) {
       const uint32_t mLocal = idx / kVecsPerRow, vec = idx % kVecsPerRow;
@@ -468,11 +463,14 @@ igemmEpilogue(char *lds, const IgemmArgs &a, floatx16 (&acc)[2][BN / 64],
         continue;
       const char *src = lds + mLocal * kOutRow + vec * 16;
       const size_t pixel = outPixel(a, m);
-      OutT *dst = out + pixel * outChans + g * d.outChansPerGroup + n;
       if constexpr (decltype(through)::value) {
-        storeThrough(dst, *reinterpret_cast<const uintx4 *>(src));
+        storeThrough(outBuf,
+                     (uint32_t(pixel) * outChans + g * d.outChansPerGroup + n) *
+                         uint32_t(sizeof(OutT)),
+                     *reinterpret_cast<const uintx4 *>(src));
         continue;
       }
+      OutT *dst = out + pixel * outChans + g * d.outChansPerGroup + n;
       if (a.outTransposed) {
         // [channel][pixel]: element stores, for small outputs
         const OutT *e = reinterpret_cast<const OutT *>(src);

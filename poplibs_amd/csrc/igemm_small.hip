@@ -50,6 +50,7 @@ struct SmallArgs {
   // 1: the result as [channel][pixel]; 2: into a larger field
   uint16_t outMode;
   uint32_t outFullH, outFullW, outOffH, outOffW;
+  uint32_t outThrough; // bytes of the output, 0 where it is out of a buffer's reach
   float scale;
   uint32_t formats; // fp8: bit 0 input, bit 1 weights in E5M2
   FastDiv divNTiles, divMTiles, divOutW, divOutH, divChunks, divKW;
@@ -336,10 +337,11 @@ __device__ __forceinline__ void igemmSmallTile(const SmallArgs &a,
       pixel = (size_t(b) * a.outFullH + oh + a.outOffH) * a.outFullW + ow +
               a.outOffW;
     }
-    OutT *at = out + pixel * a.outChans + g * a.co + n;
-    if (a.co % 4 == 0) {
-      storeOut4Through(at, v);
+    if (a.co % 4 == 0 && a.outThrough) {
+      storeOut4Through(bufferOf(out, a.outThrough),
+                       uint32_t(pixel) * a.outChans + g * a.co + n, out, v);
     } else {
+      OutT *at = out + pixel * a.outChans + g * a.co + n;
       for (int e = 0; e != 4 && n + e < a.co; ++e)
         storeOut(at, e, v[e]);
     }
@@ -578,6 +580,11 @@ hipError_t prepareSmall(const IgemmDesc &d, int inType, int outType,
   a.outMode = d.outTransposed ? 1 : d.outFullH || d.outFullW ? 2 : 0;
   a.outFullH = d.outFullH, a.outFullW = d.outFullW;
   a.outOffH = d.outOffH, a.outOffW = d.outOffW;
+  a.outThrough = reachableBytes(
+      uint64_t(d.batch) *
+      (a.outMode == 2 ? uint64_t(d.outFullH) * d.outFullW
+                      : uint64_t(d.outH) * d.outW) *
+      a.outChans * (outType == kFloat ? 4 : 2));
   a.scale = inType == kQuarter ? q.scale : 1.0f;
   a.formats = inType != kQuarter
                   ? 0

@@ -331,6 +331,7 @@ wideTile(const IgemmArgs &a, const char *__restrict__ in,
         }
     }
     __syncthreads();
+    const __amdgpu_buffer_rsrc_t outBuf = bufferOf(out, a.outThrough);
     auto copyOut = [&](auto through) {
       for (int idx = t; idx < 128 * kVecsPerRow; idx += kThreads) {
         const uint32_t mLocal = idx / kVecsPerRow, vec = idx % kVecsPerRow;
@@ -339,10 +340,13 @@ wideTile(const IgemmArgs &a, const char *__restrict__ in,
         if (m >= a.M || n >= d.outChansPerGroup)
           continue;
         const char *src = lds + mLocal * kOutRow + vec * 16;
-        OutT *dst =
-            out + outPixel(a, m) * outChans + g * d.outChansPerGroup + n;
+        const size_t pixel = outPixel(a, m);
+        OutT *dst = out + pixel * outChans + g * d.outChansPerGroup + n;
         if constexpr (decltype(through)::value) {
-          storeThrough(dst, *reinterpret_cast<const uintx4 *>(src));
+          storeThrough(outBuf,
+                       (uint32_t(pixel) * outChans + g * d.outChansPerGroup +
+                        n) * uint32_t(sizeof(OutT)),
+                       *reinterpret_cast<const uintx4 *>(src));
         } else if (n + kVecElems <= d.outChansPerGroup) {
           const uintx4 whole = *reinterpret_cast<const uintx4 *>(src);
           *reinterpret_cast<AnyWords *>(dst) = whole;

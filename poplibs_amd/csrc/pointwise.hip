@@ -283,12 +283,10 @@ __launch_bounds__(TM * 4 + 64 * LW,
 
   auto store = [&](uintx4 data, uint32_t m, uint32_t n) {
     if constexpr (THROUGH) {
-#if defined(__HIP_DEVICE_COMPILE__)
-      __builtin_amdgcn_raw_buffer_store_b128(
-          data, bufferOf(out, a.outBytes),
-          (m * outChans + g * d.outChansPerGroup + n) * uint32_t(sizeof(OutT)),
-          0, kWriteThroughStore);
-#endif
+      storeThrough(bufferOf(out, a.outBytes),
+                   (m * outChans + g * d.outChansPerGroup + n) *
+                       uint32_t(sizeof(OutT)),
+                   data);
     } else {
       // streaming (the output is not read again here): 15.2 -> 12.4 us on the
       // 56 x 56, 256 -> 64 layer.  The same hint on the loads loses a

@@ -47,7 +47,7 @@ struct ThinArgs {
   uint32_t biasByte;   // where the fp32 bias lies in LDS
   uint32_t weightByte; // ... and the packed weights, on their way to registers
   FastDiv divChunksPerRow; // by the chunks of 8 elements of a kernel row
-  uint32_t through;    // the output is stored through the L2
+  uint32_t outThrough; // bytes of the output if it is stored through the L2, else 0
   uint32_t cutElems;   // elements of a row in truncated columns
   FastDiv divCut;
 };
@@ -299,6 +299,7 @@ __global__ __launch_bounds__(kThinThreads)
       w[cb][q] = reinterpret_cast<const half8 *>(
           lds + a.weightByte)[(cb * KS + q) * 64 + lane];
 
+  const __amdgpu_buffer_rsrc_t outBuf = bufferOf(out, a.outThrough);
   for (uint32_t tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
     const uint32_t image = a.divTilesPerImage(tile);
     const uint32_t oh0 = (tile - image * a.tilesPerImage) * a.tileRows;
@@ -344,24 +345,34 @@ __global__ __launch_bounds__(kThinThreads)
       }
       const uint32_t ow = cbk * 16 + (lane & 15);
       if (ow < d.outW) {
+        // a pair of channel blocks: eight neighbouring channels per lane
+        auto pairOf = [&](int cb) {
+          const __half2 h[4] = {roundPairToHalf(acc[cb][0], acc[cb][1]),
+                                roundPairToHalf(acc[cb][2], acc[cb][3]),
+                                roundPairToHalf(acc[cb + 1][0], acc[cb + 1][1]),
+                                roundPairToHalf(acc[cb + 1][2], acc[cb + 1][3])};
+          uintx4 u;
+          __builtin_memcpy(&u, h, 16);
+          return u;
+        };
+        if constexpr (CB % 2 == 0 && sizeof(OutT) == 2) {
+          if (a.outThrough) {
+            const uint32_t byte =
+                (((image * d.outH + oh0 + r) * d.outW + ow) * d.outChans +
+                 thinChannelBase(0, quarter, CB)) * 2;
+#pragma unroll
+            for (int cb = 0; cb != CB; cb += 2)
+              storeThrough(outBuf, byte + cb * 32, pairOf(cb));
+            continue;
+          }
+        }
         OutT *dst = out + ((size_t(image) * d.outH + oh0 + r) * d.outW + ow) *
                               d.outChans;
-        // a pair of channel blocks: eight neighbouring channels per lane
 #pragma unroll
         for (int cb = 0; cb + 1 < CB; cb += 2) {
           OutT *at = dst + thinChannelBase(cb, quarter, CB);
           if constexpr (sizeof(OutT) == 2) {
-            const __half2 h[4] = {
-                roundPairToHalf(acc[cb][0], acc[cb][1]),
-                roundPairToHalf(acc[cb][2], acc[cb][3]),
-                roundPairToHalf(acc[cb + 1][0], acc[cb + 1][1]),
-                roundPairToHalf(acc[cb + 1][2], acc[cb + 1][3])};
-            uintx4 u;
-            __builtin_memcpy(&u, h, 16);
-            if (CB % 2 == 0 && a.through)
-              storeThrough(at, u);
-            else
-              *reinterpret_cast<uintx4 *>(at) = u;
+            *reinterpret_cast<uintx4 *>(at) = pairOf(cb);
           } else {
             const float v0[4] = {acc[cb][0], acc[cb][1], acc[cb][2],
                                  acc[cb][3]};
@@ -620,10 +631,12 @@ hipError_t launchThinInput(const ThinInputDesc &d, int inType, int outType,
   // 17.5 -> 14.0 (150 layers of up to 5, 20 and 60 MB of output 1.01, 1.06 and 1.13
   // times as fast); but of 48 channels, a piece and a half, 39 x 137 x 137, 5 x 5
   // 24.5 and 35.8.
-  a.through = outType == kHalf && d.outChans % 32 == 0 &&
-              reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-              uint64_t(d.batch) * d.outH * d.outW * d.outChans * 2 <=
-                  kMostThrough;
+  const uint64_t outBytes =
+      uint64_t(d.batch) * d.outH * d.outW * d.outChans * 2;
+  const bool through = outType == kHalf && d.outChans % 32 == 0 &&
+                       reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
+                       outBytes <= kMostThrough;
+  a.outThrough = through ? reachableBytes(outBytes) : 0;
   const uint32_t grid = uint32_t(l.workgroups);
   if (outType == kHalf)
     return launchBlocks<__half>(d.outChans / 16, s.kSteps, a, grid,

@@ -70,6 +70,7 @@ struct WuWindowArgs {
   uint32_t actBytes, deltaBytes;
   uint32_t strideF, strideTap; // of the result, in elements
   uint64_t chunkElems;
+  uint32_t outThrough; // bytes of a chunk's, 0 where out of a buffer's reach
   FastDiv divSegs, divOutH, divTilesPerChunk, divKH, divCiTiles, divCoTiles;
   FastDiv divCo;
 };
@@ -149,9 +150,9 @@ storeWindow(const WuWindowArgs &a, const WinPlace &w,
           continue;
         const size_t f =
             (size_t(w.g0) * a.resultCo + coIn) * a.resultCi + ciIn;
-        if (a.strideF == 1 && a.resultCi % 4 == 0) {
+        if (a.strideF == 1 && a.resultCi % 4 == 0 && a.outThrough) {
           const float v[4] = {total[0], total[1], total[2], total[3]};
-          storeOut4Through(to + f, v);
+          storeOut4Through(bufferOf(to, a.outThrough), uint32_t(f), out, v);
         } else {
 #pragma unroll
           for (uint32_t x = 0; x != 4; ++x)
@@ -824,6 +825,7 @@ hipError_t launchWuWindow(const WuTapDesc &d, int outType, const void *acts,
   const uint32_t blocks = uint32_t(s.chunks * s.tiles);
   void *to = direct ? out : workspace;
   const int toType = direct ? outType : int(kFloat);
+  a.outThrough = reachableBytes(a.chunkElems * (toType == kFloat ? 4 : 2));
   hipError_t e;
   if (d.elemBytes == 4)
     e = d.windowCo == 16
