@@ -943,19 +943,20 @@ mxconv_plan makePlanWith(const ConvParams &params,
            (l.workgroups * 2 >= gfx950::numCUs && l.rowsOut >= 4 &&
             (l.colsOut >= 4 || l.strips == 1))))
         f.dense3x3 = 2;
-      // Strips of columns for the others from some amount of work on, for 3 x 3
-      // taps more of it where channels are few and many slots' sums meet: below,
-      // the kernel's longer program and the meeting cost up to 1.5 us more than
-      // they save.  Of 420 layers (4 to 64 images of 7 to 112 squared, 32 to 960
-      // channels) the choice is 0.8, 1.0 and 0.8 % behind the faster of the two
-      // for 3, 5 and 7 taps a side, with lines at 8e6, 20e6 and 43e6 products
-      // 3.2, 2.2 and 2.7 %.
+      // Strips of columns for the others from some amount of work on, more of it
+      // where channels are few and many slots' sums meet: below, the kernel's
+      // longer program and the meeting cost up to 4 us more than they save.  Of
+      // 260 layers around the lines (1 to 128 images of 7 to 112 squared, 8 to
+      // 1040 channels) the choice is 0.7, 0.9 and 0.9 % behind the faster of the
+      // two for 3, 5 and 7 taps a side; with lines at 8e6, 20e6 and 43e6 products
+      // 4.4, 3.1 and 1.6 %, at 8e6 and 14e6 whatever the channels 2.2 (5 x 5) and
+      // 3.6 % (7 x 7, N = 16, 11 x 11 stride 2, 568 channels 14.4 us, 11.6 so).
       const double products =
           double(f.batch) * f.outH * f.outW * f.channels * f.kH * f.kW;
       const double enough =
           f.kH == 3   ? 1e6 * std::max(1.0, 192.0 / f.channels)
-          : f.kH == 5 ? 8e6
-                      : 14e6;
+          : f.kH == 5 ? 10e6 * std::max(1.0, 32.0 / f.channels)
+                      : 30e6 * std::max(1.0, 16.0 / f.channels);
       const int asked = options.planConstraints.columns;
       const bool takes = params.inputType == poplar::HALF &&
                          options.planConstraints.rowRing != 1 &&

@@ -700,6 +700,23 @@ def test_depthwise_weight_deltas_by_rings_or_columns(kw, ring):
     assert ("columns walked down in registers" in text) == (ring is False), text
 
 
+@pytest.mark.parametrize("kw,strips", [
+    # 5 x 5 and 7 x 7 taps: strips of columns from some work on, and from more
+    # of it where a few channels leave many slots' sums to meet
+    (dict(batch=26, field=(45, 45), kernel=(5, 5), groups=48, stride=2, pad=2),
+     True),
+    (dict(batch=18, field=(60, 60), kernel=(5, 5), groups=8, pad=2), False),
+    (dict(batch=18, field=(20, 20), kernel=(7, 7), groups=120, pad=3), True),
+    (dict(batch=16, field=(11, 11), kernel=(7, 7), groups=568, stride=2, pad=3),
+     False),
+    (dict(batch=3, field=(11, 11), kernel=(7, 7), groups=912, pad=3), False),
+    (dict(batch=60, field=(50, 50), kernel=(7, 7), groups=8, stride=2, pad=3),
+     False)])
+def test_depthwise_weight_deltas_in_strips_from_some_work_on(kw, strips):
+    text = pa.WeightUpdatePlan(make_params(pa.HALF, **kw)).describe()
+    assert ("columns walked down in registers" in text) == strips, text
+
+
 @pytest.mark.gpu
 def test_weight_update_applies_scaled_deltas(oracle):
     from gpu_helpers import quantize
