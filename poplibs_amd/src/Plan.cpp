@@ -966,7 +966,17 @@ mxconv_plan makePlanWith(const ConvParams &params,
             "planConstraints gfx950 columns: the weight deltas' kernel takes "
             "half tensors, 3x3, 5x5 or 7x7 taps at stride 1 or 2, without "
             "rowRing 1");
-      if (takes && (asked > 0 || (asked != 0 && products >= enough))) {
+      // (Rings whatever the estimates say where the tensors are more than the
+      // 256 MB cache in front of HBM holds: both were fitted to smaller ones.  Of
+      // 67 layers of 0.27 to 2.7 GB what they picked took 0.79 to 1.42 times the
+      // rings' time, 1.02 on average, 170 x 65 x 65, 136 channels 109 us, 77 in
+      // rings.)
+      const double tensors =
+          2.0 * f.batch * f.channels *
+          (double(f.inH) * f.inW + double(f.outH) * f.outW);
+      const bool ringsKept = f.dense3x3 == 2 && tensors > double(1 << 28);
+      if (takes && (asked > 0 ||
+                    (asked != 0 && products >= enough && !ringsKept))) {
         // The rings win where a few channels make long strips and the tensors
         // come from HBM (32 x 112 x 112 stride 2, 96 channels 24.2 us against
         // 28.1; 32 x 56 x 56, 144 19.1 against 19.8): every workgroup leaves a

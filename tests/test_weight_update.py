@@ -717,6 +717,21 @@ def test_depthwise_weight_deltas_in_strips_from_some_work_on(kw, strips):
     assert ("columns walked down in registers" in text) == strips, text
 
 
+def test_depthwise_weight_deltas_of_large_tensors_keep_the_rings():
+    # 391 MB, more than the cache in front of HBM holds; 120 MB
+    kw = dict(field=(65, 65), kernel=(3, 3), groups=136, pad=1)
+    text = pa.WeightUpdatePlan(make_params(pa.HALF, batch=170, **kw)).describe()
+    assert RING_WU in text, text
+    named = {"planConstraints": '{"gfx950": {"columns": 4}}'}
+    text = pa.WeightUpdatePlan(make_params(pa.HALF, batch=170, **kw),
+                               named).describe()
+    assert "columns walked down in registers" in text, text
+    text = pa.WeightUpdatePlan(make_params(pa.HALF, batch=48, field=(23, 23),
+                                           kernel=(3, 3), groups=976,
+                                           pad=1)).describe()
+    assert "columns walked down in registers" in text, text
+
+
 @pytest.mark.gpu
 def test_weight_update_applies_scaled_deltas(oracle):
     from gpu_helpers import quantize
