@@ -330,6 +330,9 @@ struct PointwiseDesc {
   // bytes of an input element: 2 (fp16) or 1 (fp8)
   uint32_t elemBytes = 2;
 };
+/// Bytes of an output in rows of no whole 64-byte pieces above which the planner
+/// looks at the other kernels, and the launch stores it as it does whole ones.
+constexpr uint64_t kPointwiseOddRows = 150000000;
 bool pointwiseTakes(const PointwiseDesc &d, int inType, int outType);
 /// Whether a workgroup can own `chanTiles` 64-channel tiles of this layer's
 /// output (they divide the layer's; 4 at most with 64 input channels, 2 with

@@ -712,7 +712,7 @@ hipError_t launchPointwise(const PointwiseDesc &d, int inType, int outType,
   const uint64_t outBytes = uint64_t(a.M) * outPixel;
   const bool through = outPixel % 64 != 0 &&
                        (outBytes <= 6000000 ||
-                        (outBytes >= 12000000 && outBytes <= 150000000 &&
+                        (outBytes >= 12000000 && outBytes <= kPointwiseOddRows &&
                          inPixel <= 128 && outPixel * 2 >= inPixel * 5));
   a.outBytes = through ? uint32_t(outBytes) : 0;
   a.mTiles = 0; // set for the tile height of the kernel that runs

@@ -1649,12 +1649,20 @@ mxconv_plan makePlanWith(const ConvParams &params,
     // its pieces are written one by one, whole rows of tiles at a time by the
     // others.  Of 420 layers of such rows those of 150 MB and more took 1.04 to
     // 2.4 times as long here, fp8 81 x 61 x 61, 112 -> 400 167 us, 93 in tiles of
-    // 128; smaller ones 0.6 to 1.5 times, 0.85 on average.)
+    // 128; smaller ones 0.6 to 1.5 times, 0.85 on average.  Two channel tiles to a
+    // workgroup write 128 bytes at a time: of 93 layers of 0.15 to 1.7 GB and more
+    // than 128 bytes of input to a pixel those with an odd number of tiles took
+    // 1.24 times as long here on average, those with an even one of fp8 0.74 times
+    // (128 x 56 x 56, 160 -> 368 74 us, 113 in tiles), of fp16 1.12 times up to 176
+    // bytes and 0.95 beyond.)
     const std::size_t inPixel = ci * p.numConvGroups * params.inputType.size();
     const std::size_t outPixel = co * p.numConvGroups * params.outputType.size();
+    const bool tilePairs =
+        (co + 63) / 64 % 2 == 0 && params.outputType == poplar::HALF;
+    const std::size_t mostIn = !tilePairs ? 256 : quarterIn ? 128 : 176;
     const bool largeOddRows =
-        outPixel % 64 != 0 && inPixel <= 256 && outPixel * 2 >= inPixel * 5 &&
-        std::size_t(pw.batch) * pw.pixels * outPixel > 150000000 &&
+        outPixel % 64 != 0 && inPixel <= mostIn && outPixel * 2 >= inPixel * 5 &&
+        std::size_t(pw.batch) * pw.pixels * outPixel > mxk::kPointwiseOddRows &&
         pc.pointwise != 1;
     plan.pointwiseOn =
         unitWindow && ciPadded == ci && !paddedSmall && !deepQuarter &&

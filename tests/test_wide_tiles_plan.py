@@ -85,3 +85,16 @@ def test_large_outputs_in_odd_rows_leave_the_pointwise_kernel(co, batch,
     assert ("pointwise streaming" in text) == pointwise, text
     asked = {"planConstraints": '{"gfx950": {"pointwise": 1}}'}
     assert "pointwise streaming" in pa.Plan(p, asked).describe()
+
+
+@pytest.mark.parametrize("in_type,ci,co,pointwise", [
+    # more than 128 bytes of input to a pixel, 150 MB of output and more: pairs
+    # of channel tiles write whole lines and stay where they are
+    (pa.QUARTER, 160, 368, True), (pa.QUARTER, 144, 488, True),
+    (pa.QUARTER, 160, 440, False), (pa.QUARTER, 128, 368, False),
+    (H, 80, 456, False), (H, 96, 456, True), (H, 104, 400, False)])
+def test_pairs_of_channel_tiles_in_odd_rows_stay(in_type, ci, co, pointwise):
+    p = make_params(in_type, H, batch=64, field=(64, 64), kernel=(1, 1), ci=ci,
+                    co=co)
+    text = pa.Plan(p).describe()
+    assert ("pointwise streaming" in text) == pointwise, text
