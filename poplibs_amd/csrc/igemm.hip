@@ -848,22 +848,34 @@ size_t igemmWorkspaceBytes(const IgemmDesc &d) {
 
 namespace {
 
-/// The bytes of an output that a launch stores through the L2, else 0: rows of whole vectors at a
-/// multiple of their size, and in tiles of 128 pixels no more of them than
-/// kMostThrough (of 256 pixels a CU has one tile at a time, whose outputs all
-/// leave at its end: 1.02 to 1.14 times as fast from 10 to 250 MB).  Of 290 layers
-/// and products with up to 5, 30 and 60 MB of output 1.04, 1.10 and 1.03 times as
-/// fast on average, the slowest 0.99.
-/// us, by way of the L2 and through it: 50 x 37 x 37, 1 x 1 stride 2, 272 -> 368
-/// 11.1 -> 9.5; fp8 119 x 13 x 13, 3 x 3, 176 -> 288 16.5 -> 14.9; product 3698 x
-/// 648 x 2000 17.8 -> 16.0; fp32 8 x 52 x 52, 1 x 1, 48 -> 192 11.5 -> 9.7.
+/// The bytes of an output that a launch stores through the L2, else 0.  Rows of whole
+/// vectors at a multiple of their size, and
+///  * in tiles of 128 pixels no more than kMostThrough of them: of 290 layers and
+///    products with up to 5, 30 and 60 MB of output 1.04, 1.10 and 1.03 times as
+///    fast on average, the slowest 0.99.  us, by way of the L2 and through it: 50 x
+///    37 x 37, 1 x 1 stride 2, 272 -> 368 11.1 -> 9.5; fp8 119 x 13 x 13, 3 x 3, 176
+///    -> 288 16.5 -> 14.9; product 3698 x 648 x 2000 17.8 -> 16.0; fp32 8 x 52 x 52,
+///    1 x 1, 48 -> 192 11.5 -> 9.7;
+///  * in tiles of 256 pixels, of which a CU has one at a time, whose outputs all
+///    leave at its end, any number of rows of whole 64-byte pieces (60 layers of 10 MB
+///    to 0.9 GB 1.04 times as fast on average, the slowest 1.01) and up to
+///    kMostWideThrough of others (32 of up to 120 MB 1.03 times, 18 of 0.12 to 1.1
+///    GB 0.99, fp8 109 x 42 x 42, 3 x 3, 176 -> 392 167 us, 181 through it).
+/// With K in parts the bytes are those of a part (partial sums of 0.05 to 0.2 GB in
+/// all 1.02 times as fast, the slowest 0.99), in a launch of several convolutions
+/// those of each: the phases of a backward pass at stride 2, which write every
+/// second pixel, 1.08 times as fast over 81 layers of 2 to 170 MB in all, 0.96 to
+/// 1.30.
 uint32_t throughBytes(const IgemmArgs &a, int outType, const void *out) {
   const IgemmDesc &d = a.d;
   const uint64_t pixel = uint64_t(d.groups) * d.outChansPerGroup *
                          (outType == kFloat ? 4 : 2);
-  const bool through = d.outChansPerGroup % 8 == 0 && !a.outTransposed &&
-                       reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-                       (d.blockM == 256 || a.M * pixel <= kMostThrough);
+  const uint64_t bytes = a.M * pixel;
+  const bool through =
+      d.outChansPerGroup % 8 == 0 && !a.outTransposed &&
+      reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
+      (d.blockM == 256 ? pixel % 64 == 0 || bytes <= kMostWideThrough
+                       : bytes <= kMostThrough);
   if (!through)
     return 0;
   const uint64_t pixels = a.outMapped ? uint64_t(d.batch) * d.outFullD *

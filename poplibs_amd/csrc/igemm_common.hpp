@@ -119,6 +119,8 @@ constexpr int kStreamingLoad = 2;
 /// runs, which is 0.5 to 3 % faster by leaving them to the L2 (32 x 64 x 64,
 /// 3 x 3, 80 -> 632, 166 MB 146 us, 151 through it).
 constexpr uint64_t kMostThrough = 60000000;
+/// ... and in tiles of 256 pixels, in rows of no whole 64-byte pieces (throughBytes).
+constexpr uint64_t kMostWideThrough = 120000000;
 template <int POLICY = 0>
 __device__ __forceinline__ void loadToLds(__amdgpu_buffer_rsrc_t buffer,
                                           LdsPtr dst, uint32_t vectorOffset,
