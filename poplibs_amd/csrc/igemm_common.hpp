@@ -432,19 +432,27 @@ igemmEpilogue(char *lds, const IgemmArgs &a, floatx16 (&acc)[2][BN / 64],
   constexpr int kOutRow = BN * int(sizeof(OutT)) + 16;
   if (!producer) {
     const uint32_t mRow = lane & 31, nOff4 = (lane >> 5) * 4;
+    // (the bias first, all of it: LDS answers in order, and a piece read between the
+    // writes waits for them; 26 x 24 x 24, 3 x 3, 144 -> 40 9.4 -> 9.2 us)
+    floatx4 bv[TN][4];
+#pragma unroll
+    for (int j = 0; j != TN; ++j)
+#pragma unroll
+      for (int q = 0; q != 4; ++q)
+        bv[j][q] = *reinterpret_cast<const floatx4 *>(
+            biasLds + wn * (BN / 2) + j * 32 + 8 * q + nOff4);
 #pragma unroll
     for (int j = 0; j != TN; ++j)
 #pragma unroll
       for (int q = 0; q != 4; ++q) {
         const uint32_t nLocal = wn * (BN / 2) + j * 32 + 8 * q + nOff4;
-        const floatx4 bv = *reinterpret_cast<const floatx4 *>(biasLds + nLocal);
 #pragma unroll
         for (int i = 0; i != 2; ++i) {
           const uint32_t mLocal = wm * 64 + i * 32 + mRow;
           float v[4];
 #pragma unroll
           for (int e = 0; e != 4; ++e)
-            v[e] = acc[i][j][q * 4 + e] * scale + bv[e];
+            v[e] = acc[i][j][q * 4 + e] * scale + bv[j][q][e];
           storeOut4(reinterpret_cast<OutT *>(lds + mLocal * kOutRow) + nLocal,
                     v);
         }
