@@ -42,7 +42,10 @@
 // 3 x 3 stride 2, 208 -> 64 9.7 -> 6.5 us; 21 x 39 x 39 stride 2, 32 groups of 16
 // 22.4 -> 18.7; 8 x 54 x 54, 32 -> 64 13.2 -> 11.3; tiles and chunks fitted anew).
 // Four are faster only where the tile is 32 x 32 and the chunk short (0.3 % over
-// 330 layers), a quarter slower on long ones.
+// 330 layers), a quarter slower on long ones.  A wave's fp32 sums are twice as long
+// for the same chunk, but the chunks are others: with fp32 results the deltas of 112
+// layers were off by 0.98 times as much as before on average against 64-bit sums
+// (0.77 to 1.21, at 0.6e-7 to 2.4e-7).
 //
 // With one chunk the deltas leave in weight order, one launch in all; with
 // several, fp32 sums go to the workspace as [chunk][tap][g][co][ci] and
@@ -628,12 +631,16 @@ uint64_t wuWindowWorkgroups(const WuTapDesc &d) {
 namespace {
 /// The pass's time by tile, kernel columns and stride along a row: `call`, a
 /// workgroup's k-steps at the pace of a wave (`wave` each of its own) or of the
-/// CU (`step`), `round` + `roundStep` per k-step for what does not go side by
-/// side on 256 CUs that take `places` workgroups each, and the second launch with
-/// its partial sums or the one launch's scattered results.  Fitted to 7 000
-/// measurements on 330 layers (4 to 64 images, fields of 7 to 64, 4 to 512
-/// channels, up to 32 groups), within 5 to 9 %; the tile and chunks picked by it
-/// are on average 1.8 % behind the best of those measured.
+/// CU (`step`), `round` + `roundStep` per k-step and round of workgroups beyond
+/// the first, and the second launch with its partial sums or the one launch's
+/// scattered results.  `places` rounds the workgroups of a CU up, to a whole one (1)
+/// or a third (3): a fitted number, not the workgroups that a CU holds (by registers
+/// two to three of every kernel here).  Fitted to 7 000 measurements on 330 layers
+/// (4 to 64 images, fields of 7 to 64, 4 to 512 channels, up to 32 groups), within 5
+/// to 9 %; the tile and chunks picked by it are on average 1.8 % behind the best of
+/// those measured.  Larger layers go by it too: of 70 with up to 600 GFLOP the pass
+/// is 1.06 times as fast on average as by the fit before, the slowest 0.88 (chunks of
+/// a thousand k-steps cut into rounds: 224 x 42 x 42, 136 -> 120 274 us, 312 so).
 struct WinFit {
   double call, wave, step, round, roundStep, second, partialMB, resultMB, places;
 };

@@ -978,9 +978,10 @@ mxconv_plan makePlanWith(const ConvParams &params,
       if (takes && (asked > 0 ||
                     (asked != 0 && products >= enough && !ringsKept))) {
         // The rings win where a few channels make long strips and the tensors
-        // come from HBM (32 x 112 x 112 stride 2, 96 channels 24.2 us against
-        // 28.1; 32 x 56 x 56, 144 19.1 against 19.8): every workgroup leaves a
-        // tile of all channels, whose sums their columns meet for in LDS (9 x 17
+        // are large (32 x 112 x 112 stride 2, 96 channels 23.3 us against 27.3 in
+        // strips; 64 x 56 x 56, 144 27.4 and 30.1; but 32 x 56 x 56, 144 19.2 and
+        // 17.2, where the two estimates are 0.1 us apart): every workgroup leaves
+        // a tile of all channels, whose sums their columns meet for in LDS (9 x 17
         // x 17, 856 channels 19.8 us, 10.4 in strips; 32 x 14 x 14, 504 16.8 and
         // 10.0; 11 x 56 x 56, 320 18.4 and 14.4).  Of 80 layers that the rings
         // take the choice is 1.0 % behind the best.

@@ -15,17 +15,18 @@ TILES = dict(kernel=(3, 3), ci=16 * 128, co=8)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kw", [
-    # 64, 512 and 576 pixels
-    dict(batch=1, field=(8, 8), pad=1, **TILES),
-    dict(batch=2, field=(16, 16), pad=1, **TILES),
-    dict(batch=4, field=(12, 12), pad=1, **TILES),
+@pytest.mark.parametrize("kw,chunks,pixels", [
+    # 64 (a chunk of 256), 512 and 576 pixels
+    (dict(batch=1, field=(8, 8), pad=1, **TILES), 1, 256),
+    (dict(batch=2, field=(16, 16), pad=1, **TILES), 1, 512),
+    (dict(batch=4, field=(12, 12), pad=1, **TILES), 1, 576),
     # three chunks of 1088 pixels, the last one shorter
-    dict(batch=4, field=(56, 57), pad=1, stride=2, **TILES),
+    (dict(batch=4, field=(56, 57), pad=1, stride=2, **TILES), 3, 1088),
     # one of 3136
-    dict(batch=1, field=(56, 56), pad=1, kernel=(3, 3), ci=3520, co=8),
+    (dict(batch=1, field=(56, 56), pad=1, kernel=(3, 3), ci=3520, co=8), 1,
+     3136),
 ])
-def test_long_chunks(oracle, kw):
+def test_long_chunks(oracle, kw, chunks, pixels):
     from gpu_helpers import quantize
     p = make_params(pa.HALF, pa.FLOAT, **kw)
     print("case", p, flush=True)
@@ -37,6 +38,8 @@ def test_long_chunks(oracle, kw):
         pa.HALF)
     got, plan = run_weight_update(p, xq, dq, FORCE_DENSE_WU)
     assert DENSE_WU in plan.describe(), plan.describe()
+    assert "%d chunks of %d pixels" % (chunks, pixels) in plan.describe(), \
+        plan.describe()
     # (fp32 sums of at most 3136 products)
     assert rel_l2(got, oracle.weight_deltas(p, xd, dd, threads=8)) <= 1e-5
 
