@@ -43,9 +43,9 @@
 // 22.4 -> 18.7; 8 x 54 x 54, 32 -> 64 13.2 -> 11.3; tiles and chunks fitted anew).
 // Four are faster only where the tile is 32 x 32 and the chunk short (0.3 % over
 // 330 layers), a quarter slower on long ones.  A wave's fp32 sums are twice as long
-// for the same chunk, but the chunks are others: with fp32 results the deltas of 112
-// layers were off by 0.98 times as much as before on average against 64-bit sums
-// (0.77 to 1.21, at 0.6e-7 to 2.4e-7).
+// for the same chunk, but the chunks are others: with fp32 results the deltas of 56
+// layers were off by 0.97 times as much as before on average against 64-bit sums
+// (0.77 to 1.21, at 0.6e-7 to 1.8e-7).
 //
 // With one chunk the deltas leave in weight order, one launch in all; with
 // several, fp32 sums go to the workspace as [chunk][tap][g][co][ci] and
