@@ -968,13 +968,13 @@ mxconv_plan makePlanWith(const ConvParams &params,
             "rowRing 1");
       // (Rings whatever the estimates say where the tensors are more than the
       // 256 MB cache in front of HBM holds: both were fitted to smaller ones.  Of
-      // 67 layers of 0.27 to 2.7 GB what they picked took 0.79 to 1.42 times the
+      // 69 layers of 0.26 to 2.7 GB what they picked took 0.79 to 1.42 times the
       // rings' time, 1.02 on average, 170 x 65 x 65, 136 channels 109 us, 77 in
       // rings.)
       const double tensors =
           2.0 * f.batch * f.channels *
           (double(f.inH) * f.inW + double(f.outH) * f.outW);
-      const bool ringsKept = f.dense3x3 == 2 && tensors > double(1 << 28);
+      const bool ringsKept = f.dense3x3 == 2 && tensors > 256e6;
       if (takes && (asked > 0 ||
                     (asked != 0 && products >= enough && !ringsKept))) {
         // The rings win where a few channels make long strips and the tensors
