@@ -574,22 +574,7 @@ __global__ __launch_bounds__(kThreads) void igemmKernel(
                                            blockIdx.x, gridDim.x);
 }
 
-/// Several convolutions that run the same kernel, in one launch: the grid is
-/// the concatenation of their tiles, so that convolutions too small to fill
-/// the chip share it.  (PopLibs' parallel multi-convolution plan gives each
-/// a disjoint range of tiles, lib/poplin/MultiConvolution.cpp:125-176.)
-constexpr int kMaxFused = int(kIgemmMaxFused);
-struct IgemmFusedArgs {
-  uint32_t count;
-  uint32_t firstBlock[kMaxFused + 1]; // prefix sums of the tile counts
-  IgemmArgs a[kMaxFused];
-  const char *in[kMaxFused];
-  const char *w[kMaxFused];
-  const void *bias[kMaxFused];
-  void *out[kMaxFused];
-  float scale[kMaxFused];
-};
-
+/// Several convolutions in one launch (IgemmFusedArgs).
 template <int BN, int NS, int EB, int FA, int FB, bool UNI, class OutT>
 __global__ __launch_bounds__(kThreads) void igemmFusedKernel(IgemmFusedArgs m) {
   uint32_t i = 0;
@@ -860,7 +845,10 @@ namespace {
 ///    leave at its end, any number of rows of whole 64-byte pieces (60 layers of 10 MB
 ///    to 0.9 GB 1.04 times as fast on average, the slowest 1.01) and up to
 ///    kMostWideThrough of others (32 of up to 120 MB 1.03 times, 18 of 0.12 to 1.1
-///    GB 0.99, fp8 109 x 42 x 42, 3 x 3, 176 -> 392 167 us, 181 through it).
+///    GB 0.99, fp8 109 x 42 x 42, 3 x 3, 176 -> 392 167 us, 181 through it);
+///  * in igemm_flex.hip's tiles any number in rows of whole 64-byte pieces (46 layers
+///    of 3 MB to 1.2 GB 1.03 times as fast on average, the slowest 0.97) and up to
+///    kMostThrough of others (65 layers 1.04 times, 18 larger ones 0.95).
 /// With K in parts the bytes are those of a part (partial sums of 0.05 to 0.2 GB in
 /// all 1.02 times as fast, the slowest 0.99), in a launch of several convolutions
 /// those of each: the phases of a backward pass at stride 2, which write every
@@ -874,8 +862,9 @@ uint32_t throughBytes(const IgemmArgs &a, int outType, const void *out) {
   const bool through =
       d.outChansPerGroup % 8 == 0 && !a.outTransposed &&
       reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-      (d.blockM == 256 ? pixel % 64 == 0 || bytes <= kMostWideThrough
-                       : bytes <= kMostThrough);
+      (d.flex            ? pixel % 64 == 0 || bytes <= kMostThrough
+       : d.blockM == 256 ? pixel % 64 == 0 || bytes <= kMostWideThrough
+                         : bytes <= kMostThrough);
   if (!through)
     return 0;
   const uint64_t pixels = a.outMapped ? uint64_t(d.batch) * d.outFullD *
@@ -892,9 +881,10 @@ hipError_t prepare(const IgemmDesc &d, int inType, bool haveWorkspace,
   const uint32_t bke = kRowBytes / eb;
   const int mode = igemmTapAddressing(d);
   const bool dilated = mode == kDilatedTaps;
-  const bool wide = d.blockM == 256;
-  if ((!wide && (d.blockM != kBlockM ||
-                 (d.blockN != 64 && d.blockN != 128))) ||
+  const bool wide = !d.flex && d.blockM == 256;
+  if ((d.flex && !igemmFlexTakes(d, inType, kHalf)) ||
+      (!d.flex && !wide &&
+       (d.blockM != kBlockM || (d.blockN != 64 && d.blockN != 128))) ||
       (wide && !igemmWideTakes(d, inType, kHalf)) ||
       d.blockK != bke || d.inChansPerGroup % (16 / eb) != 0 ||
       (inType != kHalf && inType != kQuarter && inType != kFloat) ||
@@ -1001,9 +991,13 @@ hipError_t launchIgemm(const IgemmDesc &d, int inType, int outType,
   hipError_t e = prepare(d, inType, workspace != nullptr, a);
   if (e != hipSuccess)
     return e;
+  if (d.flex && !igemmFlexTakes(d, inType, outType))
+    return hipErrorInvalidValue;
   const bool split = d.blockM != 256 && d.splitK != 1;
   a.outThrough = throughBytes(a, split ? int(kFloat) : outType,
                                split ? workspace : out);
+  if (d.flex)
+    return launchIgemmFlex(a, in, weightsPacked, bias, out, stream);
   if (d.blockM == 256)
     return launchIgemmWide(a, inType, outType, in, weightsPacked, bias, out, q,
                            stream);
@@ -1043,6 +1037,11 @@ hipError_t launchSplitKSum(const IgemmDesc &d, int outType,
 }
 
 bool igemmFusable(const IgemmFusedItem &x, const IgemmFusedItem &y) {
+  if (x.d->flex || y.d->flex)
+    return x.d->flex == y.d->flex && x.d->blockM == y.d->blockM &&
+           x.d->blockN == y.d->blockN &&
+           igemmFlexTakes(*x.d, x.inType, x.outType) &&
+           igemmFlexTakes(*y.d, y.inType, y.outType);
   return x.d->splitK == 1 && y.d->splitK == 1 &&
          x.d->blockM == kBlockM && y.d->blockM == kBlockM &&
          kernelKey(*x.d, x.inType, x.outType, x.q) ==
@@ -1053,13 +1052,13 @@ hipError_t launchIgemmFused(const IgemmFusedItem *items, size_t count,
                             hipStream_t stream) {
   if (count == 0)
     return hipSuccess;
-  if (count > size_t(kMaxFused))
+  if (count > size_t(kIgemmMaxFused))
     return hipErrorInvalidValue;
   // The longest tiles first: workgroups start in order, and a long one that
   // starts when the others are ending runs on alone (the backward pass of a
   // 3 x 3 stride-2 layer has phases of 1, 2, 2 and 4 taps: 25 x 57 x 57,
   // 72 -> 200 channels 26.0 us in that order, 22.5 in the other).
-  size_t order[kMaxFused];
+  size_t order[kIgemmMaxFused];
   for (size_t i = 0; i != count; ++i)
     order[i] = i;
   auto length = [&](size_t i) {
@@ -1091,6 +1090,8 @@ hipError_t launchIgemmFused(const IgemmFusedItem *items, size_t count,
     m.scale[i] = x.inType == kQuarter ? x.q.scale : 1.0f;
   }
   m.firstBlock[count] = uint32_t(blocks);
+  if (items[0].d->flex)
+    return launchIgemmFlexFused(m, stream);
   return dispatch(kernelKey(*items[0].d, items[0].inType, items[0].outType,
                             items[0].q),
                   LaunchFused{m, stream});

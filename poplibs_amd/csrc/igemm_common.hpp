@@ -36,6 +36,26 @@ struct IgemmArgs {
   FastDiv divWideBlock; // by 4 * nTiles (igemm_wide.hip)
 };
 
+/// Several convolutions that run the same kernel, in one launch: the grid is
+/// the concatenation of their tiles, so that convolutions too small to fill
+/// the chip share it.  (PopLibs' parallel multi-convolution plan gives each
+/// a disjoint range of tiles, lib/poplin/MultiConvolution.cpp:125-176.)
+struct IgemmFusedArgs {
+  uint32_t count;
+  uint32_t firstBlock[kIgemmMaxFused + 1]; // prefix sums of the tile counts
+  IgemmArgs a[kIgemmMaxFused];
+  const char *in[kIgemmMaxFused];
+  const char *w[kIgemmMaxFused];
+  const void *bias[kIgemmMaxFused];
+  void *out[kIgemmMaxFused];
+  float scale[kIgemmMaxFused];
+};
+
+/// igemm_flex.hip: tiles of any of its shapes; `a` as prepared for igemmKernel.
+hipError_t launchIgemmFlex(const IgemmArgs &a, const void *in, const void *w,
+                           const void *bias, void *out, hipStream_t stream);
+hipError_t launchIgemmFlexFused(const IgemmFusedArgs &m, hipStream_t stream);
+
 /// igemm_wide.hip: tiles of 256 pixels; `a` as prepared for igemmKernel.
 hipError_t launchIgemmWide(const IgemmArgs &a, int inType, int outType,
                            const void *in, const void *w, const void *bias,

@@ -234,7 +234,10 @@ struct IgemmDesc {
   // 16, 16 x 32, 32 x 32 or 64 x 32 pixels x channels; igemmSmallTakes); the
   // packed weights then have its layout (igemmSmallPackJob).
   uint32_t small = 0;
-  // Patch rows the tallest tile of that kernel spans (igemmPatchMaxRows),
+  // 1 or 2: the kernel of tiles of 128, 192 or 256 pixels x 64 to 256 channels
+  // in steps of 32 runs (igemmFlexTakes), 2 with two workgroups to a CU.
+  uint32_t flex = 0;
+  // Patch rows the tallest tile of the resident-patch kernel spans (igemmPatchMaxRows),
   // worked out once when the plan is made - it takes a walk over the tiles -
   // so that a launch does not repeat it; 0 = not known, work it out.
   uint32_t patchMaxRows = 0;
@@ -251,6 +254,10 @@ bool igemmAddressable(const IgemmDesc &d, int inType);
 /// Whether the kernel of 256-pixel tiles (d.blockM 256; d.blockN 192 or 256)
 /// takes the convolution, its tiles' images included.
 bool igemmWideTakes(const IgemmDesc &d, int inType, int outType);
+/// Whether the kernel of igemm_flex.hip has tiles of blockM x blockN, alone on
+/// a CU (flex 1) or two to a CU (2); whether it takes the convolution.
+bool igemmFlexTile(uint32_t blockM, uint32_t blockN, uint32_t flex);
+bool igemmFlexTakes(const IgemmDesc &d, int inType, int outType);
 int igemmTapAddressing(const IgemmDesc &d);
 size_t igemmWorkspaceBytes(const IgemmDesc &d);
 hipError_t launchIgemm(const IgemmDesc &d, int inType, int outType,

@@ -1571,6 +1571,7 @@ mxconv_status fusedWeightDeltas(const mxconv_plan *plan, const void *zDeltas,
                       !plan->paddedInputChans &&
                       plan->igemmPhases.empty() && !plan->kernelSelected &&
                       !plan->igemm.patch && !plan->igemm.small &&
+                      !plan->igemm.flex &&
                       // (tiles of 256 pixels do not write it transposed)
                       plan->igemm.blockM != 256 &&
                       // (a padded output field - the forward kernel was

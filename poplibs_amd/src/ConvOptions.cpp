@@ -221,6 +221,11 @@ void checkGfx950(const std::string &path, const Value &v, PlanConstraints &pc) {
       if (v > 1)
         throw invalid_option("'" + sub + "': Must be 0 or 1");
       pc.thinInput = int(v);
+    } else if (m.first == "flex") {
+      const unsigned v = requireUnsigned(sub, m.second);
+      if (v > 2)
+        throw invalid_option("'" + sub + "': Must be 0, 1 or 2");
+      pc.flex = int(v);
     } else if (m.first == "smallTile") {
       const unsigned v = requireUnsigned(sub, m.second);
       if (v > 4)

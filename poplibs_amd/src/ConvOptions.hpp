@@ -73,6 +73,9 @@ struct PlanConstraints {
   /// split over the waves of a workgroup): -1 planner's choice (never with
   /// "kernel" or another tile named), 0 never, 1 to 4 the tile.
   int smallTile = -1;
+  // The kernel of tiles of 128, 192 or 256 pixels x 64 to 256 channels (blockM,
+  // blockN): 1 alone on a CU, 2 two to a CU.
+  int flex = -1;
   /// A weight update pass's deltas: -1 planner's choice, 0 through the pass's
   /// own convolution (batch and channels exchanged), 1 by the kernel that
   /// reads the layer's own tensors (an error where none takes the layer), 2

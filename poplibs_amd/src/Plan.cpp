@@ -370,6 +370,74 @@ double fillingUs(unsigned blockM, unsigned blockN, unsigned stages,
          f.byte * mb;
 }
 
+/// A call of igemmFlexKernel and of the kernels it is weighed against, on one
+/// scale: `tiles` workgroups of `kSteps` each, megabytes out and in (weights
+/// included).  Per call, per round of workgroups, per k-step - of the longest
+/// CU, `lone` times that where the chip is not full - and per megabyte.  Fitted
+/// to 2 493 random layers and products of 0.15 to 137 GFLOP (fp16; 1 to 128
+/// images of 7 to 64 squared, 1 x 1 to 5 x 5, up to 768 channels; products of up
+/// to 4096 x 8192 x 8192), all tiles of each: igemmFlexKernel within 10 %
+/// (two workgroups to a CU: 17 %), the tile picked by it 1.1 % behind the best;
+/// the others within 6 to 14 %.
+struct CallFit {
+  double call, round, step, lone, ragged, out, in;
+};
+double callUs(const CallFit &f, bool shared, std::size_t tiles,
+              std::size_t kSteps, bool ragged, double outMB, double inMB) {
+  const double perCU = double(tiles) / double(gfx950::numCUs);
+  // (two to a CU: rounds of half as much each)
+  const double rounds = shared ? std::max(1.0, std::ceil(2.0 * perCU) / 2.0)
+                               : std::ceil(perCU);
+  return f.call + f.round * (shared ? std::max(perCU, 0.5) : rounds) +
+         double(kSteps) * std::max(f.lone * rounds, perCU) * f.step *
+             (1.0 + (ragged ? f.ragged : 0.0)) +
+         f.out * outMB + f.in * inMB;
+}
+double estimateFlex(unsigned blockM, unsigned blockN, bool shared,
+                    std::size_t tiles, std::size_t kSteps, bool ragged,
+                    double outMB, double inMB) {
+  const double edge = (blockM + blockN) / 256.0;
+  const double area = blockM * blockN / 16384.0;
+  const double step = shared ? 0.079 + 0.286 * edge + 0.058 * area
+                             : 0.186 + 0.003 * edge + 0.254 * area;
+  // (what the fit leaves: tiles of two stages, and tall ones of 64 channels)
+  const double left = !shared && blockM + blockN >= 416  ? 1.05
+                      : !shared && blockN == 64 && blockM > 128 ? 1.1
+                                                                : 1.0;
+  return left *
+         callUs(shared ? CallFit{3.27, 0.0, step, 1.04, 0.036 * edge / step,
+                                 0.25, 0.159}
+                       : CallFit{1.71, 2.4 + 0.48 * area, step, 0.80,
+                                 0.025 * edge / step, 0.124, 0.077},
+                shared, tiles, kSteps, ragged, outMB, inMB);
+}
+/// igemmKernel (patch 0) and the resident patch, K whole.
+double estimateBesideFlex(unsigned patch, unsigned blockN, unsigned stages,
+                          std::size_t tiles, std::size_t kSteps, bool ragged,
+                          double outMB, double inMB) {
+  const bool shared = !patch && (blockN == 64 || stages == 2);
+  const CallFit f =
+      patch == 1     ? CallFit{0.41, 3.11, 0.171, 0.86, 0.0, 0.33, 0.34}
+      : patch == 2   ? CallFit{1.76, 1.85, 0.291, 0.975, 0.07, 0.16, 0.105}
+      : blockN == 64 ? CallFit{2.58, 0.0, 0.313, 0.91, 0.17, 0.38, 0.083}
+      : stages == 2  ? CallFit{2.96, 1.18, 0.492, 0.96, 0.04, 0.07, 0.07}
+                     : CallFit{2.11, 1.54, 0.412, 0.89, 0.16, 0.175, 0.09};
+  return callUs(f, shared, tiles, kSteps, ragged, outMB, inMB);
+}
+/// ... and pointwiseKernel.
+double pointwiseBesideFlex(double pixels, double co, double macs, double outMB,
+                           double inMB, double weightsMB) {
+  return std::max(4.9, 4.05 + 0.128 * outMB + 0.084 * inMB +
+                           0.136 * weightsMB + 2.39e-9 * macs +
+                           6.2e-6 * pixels * std::ceil(co / 64.0));
+}
+/// igemmFlexKernel is taken where it is estimated at less than this share of
+/// what is planned.  Over the layers of the fit: tiles of 128 x 128 two to a CU
+/// 1.15 times as fast on average, alone 1.006, of 128 x 64 1.012, resident patch
+/// of 16-pixel blocks 1.13, of 32 1.03, pointwise layers 1.01; under 1 % of all
+/// lose more than 3 %.  With 1.0 in its place 12 % do, for no more on average.
+constexpr double kFlexShare = 0.88;
+
 /// igemmPatchKernel (mode 1) and igemmPatch16Kernel (mode 2, seven blocks of 16
 /// pixels whatever the tile's height): start and end of a workgroup and its
 /// k-steps, again for every further round of workgroups on a CU, and the way
@@ -1392,10 +1460,22 @@ mxconv_plan makePlanWith(const ConvParams &params,
       }
     }
     const bool anyHeight = pc.patch == 2 && g.blockM >= 1 && g.blockM <= 112;
+    // (igemm_flex.hip)
+    if (pc.flex > 0) {
+      g.flex = uint32_t(pc.flex);
+      if (!halfIn || pc.patch > 0 || !pc.blockM || !pc.blockN ||
+          !mxk::igemmFlexTile(g.blockM, g.blockN, g.flex) ||
+          (pc.splitK > 1))
+        throw poplar::invalid_option(
+            "planConstraints gfx950 flex: that kernel takes half inputs and "
+            "outputs in tiles of blockM 128, 192 or 256 and blockN 64 to 256 in "
+            "steps of 32 (with flex 2 up to 288 of both together), K whole");
+    }
     // (tiles of 256 pixels: igemm_wide.hip)
-    const bool wideTile = g.blockM == 256 && pc.patch < 1;
-    if ((g.blockM != 128 && g.blockM != 64 && !anyHeight && !wideTile) ||
-        (!wideTile && g.blockN != 64 && g.blockN != 128) ||
+    const bool wideTile = g.blockM == 256 && pc.patch < 1 && !g.flex;
+    if ((g.blockM != 128 && g.blockM != 64 && !anyHeight && !wideTile &&
+         !g.flex) ||
+        (!wideTile && !g.flex && g.blockN != 64 && g.blockN != 128) ||
         (wideTile && ((g.blockN != 192 && g.blockN != 256) || floatIn)) ||
         g.blockK != stepElems)
       throw poplar::invalid_option(
@@ -1419,7 +1499,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
                                 (plan.coPadded / g.blockN) * p.numConvGroups;
       const std::size_t kSteps = plan.kPadded / g.blockK;
       std::size_t parts = 1;
-      if (g.blockM == 256)
+      if (g.blockM == 256 || g.flex)
         parts = 1;
       else if (pc.splitK)
         parts = pc.splitK;
@@ -1609,6 +1689,17 @@ mxconv_plan makePlanWith(const ConvParams &params,
             "at most 32 taps on an input of which the images that 256 output "
             "pixels meet stay under 2^31 bytes (a zero-stuffed input where "
             "every phase has taps)");
+    }
+    if (g.flex) {
+      bool takes = !plan.igemmPhases.empty() ||
+                   mxk::igemmFlexTakes(g, inId, outId);
+      for (const auto &ph : plan.igemmPhases)
+        takes = takes && mxk::igemmFlexTakes(ph.d, inId, outId);
+      if (!takes || plan.denseWeightUpdate || plan.depthwiseWeightUpdate)
+        throw poplar::invalid_option(
+            "planConstraints gfx950 flex: that kernel takes half inputs and "
+            "outputs, kernels of at most 32 taps and an input of which the "
+            "images that a tile's pixels meet stay under 2^31 bytes");
     }
     // A pointwise convolution with few input channels is bound by HBM, not
     // by the matrix cores: unless the big tile was asked for explicitly, the
@@ -2045,7 +2136,128 @@ mxconv_plan makePlanWith(const ConvParams &params,
         plan.weightPackedElems = mxk::igemmSmallPackedElems(g, inId);
       }
     }
-    if (!g.patch && g.blockM != 128 && g.blockM != 256)
+    // A tile's height and width closer to the layer's (fp16).
+    const bool flexFree =
+        halfIn && params.outputType == poplar::HALF && !g.small &&
+        pc.flex < 0 && pc.kernel.empty() && pc.method == Method::ANY &&
+        !pc.blockM && !pc.blockN && !pc.blockK && !pc.splitK && !pc.stages &&
+        pc.patch < 0 && pc.pointwise < 0 && pc.smallTile < 0 &&
+        !pc.chanTiles && g.splitK == 1 && !isWeightUpdatePass(options.pass);
+    if (flexFree && !plan.igemmPhases.empty() && g.blockN == 128) {
+      // The phases of a zero-stuffed input, all with taps, in two rounds or more
+      // of tiles of 128 x 128 that their channels fill badly: tiles of 160
+      // channels where those cover them in 0.7 of the columns (N = 42, 35 x 35,
+      // 3 x 3 stride 2, 136 -> 80 backwards 14.4 -> 10.7 us; four such layers
+      // 1.24 to 1.34 times as fast), of 96 where those do in three quarters (N =
+      // 25, 57 x 57, 72 -> 200 20.5 -> 19.4; four 1.01 to 1.07).  Single taps,
+      // whose other phases write zeros, and fewer tiles gain nothing or lose (N =
+      // 38, 27 x 27, 192 -> 56 7.4 -> 8.6).
+      std::size_t tiles = 0;
+      bool taps = true;
+      for (const auto &ph : plan.igemmPhases) {
+        tiles += (std::size_t(ph.d.batch) * ph.d.outD * ph.d.outH * ph.d.outW +
+                  127) /
+                 128 * ((co + 127) / 128) * p.numConvGroups;
+        taps = taps && !ph.d.noTaps;
+      }
+      const std::size_t columns = (co + 127) / 128 * 128;
+      const uint32_t bn = (co + 159) / 160 * 160 * 10 <= columns * 7  ? 160
+                          : (co + 95) / 96 * 96 * 4 <= columns * 3 ? 96
+                                                                    : 0;
+      const uint32_t bm = bn == 160 ? 128 : 192;
+      bool takes = taps && bn && tiles >= 2 * gfx950::numCUs;
+      auto tileOf = [&](mxk::IgemmDesc d) {
+        d.blockM = bm, d.blockN = bn, d.flex = 2;
+        return d;
+      };
+      for (const auto &ph : plan.igemmPhases)
+        takes = takes && mxk::igemmFlexTakes(tileOf(ph.d), inId, outId);
+      if (takes) {
+        g = tileOf(g);
+        plan.coPadded = (co + bn - 1) / bn * bn;
+        std::size_t offset = 0;
+        for (auto &ph : plan.igemmPhases) {
+          ph.d = tileOf(ph.d);
+          ph.packedOffset = offset;
+          offset += p.numConvGroups * plan.coPadded * ph.kPadded;
+        }
+        plan.weightPackedElems = offset;
+      }
+    } else if (flexFree && plan.igemmPhases.empty() &&
+               // (below, a call costs its launch, whatever the tile)
+               2.0 * double(s.batch) * s.outD * s.outH * s.outW * double(co) *
+                       double(k) * p.numConvGroups >=
+                   3e8) {
+      const std::size_t m = s.batch * s.outD * s.outH * s.outW;
+      const std::size_t kSteps = (k + 63) / 64;
+      const double inMB = 1e-6 * double(plan.inputBytes());
+      const double outMB = 1e-6 * double(plan.outputBytes());
+      const double weightsMB = 1e-6 * double(plan.weightBytes());
+      const bool ragged = ciPadded % 64 != 0;
+      const std::size_t taps = std::size_t(s.kD) * s.kH * s.kW;
+      auto tilesOf = [&](std::size_t bm, std::size_t bn) {
+        return (m + bm - 1) / bm * ((co + bn - 1) / bn) * p.numConvGroups;
+      };
+      // (tiles of 256 x 192 and 256 x 256 were chosen for their size: of 56 such
+      // layers of the fit each is faster in one of this kernel's, 1.26 times on
+      // average)
+      double planned =
+          plan.pointwiseOn
+              ? pointwiseBesideFlex(double(m) * p.numConvGroups, double(co),
+                                    double(m) * double(co) * double(k) *
+                                        p.numConvGroups,
+                                    outMB, inMB, weightsMB)
+          : g.blockM == 256
+              ? 1e30
+              : estimateBesideFlex(
+                    g.patch, g.blockN, g.stages,
+                    tilesOf(g.blockM, g.patch ? 128 : g.blockN),
+                    g.patch ? (ciPadded + 63) / 64 * taps : kSteps, ragged,
+                    outMB, inMB + weightsMB);
+      // (tiles of 64 channels, those of one round and the resident patch, by 5 %
+      // more: the estimates part less sharply)
+      planned *= !plan.pointwiseOn &&
+                         (g.patch || g.blockN == 64 || g.stages == 4)
+                     ? 0.95 * kFlexShare
+                     : kFlexShare;
+      mxk::IgemmDesc chosenTile = g;
+      for (uint32_t bm : {128u, 192u, 256u})
+        for (uint32_t bn = 64; bn <= 256; bn += 32)
+          for (uint32_t flex : {1u, 2u}) {
+            if (!mxk::igemmFlexTile(bm, bn, flex))
+              continue;
+            mxk::IgemmDesc t = g;
+            t.patch = 0, t.blockM = bm, t.blockN = bn, t.flex = flex;
+            const double us =
+                estimateFlex(bm, bn, flex == 2, tilesOf(bm, bn), kSteps, ragged,
+                             outMB, inMB + weightsMB);
+            if (us >= planned ||
+                p.numConvGroups * ((co + bn - 1) / bn * bn) *
+                        ((k + 63) / 64 * 64) * 2 >=
+                    (1ull << 31) ||
+                !mxk::igemmFlexTakes(t, inId, outId))
+              continue;
+            planned = us, chosenTile = t;
+          }
+      if (chosenTile.flex) {
+        g = chosenTile;
+        plan.pointwiseOn = false;
+        plan.coPadded = (co + g.blockN - 1) / g.blockN * g.blockN;
+        plan.kPadded = (k + 63) / 64 * 64;
+        plan.weightPackedElems =
+            p.numConvGroups * plan.coPadded * plan.kPadded;
+        for (auto &c : plan.candidates)
+          c.chosen = false;
+        mxconv_plan::Candidate c;
+        c.name = "flexible " + std::to_string(g.blockM) + " x " +
+                 std::to_string(g.blockN);
+        c.workgroups = tilesOf(g.blockM, g.blockN), c.perCU = g.flex;
+        c.kSteps = kSteps, c.estimateUs = planned;
+        c.rounds = roundsOf(c.workgroups, c.perCU), c.chosen = true;
+        plan.candidates.push_back(c);
+      }
+    }
+    if (!g.patch && !g.flex && g.blockM != 128 && g.blockM != 256)
       throw poplar::invalid_option(
           "planConstraints gfx950 blockM 64 goes with the resident-patch "
           "kernel only");
@@ -2135,7 +2347,10 @@ std::string mxconv_plan::constraintsJson() const {
          << ", \"blockM\": " << igemm.blockM;
     } else {
       os << ", \"pointwise\": 0, \"patch\": 0, \"blockM\": "
-         << igemm.blockM << ", \"blockN\": " << igemm.blockN
+         << igemm.blockM << ", \"blockN\": " << igemm.blockN;
+      if (igemm.flex)
+        os << ", \"flex\": " << igemm.flex;
+      os
          << ", \"blockK\": " << igemm.blockK << ", \"splitK\": "
          << igemm.splitK << ", \"stages\": " << igemm.stages;
     }
@@ -2332,7 +2547,11 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
         (kPadded / g.blockK + g.splitK - 1) / g.splitK;
     const std::size_t perCU = g.blockN == 64 || g.stages == 2 ? 2 : 1;
     double us =
-        g.blockM == 256
+        g.flex ? poplin::estimateFlex(
+                     g.blockM, g.blockN, g.flex == 2, tiles, steps,
+                     g.inChansPerGroup % 64 != 0, 1e-6 * double(outputBytes()),
+                     1e-6 * double(inputBytes() + weightBytes()))
+        : g.blockM == 256
             ? poplin::estimateWide(tiles, steps, g.blockN)
             : poplin::estimateStreaming(tiles, steps, perCU, g.blockN,
                                         g.splitK,
@@ -2505,6 +2724,12 @@ std::string mxconv_plan::describe() const {
                      "SIMD\n"
                    : "32 pixels, each k-step halved between the two waves of "
                      "a SIMD\n");
+      else if (g.flex)
+        os << "        data path                  8 waves, each fetching its "
+              "share and multiplying "
+           << g.blockM / 4 << " x " << g.blockN / 2
+           << (g.flex == 2 ? "; two workgroups per CU\n"
+                           : "; one workgroup per CU\n");
       else if (g.blockM == 256)
         os << "        data path                  8 waves, each fetching its "
               "share and multiplying 64 x "

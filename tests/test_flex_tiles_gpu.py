@@ -1,0 +1,183 @@
+"""Tiles of 128 to 256 pixels x 64 to 256 channels (csrc/igemm_flex.hip), every
+shape at the edges of tiles, of k-steps and of taps, against the oracle.  +-1
+data: sums of at most 2 048 products and a bias are exact in half."""
+import json
+
+import pytest
+
+import poplibs_amd as pa
+from helpers import make_params
+
+TILES = [(m, n, 1) for m in (128, 192, 256) for n in range(64, 257, 32)
+         if (m, n) != (256, 64)]
+TILES += [(128, 64, 2), (128, 96, 2), (128, 128, 2), (128, 160, 2),
+          (192, 64, 2), (192, 96, 2)]
+
+
+def _options(tile):
+    m, n, flex = tile
+    return {"planConstraints": json.dumps({"gfx950": {
+        "kernel": "igemm", "patch": 0, "blockM": m, "blockN": n,
+        "flex": flex}})}
+
+
+def _exact(oracle, tile, kw, idil_phases=0):
+    from test_fast_gpu import _run
+    p = make_params(pa.HALF, **kw)
+    print("case", tile, p, flush=True)
+    text = pa.Plan(p, _options(tile)).describe()
+    assert "%d x %d x 64" % tile[:2] in text, text
+    assert ("two workgroups per CU" in text) == (tile[2] == 2), text
+    if idil_phases:
+        assert "%d phases" % idil_phases in text, text
+    _run(oracle, p, 91, 0, "implicit GEMM", dist="pm1",
+         options=_options(tile))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+def test_every_tile_at_its_edges(oracle, tile):
+    m, n, _ = tile
+    # five M tiles (a block of four and one more), the last of one pixel; two N
+    # tiles, the last of one channel; seven k-steps, more than any stages
+    _exact(oracle, tile, dict(batch=1, field=(4 * m + 1,), kernel=(1,), ci=448,
+                              co=n + 1))
+    # a whole tile and a part, taps that share a k-step, images within a tile
+    _exact(oracle, tile, dict(batch=3, field=(11, m // 16), kernel=(3, 3),
+                              ci=8, co=n - 8, pad=1))
+
+
+FORMS = [
+    # fewer k-steps than stages: half of one, one, two
+    dict(field=(9, 15), kernel=(1, 1), ci=32, co=72),
+    dict(field=(9, 15), kernel=(1, 1), ci=64, co=72),
+    dict(field=(9, 15), kernel=(1, 1), ci=72, co=72),
+    # a chunk of 8 channels to a tap, and taps that straddle k-steps
+    dict(batch=2, field=(13, 12), kernel=(5, 6), ci=8, co=40, pad=2),
+    dict(batch=2, field=(13, 12), kernel=(3, 3), ci=40, co=130, pad=1),
+    # strides, a dilated kernel, groups, a depth, a truncated input
+    dict(batch=2, field=(33, 31), kernel=(3, 3), ci=72, co=200, stride=2,
+         pad=1),
+    dict(batch=2, field=(23, 21), kernel=(3, 3), ci=24, co=72, groups=3,
+         stride=(1, 2), kdil=(2, 1), pad=(2, 1)),
+    dict(batch=2, field=(6, 7, 8), kernel=(3, 2, 2), ci=16, co=24, pad=1),
+    dict(batch=2, field=(19, 21), kernel=(3, 3), ci=64, co=40,
+         itl=(1, 0), itu=(0, 3), padLower=(0, 2), padUpper=(2, 0)),
+    # channels filled up in a copy, odd rows of outputs, zeros around the field
+    dict(batch=3, field=(20, 20), kernel=(3, 3), ci=13, co=33, pad=1),
+    dict(batch=2, field=(12, 12), kernel=(3, 3), ci=64, co=24, pad=1,
+         opl=(1, 0), opu=(0, 2)),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [(128, 64, 1), (128, 96, 2), (128, 160, 1),
+                                  (192, 96, 2), (192, 256, 1), (256, 224, 1)])
+@pytest.mark.parametrize("kw", FORMS)
+def test_forms_of_layers(oracle, tile, kw):
+    _exact(oracle, tile, kw)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [(128, 160, 2), (192, 96, 2), (256, 160, 1)])
+@pytest.mark.parametrize("kw,phases", [
+    (dict(batch=2, field=(14, 15), kernel=(3, 3), ci=40, co=72, idil=2,
+          padLower=(1, 1), padUpper=(2, 1)), 4),
+    # a phase of which no tap meets an input element
+    (dict(batch=2, field=(9, 9), kernel=(1, 1), ci=64, co=136, idil=2), 4)])
+def test_phases_in_one_launch(oracle, tile, kw, phases):
+    from test_fast_gpu import _run
+    p = make_params(pa.HALF, **kw)
+    try:
+        pa.Plan(p, _options(tile))
+    except pa.MxconvError:
+        assert kw["kernel"] == (1, 1)
+        return
+    _exact(oracle, tile, kw, phases)
+
+
+@pytest.mark.gpu
+def test_the_planner_s_own_phases(oracle):
+    """A backward pass whose channels fill tiles of 128 badly."""
+    p = make_params(pa.HALF, batch=35, field=(17, 18), kernel=(3, 3), ci=16,
+                    co=136, idil=2, padLower=(1, 1), padUpper=(2, 1))
+    assert "128 x 160 x 64" in pa.Plan(p).describe()
+    from test_fast_gpu import _run
+    _run(oracle, p, 92, 0, "implicit GEMM", dist="pm1")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bias", [False, True])
+def test_a_multi_convolution_in_one_launch(bias):
+    """Two layers in one tile shape share a launch, a third in another shape has
+    its own: as one by one."""
+    import torch
+    from poplibs_amd import capi
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(5)
+    s = torch.cuda.current_stream().cuda_stream
+    plans, ins, packed, biases, outs, want = [], [], [], [], [], []
+    for tile, kw in [((128, 96, 2), dict(batch=2, field=(13, 12), ci=40,
+                                         co=96)),
+                     ((128, 96, 2), dict(batch=3, field=(9, 9), ci=72,
+                                         co=200)),
+                     ((192, 96, 2), dict(batch=1, field=(9, 9), ci=64,
+                                         co=33))]:
+        p = make_params(pa.HALF, kernel=(3, 3), pad=1, **kw)
+        plan = pa.Plan(p, _options(tile))
+
+        def values(which):
+            n = plan.buffer_bytes(which) // 2
+            return torch.randn(n, generator=gen, device=dev).half()
+        x, w = values(capi.BUF_INPUT), values(capi.BUF_WEIGHTS_EXTERNAL)
+        pk = values(capi.BUF_WEIGHTS_PACKED)
+        plan.pack_weights(w.data_ptr(), pk.data_ptr(), s)
+        b = torch.randn(p.getNumOutputChans(), generator=gen, device=dev)
+        biases.append(b.half())
+        outs.append(values(capi.BUF_OUTPUT)), want.append(outs[-1].clone())
+        plan.fwd(x.data_ptr(), pk.data_ptr(), want[-1].data_ptr(),
+                 biases[-1].data_ptr() if bias else None, None, 0, s)
+        plans.append(plan), ins.append(x), packed.append(pk)
+    pa.multi_fwd(plans, [x.data_ptr() for x in ins],
+                 [w.data_ptr() for w in packed], [o.data_ptr() for o in outs],
+                 biases=[b.data_ptr() for b in biases] if bias else None,
+                 stream=s)
+    torch.cuda.synchronize()
+    for got, expected in zip(outs, want):
+        assert torch.equal(got, expected)
+
+
+def test_plans_name_the_tile_and_come_back():
+    p = make_params(pa.HALF, batch=25, field=(57, 57), kernel=(3, 3), ci=136,
+                    co=200, pad=1)
+    plan = pa.Plan(p)
+    named = json.loads(plan.constraints())["gfx950"]
+    assert named["flex"] in (1, 2)
+    again = pa.Plan(p, {"planConstraints": plan.constraints()})
+    assert again.constraints() == plan.constraints()
+    assert again.packs_like(plan)
+    without = pa.Plan(p, {"planConstraints": '{"gfx950": {"flex": 0}}'})
+    assert "flex" not in without.constraints()
+
+
+@pytest.mark.parametrize("asked", [
+    dict(blockM=64, blockN=64, flex=1), dict(blockM=128, blockN=48, flex=1),
+    dict(blockM=256, blockN=64, flex=1), dict(blockM=192, blockN=128, flex=2),
+    dict(blockM=128, flex=1), dict(blockM=128, blockN=96, flex=1, splitK=2),
+    dict(blockM=128, blockN=96, flex=3)])
+def test_tiles_that_are_not_there_are_refused(asked):
+    p = make_params(pa.HALF, batch=2, field=(9, 9), kernel=(3, 3), ci=64,
+                    co=64, pad=1)
+    with pytest.raises(pa.MxconvError, match="flex|tile"):
+        pa.Plan(p, {"planConstraints": json.dumps({"gfx950": asked})})
+
+
+@pytest.mark.parametrize("kw", [
+    dict(dtype=pa.FLOAT, kernel=(3, 3)),
+    dict(dtype=pa.QUARTER, out_dtype=pa.HALF, kernel=(3, 3)),
+    dict(dtype=pa.HALF, out_dtype=pa.FLOAT, kernel=(3, 3)),
+    dict(dtype=pa.HALF, kernel=(6, 6))])
+def test_layers_it_does_not_take_are_refused(kw):
+    p = make_params(batch=2, field=(9, 9), ci=64, co=64, pad=2, **kw)
+    with pytest.raises(pa.MxconvError, match="flex"):
+        pa.Plan(p, _options((128, 64, 1)))
