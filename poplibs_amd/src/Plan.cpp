@@ -396,19 +396,20 @@ double callUs(const CallFit &f, bool shared, std::size_t tiles,
 double estimateFlex(unsigned blockM, unsigned blockN, bool shared,
                     std::size_t tiles, std::size_t kSteps, bool ragged,
                     double outMB, double inMB) {
-  const double edge = (blockM + blockN) / 256.0;
+  // (odd multiples of 32 channels load as many rows as the next even one; two
+  // stages, and 64 channels under a tall tile, cost a step more)
+  const double edge = (blockM + (blockN + 63) / 64 * 64) / 256.0;
   const double area = blockM * blockN / 16384.0;
-  const double step = shared ? 0.079 + 0.286 * edge + 0.058 * area
-                             : 0.186 + 0.003 * edge + 0.254 * area;
-  // (what the fit leaves: tiles of two stages, and tall ones of 64 channels)
-  const double left = !shared && blockM + blockN >= 416  ? 1.05
-                      : !shared && blockN == 64 && blockM > 128 ? 1.1
-                                                                : 1.0;
-  return left *
-         callUs(shared ? CallFit{3.27, 0.0, step, 1.04, 0.036 * edge / step,
+  const double base = shared ? 0.127 + 0.225 * edge + 0.063 * area
+                             : 0.167 + 0.073 * edge + 0.189 * area;
+  const double more = shared                             ? 1.0
+                      : blockM + blockN >= 416           ? 1.15
+                      : blockN == 64 && blockM > 128 ? 1.10
+                                                         : 1.0;
+  return callUs(shared ? CallFit{3.26, 0.0, base, 1.015, 0.035 * edge / base,
                                  0.25, 0.159}
-                       : CallFit{1.71, 2.4 + 0.48 * area, step, 0.80,
-                                 0.025 * edge / step, 0.124, 0.077},
+                       : CallFit{1.75, 2.37 + 0.45 * area, more * base, 0.80,
+                                 0.024 * edge / base, 0.129, 0.078},
                 shared, tiles, kSteps, ragged, outMB, inMB);
 }
 /// igemmKernel (patch 0) and the resident patch, K whole.
@@ -417,26 +418,31 @@ double estimateBesideFlex(unsigned patch, unsigned blockN, unsigned stages,
                           double outMB, double inMB) {
   const bool shared = !patch && (blockN == 64 || stages == 2);
   const CallFit f =
-      patch == 1     ? CallFit{0.41, 3.11, 0.171, 0.86, 0.0, 0.33, 0.34}
-      : patch == 2   ? CallFit{1.76, 1.85, 0.291, 0.975, 0.07, 0.16, 0.105}
+      patch == 1     ? CallFit{0.52, 2.98, 0.172, 0.86, 0.0, 0.34, 0.34}
+      : patch == 2   ? CallFit{1.74, 1.92, 0.291, 0.97, 0.07, 0.15, 0.104}
       : blockN == 64 ? CallFit{2.58, 0.0, 0.313, 0.91, 0.17, 0.38, 0.083}
-      : stages == 2  ? CallFit{2.96, 1.18, 0.492, 0.96, 0.04, 0.07, 0.07}
-                     : CallFit{2.11, 1.54, 0.412, 0.89, 0.16, 0.175, 0.09};
+      : stages == 2  ? CallFit{2.98, 0.99, 0.492, 0.96, 0.04, 0.095, 0.07}
+                     : CallFit{2.02, 1.63, 0.412, 0.89, 0.16, 0.175, 0.09};
   return callUs(f, shared, tiles, kSteps, ragged, outMB, inMB);
 }
 /// ... and pointwiseKernel.
 double pointwiseBesideFlex(double pixels, double co, double macs, double outMB,
                            double inMB, double weightsMB) {
-  return std::max(4.9, 4.05 + 0.128 * outMB + 0.084 * inMB +
-                           0.136 * weightsMB + 2.39e-9 * macs +
-                           6.2e-6 * pixels * std::ceil(co / 64.0));
+  return std::max(4.9, 4.14 + 0.02 * outMB + 0.083 * inMB +
+                           0.112 * weightsMB + 2.51e-9 * macs +
+                           7.95e-6 * pixels * std::ceil(co / 64.0));
 }
-/// igemmFlexKernel is taken where it is estimated at less than this share of
-/// what is planned.  Over the layers of the fit: tiles of 128 x 128 two to a CU
-/// 1.15 times as fast on average, alone 1.006, of 128 x 64 1.012, resident patch
-/// of 16-pixel blocks 1.13, of 32 1.03, pointwise layers 1.01; under 1 % of all
-/// lose more than 3 %.  With 1.0 in its place 12 % do, for no more on average.
-constexpr double kFlexShare = 0.88;
+/// igemmFlexKernel is taken where it is estimated at less than these shares of
+/// what is planned.  Over the layers of the fit, at the share and (in brackets)
+/// wherever the estimate is lower at all: tiles of 128 x 128, two to a CU, 1.155
+/// times as fast on average (1.17), one round of them 1.0075 (under 1), of 128 x
+/// 64 1.013 (1.01), resident patch of 16-pixel blocks 1.13 (1.15), of 32 1.03,
+/// pointwise layers 1.014 (1.02, one in seven slower); at the share 7 of 1 400 are
+/// slower by more than 3 %, the worst 0.85 times as fast, in brackets 190.
+double flexShare(bool pointwise, unsigned patch, unsigned blockN,
+                 unsigned stages) {
+  return pointwise ? 0.9 : patch ? 0.82 : blockN == 64 || stages == 4 ? 0.85 : 0.88;
+}
 
 /// igemmPatchKernel (mode 1) and igemmPatch16Kernel (mode 2, seven blocks of 16
 /// pixels whatever the tile's height): start and end of a workgroup and its
@@ -2184,6 +2190,11 @@ mxconv_plan makePlanWith(const ConvParams &params,
         plan.weightPackedElems = offset;
       }
     } else if (flexFree && plan.igemmPhases.empty() &&
+               // (the resident patch and the pointwise kernel fetch a group's
+               // channels, a piece of every pixel, once, not once per tap and
+               // tile: 190 x 15 x 15, 5 x 5, 4 groups of 720 -> 80 532 us, 799 in
+               // tiles of 256 x 96)
+               (p.numConvGroups == 1 || (!g.patch && !plan.pointwiseOn)) &&
                // (below, a call costs its launch, whatever the tile)
                2.0 * double(s.batch) * s.outD * s.outH * s.outW * double(co) *
                        double(k) * p.numConvGroups >=
@@ -2198,33 +2209,36 @@ mxconv_plan makePlanWith(const ConvParams &params,
       auto tilesOf = [&](std::size_t bm, std::size_t bn) {
         return (m + bm - 1) / bm * ((co + bn - 1) / bn) * p.numConvGroups;
       };
-      // (tiles of 256 x 192 and 256 x 256 were chosen for their size: of 56 such
-      // layers of the fit each is faster in one of this kernel's, 1.26 times on
-      // average)
       double planned =
           plan.pointwiseOn
               ? pointwiseBesideFlex(double(m) * p.numConvGroups, double(co),
-                                    double(m) * double(co) * double(k) *
+                                    double(m) * double(co) *
+                                        double((k + 127) / 128 * 128) *
                                         p.numConvGroups,
                                     outMB, inMB, weightsMB)
-          : g.blockM == 256
-              ? 1e30
               : estimateBesideFlex(
                     g.patch, g.blockN, g.stages,
                     tilesOf(g.blockM, g.patch ? 128 : g.blockN),
                     g.patch ? (ciPadded + 63) / 64 * taps : kSteps, ragged,
                     outMB, inMB + weightsMB);
-      // (tiles of 64 channels, those of one round and the resident patch, by 5 %
-      // more: the estimates part less sharply)
-      planned *= !plan.pointwiseOn &&
-                         (g.patch || g.blockN == 64 || g.stages == 4)
-                     ? 0.95 * kFlexShare
-                     : kFlexShare;
+      planned *= flexShare(plan.pointwiseOn, g.patch, g.blockN, g.stages);
       mxk::IgemmDesc chosenTile = g;
+      // (Tiles of 256 x 192 and 256 x 256 were chosen for their size: this
+      // kernel's of the same shape are faster for each of 56 such layers of the
+      // fit, 4096 x 4096 x 4096 118 -> 105 us.  Others have to be 8 % below: 2320 x
+      // 10111 x 12070 500 us in 256 x 256 tiles of either, 568 in 192 x 192.)
+      if (!plan.pointwiseOn && !g.patch && g.blockM == 256) {
+        chosenTile.flex = 1;
+        planned = 0.92 * estimateFlex(256, g.blockN, false,
+                                      tilesOf(256, g.blockN), kSteps, ragged,
+                                      outMB, inMB + weightsMB);
+        if (!mxk::igemmFlexTakes(chosenTile, inId, outId))
+          chosenTile = g, planned = 0.0;
+      }
       for (uint32_t bm : {128u, 192u, 256u})
         for (uint32_t bn = 64; bn <= 256; bn += 32)
           for (uint32_t flex : {1u, 2u}) {
-            if (!mxk::igemmFlexTile(bm, bn, flex))
+            if (!mxk::igemmFlexTile(bm, bn, flex) || (bn > 64 && co <= 64))
               continue;
             mxk::IgemmDesc t = g;
             t.patch = 0, t.blockM = bm, t.blockN = bn, t.flex = flex;
