@@ -996,8 +996,13 @@ hipError_t launchIgemm(const IgemmDesc &d, int inType, int outType,
   const bool split = d.blockM != 256 && d.splitK != 1;
   a.outThrough = throughBytes(a, split ? int(kFloat) : outType,
                                split ? workspace : out);
-  if (d.flex)
-    return launchIgemmFlex(a, in, weightsPacked, bias, out, stream);
+  if (d.flex) {
+    e = launchIgemmFlex(a, in, weightsPacked, bias,
+                        d.splitK == 1 ? out : workspace, stream);
+    return e != hipSuccess || d.splitK == 1
+               ? e
+               : launchSplitKSum(d, outType, workspace, bias, out, stream);
+  }
   if (d.blockM == 256)
     return launchIgemmWide(a, inType, outType, in, weightsPacked, bias, out, q,
                            stream);
@@ -1039,8 +1044,8 @@ hipError_t launchSplitKSum(const IgemmDesc &d, int outType,
 bool igemmFusable(const IgemmFusedItem &x, const IgemmFusedItem &y) {
   if (x.d->flex || y.d->flex)
     return x.d->flex == y.d->flex && x.d->blockM == y.d->blockM &&
-           x.d->blockN == y.d->blockN &&
-           igemmFlexTakes(*x.d, x.inType, x.outType) &&
+           x.d->blockN == y.d->blockN && x.d->splitK == 1 &&
+           y.d->splitK == 1 && igemmFlexTakes(*x.d, x.inType, x.outType) &&
            igemmFlexTakes(*y.d, y.inType, y.outType);
   return x.d->splitK == 1 && y.d->splitK == 1 &&
          x.d->blockM == kBlockM && y.d->blockM == kBlockM &&

@@ -62,8 +62,9 @@ __device__ __forceinline__ uint16_t loadHalf(__amdgpu_buffer_rsrc_t from,
 #endif
 }
 
-/// AHEAD: operands are read a whole k-step ahead.
-template <int MB, int NB, int NS, bool AHEAD, class OutT>
+/// AHEAD: operands are read a whole k-step ahead.  SPLIT: one part of K, whose
+/// fp32 sums go to a workspace [part][pixel][channel], without a bias.
+template <int MB, int NB, int NS, bool AHEAD, bool SPLIT, class OutT>
 __device__ __forceinline__ void
 flexTile(const IgemmArgs &a, const char *__restrict__ in,
          const char *__restrict__ w, const OutT *__restrict__ bias,
@@ -80,10 +81,13 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wm = wave >> 1, wn = wave & 1;
 
-  // workgroup -> (group of convolution, block of M tiles, N tile, M tile)
+  // workgroup -> (part of K, group of convolution, block of M tiles, N tile, M
+  // tile)
   const uint32_t tile = xcdSwizzle(block, blocks);
-  const uint32_t g = a.divMTiles(a.divNTiles(tile));
-  const uint32_t within = tile - g * (a.mTiles * a.nTiles);
+  const uint32_t partGroup = a.divMTiles(a.divNTiles(tile));
+  const uint32_t part = SPLIT ? a.divGroups(partGroup) : 0;
+  const uint32_t g = partGroup - part * d.groups;
+  const uint32_t within = tile - partGroup * (a.mTiles * a.nTiles);
   const uint32_t mBlock = a.divWideBlock(within);
   const uint32_t inBlock = within - mBlock * (kFlexGroup * a.nTiles);
   const uint32_t mLeft = a.mTiles - mBlock * kFlexGroup;
@@ -112,11 +116,12 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
                uint32_t(left < kOutOfRange - 1 ? left : kOutOfRange - 1));
   const __amdgpu_buffer_rsrc_t wBuf = bufferOf(w, a.wBytes);
 
-  // The bias: asked for first, into LDS in front of the loop.
+  // The bias: asked for first, into LDS in front of the loop.  (The parts' sum
+  // adds it where K is split.)
   // (without a bias its buffer is empty and reads as zeros)
   const uint32_t biasChan = nTile * W + t;
   const uint16_t biasOwn = loadHalf(
-      bufferOf(bias, bias ? d.groups * d.outChansPerGroup * 2 : 0),
+      bufferOf(bias, bias && !SPLIT ? d.groups * d.outChansPerGroup * 2 : 0),
       t < W && biasChan < d.outChansPerGroup
           ? (g * d.outChansPerGroup + biasChan) * 2
           : kOutOfRange);
@@ -129,7 +134,8 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
                             a.kPadded * 2 +
                         chunk * 16;
   const uint32_t bStep = 64 * a.kPadded * 2; // 64 rows on
-  uint32_t kByte = 0;
+  const uint32_t kFirst = part * a.kSteps * kRowBytes;
+  uint32_t kByte = kFirst;
   auto loadBOne = [&](char *__restrict__ into, int r) {
     char *dst = into + (H + wave * 8 + r * 64) * kRowBytes;
     uint32_t outside = kByte < a.kPadded * 2 ? 0u : kOutOfRange;
@@ -188,8 +194,8 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
   // Where in K the input data loaded next is, this lane's own chunk of it: tap
   // and byte within the tap's channels; `place`: the two in the input, with
   // the top bit for a tap beyond the kernel.
-  uint32_t tap = a.divCiBytes(chunk * 16);
-  uint32_t ciOff = chunk * 16 - tap * ciBytes;
+  uint32_t tap = a.divCiBytes(kFirst + chunk * 16);
+  uint32_t ciOff = kFirst + chunk * 16 - tap * ciBytes;
   const uint32_t stepTaps = a.divCiBytes(kRowBytes);
   const uint32_t stepBytes = kRowBytes - stepTaps * ciBytes;
   uint32_t toTop, place;
@@ -380,6 +386,29 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
   MXK_WAIT_VMCNT(0);
   MXK_WAIT_LGKMCNT0();
 
+  const uint32_t outChans = d.groups * d.outChansPerGroup;
+  const __amdgpu_buffer_rsrc_t outBuf = bufferOf(out, a.outThrough);
+  if constexpr (SPLIT) {
+    // A lane has four consecutive channels of a pixel: 16 bytes each, 64 of a
+    // pixel side by side, straight from the registers.
+    float *own = reinterpret_cast<float *>(out) +
+                 size_t(part) * a.M * outChans + g * d.outChansPerGroup;
+    const __amdgpu_buffer_rsrc_t partBuf =
+        bufferOf(own, a.M * outChans * uint32_t(sizeof(float)));
+#pragma unroll
+    for (int i = 0; i != MB; ++i) {
+      const uint32_t m = mTile * H + (wm * MB + i) * 16 + (lane & 15);
+#pragma unroll
+      for (int j = 0; j != NB; ++j) {
+        const uint32_t n = nTile * W + (wn * NB + j) * 16 + (lane >> 4) * 4;
+        if (m < a.M && n < d.outChansPerGroup)
+          storeThrough(partBuf, (m * outChans + n) * uint32_t(sizeof(float)),
+                       __builtin_bit_cast(ThroughWords4, acc[i][j]));
+      }
+    }
+    return;
+  }
+
   // The tile as [H rows][W outputs] (+ 16 bytes of padding per row) into LDS -
   // a lane has four consecutive channels of a pixel - then whole 16-byte
   // vectors out.
@@ -408,8 +437,6 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
     }
   }
   __syncthreads();
-  const uint32_t outChans = d.groups * d.outChansPerGroup;
-  const __amdgpu_buffer_rsrc_t outBuf = bufferOf(out, a.outThrough);
   auto copyOut = [&](auto through) {
     for (int idx = t; idx < H * kVecsPerRow; idx += kThreads) {
       const uint32_t mLocal = idx / kVecsPerRow, vec = idx % kVecsPerRow;
@@ -447,11 +474,12 @@ constexpr bool flexAhead(int mb, int nb, int perCU) {
 }
 
 /// PER_CU: workgroups that share a CU.
-template <int MB, int NB, int NS, int PER_CU, class OutT>
+template <int MB, int NB, int NS, int PER_CU, bool SPLIT, class OutT>
 __global__ __launch_bounds__(kThreads, 2 * PER_CU) void igemmFlexKernel(
     IgemmArgs a, const char *__restrict__ in, const char *__restrict__ w,
     const OutT *__restrict__ bias, OutT *__restrict__ out) {
-  flexTile<MB, NB, NS, flexAhead(MB, NB, PER_CU), OutT>(a, in, w, bias, out, blockIdx.x, gridDim.x);
+  flexTile<MB, NB, NS, flexAhead(MB, NB, PER_CU), SPLIT, OutT>(
+      a, in, w, bias, out, blockIdx.x, gridDim.x);
 }
 
 /// Several convolutions in one launch, as igemmFusedKernel.
@@ -461,7 +489,7 @@ __global__ __launch_bounds__(kThreads, 2 * PER_CU) void igemmFlexFusedKernel(
   uint32_t i = 0;
   while (i + 1 < m.count && blockIdx.x >= m.firstBlock[i + 1])
     ++i;
-  flexTile<MB, NB, NS, flexAhead(MB, NB, PER_CU), OutT>(
+  flexTile<MB, NB, NS, flexAhead(MB, NB, PER_CU), false, OutT>(
       m.a[i], m.in[i], m.w[i], static_cast<const OutT *>(m.bias[i]),
       static_cast<OutT *>(m.out[i]), blockIdx.x - m.firstBlock[i],
       m.firstBlock[i + 1] - m.firstBlock[i]);
@@ -489,15 +517,21 @@ struct FlexOne {
   void *out;
   hipStream_t stream;
   template <int MB, int NB, int NS, int PER_CU> hipError_t go() const {
+    return a.d.splitK > 1 ? run<MB, NB, NS, PER_CU, true>()
+                          : run<MB, NB, NS, PER_CU, false>();
+  }
+  template <int MB, int NB, int NS, int PER_CU, bool SPLIT>
+  hipError_t run() const {
     using OutT = __half;
-    const uint64_t blocks = uint64_t(a.mTiles) * a.nTiles * a.d.groups;
+    const uint64_t blocks =
+        uint64_t(a.mTiles) * a.nTiles * a.d.groups * a.d.splitK;
     if (blocks == 0)
       return hipSuccess;
     if (blocks > 0x7fffffffull)
       return hipErrorInvalidConfiguration;
     constexpr int kLds = FlexShape<MB, NB, NS>::template ldsBytes<OutT>();
     static_assert(kLds * PER_CU <= 160 * 1024, "a CU's LDS");
-    const auto kernel = &igemmFlexKernel<MB, NB, NS, PER_CU, OutT>;
+    const auto kernel = &igemmFlexKernel<MB, NB, NS, PER_CU, SPLIT, OutT>;
     static const hipError_t attr = raiseLds(kernel, kLds);
     if (attr != hipSuccess)
       return attr;
@@ -585,7 +619,13 @@ bool igemmFlexTile(uint32_t blockM, uint32_t blockN, uint32_t flex) {
 
 bool igemmFlexTakes(const IgemmDesc &d, int inType, int outType) {
   return inType == kHalf && outType == kHalf &&
-         igemmFlexTile(d.blockM, d.blockN, d.flex) && d.splitK == 1 &&
+         igemmFlexTile(d.blockM, d.blockN, d.flex) &&
+         // (whole vectors of fp32 sums, a part of them within a buffer's reach)
+         (d.splitK == 1 ||
+          (d.outChansPerGroup % 4 == 0 && !d.outFullH && !d.outFullW &&
+           uint64_t(d.batch) * d.outD * d.outH * d.outW * d.groups *
+                   d.outChansPerGroup * 4 <
+               kOutOfRange)) &&
          !d.patch && !d.small && !d.outTransposed &&
          igemmTapAddressing(d) == kMaskTaps && igemmAddressable(d, inType);
 }

@@ -432,6 +432,41 @@ double pointwiseBesideFlex(double pixels, double co, double macs, double outMB,
                            0.112 * weightsMB + 2.51e-9 * macs +
                            7.95e-6 * pixels * std::ceil(co / 64.0));
 }
+/// Long sums over few outputs (K of 2 000 and more, up to 260 tiles of 128 x 64):
+/// a call of igemmFlexKernel with K in `parts`, one round of workgroups of `kSteps`
+/// each and the kernel that adds the parts, and of igemmKernel, K whole or in
+/// parts.  Fitted to 569 random layers and products of 0.4 to 60 GFLOP, all tiles
+/// and up to two numbers of parts each, within 8 % (igemmKernel 6 to 11); the tile
+/// picked by it is 1.4 % behind the best.
+double estimateFlexParts(unsigned blockM, unsigned blockN,
+                         std::size_t workgroups, std::size_t kSteps,
+                         std::size_t parts, bool ragged, double partialMB) {
+  const double perCU = double(workgroups) / double(gfx950::numCUs);
+  const double edge = (blockM + (blockN + 63) / 64 * 64) / 256.0;
+  const double area = blockM * blockN / 16384.0;
+  const double step = (0.175 + 0.044 * edge + 0.145 * area) *
+                          (blockM + blockN >= 416 ? 1.15 : 1.0) +
+                      (ragged ? 0.073 * edge : 0.0);
+  return 5.9 + 1.03 * area + 0.0049 * blockM +
+         double(kSteps) * step * (0.895 + 0.105 * perCU) +
+         0.45 * std::min(partialMB, 15.0) +
+         0.24 * std::max(partialMB - 15.0, 0.0) + 0.05 * double(parts);
+}
+double estimateBesideFlexParts(unsigned blockN, std::size_t parts,
+                               std::size_t workgroups, std::size_t kSteps,
+                               bool ragged, double outMB, double inMB) {
+  if (parts == 1)
+    return callUs(CallFit{1.44, 0.05, 0.272, 0.94, 0.23, 0.83, 0.18}, true,
+                  workgroups, kSteps, ragged, outMB, inMB);
+  // (a part's sums are fp32)
+  const double partialMB = 2.0 * outMB * double(parts);
+  return blockN == 64
+             ? callUs(CallFit{4.86, 2.1, 0.282, 0.95, 0.31, 0.52, 0.0}, false,
+                      workgroups, kSteps, ragged, partialMB, inMB)
+             : callUs(CallFit{1.62, 0.3, 0.351, 1.06, 0.28, 0.59, 0.097}, false,
+                      workgroups, kSteps, ragged, partialMB, inMB);
+}
+
 /// igemmFlexKernel is taken where it is estimated at less than these shares of
 /// what is planned.  Over the layers of the fit, at the share and (in brackets)
 /// wherever the estimate is lower at all: tiles of 128 x 128, two to a CU, 1.155
@@ -1470,12 +1505,11 @@ mxconv_plan makePlanWith(const ConvParams &params,
     if (pc.flex > 0) {
       g.flex = uint32_t(pc.flex);
       if (!halfIn || pc.patch > 0 || !pc.blockM || !pc.blockN ||
-          !mxk::igemmFlexTile(g.blockM, g.blockN, g.flex) ||
-          (pc.splitK > 1))
+          !mxk::igemmFlexTile(g.blockM, g.blockN, g.flex))
         throw poplar::invalid_option(
             "planConstraints gfx950 flex: that kernel takes half inputs and "
             "outputs in tiles of blockM 128, 192 or 256 and blockN 64 to 256 in "
-            "steps of 32 (with flex 2 up to 288 of both together), K whole");
+            "steps of 32 (with flex 2 up to 288 of both together)");
     }
     // (tiles of 256 pixels: igemm_wide.hip)
     const bool wideTile = g.blockM == 256 && pc.patch < 1 && !g.flex;
@@ -1505,7 +1539,9 @@ mxconv_plan makePlanWith(const ConvParams &params,
                                 (plan.coPadded / g.blockN) * p.numConvGroups;
       const std::size_t kSteps = plan.kPadded / g.blockK;
       std::size_t parts = 1;
-      if (g.blockM == 256 || g.flex)
+      if (pc.splitK && g.flex)
+        parts = pc.splitK;
+      else if (g.blockM == 256 || g.flex)
         parts = 1;
       else if (pc.splitK)
         parts = pc.splitK;
@@ -2271,6 +2307,97 @@ mxconv_plan makePlanWith(const ConvParams &params,
         plan.candidates.push_back(c);
       }
     }
+    // A long sum over few outputs (fp16): large tiles with K in parts, which
+    // fetch half as much for a product as tiles of 128 x 64 with K whole.  133 x
+    // 4872 x 5488 35.5 -> 20.7 us, 450 x 7416 x 1400 31.8 -> 23.4, N = 8, 31 x 31, 5
+    // x 5 stride 2, 376 -> 392 34.7 -> 28.8.  Taken below 0.92 of the estimate for
+    // tiles of 128 x 64 with K whole (106 such layers of the fit 1.08 times as fast
+    // on average, two slower by more than 3 %), 0.88 with K in parts already (117,
+    // 1.02), 0.95 for 128 x 128 in parts (15, 1.10).  Shorter sums do not pay for
+    // the second kernel (K of 1 500 to 2 000 0.7 to 0.9 times as fast), nor do 64
+    // channels and fewer, whose windows are most of what is fetched (7 x 36 x 36,
+    // 5 x 5, 552 -> 40 33.7 -> 44.6).
+    if (halfIn && params.outputType == poplar::HALF && !g.small && !g.patch &&
+        (g.flex || g.blockM == 128) && !plan.pointwiseOn &&
+        plan.igemmPhases.empty() && !s.outputPadded() && pc.flex < 0 &&
+        pc.kernel.empty() && pc.method == Method::ANY && !pc.blockM &&
+        !pc.blockN && !pc.blockK && !pc.splitK && !pc.stages && pc.patch < 0 &&
+        pc.pointwise < 0 && pc.smallTile < 0 && !pc.chanTiles &&
+        !isWeightUpdatePass(options.pass) && p.numConvGroups == 1 &&
+        co % 4 == 0 && co > 64 && k >= 2000) {
+      const std::size_t m = s.batch * s.outD * s.outH * s.outW;
+      const std::size_t kSteps = (k + 63) / 64;
+      const double outMB = 1e-6 * double(plan.outputBytes());
+      const double inMB = 1e-6 * double(plan.inputBytes() + plan.weightBytes());
+      const bool ragged = ciPadded % 64 != 0;
+      auto tilesOf = [&](std::size_t bm, std::size_t bn) {
+        return (m + bm - 1) / bm * ((co + bn - 1) / bn);
+      };
+      const std::size_t tiles = tilesOf(g.blockM, g.blockN);
+      const std::size_t planSteps = (kSteps + g.splitK - 1) / g.splitK;
+      double planned =
+          g.flex ? 0.9 * estimateFlex(g.blockM, g.blockN, g.flex == 2, tiles,
+                                      kSteps, ragged, outMB, inMB)
+                 : (g.splitK == 1       ? 0.92
+                    : g.blockN == 64 ? 0.88
+                                        : 0.95) *
+                       estimateBesideFlexParts(g.blockN, g.splitK,
+                                               tiles * g.splitK, planSteps,
+                                               ragged, outMB, inMB);
+      const std::size_t copy =
+          plan.paddedInputChans
+              ? s.batch * s.inD * s.inH * s.inW * ciPadded * 2
+              : 0;
+      // (callers that bring no workspace have 32 MB of it)
+      const std::size_t most =
+          std::max<std::size_t>(plan.workspaceBytes, std::size_t(32) << 20);
+      mxk::IgemmDesc chosenTile = g;
+      chosenTile.flex = 0;
+      if (tilesOf(128, 64) <= 260 &&
+          2.0 * double(m) * double(co) * double(k) >= 4e8 &&
+          (g.flex || g.splitK > 1 || g.blockN == 64))
+        for (uint32_t bm : {128u, 192u, 256u})
+          for (uint32_t bn = 64; bn <= 256; bn += 32)
+            for (std::size_t slots :
+                 {std::size_t(gfx950::numCUs), std::size_t(gfx950::numCUs / 2)}) {
+              const std::size_t own = tilesOf(bm, bn);
+              const std::size_t parts = std::min(slots / own, kSteps / 3);
+              if (parts < 2 || !mxk::igemmFlexTile(bm, bn, 1))
+                continue;
+              mxk::IgemmDesc t = g;
+              t.blockM = bm, t.blockN = bn, t.flex = 1;
+              t.splitK = uint32_t(parts);
+              const double us = estimateFlexParts(
+                  bm, bn, own * parts, (kSteps + parts - 1) / parts, parts,
+                  ragged, 2.0 * outMB * double(parts));
+              if (us >= planned ||
+                  mxk::igemmWorkspaceBytes(t) + copy + 256 > most ||
+                  !mxk::igemmFlexTakes(t, inId, outId))
+                continue;
+              planned = us, chosenTile = t;
+            }
+      if (chosenTile.flex) {
+        g = chosenTile;
+        plan.coPadded = (co + g.blockN - 1) / g.blockN * g.blockN;
+        plan.kPadded = kSteps * 64;
+        plan.weightPackedElems = plan.coPadded * plan.kPadded;
+        plan.workspaceBytes = mxk::igemmWorkspaceBytes(g);
+        if (plan.paddedInputChans) {
+          plan.paddedInputOffset = (plan.workspaceBytes + 255) / 256 * 256;
+          plan.workspaceBytes = plan.paddedInputOffset + copy;
+        }
+        for (auto &c : plan.candidates)
+          c.chosen = false;
+        mxconv_plan::Candidate c;
+        c.name = "flexible " + std::to_string(g.blockM) + " x " +
+                 std::to_string(g.blockN) + ", K in " +
+                 std::to_string(g.splitK) + " parts";
+        c.workgroups = tilesOf(g.blockM, g.blockN) * g.splitK, c.perCU = 1;
+        c.kSteps = (kSteps + g.splitK - 1) / g.splitK, c.estimateUs = planned;
+        c.rounds = 1.0, c.chosen = true;
+        plan.candidates.push_back(c);
+      }
+    }
     if (!g.patch && !g.flex && g.blockM != 128 && g.blockM != 256)
       throw poplar::invalid_option(
           "planConstraints gfx950 blockM 64 goes with the resident-patch "
@@ -2540,7 +2667,7 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
     // kernel, see splitPenaltyUs)
     const std::size_t partialBytes = mxk::igemmWorkspaceBytes(igemm);
     const double kSplitUs = igemm.splitK <= 1 ? 0.0
-                            : igemm.patch
+                            : igemm.patch || igemm.flex
                                 ? poplin::patchSplitUs(partialBytes)
                                 : poplin::splitPenaltyUs(partialBytes);
     e.reductionUs = kSplitUs;

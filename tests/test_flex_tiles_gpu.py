@@ -79,6 +79,47 @@ def test_forms_of_layers(oracle, tile, kw):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("parts,kw", [
+    # parts of three k-steps, the last of one; of one each; of two, the last of
+    # none; taps that a part's first chunk starts in the middle of
+    (3, dict(field=(9, 31), kernel=(1, 1), ci=448, co=260)),
+    (7, dict(batch=2, field=(9, 15), kernel=(1, 1), ci=448, co=36)),
+    (5, dict(field=(5, 15), kernel=(1, 1), ci=448, co=68)),
+    (4, dict(batch=3, field=(9, 11), kernel=(3, 3), ci=40, co=136, pad=1,
+             stride=(1, 2)))])
+def test_k_in_parts(oracle, tile, parts, kw):
+    from test_fast_gpu import _run
+    options = _options(tile)
+    named = json.loads(options["planConstraints"])
+    named["gfx950"]["splitK"] = parts
+    options = {"planConstraints": json.dumps(named)}
+    p = make_params(pa.HALF, **kw)
+    print("case", tile, parts, p, flush=True)
+    assert "parts         %d" % parts in pa.Plan(p, options).describe()
+    for bias in (True, False):
+        _run(oracle, p, 93, 0, "implicit GEMM", dist="pm1", bias=bias,
+             options=options)
+
+
+@pytest.mark.gpu
+def test_the_planner_s_own_parts(oracle):
+    """A long sum over few outputs, ragged channels filled up in a copy behind
+    the parts' sums."""
+    from test_fast_gpu import _run
+    p = make_params(pa.HALF, batch=6, field=(16, 15), kernel=(3, 3), ci=845,
+                    co=132, pad=1)
+    options = {"planConstraints": '{"gfx950": {"kernel": "igemm", "patch": 0, '
+                                  '"blockM": 192, "blockN": 160, "flex": 1, '
+                                  '"splitK": 20}}'}
+    assert "845 -> 848" in pa.Plan(p, options).describe()
+    _run(oracle, p, 94, 1e-3, "implicit GEMM", wscale=0.05, options=options)
+    q = pa.matMulParams(pa.HALF, pa.HALF, 1, 133, 4872, 5488)
+    named = json.loads(pa.Plan(q).constraints())["gfx950"]
+    assert named["flex"] == 1 and named["splitK"] > 1
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("tile", [(128, 160, 2), (192, 96, 2), (256, 160, 1)])
 @pytest.mark.parametrize("kw,phases", [
     (dict(batch=2, field=(14, 15), kernel=(3, 3), ci=40, co=72, idil=2,
@@ -163,8 +204,7 @@ def test_plans_name_the_tile_and_come_back():
 @pytest.mark.parametrize("asked", [
     dict(blockM=64, blockN=64, flex=1), dict(blockM=128, blockN=48, flex=1),
     dict(blockM=256, blockN=64, flex=1), dict(blockM=192, blockN=128, flex=2),
-    dict(blockM=128, flex=1), dict(blockM=128, blockN=96, flex=1, splitK=2),
-    dict(blockM=128, blockN=96, flex=3)])
+    dict(blockM=128, flex=1), dict(blockM=128, blockN=96, flex=3)])
 def test_tiles_that_are_not_there_are_refused(asked):
     p = make_params(pa.HALF, batch=2, field=(9, 9), kernel=(3, 3), ci=64,
                     co=64, pad=1)
@@ -181,3 +221,22 @@ def test_layers_it_does_not_take_are_refused(kw):
     p = make_params(batch=2, field=(9, 9), ci=64, co=64, pad=2, **kw)
     with pytest.raises(pa.MxconvError, match="flex"):
         pa.Plan(p, _options((128, 64, 1)))
+
+
+@pytest.mark.parametrize("m,k,n", [(133, 4872, 5488), (298, 3528, 3712),
+                                   (450, 7416, 1400), (2048, 8192, 1024)])
+def test_parts_leave_room_in_the_static_scratch(m, k, n):
+    """Callers that bring no workspace have 32 MB of it: products that ran
+    without any before K was cut run in it still."""
+    from poplibs_amd import capi
+    plan = pa.MatMulPlan(pa.HALF, pa.HALF, 1, m, k, n)
+    assert plan.buffer_bytes(capi.BUF_WORKSPACE) <= 32 << 20
+
+
+def test_parts_want_whole_vectors():
+    p = make_params(pa.HALF, batch=2, field=(9, 9), kernel=(3, 3), ci=64,
+                    co=66, pad=1)
+    with pytest.raises(pa.MxconvError, match="flex"):
+        pa.Plan(p, {"planConstraints": json.dumps({"gfx950": {
+            "kernel": "igemm", "patch": 0, "blockM": 128, "blockN": 96,
+            "flex": 1, "splitK": 2}})})
