@@ -723,7 +723,9 @@ hipError_t dispatch(const KernelKey &k, const Launch &launch) {
 
 /// out[i] = sum over parts of partial[part][i] (+ bias of i's channel).  The
 /// parts are added in a fixed order: four interleaved running sums (so that
-/// four loads are in flight per lane), combined at the end.  A thread takes V
+/// four loads are in flight per lane), combined at the end; the last one to three
+/// parts together too, those beyond the last the last again and left out (seven
+/// parts of 222 x 1040, the call 13.4 -> 12.9 us).  A thread takes V
 /// neighbouring channels of one pixel: 4 where the channel count is a multiple
 /// of 4 (one 16-byte load per part), else 1.
 template <class OutT, int V>
@@ -750,8 +752,26 @@ __global__ __launch_bounds__(64) void splitKReduceKernel(
     for (int u = 0; u != 4; ++u)
       add(u, p + u);
   }
-  for (; p != parts; ++p)
-    add(0, p);
+  if (p != parts) {
+    float rest[3][V];
+#pragma unroll
+    for (uint32_t u = 0; u != 3; ++u) {
+      const uint32_t part = p + u < parts ? p + u : parts - 1;
+      const float *src = partial + uint64_t(part) * elems + i;
+      if constexpr (V == 4) {
+        const float4 r = *reinterpret_cast<const float4 *>(src);
+        rest[u][0] = r.x, rest[u][1] = r.y, rest[u][2] = r.z, rest[u][3] = r.w;
+      } else {
+        rest[u][0] = *src;
+      }
+    }
+#pragma unroll
+    for (uint32_t u = 0; u != 3; ++u)
+      if (p + u < parts)
+#pragma unroll
+        for (int e = 0; e != V; ++e)
+          sum[u][e] += rest[u][e];
+  }
   float v[V];
 #pragma unroll
   for (int e = 0; e != V; ++e)
