@@ -24,8 +24,49 @@
 // 1.25, 1.43 and 1.49 in one of 256 x 256.
 #include "igemm_common.hpp"
 
+#include <algorithm>
+
 namespace mxk {
 namespace {
+
+/// A word of every 64-byte line of a convolution's arguments, asked for together:
+/// the compiler fetches an argument where it is first used, and each line's first
+/// fetch is a trip to memory (the scalar cache starts a launch cold).
+__device__ __forceinline__ void fetchArgs(const IgemmArgs &a) {
+  asm volatile("" ::"s"(a.d.groups), "s"(a.d.loH), "s"(a.d.outStepH),
+               "s"(a.divOutW.mul), "s"(a.divKW.mul), "s"(a.divKH.mul),
+               "s"(a.mTiles), "s"(a.wBytes), "s"(a.divWideBlock.mul));
+}
+
+/// The convolution of a fused launch that workgroup `block` belongs to: all the
+/// counts compared at once, not one trip each.
+__device__ __forceinline__ uint32_t fusedMember(const IgemmFusedArgs &m,
+                                                uint32_t block) {
+  uint32_t i = 0;
+#pragma unroll
+  for (uint32_t k = 1; k != kIgemmMaxFused; ++k)
+    i += uint32_t(k < m.count) & uint32_t(block >= m.firstBlock[k]);
+  return i;
+}
+
+/// What a workgroup of convolution i of a fused launch needs besides, fetched with
+/// the first line of its arguments.
+struct FusedPointers {
+  const char *in, *w;
+  const void *bias;
+  void *out;
+  uint32_t first, end;
+};
+__device__ __forceinline__ FusedPointers fusedPointers(const IgemmFusedArgs &m,
+                                                       uint32_t i) {
+  const FusedPointers p = {m.in[i],         m.w[i],
+                           m.bias[i],       m.out[i],
+                           m.firstBlock[i], m.firstBlock[i + 1]};
+  fetchArgs(m.a[i]);
+  asm volatile("" ::"s"(p.in), "s"(p.w), "s"(p.bias), "s"(p.out), "s"(p.first),
+               "s"(p.end));
+  return p;
+}
 
 constexpr int kFlexGroup = 4; // M tiles of a block of workgroups
 constexpr int kFlexTaps = 32; // (kMaskTaps)
@@ -43,13 +84,17 @@ template <int MB, int NB, int NS> struct FlexShape {
   template <class OutT> static constexpr int outRow() {
     return W * int(sizeof(OutT)) + 16;
   }
-  // the tile's bias as fp32, behind both what the loop and what the end needs
+  // the tile's bias as fp32, behind both what the loop and what the end needs,
+  // and where each of its rows goes
   template <class OutT> static constexpr int biasByte() {
     constexpr int end = H * outRow<OutT>();
     return ((kLoop > end ? kLoop : end) + 15) / 16 * 16;
   }
-  template <class OutT> static constexpr int ldsBytes() {
+  template <class OutT> static constexpr int rowOutByte() {
     return biasByte<OutT>() + W * int(sizeof(float));
+  }
+  template <class OutT> static constexpr int ldsBytes() {
+    return rowOutByte<OutT>() + H * int(sizeof(uint32_t));
   }
 };
 
@@ -76,6 +121,9 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
   uint2 *rowTable = reinterpret_cast<uint2 *>(lds + Shape::kRows);
   uint32_t *tapTable = reinterpret_cast<uint32_t *>(lds + Shape::kTaps);
   float *biasLds = reinterpret_cast<float *>(lds + Shape::template biasByte<OutT>());
+  fetchArgs(a);
+  uint32_t *rowOut =
+      reinterpret_cast<uint32_t *>(lds + Shape::template rowOutByte<OutT>());
   const IgemmDesc &d = a.d;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -149,28 +197,50 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
       kByte += kRowBytes;
   };
 
+  // (the first stage's weights are on their way while the tables are made)
+#pragma unroll
+  for (int r = 0; r != BLOADS; ++r)
+    loadBOne(lds, r);
+
   // The row table: per output pixel the byte offset of the input element
-  // under tap (0, 0), and the complement of the taps that read inside; and
-  // every tap's place in the input.
-  if (t < H) {
-    const uint32_t m = mTile * H + t;
+  // under tap (0, 0) - and the pixel's place in the output - by one thread, the
+  // complement of the taps that read inside by another; and every tap's place
+  // in the input.  (Places of mapped outputs worked out when they are stored,
+  // three divisions to a vector: N = 42, 35 x 35, 3 x 3 stride 2, 136 -> 80
+  // backwards 10.8 us, 10.2 so; 25 x 57 x 57, 72 -> 200 20.2 and 19.5.)
+  const uint32_t half = uint32_t(t) / (kThreads / 2);
+  const uint32_t row = uint32_t(t) % (kThreads / 2);
+  if (row < H) {
+    const uint32_t m = mTile * H + row;
     const bool rowValid = m < a.M;
     const uint32_t mm = rowValid ? m : 0;
     const uint32_t q = a.divOutW(mm), ow = mm - q * d.outW;
     const uint32_t q2 = a.divOutH(q), oh = q - q2 * d.outH;
     const uint32_t image = a.divOutD(q2), od = q2 - image * d.outD;
-    const uint32_t b = image - firstImage;
     const int idBase = int(od * d.strideD) - d.padD;
     const int ihBase = int(oh * d.strideH) - d.padH;
     const int iwBase = int(ow * d.strideW) - d.padW;
-    const uint32_t offset =
-        shift +
-        (((b * d.inD + uint32_t(idBase)) * d.inH + uint32_t(ihBase)) * d.inW +
-         uint32_t(iwBase)) *
-            pixelBytes +
-        g * ciBytes;
-    rowTable[t] =
-        uint2{offset, rowValid ? ~tapMaskOf(a, idBase, ihBase, iwBase) : ~0u};
+    if (half == 0) {
+      const uint32_t b = image - firstImage;
+      rowTable[row].x =
+          shift +
+          (((b * d.inD + uint32_t(idBase)) * d.inH + uint32_t(ihBase)) *
+               d.inW +
+           uint32_t(iwBase)) *
+              pixelBytes +
+          g * ciBytes;
+      uint32_t pixel = m;
+      if (a.outMapped)
+        pixel = ((image * d.outFullD + od * d.outStepD + d.outOffD) *
+                     d.outFullH +
+                 oh * d.outStepH + d.outOffH) *
+                    d.outFullW +
+                ow * d.outStepW + d.outOffW;
+      rowOut[row] = rowValid ? pixel : ~0u;
+    } else {
+      rowTable[row].y =
+          rowValid ? ~tapMaskOf(a, idBase, ihBase, iwBase) : ~0u;
+    }
   }
   if (uint32_t(kThreads - 1 - t) <= taps) {
     const uint32_t tap = kThreads - 1 - t;
@@ -227,10 +297,12 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
   // stride 2, 72 -> 200 12.9 us with all of them behind the barrier, 12.5).
   // A k-step has SLOTS slots, and `loadSlot` issues what belongs to one.
   constexpr int SLOTS = NS > 2 || AHEAD ? 2 * PRODUCTS : PRODUCTS;
-  auto loadSlot = [&](char *__restrict__ into, auto slot) {
+  auto loadSlot = [&](char *__restrict__ into, auto slot, auto most) {
     constexpr int K = decltype(slot)::value;
+    constexpr int MOST = decltype(most)::value;
     constexpr int FROM = (K * LOADS + SLOTS - 1) / SLOTS;
-    constexpr int TO = ((K + 1) * LOADS + SLOTS - 1) / SLOTS;
+    constexpr int UP = ((K + 1) * LOADS + SLOTS - 1) / SLOTS;
+    constexpr int TO = UP < MOST ? UP : MOST;
     staticFor<FROM, TO>([&](auto load) {
       constexpr int L = decltype(load)::value;
       if constexpr (L < ALOADS) {
@@ -242,6 +314,7 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
       }
     });
   };
+  using All = std::integral_constant<int, LOADS>;
   // The stages before the loop: all of them, or all but what the loop's first
   // half k-step sends.
   constexpr bool ACROSS = NS > 2 && !AHEAD; // over the end of a k-step
@@ -249,8 +322,10 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
   constexpr int AHEAD_OF_LAST = (LAST * LOADS + SLOTS - 1) / SLOTS;
   staticFor<0, NS>([&](auto stage) {
     constexpr int N = decltype(stage)::value;
+    // (the first stage's weights went out above)
+    using Most = std::integral_constant<int, N == 0 ? ALOADS : LOADS>;
     staticFor<0, N == NS - 1 ? LAST : SLOTS>(
-        [&](auto slot) { loadSlot(lds + N * kStage, slot); });
+        [&](auto slot) { loadSlot(lds + N * kStage, slot, Most{}); });
   });
   if (t < W)
     biasLds[t] = __half2float(__ushort_as_half(biasOwn));
@@ -321,7 +396,7 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
           readOne(next.half[0], from, Half0{}, K);
           readOne(next.half[1], from, Half1{}, K);
         }
-        loadSlot(freed, product);
+        loadSlot(freed, product, All{});
         pin();
       });
     };
@@ -356,7 +431,8 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
         if constexpr (K < OPERANDS)
           readOne(second, cur, Half1{}, K);
         if constexpr (ACROSS)
-          loadSlot(before, std::integral_constant<int, PRODUCTS + K>{});
+          loadSlot(before, std::integral_constant<int, PRODUCTS + K>{},
+                     All{});
         pin();
       });
       MXK_WAIT_LGKMCNT0(); // this wave has read all it needs of `cur`
@@ -369,7 +445,7 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
         pin();
         if constexpr (K < OPERANDS)
           readOne(first, next, Half0{}, K);
-        loadSlot(cur, product);
+        loadSlot(cur, product, All{});
         pin();
       });
     };
@@ -440,16 +516,15 @@ flexTile(const IgemmArgs &a, const char *__restrict__ in,
   auto copyOut = [&](auto through) {
     for (int idx = t; idx < H * kVecsPerRow; idx += kThreads) {
       const uint32_t mLocal = idx / kVecsPerRow, vec = idx % kVecsPerRow;
-      const uint32_t m = mTile * H + mLocal;
+      const uint32_t pixel = rowOut[mLocal];
       const uint32_t n = nTile * W + vec * kVecElems;
-      if (m >= a.M || n >= d.outChansPerGroup)
+      if (pixel == ~0u || n >= d.outChansPerGroup)
         continue;
       const char *src = lds + mLocal * kOutRow + vec * 16;
-      const size_t pixel = outPixel(a, m);
-      OutT *dst = out + pixel * outChans + g * d.outChansPerGroup + n;
+      OutT *dst = out + size_t(pixel) * outChans + g * d.outChansPerGroup + n;
       if constexpr (decltype(through)::value) {
         storeThrough(outBuf,
-                     (uint32_t(pixel) * outChans + g * d.outChansPerGroup + n) *
+                     (pixel * outChans + g * d.outChansPerGroup + n) *
                          uint32_t(sizeof(OutT)),
                      *reinterpret_cast<const uintx4 *>(src));
       } else if (n + kVecElems <= d.outChansPerGroup) {
@@ -486,13 +561,11 @@ __global__ __launch_bounds__(kThreads, 2 * PER_CU) void igemmFlexKernel(
 template <int MB, int NB, int NS, int PER_CU, class OutT>
 __global__ __launch_bounds__(kThreads, 2 * PER_CU) void igemmFlexFusedKernel(
     IgemmFusedArgs m) {
-  uint32_t i = 0;
-  while (i + 1 < m.count && blockIdx.x >= m.firstBlock[i + 1])
-    ++i;
+  const uint32_t i = fusedMember(m, blockIdx.x);
+  const FusedPointers p = fusedPointers(m, i);
   flexTile<MB, NB, NS, flexAhead(MB, NB, PER_CU), false, OutT>(
-      m.a[i], m.in[i], m.w[i], static_cast<const OutT *>(m.bias[i]),
-      static_cast<OutT *>(m.out[i]), blockIdx.x - m.firstBlock[i],
-      m.firstBlock[i + 1] - m.firstBlock[i]);
+      m.a[i], p.in, p.w, static_cast<const OutT *>(p.bias),
+      static_cast<OutT *>(p.out), blockIdx.x - p.first, p.end - p.first);
 }
 
 /// Stages of a tile's kernel that has its CU to itself, or shares it (0: the
@@ -627,6 +700,10 @@ bool igemmFlexTakes(const IgemmDesc &d, int inType, int outType) {
                    d.outChansPerGroup * 4 <
                kOutOfRange)) &&
          !d.patch && !d.small && !d.outTransposed &&
+         // (places in the output are 32-bit numbers of pixels)
+         uint64_t(d.batch) * std::max(d.outFullD, d.outD) *
+                 std::max(d.outFullH, d.outH) * std::max(d.outFullW, d.outW) <
+             0xffffffffull &&
          igemmTapAddressing(d) == kMaskTaps && igemmAddressable(d, inType);
 }
 
