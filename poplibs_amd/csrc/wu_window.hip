@@ -317,7 +317,13 @@ __global__ __launch_bounds__(64 * NW) void wuWindowKernel(
   };
 
   // The loads of the wave's next k-step go out before this one's MFMAs.
-  // (Pinned: left to itself the compiler issues them behind those.)
+  // (Pinned: left to itself the compiler issues them behind those.)  No k-step
+  // beyond the wave's last is multiplied: an odd count rounded up cost 5 % of
+  // the pass over 42 layers, up to 15 (10 x 31 x 31 stride 2, 56 -> 56 8.8 us,
+  // 7.6; 5 x 30 x 30 stride 2, 160 -> 88 10.1, 8.8).  Loads a k-step further ahead
+  // gain nothing, and neither do fewer instructions: 82 requests of 128 bytes
+  // to the L2 per k-step of 64 x 32 channels, most of them for half a line or
+  // two halves, keep the way from there busy.
   constexpr uint32_t kStride = NW * kWinUnits;
   uint32_t at = u0 + wave * kWinUnits;
   Raw even, odd;
@@ -327,11 +333,14 @@ __global__ __launch_bounds__(64 * NW) void wuWindowKernel(
     __builtin_amdgcn_sched_barrier(0);
     multiply(even);
     __builtin_amdgcn_sched_barrier(0);
-    load(even, at + 2 * kStride);
+    at += kStride;
+    if (at >= u1)
+      break;
+    load(even, at + kStride);
     __builtin_amdgcn_sched_barrier(0);
     multiply(odd);
     __builtin_amdgcn_sched_barrier(0);
-    at += 2 * kStride;
+    at += kStride;
   }
 
   storeWindow<JO, JI, KW, NW>(a, place, acc, lds, out);
@@ -474,11 +483,14 @@ __global__ __launch_bounds__(64 * NW) void wuWindowFloatKernel(
     __builtin_amdgcn_sched_barrier(0);
     both(even);
     __builtin_amdgcn_sched_barrier(0);
-    load(even, at + 2 * kStride);
+    at += kStride;
+    if (at >= u1)
+      break;
+    load(even, at + kStride);
     __builtin_amdgcn_sched_barrier(0);
     both(odd);
     __builtin_amdgcn_sched_barrier(0);
-    at += 2 * kStride;
+    at += kStride;
   }
   storeWindow<J, J, KW, NW>(a, place, acc, lds, out);
 }
