@@ -432,7 +432,7 @@ double pointwiseBesideFlex(double pixels, double co, double macs, double outMB,
                            0.112 * weightsMB + 2.51e-9 * macs +
                            7.95e-6 * pixels * std::ceil(co / 64.0));
 }
-/// Long sums over few outputs (K of 2 000 and more, up to 260 tiles of 128 x 64):
+/// Long sums over few outputs (K of 2 000 and more, up to 800 tiles of 128 x 64):
 /// a call of igemmFlexKernel with K in `parts`, one round of workgroups of `kSteps`
 /// each and the kernel that adds the parts, and of igemmKernel, K whole or in
 /// parts.  Fitted to 569 random layers and products of 0.4 to 60 GFLOP, all tiles
@@ -2316,7 +2316,12 @@ mxconv_plan makePlanWith(const ConvParams &params,
     // 1.02), 0.95 for 128 x 128 in parts (15, 1.10).  Shorter sums do not pay for
     // the second kernel (K of 1 500 to 2 000 0.7 to 0.9 times as fast), nor do 64
     // channels and fewer, whose windows are most of what is fetched (7 x 36 x 36,
-    // 5 x 5, 552 -> 40 33.7 -> 44.6).
+    // 5 x 5, 552 -> 40 33.7 -> 44.6).  Of 260 to 800 such tiles, planned in tiles of
+    // 128 x 128 that leave the last round of workgroups part empty, 10 % below the
+    // estimate for those: 388 x 6240 x 5568 50.9 -> 39.2 us, 10 x 53 x 53, 5 x 5 stride
+    // 2, 352 -> 320 57.8 -> 49.0.  There windows with fewer than 192 channels lose (7
+    // x 54 x 54, 5 x 5, 704 -> 128 88.9 -> 109), and tiles of 128 x 256 are as often
+    // slower as faster than estimated (340 x 7072 x 6816 48.1 -> 54.2).
     if (halfIn && params.outputType == poplar::HALF && !g.small && !g.patch &&
         (g.flex || g.blockM == 128) && !plan.pointwiseOn &&
         plan.igemmPhases.empty() && !s.outputPadded() && pc.flex < 0 &&
@@ -2338,6 +2343,9 @@ mxconv_plan makePlanWith(const ConvParams &params,
       double planned =
           g.flex ? 0.9 * estimateFlex(g.blockM, g.blockN, g.flex == 2, tiles,
                                       kSteps, ragged, outMB, inMB)
+          : g.splitK == 1 && g.blockN == 128
+              ? 0.9 * estimateBesideFlex(0, 128, g.stages, tiles, kSteps, ragged,
+                                         outMB, inMB)
                  : (g.splitK == 1       ? 0.92
                     : g.blockN == 64 ? 0.88
                                         : 0.95) *
@@ -2353,16 +2361,18 @@ mxconv_plan makePlanWith(const ConvParams &params,
           std::max<std::size_t>(plan.workspaceBytes, std::size_t(32) << 20);
       mxk::IgemmDesc chosenTile = g;
       chosenTile.flex = 0;
-      if (tilesOf(128, 64) <= 260 &&
-          2.0 * double(m) * double(co) * double(k) >= 4e8 &&
-          (g.flex || g.splitK > 1 || g.blockN == 64))
+      const std::size_t narrow = tilesOf(128, 64);
+      if ((narrow <= 260 ? g.flex || g.splitK > 1 || g.blockN == 64
+                         : narrow <= 800 && co >= 192) &&
+          2.0 * double(m) * double(co) * double(k) >= 4e8)
         for (uint32_t bm : {128u, 192u, 256u})
           for (uint32_t bn = 64; bn <= 256; bn += 32)
             for (std::size_t slots :
                  {std::size_t(gfx950::numCUs), std::size_t(gfx950::numCUs / 2)}) {
               const std::size_t own = tilesOf(bm, bn);
               const std::size_t parts = std::min(slots / own, kSteps / 3);
-              if (parts < 2 || !mxk::igemmFlexTile(bm, bn, 1))
+              if (parts < 2 || !mxk::igemmFlexTile(bm, bn, 1) ||
+                  (narrow > 260 && bm == 128 && bn == 256))
                 continue;
               mxk::IgemmDesc t = g;
               t.blockM = bm, t.blockN = bn, t.flex = 1;

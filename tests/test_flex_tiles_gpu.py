@@ -233,6 +233,20 @@ def test_parts_leave_room_in_the_static_scratch(m, k, n):
     assert plan.buffer_bytes(capi.BUF_WORKSPACE) <= 32 << 20
 
 
+@pytest.mark.parametrize("m,k,n,parts", [
+    # more than 260 tiles of 128 x 64, in a part empty round of 128 x 128 with K
+    # whole; more than 800; fewer than 192 channels
+    (388, 6240, 5568, True), (1088, 6408, 2576, True),
+    (3000, 6408, 2576, False), (32000, 2400, 128, False)])
+def test_parts_of_sums_over_more_outputs(m, k, n, parts):
+    from poplibs_amd import capi
+    plan = pa.MatMulPlan(pa.HALF, pa.HALF, 1, m, k, n)
+    chosen = [line for line in plan.describe().split("\n")
+              if line.strip().startswith("*")]
+    assert ("parts" in chosen[0]) == parts
+    assert plan.buffer_bytes(capi.BUF_WORKSPACE) <= 32 << 20
+
+
 def test_parts_want_whole_vectors():
     p = make_params(pa.HALF, batch=2, field=(9, 9), kernel=(3, 3), ci=64,
                     co=66, pad=1)
