@@ -514,13 +514,20 @@ __global__ __launch_bounds__(256) void biasUpdateKernel(
   const uint32_t cLocal = threadIdx.x % kBiasChans;
   const uint32_t lane = threadIdx.x / kBiasChans;
   const uint64_t c = uint64_t(blockIdx.x) * kBiasChans + cLocal;
+  const uint64_t cIn = c < channels ? c : channels - 1;
+  const float before = Load<T>::at(biases, cIn, 0);
+  // (splits beyond the last: the last again, and not added.  Under a condition
+  // each, the first was waited for on its own: 77 updates 1.04 times as fast so, up
+  // to 1.14)
   float v[kBiasSplits / kBiasLanes];
 #pragma unroll
   for (uint32_t i = 0; i != kBiasSplits / kBiasLanes; ++i) {
     const uint32_t s = i * kBiasLanes + lane;
-    v[i] = s < splits && c < channels ? partial[uint64_t(s) * channels + c]
-                                      : 0.f;
+    v[i] = partial[uint64_t(s < splits ? s : splits - 1) * channels + cIn];
   }
+#pragma unroll
+  for (uint32_t i = 0; i != kBiasSplits / kBiasLanes; ++i)
+    v[i] = i * kBiasLanes + lane < splits ? v[i] : 0.f;
   float sum = 0.f;
 #pragma unroll
   for (uint32_t i = 0; i != kBiasSplits / kBiasLanes; ++i)
@@ -533,7 +540,7 @@ __global__ __launch_bounds__(256) void biasUpdateKernel(
 #pragma unroll
   for (uint32_t l = 1; l != kBiasLanes; ++l)
     total += lanes[l][cLocal];
-  storeOut(biases, c, Load<T>::at(biases, c, 0) + scale * total);
+  storeOut(biases, c, before + scale * total);
 }
 
 /// The same in one launch, for few rows: a workgroup takes 32 channels (64
