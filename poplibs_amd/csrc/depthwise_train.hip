@@ -168,8 +168,13 @@ struct BlockArgs {
 /// once, and every output then takes exactly its own taps - no tests, no
 /// divergence between neighbouring outputs, each input vector loaded once per
 /// thread.
+/// What bounds it is a wave's chain of instructions, 1 200 with two blocks of 5 x 5
+/// taps: with one block to a thread instead of two (5 x 5) or four (3 x 3), and no
+/// load under a condition of its own, 17 x 44 x 44, 400 channels, 5 x 5 17.8 -> 13.2
+/// us, 19 x 25 x 25, 40, 3 x 3 4.4 -> 2.8; 70 layers 1.32 times as fast.
 template <int S, int K, int R, class OutT>
-__global__ __launch_bounds__(256) void depthwiseDilatedBlockKernel(
+__global__ __launch_bounds__(256, K == 5 ? 2 : 4) void
+depthwiseDilatedBlockKernel(
     BlockArgs a, const __half *__restrict__ in, const __half *__restrict__ w,
     const OutT *__restrict__ bias, OutT *__restrict__ out) {
   const DepthwiseDesc &d = a.d;
@@ -195,22 +200,33 @@ __global__ __launch_bounds__(256) void depthwiseDilatedBlockKernel(
   for (int i = 0; i != ROWS; ++i)
 #pragma unroll
     for (int j = 0; j != ND; ++j) {
-      const int ih = qh0 + i, iw = qw + j;
-      x[i][j].raw = uint4{0, 0, 0, 0};
-      if (ih >= int(d.loH) && ih < int(d.hiH) && iw >= int(d.loW) &&
-          iw < int(d.hiW))
-        x[i][j].raw = *reinterpret_cast<const uint4 *>(
-            image + (size_t(ih) * d.inW + size_t(iw)) * d.channels);
+      // (an element outside is answered with one inside and put to zero below:
+      // every load is unconditional)
+      const int ih = min(max(qh0 + i, int(d.loH)), int(d.hiH) - 1);
+      const int iw = min(max(qw + j, int(d.loW)), int(d.hiW) - 1);
+      x[i][j].raw = *reinterpret_cast<const uint4 *>(
+          image + (size_t(ih) * d.inW + size_t(iw)) * d.channels);
     }
   Vec8 k[K * K];
 #pragma unroll
   for (int tap = 0; tap != K * K; ++tap)
     k[tap].raw =
         *reinterpret_cast<const uint4 *>(w + size_t(tap) * d.channels + c);
+  BiasVec<OutT, 8> biasRaw;
+  biasRaw.load(bias, c);
   float biasV[8];
 #pragma unroll
   for (int i = 0; i != 8; ++i)
-    biasV[i] = bias ? Load<OutT>::at(bias, c + i, 0) : 0.0f;
+    biasV[i] = biasRaw.at(i);
+#pragma unroll
+  for (int i = 0; i != ROWS; ++i)
+#pragma unroll
+    for (int j = 0; j != ND; ++j) {
+      const bool inside =
+          uint32_t(qh0 + i) - d.loH < d.hiH - d.loH &&
+          uint32_t(qw + j) - d.loW < d.hiW - d.loW;
+      x[i][j].raw = inside ? x[i][j].raw : uint4{0, 0, 0, 0};
+    }
 
   OutT *outImage = out + size_t(b) * d.outH * d.outW * d.channels + c;
 #pragma unroll
@@ -240,6 +256,12 @@ __global__ __launch_bounds__(256) void depthwiseDilatedBlockKernel(
       }
     }
 }
+
+/// Blocks of 3 x 3 taps up to which a thread takes one, not two: a short chain of
+/// instructions counts where the chip is not filled, the taps' loads shared by two
+/// beyond (9 x 58 x 58, 256 channels, 259 000 blocks 6.6 and 6.0 us; 10 x 42 x 42,
+/// 192, 116 000 3.9 and 4.0; 25 x 9 x 9, 72, 8 100 2.8 and 3.1 - with four 4.3).
+constexpr uint64_t kFewBlocks = 120000;
 
 inline int floorDiv(int n, int d) { return n >= 0 ? n / d : -((-n + d - 1) / d); }
 
@@ -511,7 +533,7 @@ bool depthwiseDirectInBlocks(const DepthwiseDesc &d) {
   return d.inDilH == 2 && d.inDilW == 2 && d.strideH == 1 && d.strideW == 1 &&
          d.dilH == 1 && d.dilW == 1 && d.kH == d.kW &&
          (d.kH == 3 || d.kH == 5) && d.outH < (1u << 30) &&
-         d.outW < (1u << 30);
+         d.outW < (1u << 30) && d.loH < d.hiH && d.loW < d.hiW;
 }
 
 hipError_t launchDepthwiseDirect(const DepthwiseDesc &d, int inType,
@@ -534,12 +556,12 @@ hipError_t launchDepthwiseDirect(const DepthwiseDesc &d, int inType,
     return hipErrorInvalidConfiguration;
   if (inType == kHalf && (outType == kHalf || outType == kFloat) &&
       depthwiseDirectInBlocks(d)) {
-    if (d.kH == 3)
-      return launchDilatedBlock<2, 3, 4>(d, outType, in, weightsPacked, bias,
-                                         out, stream);
-    if (d.kH == 5)
-      return launchDilatedBlock<2, 5, 2>(d, outType, in, weightsPacked, bias,
-                                         out, stream);
+    const uint64_t blocks =
+        uint64_t(d.batch) * (d.outH / 2 + 1) * (d.outW / 2 + 1) * a.vecs;
+    const auto go = d.kH == 5                ? &launchDilatedBlock<2, 5, 1>
+                    : blocks <= kFewBlocks ? &launchDilatedBlock<2, 3, 1>
+                                             : &launchDilatedBlock<2, 3, 2>;
+    return go(d, outType, in, weightsPacked, bias, out, stream);
   }
   a.divVecs = makeFastDiv(a.vecs);
   a.divOutW = makeFastDiv(d.outW);
