@@ -514,15 +514,28 @@ void deltaBlockShape(const DepthwiseDesc &d, uint32_t &itemsPerBlock,
 }
 
 uint32_t deltaSlices(const DepthwiseDesc &d) {
-  // About 4 workgroups per CU in all; a slot walks at least 16 pixels.
+  // About 4 workgroups per CU in all; a slot walks at least 16 pixels, or 8 or 4
+  // where that leaves no more slices than the sum's 64 parts have in one round of
+  // loads, and sums of 2 MB.  (The walk is a chain of latencies: 13 x 12 x 12, 40
+  // channels, 3 x 3 6.7 us with 16, 5.2 with 4; but 46 x 13 x 13, 40 6.2 with 195
+  // slices, 7.5 with 389, and 11 x 12 x 12 stride 2, 808, 5 x 5 8.5 with 2 MB, 9.9
+  // with 4.)
   uint32_t itemsPerBlock, slots;
   deltaBlockShape(d, itemsPerBlock, slots);
   const uint64_t pixels = uint64_t(d.batch) * d.outH * d.outW;
   const uint64_t items =
       uint64_t(d.kH) * d.kW * (uint64_t(d.channels) * d.elemBytes / 16);
   const uint64_t itemBlocks = (items + itemsPerBlock - 1) / itemsPerBlock;
-  uint64_t slices = (1024 + itemBlocks - 1) / std::max<uint64_t>(itemBlocks, 1);
-  slices = std::min<uint64_t>(slices, (pixels + 16 * slots - 1) / (16 * slots));
+  const uint64_t most =
+      (1024 + itemBlocks - 1) / std::max<uint64_t>(itemBlocks, 1);
+  uint64_t slices = 1;
+  for (uint32_t walk : {4u, 8u, 16u}) {
+    slices = std::min<uint64_t>(most, (pixels + walk * slots - 1) /
+                                          (walk * slots));
+    if (slices <= 256 &&
+        slices * d.kH * d.kW * d.channels * sizeof(float) <= 2000000)
+      break;
+  }
   slices = std::min<uint64_t>(std::max<uint64_t>(slices, 1), 65535);
   return uint32_t(slices);
 }
