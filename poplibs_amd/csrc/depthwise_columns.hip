@@ -1,4 +1,4 @@
-// Depthwise convolution with 5 x 5 or 7 x 7 taps at stride 1 or 2: a lane
+// Depthwise convolution with 3 x 3, 5 x 5 or 7 x 7 taps at stride 1 or 2: a lane
 // walks down a strip of output columns of two neighbouring channels.
 //
 // Twenty-five or forty-nine multiply-adds per output and channel make the
@@ -32,9 +32,10 @@
 // stride 2, 13 x 106 x 106, 304: 191 -> 31.5 (its tensors' bytes take 21);
 // 5 x 5 taps 32 x 28 x 28, 240: 15.8 -> 10.4; 8 x 90 x 90, 48: 13.2 -> 7.6;
 // stride 2, 32 x 28 x 28, 240: 10.1 -> 6.5; 32 x 112 x 112, 96: 25.2 -> 20.4.
-// 3 x 3 taps stay with their own kernels, which are bound by the bytes: this
-// one (of one channel to a lane) was within 10 % of them either way for most
-// layers and 1.3 to 1.5 us slower for small ones.
+// 3 x 3 taps go here from the row ring where the two estimates say so (Plan.cpp):
+// 43 x 26 x 26, 336 channels 14.4 -> 9.2, 47 x 19 x 19, 488 11.6 -> 8.8, 11 x 7 x 7
+// stride 2, 688 3.1 -> 2.3; the small-workgroup kernel of up to 224 channels keeps
+// its layers, which are within 10 % either way.
 //
 // The reference's role: depthwise layers go through
 // lib/poplin/codelets/ConvPartialHorizontalMac.cpp there.
@@ -240,7 +241,7 @@ bool depthwiseColumnsTakes(const DepthwiseDesc &d, int inType, int outType) {
                             (outType == kHalf ? 2 : 4);
   const int most = 1 << 20;
   return inType == kHalf && (outType == kHalf || outType == kFloat) &&
-         d.elemBytes == 2 && d.kH == d.kW && (d.kH == 5 || d.kH == 7) &&
+         d.elemBytes == 2 && d.kH == d.kW && (d.kH == 3 || d.kH == 5 || d.kH == 7) &&
          d.strideH == d.strideW && (d.strideH == 1 || d.strideH == 2) &&
          d.dilH == 1 && d.dilW == 1 && d.inDilH == 1 && d.inDilW == 1 &&
          d.loH < d.hiH && d.hiH <= d.inH && d.loW < d.hiW && d.hiW <= d.inW &&
@@ -249,12 +250,46 @@ bool depthwiseColumnsTakes(const DepthwiseDesc &d, int inType, int outType) {
          d.padH < most && d.padW > -most && d.padW < most;
 }
 
+// 3 x 3 taps: the same with their own figures, fitted to 6 100 timings of 500
+// random layers (1 to 64 images of 7 to 112 squared, 32 to 960 channels) within 8
+// to 9 %; the choice by it is 1 % behind the best.
+double threeEstimateUs(const DepthwiseDesc &d) {
+  struct Fit {
+    double call, product, row, perRow, rate, start;
+    int resident[2];
+  };
+  constexpr Fit fits[2] = {{1.62, 1.98, 11.7, 4.55, 4.78e6, 2.07, {8, 6}},
+                           {1.78, 1.03, 6.47, 8.14, 5.53e6, 1.35, {8, 5}}};
+  const uint32_t s = d.strideH, strip = d.columns;
+  const Fit &f = fits[s - 1];
+  const double rows = std::min(d.columnRows, d.outH);
+  const double bands = std::ceil(d.outH / rows);
+  const double blocks =
+      std::ceil(double(columnItems(d)) / kColThreads) * bands;
+  const double rowsIn = (rows - 1) * s + 3;
+  const double columnsIn = s * (strip - 1) + 3;
+  const double waveUs = (f.product * 12 * rows * strip +
+                         f.row * rowsIn * (3 * columnsIn + f.perRow)) *
+                        1e-3 / 2.4;
+  const double resident = f.resident[strip / 2 - 1];
+  const double perCu = blocks / 256;
+  const double full = std::floor(perCu / resident);
+  const double rest = std::ceil(perCu - full * resident);
+  const double us = full * (resident + f.start) * waveUs +
+                    (rest > 0 ? (rest + f.start) * waveUs : 0.0);
+  const double bytes = 2.0 * d.batch * d.channels *
+                       (double(d.inH) * d.inW + double(d.outH) * d.outW);
+  return f.call + std::sqrt(std::hypot(us * us, std::pow(bytes / f.rate, 2)));
+}
+
 // What a strip and a band cost, fitted to 1700 timings of 130 random layers
 // (the choice by it is within 2 % of the best on average): a wave issues its
 // multiply-adds and, for each input row, three instructions a column and some
 // twenty around them; the waves of a SIMD take turns, as if there were two
 // thirds of one more (their waits), and the tensors pass at 5 TB/s beside it.
 double depthwiseColumnsEstimateUs(const DepthwiseDesc &d) {
+  if (d.kH == 3)
+    return threeEstimateUs(d);
   const uint32_t k = d.kH, s = d.strideH, strip = d.columns;
   const double rows = std::min(d.columnRows, d.outH);
   const double bands = std::ceil(d.outH / rows);
@@ -357,8 +392,11 @@ hipError_t launchDepthwiseColumns(const DepthwiseDesc &d, int inType,
   };
   using One = std::integral_constant<int, 1>;
   using Two = std::integral_constant<int, 2>;
+  using Three = std::integral_constant<int, 3>;
   using Five = std::integral_constant<int, 5>;
   using Seven = std::integral_constant<int, 7>;
+  if (d.kH == 3)
+    return d.strideH == 1 ? go(Three{}, One{}) : go(Three{}, Two{});
   if (d.kH == 5)
     return d.strideH == 1 ? go(Five{}, One{}) : go(Five{}, Two{});
   return d.strideH == 1 ? go(Seven{}, One{}) : go(Seven{}, Two{});

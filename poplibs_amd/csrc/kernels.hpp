@@ -437,7 +437,7 @@ bool depthwiseStripTakes(const DepthwiseDesc &d);
 /// and, with strips, the taps; what it may take at most.
 uint64_t depthwiseTileLdsBytes(const DepthwiseDesc &d);
 constexpr uint32_t kDepthwiseTileLdsMost = 80 * 1024;
-/// fp16, 5 x 5 or 7 x 7 taps, stride 1 or 2: a lane walks down a strip of
+/// fp16, 3 x 3, 5 x 5 or 7 x 7 taps, stride 1 or 2: a lane walks down a strip of
 /// output columns of two neighbouring channels.
 bool depthwiseColumnsTakes(const DepthwiseDesc &d, int inType, int outType);
 /// Strip (2 or 4 columns; 0: the faster) and band for d, and what they take.
@@ -472,6 +472,8 @@ struct DepthwiseRowsLaunch {
   uint64_t workgroups;
 };
 DepthwiseRowsLaunch depthwiseRowsLaunchShape(const DepthwiseDesc &d);
+/// Estimated microseconds of a call, 3 x 3 taps on half tensors.
+double depthwiseRowsEstimateUs(const DepthwiseDesc &d);
 hipError_t launchDepthwiseRows(const DepthwiseDesc &d, int inType, int outType,
                                const void *in, const void *weightsPacked,
                                const void *bias, void *out,

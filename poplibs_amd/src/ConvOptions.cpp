@@ -211,6 +211,11 @@ void checkGfx950(const std::string &path, const Value &v, PlanConstraints &pc) {
       if (v != 0 && v != 2 && v != 4)
         throw invalid_option("'" + sub + "': Must be 0, 2 or 4");
       pc.columns = int(v);
+    } else if (m.first == "strips") {
+      const unsigned v = requireUnsigned(sub, m.second);
+      if (v != 2 && v != 4)
+        throw invalid_option("'" + sub + "': Must be 2 or 4");
+      pc.strips = int(v);
     } else if (m.first == "pointwise") {
       const unsigned v = requireUnsigned(sub, m.second);
       if (v > 1)

@@ -58,6 +58,8 @@ struct PlanConstraints {
   /// (never with a tile or rowRing 1), 0 never, 2 or 4 that strip (an error
   /// where they cannot take the layer).
   int columns = -1;
+  /// 3 x 3 taps forward the same way, by strips of 2 or 4 (0: as planned).
+  int strips = 0;
   /// 64-channel tiles of the output per workgroup of the pointwise streaming
   /// kernel (1 to 4); 0 = planner's choice.
   unsigned chanTiles = 0;

@@ -2437,15 +2437,44 @@ mxconv_plan makePlanWith(const ConvParams &params,
         mxk::depthwiseColumnsTakes(d, dwType,
                                    params.outputType == poplar::HALF
                                        ? mxk::kHalf
-                                       : mxk::kFloat);
+                                       : mxk::kFloat) &&
+        (d.kH != 3 || pc.strips);
+    if (pc.strips && !plan.depthwiseWeightUpdate &&
+        (!columns || d.kH != 3 || pc.columns > 0))
+      throw poplar::invalid_option(
+          "planConstraints gfx950 strips: fp16 inputs and 3x3 taps at stride 1 "
+          "or 2, without columns, a tile or rowRing named");
     if (columns)
-      mxk::chooseDepthwiseColumns(d, pc.columns > 0 ? uint32_t(pc.columns) : 0);
+      mxk::chooseDepthwiseColumns(d, pc.strips        ? uint32_t(pc.strips)
+                                     : pc.columns > 0 ? uint32_t(pc.columns)
+                                                      : 0);
     else if (pc.columns > 0 && !plan.depthwiseWeightUpdate)
       throw poplar::invalid_option(
           "planConstraints gfx950 columns: that kernel takes fp16 inputs, 5x5 "
           "or 7x7 taps at stride 1 or 2, without a tile or rowRing named");
     else
       chooseDepthwiseTileOrRing(d, pc, s.inputDilated(), dwType);
+    // 3 x 3 taps that would go to the ring, whose workgroups walk a band each and
+    // wait for its first rows: strips of columns where they are estimated at 5 %
+    // less.  Of 260 such layers 150 change, and all together are 1.11 times as fast
+    // (four in ten of those with more than 224 channels by 1.25 and more, 43 x 26 x
+    // 26, 336 channels 14.4 -> 9.2 us; the slowest 0.90).  Tensors of more than the
+    // 256 MB cache in front of HBM were not among them.
+    if (!columns && d.kH == 3 && d.kW == 3 && d.dense3x3 == 2 &&
+        !plan.depthwiseWeightUpdate && pc.columns < 0 && pc.rowRing < 0 &&
+        params.outputType == poplar::HALF &&
+        2.0 * double(d.batch) * double(d.channels) *
+                (double(d.inH) * d.inW + double(d.outH) * d.outW) <=
+            256e6 &&
+        mxk::depthwiseColumnsTakes(d, dwType, mxk::kHalf)) {
+      mxk::DepthwiseDesc c = d;
+      mxk::chooseDepthwiseColumns(c, 0);
+      if (mxk::depthwiseColumnsEstimateUs(c) <
+          0.95 * mxk::depthwiseRowsEstimateUs(d)) {
+        d = c;
+        d.dense3x3 = 0;
+      }
+    }
     plan.weightPackedElems = plan.weightElems; // [kH*kW][C]
   } else {
     plan.weightPackedElems = plan.weightElems; // [G][K][Ci][Co]
@@ -2477,7 +2506,8 @@ std::string mxconv_plan::constraintsJson() const {
        << (depthwise.dense3x3 == 2 ? 1 : 0);
     // (an explicit tile names the LDS-tiled kernel)
     if (depthwise.columns)
-      os << ", \"columns\": " << depthwise.columns;
+      os << (depthwise.kH == 3 ? ", \"strips\": " : ", \"columns\": ")
+         << depthwise.columns;
     else if (!depthwise.dense3x3 && depthwise.inDilH == 1 && depthwise.inDilW == 1)
       os << ", \"tileH\": " << depthwise.tileH << ", \"tileW\": "
          << depthwise.tileW;
