@@ -407,21 +407,23 @@ __global__ __launch_bounds__(256) void depthwiseWeightDeltaKernel(
 constexpr uint32_t kManyOutputs = 3500, kManyOutputsPerSlice = 25;
 
 /// out[c][tap] = sum over slices of partial[slice][tap][c], in a fixed order:
-/// a workgroup takes COLUMNS outputs and cuts the slices into PARTS contiguous
-/// parts, COLUMNS lanes (contiguous in a slice) to each; a lane adds up its
-/// part with up to sixteen loads in flight, then the sums of an output meet in steps
-/// of eight, each in order (one thread adding all 64 is a chain of 64 LDS reads
-/// at the kernel's end).
+/// a workgroup takes COLUMNS outputs and deals the slices to PARTS parts in turn,
+/// COLUMNS lanes (contiguous in a slice) to each; a lane adds up its part's with
+/// four loads in flight, then the sums of an output meet in steps of eight, each in
+/// order (one thread adding all 64 is a chain of 64 LDS reads at the kernel's end).
 ///
-/// The walk over the slices is a chain of memory latencies.  64 parts of 16
-/// outputs make it short, but launch a wave for every output: with many of
-/// those, eight parts of 32 take a quarter of the time (5 x 5 taps, 960
-/// channels, 16 slices: 8.0 -> 3.2 us).  Their chain is eight times as long,
-/// which shows right behind the kernel that writes the slices: of 70 passes the
-/// line below is where both are level (3 x 3, 128 channels, 80 slices 7.5 us
-/// with 64 parts, 8.4 with eight; 688, 256 slices 17.8 and 20.5; 920, 31
-/// slices 9.4 and 7.7; 5 x 5, 904, 93 slices 29.3 and 26.5).
-template <class OutT, int PARTS, int COLUMNS>
+/// What it costs is the chain of instructions of a wave: 32-bit offsets into a
+/// buffer, beyond whose end zeros arrive, take one or two to a load, where slices
+/// in runs with the loads' addresses and conditions worked out took ten and more (16
+/// parts of 16 loads 1.5 us longer than 64 of four; the pass over 120 layers 1.014
+/// times as fast with the offsets, 12 x 19 x 19, 5 x 5 stride 2 10.5 -> 9.6 us).  64
+/// parts of 16 outputs make it short, but launch a wave for every output: with many
+/// of those, eight parts of 32 take a quarter of the time (5 x 5 taps, 960 channels,
+/// 16 slices: 8.0 -> 3.2 us).  Their chain is eight times as long, which shows right
+/// behind the kernel that writes the slices: the line below is where both were level
+/// over 70 passes.
+/// WIDE: offsets beyond 31 bits.
+template <class OutT, int PARTS, int COLUMNS, bool WIDE>
 __global__ __launch_bounds__(PARTS *COLUMNS) void depthwiseDeltaSumKernel(
     const float *__restrict__ partial, uint32_t slices, uint32_t taps,
     uint32_t channels, OutT *__restrict__ out) {
@@ -430,38 +432,28 @@ __global__ __launch_bounds__(PARTS *COLUMNS) void depthwiseDeltaSumKernel(
   const uint32_t column = threadIdx.x % COLUMNS, part = threadIdx.x / COLUMNS;
   const uint32_t outputs = taps * channels;
   const uint32_t i = blockIdx.x * COLUMNS + column; // tap * C + c
-  const uint32_t per = (slices + PARTS - 1) / PARTS;
-  const uint32_t from = min(part * per, slices), to = min(from + per, slices);
-  // (sixteen, eight or four loads at once, those beyond the part's last the last
-  // again and not added: under a condition each, as the last fifteen were, a wave
-  // waits for one after the other.  The pass over 38 layers 1.12 times as fast so,
-  // 16 x 52 x 52, 3 x 3 10.0 -> 8.4 us, 7 x 65 x 65 at stride 2 8.7 -> 7.3)
   float sum = 0.0f;
-  if (i < outputs) {
-    uint32_t s = from;
-    auto add = [&](auto at_once) {
-      constexpr int N = decltype(at_once)::value;
-      float v[N];
+  if constexpr (WIDE) {
+    if (i < outputs)
+      for (uint32_t s = part; s < slices; s += PARTS)
+        sum += partial[size_t(s) * outputs + i];
+  } else {
+    const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(partial), short(0), int(slices * outputs * 4),
+        0x00020000);
+    const uint32_t step = PARTS * outputs * 4;
+    uint32_t at = i < outputs ? (part * outputs + i) * 4 : 0x80000000u;
+    constexpr int kInFlight = 4;
+    for (uint32_t s = 0; s < slices; s += kInFlight * PARTS) {
+      float v[kInFlight];
 #pragma unroll
-      for (uint32_t u = 0; u != N; ++u)
-        v[u] = partial[size_t(min(s + u, to - 1)) * outputs + i];
-#pragma unroll
-      for (uint32_t u = 0; u != N; ++u)
-        v[u] = s + u < to ? v[u] : 0.0f;
-#pragma unroll
-      for (int width = N / 2; width != 0; width /= 2)
-#pragma unroll
-        for (int u = 0; u != width; ++u)
-          v[u] += v[u + width];
-      sum += v[0];
-      s += N;
-    };
-    while (s + 8 < to)
-      add(std::integral_constant<int, 16>{});
-    if (s + 4 < to)
-      add(std::integral_constant<int, 8>{});
-    else if (s < to)
-      add(std::integral_constant<int, 4>{});
+      for (uint32_t u = 0; u != kInFlight; ++u)
+        v[u] = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(buffer, at + u * step,
+                                                        0, 0));
+      at += kInFlight * step;
+      sum += (v[0] + v[1]) + (v[2] + v[3]);
+    }
   }
   meet[part][column] = sum;
   __syncthreads();
@@ -488,20 +480,28 @@ __global__ __launch_bounds__(PARTS *COLUMNS) void depthwiseDeltaSumKernel(
   storeOut(out, size_t(c) * taps + tap, total);
 }
 
+template <class OutT, int PARTS, int COLUMNS>
+void launchDeltaSumIn(const float *partial, uint32_t slices, uint32_t taps,
+                      uint32_t channels, void *out, hipStream_t stream) {
+  const uint32_t outputs = taps * channels;
+  // (offsets up to four rounds of parts beyond the slices)
+  const bool wide = (uint64_t(slices) + 5 * PARTS) * outputs * 4 >= (1ull << 31);
+  const auto kernel = wide
+                          ? &depthwiseDeltaSumKernel<OutT, PARTS, COLUMNS, true>
+                          : &depthwiseDeltaSumKernel<OutT, PARTS, COLUMNS, false>;
+  hipLaunchKernelGGL(kernel, dim3((outputs + COLUMNS - 1) / COLUMNS),
+                     dim3(PARTS * COLUMNS), 0, stream, partial, slices, taps,
+                     channels, static_cast<OutT *>(out));
+}
+
 template <class OutT>
 void launchDeltaSum(const float *partial, uint32_t slices, uint32_t taps,
                     uint32_t channels, void *out, hipStream_t stream) {
-  const uint32_t outputs = taps * channels;
-  if (outputs < kManyOutputs + uint64_t(kManyOutputsPerSlice) * slices)
-    hipLaunchKernelGGL((depthwiseDeltaSumKernel<OutT, 64, 16>),
-                       dim3((outputs + 15) / 16), dim3(1024), 0, stream,
-                       partial, slices, taps, channels,
-                       static_cast<OutT *>(out));
+  if (taps * channels < kManyOutputs + uint64_t(kManyOutputsPerSlice) * slices)
+    launchDeltaSumIn<OutT, 64, 16>(partial, slices, taps, channels, out,
+                                   stream);
   else
-    hipLaunchKernelGGL((depthwiseDeltaSumKernel<OutT, 8, 32>),
-                       dim3((outputs + 31) / 32), dim3(256), 0, stream,
-                       partial, slices, taps, channels,
-                       static_cast<OutT *>(out));
+    launchDeltaSumIn<OutT, 8, 32>(partial, slices, taps, channels, out, stream);
 }
 
 /// Threads of a workgroup: itemsPerBlock items by `slots` parts of a slice.

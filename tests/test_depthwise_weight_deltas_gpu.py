@@ -152,3 +152,21 @@ def test_columns_plan_choice():
         assert COLUMNS not in plan(**bad).describe()
         with pytest.raises(pa.MxconvError):
             plan(_options(4), **bad)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kw", [
+    # walks of four pixels: one slice, a last slice of one pixel
+    dict(batch=1, field=(3, 3), kernel=(3, 3), groups=8, pad=1),
+    dict(batch=1, field=(29, 7), kernel=(3, 3), groups=24, pad=1),
+    # 256 slices of four pixels, and a pixel more: of eight
+    dict(batch=2, field=(32, 32), kernel=(3, 3), groups=104, pad=1),
+    dict(batch=1, field=(2049, 1), kernel=(3, 3), groups=104, pad=1),
+    # of sixteen (more than 2 MB of sums with eight), stride 2, uneven padding
+    dict(batch=11, field=(12, 11), kernel=(5, 5), groups=808, stride=2, pad=2),
+    dict(batch=9, field=(11, 12), kernel=(3, 3), groups=48, stride=2,
+         padLower=(2, 0), padUpper=(0, 1))])
+def test_walks_of_small_layers_are_exact(oracle, kw):
+    """A slot's walk over the pixels is as short as the number of slices and the
+    size of their sums allow (depthwiseWeightDeltaKernel)."""
+    _signs(oracle, kw, options=_options(0))
