@@ -680,6 +680,15 @@ hipError_t launchHeight(const IgemmDesc &d, const Launch &launch) {
   return hipErrorInvalidValue;
 }
 
+/// Bytes of the weights packed for d's tile width, which a buffer has to reach.
+uint64_t flexWeightBytes(const IgemmDesc &d) {
+  const uint64_t co =
+      (uint64_t(d.outChansPerGroup) + d.blockN - 1) / d.blockN * d.blockN;
+  const uint64_t k = (uint64_t(d.kD) * d.kH * d.kW * d.inChansPerGroup + 63) /
+                     64 * 64;
+  return d.groups * co * k * 2;
+}
+
 } // namespace
 
 bool igemmFlexTile(uint32_t blockM, uint32_t blockN, uint32_t flex) {
@@ -693,6 +702,7 @@ bool igemmFlexTile(uint32_t blockM, uint32_t blockN, uint32_t flex) {
 bool igemmFlexTakes(const IgemmDesc &d, int inType, int outType) {
   return inType == kHalf && outType == kHalf &&
          igemmFlexTile(d.blockM, d.blockN, d.flex) &&
+         flexWeightBytes(d) < kOutOfRange &&
          // (whole vectors of fp32 sums, a part of them within a buffer's reach)
          (d.splitK == 1 ||
           (d.outChansPerGroup % 4 == 0 && !d.outFullH && !d.outFullW &&

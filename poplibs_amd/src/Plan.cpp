@@ -1740,8 +1740,9 @@ mxconv_plan makePlanWith(const ConvParams &params,
       if (!takes || plan.denseWeightUpdate || plan.depthwiseWeightUpdate)
         throw poplar::invalid_option(
             "planConstraints gfx950 flex: that kernel takes half inputs and "
-            "outputs, kernels of at most 32 taps and an input of which the "
-            "images that a tile's pixels meet stay under 2^31 bytes");
+            "outputs, kernels of at most 32 taps, packed weights under 2^31 "
+            "bytes and an input of which the images that a tile's pixels meet "
+            "do so too");
     }
     // A pointwise convolution with few input channels is bound by HBM, not
     // by the matrix cores: unless the big tile was asked for explicitly, the
@@ -2281,11 +2282,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
             const double us =
                 estimateFlex(bm, bn, flex == 2, tilesOf(bm, bn), kSteps, ragged,
                              outMB, inMB + weightsMB);
-            if (us >= planned ||
-                p.numConvGroups * ((co + bn - 1) / bn * bn) *
-                        ((k + 63) / 64 * 64) * 2 >=
-                    (1ull << 31) ||
-                !mxk::igemmFlexTakes(t, inId, outId))
+            if (us >= planned || !mxk::igemmFlexTakes(t, inId, outId))
               continue;
             planned = us, chosenTile = t;
           }

@@ -254,3 +254,29 @@ def test_parts_want_whole_vectors():
         pa.Plan(p, {"planConstraints": json.dumps({"gfx950": {
             "kernel": "igemm", "patch": 0, "blockM": 128, "blockN": 96,
             "flex": 1, "splitK": 2}})})
+
+
+@pytest.mark.parametrize("m,k,n", [
+    # columns that tiles of 128 fill to the last and wider ones of their own do
+    # not, whose packed weights would be 2^31 bytes and more
+    (128, 32768, 32640), (16, 70272, 15136), (300, 376192, 2816),
+    (128, 62016, 17272), (200, 89152, 12000), (512, 524096, 2048),
+    # ... and the last a buffer reaches in tiles of 128
+    (128, 16320, 65408), (4096, 8128, 130944)])
+def test_packed_weights_stay_within_a_buffer_s_reach(m, k, n):
+    from poplibs_amd import capi
+    plan = pa.MatMulPlan(pa.HALF, pa.HALF, 1, m, k, n)
+    assert "implicit GEMM" in plan.describe()
+    assert plan.buffer_bytes(capi.BUF_WEIGHTS_PACKED) < 2 ** 31
+
+
+@pytest.mark.parametrize("width,fits", [(128, True), (192, False)])
+def test_a_named_tile_whose_weights_no_buffer_reaches_is_refused(width, fits):
+    p = make_params(pa.HALF, batch=1, field=(16,), kernel=(1,), ci=32960,
+                    co=32512)
+    assert (-(-32512 // width) * width * 32960 * 2 < 2 ** 31) == fits
+    if fits:
+        pa.Plan(p, _options((128, width, 1)))
+    else:
+        with pytest.raises(pa.MxconvError, match="flex"):
+            pa.Plan(p, _options((128, width, 1)))
