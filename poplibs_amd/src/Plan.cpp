@@ -467,6 +467,46 @@ double estimateBesideFlexParts(unsigned blockN, std::size_t parts,
                       workgroups, kSteps, ragged, partialMB, inMB);
 }
 
+/// The same two for up to 128 pixels, one tile of rows, where the weights' way from
+/// memory counts beside the products, and rows that start in the middle of a line
+/// (`ragged`) cost a k-step more.  Fitted to 855 random products and layers of 4 to
+/// 128 pixels with 3 MB to 1.7 GB of weights that no cache holds, igemmFlexKernel
+/// within 5 %, igemmKernel 3 to 4.
+double besideBytes(double computeUs, double bytesUs) {
+  return std::sqrt(std::hypot(computeUs * computeUs, bytesUs * bytesUs));
+}
+double estimateFlexPartsOfFewRows(unsigned blockM, unsigned blockN,
+                                  std::size_t kSteps, std::size_t parts,
+                                  double partialMB, double weightsMB) {
+  const double area = blockM * blockN / 16384.0;
+  return 4.375 +
+         besideBytes(double(kSteps) * (0.21 + 0.412 * area),
+                     0.151 * weightsMB) +
+         0.901 * partialMB + 0.097 * double(parts);
+}
+double estimateBesideFlexPartsOfFewRows(unsigned blockN, std::size_t parts,
+                                        std::size_t workgroups,
+                                        std::size_t kSteps, std::size_t rows,
+                                        bool ragged, double partialMB,
+                                        double weightsMB) {
+  struct Fit {
+    double call, lone, step, byte, partial, ragged, whole;
+  };
+  const Fit f =
+      blockN == 64
+          ? parts == 1 ? Fit{2.926, 0.984, 0.359, 0.222, 0.256, 0.257, 0.113}
+                       : Fit{7.241, 1.013, 0.364, 0.192, 0.098, 0.225, 0.101}
+      : parts == 1 ? Fit{4.253, 0.98, 0.408, 0.151, 0.389, 0.426, 0.253}
+                   : Fit{6.55, 0.941, 0.407, 0.156, 0.673, 0.487, 0.333};
+  const double perCU = double(workgroups) / double(gfx950::numCUs);
+  const double step =
+      f.step + double(rows) / 128.0 * (ragged ? f.ragged : f.whole);
+  return f.call +
+         besideBytes(double(kSteps) * std::max(f.lone, perCU) * step,
+                     f.byte * weightsMB) +
+         f.partial * partialMB;
+}
+
 /// igemmFlexKernel is taken where it is estimated at less than these shares of
 /// what is planned.  Over the layers of the fit, at the share and (in brackets)
 /// wherever the estimate is lower at all: tiles of 128 x 128, two to a CU, 1.155
@@ -2383,6 +2423,30 @@ mxconv_plan makePlanWith(const ConvParams &params,
                 continue;
               planned = us, chosenTile = t;
             }
+      // Up to 128 pixels, where the weights' bytes count, beside tiles of igemmKernel:
+      // 3 % below the estimates that know of them.  Of 855 products and layers that
+      // the estimates above chose parts for, 217 stay as they were, among them 78 of
+      // the 82 that were more than 3 % slower in parts (12 x 2384 x 31152 30.1 ->
+      // 37.7 us, 99 x 4096 x 23768 53.0 -> 65.0); all are 1.155 times as fast as
+      // without parts, 1.145 with all of them in parts.  Beside these tiles with K
+      // whole, from K of 5 000 on: 41 such products 1.16 times as fast, ten of
+      // shorter sums 0.97.
+      if (chosenTile.flex && m <= 128) {
+        const double partialMB = 2.0 * outMB;
+        const double weightsMB = 1e-6 * double(plan.weightBytes());
+        if (g.flex
+                ? k < 5000
+                : estimateFlexPartsOfFewRows(
+                      chosenTile.blockM, chosenTile.blockN,
+                      (kSteps + chosenTile.splitK - 1) / chosenTile.splitK,
+                      chosenTile.splitK, partialMB * chosenTile.splitK,
+                      weightsMB) >=
+                      0.97 * estimateBesideFlexPartsOfFewRows(
+                                 g.blockN, g.splitK, tiles * g.splitK,
+                                 planSteps, m, ragged, partialMB * g.splitK,
+                                 weightsMB))
+          chosenTile.flex = 0;
+      }
       if (chosenTile.flex) {
         g = chosenTile;
         plan.coPadded = (co + g.blockN - 1) / g.blockN * g.blockN;

@@ -280,3 +280,20 @@ def test_a_named_tile_whose_weights_no_buffer_reaches_is_refused(width, fits):
     else:
         with pytest.raises(pa.MxconvError, match="flex"):
             pa.Plan(p, _options((128, width, 1)))
+
+
+@pytest.mark.parametrize("m,k,n,parts", [
+    # the weights' way from memory is the time: tiles of 128 x 128 and 64, K whole
+    # or in parts, fill the chip
+    (12, 2384, 31152, False), (99, 4096, 23768, False), (77, 2240, 16232, False),
+    (35, 6784, 9688, False),
+    # so do tiles of 128 x 96, of which only a longer sum leaves
+    (26, 4048, 20192, False), (14, 25184, 18648, True),
+    # ... and do not
+    (34, 10088, 5712, True), (97, 44912, 18728, True), (117, 2288, 4552, True)])
+def test_parts_of_few_rows(m, k, n, parts):
+    plan = pa.MatMulPlan(pa.HALF, pa.HALF, 1, m, k, n)
+    chosen = [line for line in plan.describe().split("\n")
+              if line.strip().startswith("*")]
+    flexible = "flexible" in chosen[0] and "parts" in chosen[0]
+    assert flexible == parts, chosen
