@@ -2517,21 +2517,26 @@ mxconv_plan makePlanWith(const ConvParams &params,
       chooseDepthwiseTileOrRing(d, pc, s.inputDilated(), dwType);
     // 3 x 3 taps that would go to the ring, whose workgroups walk a band each and
     // wait for its first rows: strips of columns where they are estimated at 5 %
-    // less.  Of 260 such layers 150 change, and all together are 1.11 times as fast
-    // (four in ten of those with more than 224 channels by 1.25 and more, 43 x 26 x
-    // 26, 336 channels 14.4 -> 9.2 us; the slowest 0.90).  Tensors of more than the
-    // 256 MB cache in front of HBM were not among them.
+    // less, 10 % below 24 MB of tensors, up to 96 MB (43 x 26 x 26, 336 channels 14.4
+    // -> 9.2 us).  With three calls' tensors in turn the 337 such layers of 467 with
+    // a lower estimate are 1.13 times as fast as in rings, the slowest 0.97; of the
+    // 130 left in rings 71 would be more than 3 % slower in strips, with up to 24 MB
+    // down to 0.92 (13 x 19 x 19, 912) and with more than 96 - which the cache of 256
+    // MB in front of HBM does not hold three times - 0.94 on average (28 x 46 x 46,
+    // 424 23.9 -> 29.0).  Strips want their input in that cache: behind a kernel that
+    // has just written it they are 1.08 and 1.03 times as fast at stride 1 and 2,
+    // from HBM 0.95 and 1.00.
+    const double tensorBytes =
+        2.0 * double(d.batch) * double(d.channels) *
+        (double(d.inH) * d.inW + double(d.outH) * d.outW);
     if (!columns && d.kH == 3 && d.kW == 3 && d.dense3x3 == 2 &&
         !plan.depthwiseWeightUpdate && pc.columns < 0 && pc.rowRing < 0 &&
-        params.outputType == poplar::HALF &&
-        2.0 * double(d.batch) * double(d.channels) *
-                (double(d.inH) * d.inW + double(d.outH) * d.outW) <=
-            256e6 &&
+        params.outputType == poplar::HALF && tensorBytes <= 96e6 &&
         mxk::depthwiseColumnsTakes(d, dwType, mxk::kHalf)) {
       mxk::DepthwiseDesc c = d;
       mxk::chooseDepthwiseColumns(c, 0);
       if (mxk::depthwiseColumnsEstimateUs(c) <
-          0.95 * mxk::depthwiseRowsEstimateUs(d)) {
+          (tensorBytes < 24e6 ? 0.9 : 0.95) * mxk::depthwiseRowsEstimateUs(d)) {
         d = c;
         d.dense3x3 = 0;
       }

@@ -110,3 +110,16 @@ def test_strips_plan_choice():
             pa.Plan(make_params(pa.HALF, **bad), options)
     with pytest.raises(pa.MxconvError):
         pa.Plan(make_params(pa.FLOAT, **kw), _options(2))
+
+
+@pytest.mark.parametrize("batch,field,groups,strips", [
+    # up to 24 MB of tensors, to 96 MB and beyond; rings that are near or ahead
+    (47, 19, 488, True), (13, 19, 912, False), (12, 43, 144, False),
+    (43, 26, 336, True), (17, 39, 792, True), (28, 46, 424, False),
+    (8, 98, 800, False)])
+def test_layers_that_rings_are_faster_for_stay(batch, field, groups, strips):
+    plan = pa.Plan(make_params(pa.HALF, batch=batch, field=(field, field),
+                               kernel=(3, 3), groups=groups, pad=1))
+    named = json.loads(plan.constraints())["gfx950"]
+    assert ("strips" in named) == strips, named
+    assert named["rowRing"] == (0 if strips else 1)
