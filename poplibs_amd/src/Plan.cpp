@@ -2339,7 +2339,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
         c.name = "flexible " + std::to_string(g.blockM) + " x " +
                  std::to_string(g.blockN);
         c.workgroups = tilesOf(g.blockM, g.blockN), c.perCU = g.flex;
-        c.kSteps = kSteps, c.estimateUs = planned;
+        c.kSteps = kSteps, c.estimateUs = plan.flexEstimateUs();
         c.rounds = roundsOf(c.workgroups, c.perCU), c.chosen = true;
         plan.candidates.push_back(c);
       }
@@ -2464,7 +2464,8 @@ mxconv_plan makePlanWith(const ConvParams &params,
                  std::to_string(g.blockN) + ", K in " +
                  std::to_string(g.splitK) + " parts";
         c.workgroups = tilesOf(g.blockM, g.blockN) * g.splitK, c.perCU = 1;
-        c.kSteps = (kSteps + g.splitK - 1) / g.splitK, c.estimateUs = planned;
+        c.kSteps = (kSteps + g.splitK - 1) / g.splitK;
+        c.estimateUs = plan.flexEstimateUs();
         c.rounds = 1.0, c.chosen = true;
         plan.candidates.push_back(c);
       }
@@ -2617,6 +2618,30 @@ std::string mxconv_plan::constraintsJson() const {
   }
   os << "}}";
   return os.str();
+}
+
+double mxconv_plan::flexEstimateUs() const {
+  const mxk::IgemmDesc &g = igemm;
+  const std::size_t m = std::size_t(g.batch) * g.outD * g.outH * g.outW;
+  const std::size_t workgroups =
+      (m + g.blockM - 1) / g.blockM *
+      ((g.outChansPerGroup + g.blockN - 1) / g.blockN) * g.groups * g.splitK;
+  const std::size_t steps = (kPadded / g.blockK + g.splitK - 1) / g.splitK;
+  const bool ragged = g.inChansPerGroup % 64 != 0;
+  const double outMB = 1e-6 * double(outputBytes());
+  const double weightsMB = 1e-6 * double(weightBytes());
+  // (a part's sums are fp32)
+  const double partialMB = 2.0 * outMB * double(g.splitK);
+  if (g.splitK == 1)
+    return poplin::estimateFlex(g.blockM, g.blockN, g.flex == 2, workgroups,
+                                steps, ragged, outMB,
+                                1e-6 * double(inputBytes()) + weightsMB);
+  return m <= 128 ? poplin::estimateFlexPartsOfFewRows(
+                        g.blockM, g.blockN, steps, g.splitK, partialMB,
+                        weightsMB)
+                  : poplin::estimateFlexParts(g.blockM, g.blockN, workgroups,
+                                              steps, g.splitK, ragged,
+                                              partialMB);
 }
 
 mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
@@ -2794,10 +2819,7 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
         (kPadded / g.blockK + g.splitK - 1) / g.splitK;
     const std::size_t perCU = g.blockN == 64 || g.stages == 2 ? 2 : 1;
     double us =
-        g.flex ? poplin::estimateFlex(
-                     g.blockM, g.blockN, g.flex == 2, tiles, steps,
-                     g.inChansPerGroup % 64 != 0, 1e-6 * double(outputBytes()),
-                     1e-6 * double(inputBytes() + weightBytes()))
+        g.flex ? flexEstimateUs()
         : g.blockM == 256
             ? poplin::estimateWide(tiles, steps, g.blockN)
             : poplin::estimateStreaming(tiles, steps, perCU, g.blockN,

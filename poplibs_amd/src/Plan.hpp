@@ -179,6 +179,8 @@ struct mxconv_plan {
     }
   };
   DetailedEstimate detailedEstimate() const;
+  /// What a call in flexible tiles (igemm.flex) is estimated at.
+  double flexEstimateUs() const;
   /// The shader clock the estimate is converted to cycles with
   /// (MXCONV_ESTIMATE_CLOCK_MHZ): what the chip holds with the matrix cores
   /// of most CUs busy.

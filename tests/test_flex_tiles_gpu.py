@@ -201,6 +201,22 @@ def test_plans_name_the_tile_and_come_back():
     assert "flex" not in without.constraints()
 
 
+@pytest.mark.parametrize("m,k,n", [
+    # taken from tiles of 256 x 256 of the other kernel, from 128 x 128; parts,
+    # of few rows too
+    (4096, 4096, 4096), (1026, 1080, 4604), (450, 7416, 1400),
+    (97, 44912, 18728)])
+def test_the_estimate_shown_is_the_call_s(m, k, n):
+    """... and not the share of it that the choice was made by: the same for the
+    plan made again from its constraints, which weighs nothing."""
+    p = pa.matMulParams(pa.HALF, pa.HALF, 1, m, k, n)
+    plan = pa.Plan(p)
+    assert json.loads(plan.constraints())["gfx950"]["flex"]
+    again = pa.Plan(p, {"planConstraints": plan.constraints()})
+    (cycles, _), (expected, _) = plan.estimated_costs(), again.estimated_costs()
+    assert abs(cycles - expected) <= 1
+
+
 @pytest.mark.parametrize("asked", [
     dict(blockM=64, blockN=64, flex=1), dict(blockM=128, blockN=48, flex=1),
     dict(blockM=256, blockN=64, flex=1), dict(blockM=192, blockN=128, flex=2),
