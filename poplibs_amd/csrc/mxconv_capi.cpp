@@ -1032,6 +1032,21 @@ mxconv_status mxconv_multi_fwd(size_t n, const mxconv_plan *const *plans,
     const uint64_t k = uint64_t(d.kD) * d.kH * d.kW * d.inChansPerGroup;
     return (k + d.blockK - 1) / d.blockK;
   };
+  // A plan of flexible tiles with K in parts can run in the tiles of another
+  // member as well: its packed weights hold whole tiles of 128 columns.  (Without
+  // that N = 15, 22 x 22, 248 channels, four layers, 5 x 5 -> 168 and -> 48 in one
+  // launch, 64.8 us instead of 55.7; N = 45, 32 x 32 stride 2, 312 -> 80 beside N =
+  // 27, 13 x 13 stride 2, 392 -> 232 38.3 instead of 31.0.)
+  auto streams = [](const mxk::IgemmDesc &d) {
+    return !d.small && !d.patch && !d.flex && d.blockM == 128;
+  };
+  auto adapts = [](const mxk::IgemmDesc &d) {
+    return d.flex && d.splitK > 1 && d.groups == 1;
+  };
+  auto asTile = [](mxk::IgemmDesc &d, const mxk::IgemmDesc &tile) {
+    d.flex = 0;
+    d.blockM = tile.blockM, d.blockN = tile.blockN, d.stages = tile.stages;
+  };
   auto fusedItem = [&](size_t i, size_t slot, mxk::IgemmFusedItem &item) {
     const mxconv_plan *p = plans[i];
     // (a plan with more to a launch than its one kernel - a padded copy of
@@ -1053,6 +1068,11 @@ mxconv_status mxconv_multi_fwd(size_t n, const mxconv_plan *const *plans,
             quarter(i)};
     return true;
   };
+  const auto fusable = [&](const mxk::IgemmFusedItem &x,
+                           const mxk::IgemmFusedItem &y) {
+    return x.d->small || y.d->small ? mxk::igemmSmallFusable(x, y)
+                                    : mxk::igemmFusable(x, y);
+  };
   std::vector<bool> done(n, false);
   for (size_t i = 0; i != n; ++i) {
     if (done[i])
@@ -1061,43 +1081,76 @@ mxconv_status mxconv_multi_fwd(size_t n, const mxconv_plan *const *plans,
     mxk::IgemmFusedItem group[mxk::kIgemmMaxFused];
     size_t member[mxk::kIgemmMaxFused] = {i};
     size_t members = 0;
-    double alone = 0, together = 0;
-    const auto fusable = [&](const mxk::IgemmFusedItem &x,
-                             const mxk::IgemmFusedItem &y) {
-      return x.d->small || y.d->small ? mxk::igemmSmallFusable(x, y)
-                                      : mxk::igemmFusable(x, y);
-    };
-    if (parallel && fusedItem(i, 0, group[0])) {
+    bool adapted = false;
+    // Members that share convolution i's launch (adapt: in another member's
+    // tiles, too); whether they are estimated to gain by it.
+    const auto gather = [&](bool adapt) {
+      members = 0, adapted = false;
+      if (!fusedItem(i, 0, group[0]))
+        return false;
       members = 1;
+      if (adapt && adapts(plans[i]->igemm)) {
+        // the tiles of the first other member that has some of igemmKernel, or
+        // tiles of 128 x 64 where two such plans differ
+        const mxk::IgemmDesc own = unsplit[0];
+        mxk::IgemmDesc narrow = own;
+        narrow.blockM = 128, narrow.blockN = 64, narrow.stages = 4;
+        for (size_t j = i + 1; j != n && unsplit[0].flex; ++j) {
+          mxk::IgemmFusedItem item;
+          if (done[j] || !fusedItem(j, 1, item))
+            continue;
+          if (adapts(plans[j]->igemm) && !fusable(group[0], item))
+            asTile(unsplit[1], narrow);
+          if (!streams(unsplit[1]))
+            continue;
+          asTile(unsplit[0], unsplit[1]);
+          if (!fusable(group[0], item))
+            unsplit[0] = own;
+        }
+        adapted = !unsplit[0].flex;
+      }
       for (size_t j = i + 1; j != n && members != mxk::kIgemmMaxFused; ++j) {
         mxk::IgemmFusedItem item;
-        if (!done[j] && fusedItem(j, members, item) &&
-            fusable(group[0], item)) {
-          member[members] = j;
-          group[members++] = item;
-        }
+        if (done[j] || !fusedItem(j, members, item))
+          continue;
+        const bool other = adapt && adapts(plans[j]->igemm) &&
+                           streams(unsplit[0]);
+        if (other)
+          asTile(unsplit[members], unsplit[0]);
+        if (!fusable(group[0], item))
+          continue;
+        adapted = adapted || other;
+        member[members] = j;
+        group[members++] = item;
       }
+      double alone = 0;
       uint64_t tiles = 0, longest = 0;
       for (size_t k = 0; k != members; ++k) {
         const mxk::IgemmDesc &planned = plans[member[k]]->igemm;
-        const uint64_t steps = kStepsOf(planned), own = tilesOf(planned);
-        const uint64_t rounds = (own * planned.splitK + 255) / 256;
-        alone += 6 + 0.3 * double((steps + planned.splitK - 1) /
-                                  planned.splitK * rounds) +
-                 (planned.splitK != 1 ? 5 : 0);
-        tiles += own;
+        const uint64_t steps = kStepsOf(planned);
+        const uint64_t rounds = (tilesOf(planned) * planned.splitK + 255) / 256;
+        alone += planned.flex && !unsplit[k].flex
+                     ? plans[member[k]]->flexEstimateUs()
+                     : 6 + 0.3 * double((steps + planned.splitK - 1) /
+                                        planned.splitK * rounds) +
+                           (planned.splitK != 1 ? 5 : 0);
+        tiles += tilesOf(unsplit[k]);
         longest = std::max(longest, steps);
       }
-      together = 6 + 0.3 * double(longest * ((tiles + 255) / 256));
-    }
+      const double together = 6 + 0.3 * double(longest * ((tiles + 255) / 256));
+      // (small-tile convolutions cost little but their launch)
+      return members >= 2 && (group[0].d->small || together < alone);
+    };
+    bool fuse = parallel && gather(true);
+    if (!fuse && adapted)
+      fuse = gather(false);
     mxconv_status st;
-    // (small-tile convolutions cost little but their launch)
-    const bool small = members != 0 && group[0].d->small;
-    if (members >= 2 && (small || together < alone)) {
+    if (fuse) {
       for (size_t k = 0; k != members; ++k)
         done[member[k]] = true;
-      st = hipStatus(small ? mxk::launchIgemmSmallFused(group, members, s)
-                           : mxk::launchIgemmFused(group, members, s),
+      st = hipStatus(group[0].d->small
+                         ? mxk::launchIgemmSmallFused(group, members, s)
+                         : mxk::launchIgemmFused(group, members, s),
                      "fused implicit-GEMM convolution launch");
     } else {
       st = forward(plans[i], in[i], weights_packed[i],

@@ -507,6 +507,13 @@ double estimateBesideFlexPartsOfFewRows(unsigned blockN, std::size_t parts,
          f.partial * partialMB;
 }
 
+/// Columns of the packed weights of a product in flexible tiles with K in parts:
+/// whole tiles of 128 besides its own, so that it can share the launch of several
+/// convolutions in tiles of igemmKernel (mxconv_multi_fwd).
+std::size_t flexPartsColumns(std::size_t co, std::size_t blockN) {
+  return std::max((co + blockN - 1) / blockN * blockN, (co + 127) / 128 * 128);
+}
+
 /// igemmFlexKernel is taken where it is estimated at less than these shares of
 /// what is planned.  Over the layers of the fit, at the share and (in brackets)
 /// wherever the estimate is lower at all: tiles of 128 x 128, two to a CU, 1.155
@@ -1615,6 +1622,10 @@ mxconv_plan makePlanWith(const ConvParams &params,
       if (s.hasDepth() && s.inputDilated())
         parts = 1;
       g.splitK = uint32_t(parts);
+      if (g.flex && parts > 1 && p.numConvGroups == 1) {
+        plan.coPadded = flexPartsColumns(co, g.blockN);
+        plan.weightPackedElems = plan.coPadded * plan.kPadded;
+      }
       plan.workspaceBytes = mxk::igemmWorkspaceBytes(g);
       if (ciPadded != ci) {
         plan.paddedInputChans = ciPadded;
@@ -2449,7 +2460,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
       }
       if (chosenTile.flex) {
         g = chosenTile;
-        plan.coPadded = (co + g.blockN - 1) / g.blockN * g.blockN;
+        plan.coPadded = flexPartsColumns(co, g.blockN);
         plan.kPadded = kSteps * 64;
         plan.weightPackedElems = plan.coPadded * plan.kPadded;
         plan.workspaceBytes = mxk::igemmWorkspaceBytes(g);
@@ -2813,8 +2824,9 @@ mxconv_plan::DetailedEstimate mxconv_plan::detailedEstimate() const {
       break;
     const auto &g = igemm;
     const std::size_t m = std::size_t(g.batch) * g.outD * g.outH * g.outW;
-    const std::size_t tiles = (m + g.blockM - 1) / g.blockM * (coPadded / g.blockN) *
-                              g.groups * g.splitK;
+    const std::size_t tiles =
+        (m + g.blockM - 1) / g.blockM *
+        ((g.outChansPerGroup + g.blockN - 1) / g.blockN) * g.groups * g.splitK;
     const std::size_t steps =
         (kPadded / g.blockK + g.splitK - 1) / g.splitK;
     const std::size_t perCU = g.blockN == 64 || g.stages == 2 ? 2 : 1;
@@ -2929,8 +2941,9 @@ std::string mxconv_plan::describe() const {
     const std::size_t m = std::size_t(g.batch) * g.outD * g.outH * g.outW;
     const std::size_t k =
         std::size_t(g.kD) * g.kH * g.kW * g.inChansPerGroup;
-    const std::size_t tiles = (m + g.blockM - 1) / g.blockM *
-                              (coPadded / g.blockN) * g.groups;
+    const std::size_t tiles =
+        (m + g.blockM - 1) / g.blockM *
+        ((g.outChansPerGroup + g.blockN - 1) / g.blockN) * g.groups;
     os << "        gemm M x N x K             " << m << " x "
        << g.outChansPerGroup << " x " << k << " (x " << g.groups
        << " groups)\n";

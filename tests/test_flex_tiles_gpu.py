@@ -188,6 +188,82 @@ def test_a_multi_convolution_in_one_launch(bias):
         assert torch.equal(got, expected)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("layers,shared", [
+    # (batch, field, kernel, channels, stride): K in parts beside tiles of 128 x
+    # 64, before and behind them; in two shapes of its own; beside too many tiles
+    # to gain by it
+    ([(27, 13, 3, 392, 232, 2), (45, 32, 3, 312, 80, 2)], True),
+    ([(15, 22, 5, 248, 168, 1), (15, 22, 5, 248, 48, 1)], True),
+    ([(7, 22, 5, 392, 312, 1), (6, 21, 5, 392, 264, 1)], True),
+    ([(45, 32, 3, 312, 80, 2), (15, 22, 5, 248, 168, 1)], False),
+    ([(22, 27, 5, 352, 72, 1), (22, 27, 3, 352, 56, 1)], False)])
+def test_k_in_parts_shares_a_launch(layers, shared):
+    """Sums of K in parts are rounded elsewhere than those of K whole: the bytes
+    tell which of the two ran."""
+    import torch
+    from poplibs_amd import capi
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(6)
+    s = torch.cuda.current_stream().cuda_stream
+
+    def run(plan, x, w, bias, out, work):
+        packed = torch.empty(plan.buffer_bytes(capi.BUF_WEIGHTS_PACKED),
+                             dtype=torch.uint8, device=dev)
+        plan.pack_weights(w.data_ptr(), packed.data_ptr(), s)
+        plan.fwd(x.data_ptr(), packed.data_ptr(), out.data_ptr(),
+                 bias.data_ptr(), work.data_ptr(), work.numel(), s)
+        return packed
+
+    plans, ins, packed, biases, outs, works = [], [], [], [], [], []
+    own, whole, flexible = [], [], []
+    for batch, field, kernel, ci, co, stride in layers:
+        p = make_params(pa.HALF, batch=batch, field=(field, field),
+                        kernel=(kernel, kernel), ci=ci, co=co, stride=stride,
+                        pad=kernel // 2)
+        plan = pa.Plan(p)
+        named = json.loads(plan.constraints())["gfx950"]
+        flexible.append(bool(named.get("flex")) and named["splitK"] > 1)
+
+        def values(which):
+            n = plan.buffer_bytes(which) // 2
+            return torch.randn(n, generator=gen, device=dev).half()
+        x, w = values(capi.BUF_INPUT), values(capi.BUF_WEIGHTS_EXTERNAL)
+        bias = torch.randn(co, generator=gen, device=dev).half()
+        out = values(capi.BUF_OUTPUT)
+        work = torch.empty(max(plan.buffer_bytes(capi.BUF_WORKSPACE), 16),
+                           dtype=torch.uint8, device=dev)
+        own.append(out.clone()), whole.append(out.clone())
+        packed.append(run(plan, x, w, bias, own[-1], work))
+        run(pa.Plan(p, {"planConstraints": json.dumps({"gfx950": dict(
+            kernel="igemm", patch=0, pointwise=0, blockM=128, blockN=64,
+            splitK=1)})}), x, w, bias, whole[-1], work)
+        plans.append(plan), ins.append(x), biases.append(bias)
+        outs.append(out), works.append(work)
+    assert any(flexible)
+    pa.multi_fwd(plans, [x.data_ptr() for x in ins],
+                 [w.data_ptr() for w in packed], [o.data_ptr() for o in outs],
+                 biases=[b.data_ptr() for b in biases],
+                 workspaces=[w.data_ptr() for w in works],
+                 workspace_bytes=[w.numel() for w in works], stream=s)
+    torch.cuda.synchronize()
+    for got, alone, k_whole, parts in zip(outs, own, whole, flexible):
+        assert torch.equal(got, k_whole if shared else alone)
+        assert not parts or not torch.equal(alone, k_whole)
+
+
+@pytest.mark.parametrize("m,k,n", [(133, 4872, 5488), (450, 7416, 1400)])
+def test_packed_weights_of_parts_hold_whole_tiles_of_128(m, k, n):
+    from poplibs_amd import capi
+    p = pa.matMulParams(pa.HALF, pa.HALF, 1, m, k, n)
+    plan = pa.Plan(p)
+    again = pa.Plan(p, {"planConstraints": plan.constraints()})
+    assert json.loads(plan.constraints())["gfx950"]["splitK"] > 1
+    rows = plan.buffer_bytes(capi.BUF_WEIGHTS_PACKED) // (-(-k // 64) * 128)
+    assert rows >= -(-n // 128) * 128
+    assert again.packs_like(plan)
+
+
 def test_plans_name_the_tile_and_come_back():
     p = make_params(pa.HALF, batch=25, field=(57, 57), kernel=(3, 3), ci=136,
                     co=200, pad=1)
