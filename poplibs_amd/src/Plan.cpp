@@ -2283,6 +2283,16 @@ mxconv_plan makePlanWith(const ConvParams &params,
                // tile: 190 x 15 x 15, 5 x 5, 4 groups of 720 -> 80 532 us, 799 in
                // tiles of 256 x 96)
                (p.numConvGroups == 1 || (!g.patch && !plan.pointwiseOn)) &&
+               // (large pointwise layers of 392 to 512 input channels: their time
+               // is their tensors' way, which igemmFlexKernel's estimate, of
+               // tensors in the cache, makes too little of.  111 layers of 50 to
+               // 200 MB, 136 to 800 channels out, were 0.93 times as fast with
+               // three calls' tensors in turn and 0.98 with one's, N = 101, 49 x
+               // 14, 408 -> 432 44.4 us and 56.9; 38 larger ones 1.32 and 0.93, 101
+               // of 264 to 384 channels in 1.08 and 1.14)
+               !(plan.pointwiseOn && k > 384 && co <= 800 &&
+                 plan.inputBytes() + plan.outputBytes() > 50000000 &&
+                 plan.inputBytes() + plan.outputBytes() < 200000000) &&
                // (below, a call costs its launch, whatever the tile)
                2.0 * double(s.batch) * s.outD * s.outH * s.outW * double(co) *
                        double(k) * p.numConvGroups >=

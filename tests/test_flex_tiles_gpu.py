@@ -339,6 +339,22 @@ def test_parts_of_sums_over_more_outputs(m, k, n, parts):
     assert plan.buffer_bytes(capi.BUF_WORKSPACE) <= 32 << 20
 
 
+@pytest.mark.parametrize("batch,field,ci,co,flexible", [
+    # many input channels, tensors of 116, 110 and 153 MB; of 41 and 390; fewer
+    # channels; a large product of few rows
+    (101, (49, 14), 408, 432, False), (109, (26, 26), 432, 312, False),
+    (88, (31, 31), 432, 472, False), (27, (32, 30), 416, 464, True),
+    (112, (28, 52), 448, 744, True), (81, (45, 32), 280, 504, True),
+    (1, (6972,), 464, 9976, True)])
+def test_large_pointwise_layers_stay_with_their_kernel(batch, field, ci, co,
+                                                       flexible):
+    p = make_params(pa.HALF, batch=batch, field=field, kernel=(1,) * len(field),
+                    ci=ci, co=co)
+    named = json.loads(pa.Plan(p).constraints())["gfx950"]
+    assert ("flex" in named) == flexible, named
+    assert bool(named["pointwise"]) != flexible
+
+
 def test_parts_want_whole_vectors():
     p = make_params(pa.HALF, batch=2, field=(9, 9), kernel=(3, 3), ci=64,
                     co=66, pad=1)
