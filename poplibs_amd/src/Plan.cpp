@@ -2420,7 +2420,17 @@ mxconv_plan makePlanWith(const ConvParams &params,
       mxk::IgemmDesc chosenTile = g;
       chosenTile.flex = 0;
       const std::size_t narrow = tilesOf(128, 64);
-      if ((narrow <= 260 ? g.flex || g.splitK > 1 || g.blockN == 64
+      // (windows of up to 128 channels on many pixels fetch more than they
+      // multiply once the L2s no longer hold their input: of 56 layers of 8 200 to
+      // 16 300 pixels whose input is larger than the bounds below 37 were more than
+      // 3 % slower in parts, 0.95 times as fast on average, N = 9, 45 x 30, 3 x 3, 616
+      // -> 120 33.5 us and 41.9; of 65 with fewer pixels or a smaller input two,
+      // 1.13)
+      const bool wideWindows =
+          s.kD * s.kH * s.kW > 1 && co <= 128 && m > 8200 &&
+          plan.inputBytes() > (g.splitK > 1 ? 7500000u : 10500000u);
+      if (!wideWindows &&
+          (narrow <= 260 ? g.flex || g.splitK > 1 || g.blockN == 64
                          : narrow <= 800 && co >= 192) &&
           2.0 * double(m) * double(co) * double(k) >= 4e8)
         for (uint32_t bm : {128u, 192u, 256u})

@@ -355,6 +355,19 @@ def test_large_pointwise_layers_stay_with_their_kernel(batch, field, ci, co,
     assert bool(named["pointwise"]) != flexible
 
 
+@pytest.mark.parametrize("kw,parts", [
+    # up to 128 channels: many pixels of a large input, planned with K whole or
+    # in parts; fewer of them, a smaller input; more channels
+    (dict(batch=9, field=(45, 30), kernel=(3, 3), ci=616, co=120, pad=1), False),
+    (dict(batch=7, field=(35, 35), kernel=(5, 5), ci=520, co=104, pad=2), False),
+    (dict(batch=6, field=(31, 31), kernel=(5, 5), ci=696, co=80, pad=2), True),
+    (dict(batch=15, field=(35, 25), kernel=(5, 5), ci=312, co=72, pad=2), True),
+    (dict(batch=9, field=(32, 32), kernel=(5, 5), ci=576, co=136, pad=2), True)])
+def test_parts_of_windows_on_many_pixels(kw, parts):
+    named = json.loads(pa.Plan(make_params(pa.HALF, **kw)).constraints())["gfx950"]
+    assert ("flex" in named and named["splitK"] > 1) == parts, named
+
+
 def test_parts_want_whole_vectors():
     p = make_params(pa.HALF, batch=2, field=(9, 9), kernel=(3, 3), ci=64,
                     co=66, pad=1)
