@@ -2338,6 +2338,12 @@ mxconv_plan makePlanWith(const ConvParams &params,
           for (uint32_t flex : {1u, 2u}) {
             if (!mxk::igemmFlexTile(bm, bn, flex) || (bn > 64 && co <= 64))
               continue;
+            // (two workgroups to a CU fetch windows of an input beyond the L2s
+            // twice as far apart: seven such layers of 48 to 242 MB 0.96 times as
+            // fast as in tiles of 128 x 64, N = 99, 61 x 61, 5 x 5, 328 -> 40 626 us
+            // and 834, one to a CU 550; up to 45 MB eight 1.09)
+            if (flex == 2 && bn == 64 && taps > 1 && plan.inputBytes() > 45000000)
+              continue;
             mxk::IgemmDesc t = g;
             t.patch = 0, t.blockM = bm, t.blockN = bn, t.flex = flex;
             const double us =

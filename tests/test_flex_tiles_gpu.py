@@ -368,6 +368,18 @@ def test_parts_of_windows_on_many_pixels(kw, parts):
     assert ("flex" in named and named["splitK"] > 1) == parts, named
 
 
+@pytest.mark.parametrize("batch,field,ci,co,shared", [
+    # 242 and 49 MB of input; 13 and 37
+    (99, 61, 328, 40, False), (99, 27, 336, 24, False),
+    (18, 61, 96, 48, True), (28, 50, 264, 56, True)])
+def test_two_narrow_tiles_to_a_cu_want_a_small_input(batch, field, ci, co,
+                                                     shared):
+    p = make_params(pa.HALF, batch=batch, field=(field, field), kernel=(5, 5),
+                    ci=ci, co=co, pad=2)
+    named = json.loads(pa.Plan(p).constraints())["gfx950"]
+    assert (named.get("flex") == 2) == shared, named
+
+
 def test_parts_want_whole_vectors():
     p = make_params(pa.HALF, batch=2, field=(9, 9), kernel=(3, 3), ci=64,
                     co=66, pad=1)
