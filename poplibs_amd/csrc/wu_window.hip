@@ -320,7 +320,10 @@ __global__ __launch_bounds__(64 * NW) void wuWindowKernel(
   // (Pinned: left to itself the compiler issues them behind those.)  No k-step
   // beyond the wave's last is multiplied: an odd count rounded up cost 5 % of
   // the pass over 42 layers, up to 15 (10 x 31 x 31 stride 2, 56 -> 56 8.8 us,
-  // 7.6; 5 x 30 x 30 stride 2, 160 -> 88 10.1, 8.8).  Loads a k-step further ahead
+  // 7.6; 5 x 30 x 30 stride 2, 160 -> 88 10.1, 8.8).  It is the loop that ends
+  // early, not its body in the middle: with a way out between the two halves 446
+  // layers are 4 % slower, those of long walks and 32 groups up to 10 (32 x 42 x 42,
+  // 32 groups of 8 30.5 us, 26.8).  Loads a k-step further ahead
   // gain nothing, and neither do fewer instructions: 82 requests of 128 bytes
   // to the L2 per k-step of 64 x 32 channels, most of them for half a line or
   // two halves, keep the way from there busy.
@@ -328,20 +331,18 @@ __global__ __launch_bounds__(64 * NW) void wuWindowKernel(
   uint32_t at = u0 + wave * kWinUnits;
   Raw even, odd;
   load(even, at);
-  while (at < u1) {
+  for (; at + kStride < u1; at += 2 * kStride) {
     load(odd, at + kStride);
     __builtin_amdgcn_sched_barrier(0);
     multiply(even);
     __builtin_amdgcn_sched_barrier(0);
-    at += kStride;
-    if (at >= u1)
-      break;
-    load(even, at + kStride);
+    load(even, at + 2 * kStride);
     __builtin_amdgcn_sched_barrier(0);
     multiply(odd);
     __builtin_amdgcn_sched_barrier(0);
-    at += kStride;
   }
+  if (at < u1)
+    multiply(even);
 
   storeWindow<JO, JI, KW, NW>(a, place, acc, lds, out);
 }
@@ -478,20 +479,18 @@ __global__ __launch_bounds__(64 * NW) void wuWindowFloatKernel(
   uint32_t at = u0 + wave * kWinUnits;
   Raw even, odd;
   load(even, at);
-  while (at < u1) {
+  for (; at + kStride < u1; at += 2 * kStride) {
     load(odd, at + kStride);
     __builtin_amdgcn_sched_barrier(0);
     both(even);
     __builtin_amdgcn_sched_barrier(0);
-    at += kStride;
-    if (at >= u1)
-      break;
-    load(even, at + kStride);
+    load(even, at + 2 * kStride);
     __builtin_amdgcn_sched_barrier(0);
     both(odd);
     __builtin_amdgcn_sched_barrier(0);
-    at += kStride;
   }
+  if (at < u1)
+    both(even);
   storeWindow<J, J, KW, NW>(a, place, acc, lds, out);
 }
 

@@ -75,6 +75,27 @@ def test_window_weight_deltas_of_signs_are_exact(oracle, kw):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [pa.HALF, pa.FLOAT])
+@pytest.mark.parametrize("steps", [7, 8, 9, 16, 17, 25])
+def test_waves_with_odd_and_even_counts_of_steps(oracle, dtype, steps):
+    """A workgroup's waves (eight, or sixteen or four with fp32 tensors) take a
+    chunk's k-steps in turn, two to a round of their loop: none, an even number,
+    an odd one, and both in one workgroup."""
+    from test_weight_update import run_weight_update
+    p = make_params(dtype, pa.FLOAT, batch=1, field=(4 * steps - 1, 8),
+                    kernel=(3, 3), ci=256, co=512, pad=1)
+    print("case", dtype, steps, flush=True)
+    x, dz = _signs(p, 76)
+    np_type = np.float16 if dtype == pa.HALF else np.float32
+    got, plan = run_weight_update(p, x.astype(np_type), dz.astype(np_type),
+                                  BY_NAME if dtype == pa.HALF else {})
+    assert WINDOW in plan.describe(), plan.describe()
+    assert "chunks of %d k-steps" % steps in plan.describe(), plan.describe()
+    np.testing.assert_array_equal(
+        got, oracle.weight_deltas(p, x, dz, threads=8))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kw", [
     # odd channels in groups: copies filled up to whole vectors, of both
     # tensors or of one; groups that stay by themselves, that run as one, a
