@@ -1034,9 +1034,8 @@ mxconv_status mxconv_multi_fwd(size_t n, const mxconv_plan *const *plans,
   };
   // A plan of flexible tiles with K in parts can run in the tiles of another
   // member as well: its packed weights hold whole tiles of 128 columns.  (Without
-  // that N = 15, 22 x 22, 248 channels, four layers, 5 x 5 -> 168 and -> 48 in one
-  // launch, 64.8 us instead of 55.7; N = 45, 32 x 32 stride 2, 312 -> 80 beside N =
-  // 27, 13 x 13 stride 2, 392 -> 232 38.3 instead of 31.0.)
+  // that N = 15, 22 x 22, 248 channels, four layers, of which 5 x 5 -> 168 and -> 48
+  // share one, 64.8 us, 56.2 so.)
   auto streams = [](const mxk::IgemmDesc &d) {
     return !d.small && !d.patch && !d.flex && d.blockM == 128;
   };

@@ -322,7 +322,7 @@ __global__ __launch_bounds__(64 * NW) void wuWindowKernel(
   // the pass over 42 layers, up to 15 (10 x 31 x 31 stride 2, 56 -> 56 8.8 us,
   // 7.6; 5 x 30 x 30 stride 2, 160 -> 88 10.1, 8.8).  It is the loop that ends
   // early, not its body in the middle: with a way out between the two halves 446
-  // layers are 4 % slower, those of long walks and 32 groups up to 10 (32 x 42 x 42,
+  // layers are 3 % slower, those of long walks and 32 groups up to 10 (32 x 42 x 42,
   // 32 groups of 8 30.5 us, 26.8).  Loads a k-step further ahead
   // gain nothing, and neither do fewer instructions: 82 requests of 128 bytes
   // to the L2 per k-step of 64 x 32 channels, most of them for half a line or

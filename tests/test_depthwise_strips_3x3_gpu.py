@@ -74,6 +74,33 @@ def test_infinities_stay_in_their_windows(oracle, stride, strips):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("which", ["acts", "weights", "both"])
+@pytest.mark.parametrize("strips", [2, 4])
+@pytest.mark.parametrize("stride", [1, 2])
+def test_subnormal_halves_are_exact(oracle, stride, strips, which):
+    """Subnormals (multiples of 2^-24 below 2^-14) against signs, and against
+    each other: the sums are below 2^24 of their unit, which fp32 holds."""
+    from gpu_helpers import run_conv
+    p = make_params(pa.HALF, pa.FLOAT, batch=2, field=(17, 13), kernel=(3, 3),
+                    groups=24, stride=stride, pad=1)
+    print("case", stride, strips, which, flush=True)
+    acts, weights, _ = random_data(p, 73, "pm1")
+    rng = np.random.default_rng(73)
+
+    def small(like):
+        return like * rng.integers(1, 256, like.shape) * 2.0 ** -24
+
+    if which != "weights":
+        acts = small(acts)
+    if which != "acts":
+        weights = small(weights)
+    got = run_conv(p, acts.astype(np.float16), weights.astype(np.float16),
+                   None, _options(strips))
+    np.testing.assert_array_equal(
+        got, oracle.convolution(p, acts, weights, threads=8))
+
+
+@pytest.mark.gpu
 def test_the_planner_s_own_strips(oracle):
     from gpu_helpers import quantize, run_conv
     p = make_params(pa.HALF, pa.HALF, batch=12, field=(13, 13), kernel=(3, 3),

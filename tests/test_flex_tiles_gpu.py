@@ -103,9 +103,9 @@ def test_k_in_parts(oracle, tile, parts, kw):
 
 
 @pytest.mark.gpu
-def test_the_planner_s_own_parts(oracle):
-    """A long sum over few outputs, ragged channels filled up in a copy behind
-    the parts' sums."""
+def test_channels_filled_up_behind_the_parts_sums(oracle):
+    """Ragged channels, whose copy lies behind the parts' sums in the
+    workspace."""
     from test_fast_gpu import _run
     p = make_params(pa.HALF, batch=6, field=(16, 15), kernel=(3, 3), ci=845,
                     co=132, pad=1)
@@ -114,9 +114,25 @@ def test_the_planner_s_own_parts(oracle):
                                   '"splitK": 20}}'}
     assert "845 -> 848" in pa.Plan(p, options).describe()
     _run(oracle, p, 94, 1e-3, "implicit GEMM", wscale=0.05, options=options)
-    q = pa.matMulParams(pa.HALF, pa.HALF, 1, 133, 4872, 5488)
-    named = json.loads(pa.Plan(q).constraints())["gfx950"]
-    assert named["flex"] == 1 and named["splitK"] > 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p,filled", [
+    (pa.matMulParams(pa.HALF, pa.HALF, 1, 133, 4872, 2744), None),
+    (pa.matMulParams(pa.HALF, pa.HALF, 1, 480, 2407, 1040), "2407 -> 2408"),
+    (make_params(pa.HALF, batch=8, field=(28, 33), kernel=(3, 3), ci=515,
+                 co=144, pad=1), "515 -> 520")])
+def test_the_planner_s_own_parts(oracle, p, filled):
+    """K in parts as the planner itself cuts it, channels filled up in a copy
+    among them."""
+    from test_fast_gpu import _run
+    plan = pa.Plan(p)
+    print("case", p, flush=True)
+    named = json.loads(plan.constraints())["gfx950"]
+    assert named["flex"] == 1 and named["splitK"] > 1, named
+    assert ("input channels padded" in plan.describe()) == bool(filled)
+    assert not filled or filled in plan.describe(), plan.describe()
+    _run(oracle, p, 95, 1e-3, "implicit GEMM", wscale=0.05)
 
 
 @pytest.mark.gpu
@@ -127,13 +143,6 @@ def test_the_planner_s_own_parts(oracle):
     # a phase of which no tap meets an input element
     (dict(batch=2, field=(9, 9), kernel=(1, 1), ci=64, co=136, idil=2), 4)])
 def test_phases_in_one_launch(oracle, tile, kw, phases):
-    from test_fast_gpu import _run
-    p = make_params(pa.HALF, **kw)
-    try:
-        pa.Plan(p, _options(tile))
-    except pa.MxconvError:
-        assert kw["kernel"] == (1, 1)
-        return
     _exact(oracle, tile, kw, phases)
 
 
@@ -145,6 +154,98 @@ def test_the_planner_s_own_phases(oracle):
     assert "128 x 160 x 64" in pa.Plan(p).describe()
     from test_fast_gpu import _run
     _run(oracle, p, 92, 0, "implicit GEMM", dist="pm1")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,parts,co", [
+    *[(tile, 1, co) for tile in ((128, 96, 2), (192, 160, 1), (256, 256, 1))
+      for co in (33, 72, 268)],
+    ((128, 128, 1), 3, 72), ((128, 128, 1), 3, 268)])
+def test_results_and_biases_anywhere(tile, parts, co):
+    """A result that starts at a multiple of 16 bytes leaves through the L2 in
+    rows of whole vectors, from 8 bytes or an element further on as whole vectors
+    by way of it; a bias may start at any element.  The same bytes each time,
+    nothing in front or behind."""
+    import torch
+    from poplibs_amd import capi
+    options = _options(tile)
+    named = json.loads(options["planConstraints"])
+    named["gfx950"]["splitK"] = parts
+    p = make_params(pa.HALF, batch=3, field=(11, 12), kernel=(3, 3), ci=72,
+                    co=co, pad=1)
+    print("case", tile, parts, co, flush=True)
+    plan = pa.Plan(p, {"planConstraints": json.dumps(named)})
+    dev, s = torch.device("cuda:0"), torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator(device=dev).manual_seed(8)
+
+    def randoms(n):
+        return torch.randn(n, generator=gen, device=dev).half()
+    x, w = randoms(3 * 11 * 12 * 72), randoms(co * 72 * 9)
+    bias = randoms(co)
+    packed = torch.empty(plan.buffer_bytes(capi.BUF_WEIGHTS_PACKED),
+                         dtype=torch.uint8, device=dev)
+    work = torch.empty(max(plan.buffer_bytes(capi.BUF_WORKSPACE), 16),
+                       dtype=torch.uint8, device=dev)
+    plan.pack_weights(w.data_ptr(), packed.data_ptr(), s)
+    size, guard, outs = 3 * 11 * 12 * co * 2, 64, []
+    for off in (0, 8, 2):
+        for first in (0, 1):
+            moved = torch.zeros(co + 1, device=dev).half()
+            moved[first:first + co] = bias
+            buf = torch.full((size + 2 * guard + 8,), 0x5A, dtype=torch.uint8,
+                             device=dev)
+            assert buf.data_ptr() % 16 == 0 and moved.data_ptr() % 16 == 0
+            plan.fwd(x.data_ptr(), packed.data_ptr(),
+                     buf.data_ptr() + guard + off, moved.data_ptr() + 2 * first,
+                     work.data_ptr(), work.numel(), s)
+            torch.cuda.synchronize()
+            assert bool((buf[:guard + off] == 0x5A).all())
+            assert bool((buf[guard + off + size:] == 0x5A).all())
+            outs.append(buf[guard + off:guard + off + size].clone())
+    for other in outs[1:]:
+        assert torch.equal(outs[0], other)
+    ref = torch.nn.functional.conv2d(
+        x.float().cpu().reshape(3, 11, 12, 72).permute(0, 3, 1, 2),
+        w.float().cpu().reshape(co, 72, 3, 3), bias.float().cpu(), padding=1)
+    got = outs[0].view(torch.float16).float().cpu().reshape(
+        3, 11, 12, co).permute(0, 3, 1, 2)
+    # fp32 sums of halves, rounded once
+    assert (got - ref).norm() <= 1e-3 * ref.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [(128, 64, 1), (192, 96, 2)])
+def test_an_input_beyond_two_gigabytes(tile):
+    """Offsets count from the first image that a tile reads: every image of such
+    a batch as it comes out alone."""
+    import torch
+    from poplibs_amd import capi
+    kw = dict(field=(512, 512), kernel=(3, 3), ci=256, co=16, pad=1)
+    plans = [pa.Plan(make_params(pa.HALF, batch=b, **kw), _options(tile))
+             for b in (17, 1)]
+    assert plans[0].buffer_bytes(capi.BUF_INPUT) > 2 ** 31
+    print("case", tile, flush=True)
+    dev, s = torch.device("cuda:0"), torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator(device=dev).manual_seed(9)
+    x = torch.randn((17, 512, 512, 256), generator=gen, device=dev,
+                    dtype=torch.float16)
+    w = torch.randn((16, 256, 3, 3), generator=gen, device=dev,
+                    dtype=torch.float16) * 0.02
+
+    def run(plan, images):
+        packed, out = (torch.empty(plan.buffer_bytes(b), dtype=torch.uint8,
+                                   device=dev)
+                       for b in (capi.BUF_WEIGHTS_PACKED, capi.BUF_OUTPUT))
+        plan.pack_weights(w.data_ptr(), packed.data_ptr(), s)
+        plan.fwd(images.data_ptr(), packed.data_ptr(), out.data_ptr(), None,
+                 None, 0, s)
+        torch.cuda.synchronize()
+        return out.view(torch.float16).view(-1, 512, 512, 16)
+
+    got = run(plans[0], x)
+    for image in (0, 7, 8, 15, 16):
+        assert torch.equal(got[image], run(plans[1], x[image])[0]), image
+    assert torch.isfinite(got).all() and got.abs().max() > 0
 
 
 @pytest.mark.gpu
@@ -190,14 +291,14 @@ def test_a_multi_convolution_in_one_launch(bias):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("layers,shared", [
-    # (batch, field, kernel, channels, stride): K in parts beside tiles of 128 x
-    # 64, before and behind them; in two shapes of its own; beside too many tiles
-    # to gain by it
-    ([(27, 13, 3, 392, 232, 2), (45, 32, 3, 312, 80, 2)], True),
+    # (batch, field, kernel, channels, stride): K in parts in front of tiles of 128
+    # x 64 and behind them; in two shapes of its own; beside too many tiles to gain
+    # by it
     ([(15, 22, 5, 248, 168, 1), (15, 22, 5, 248, 48, 1)], True),
+    ([(15, 22, 5, 248, 48, 1), (15, 22, 5, 248, 168, 1)], True),
     ([(7, 22, 5, 392, 312, 1), (6, 21, 5, 392, 264, 1)], True),
-    ([(45, 32, 3, 312, 80, 2), (15, 22, 5, 248, 168, 1)], False),
-    ([(22, 27, 5, 352, 72, 1), (22, 27, 3, 352, 56, 1)], False)])
+    ([(7, 22, 5, 392, 312, 1), (15, 22, 5, 248, 168, 1)], False),
+    ([(15, 22, 5, 248, 168, 1), (22, 27, 3, 352, 56, 1)], False)])
 def test_k_in_parts_shares_a_launch(layers, shared):
     """Sums of K in parts are rounded elsewhere than those of K whole: the bytes
     tell which of the two ran."""
