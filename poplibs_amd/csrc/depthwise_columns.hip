@@ -250,6 +250,7 @@ bool depthwiseColumnsTakes(const DepthwiseDesc &d, int inType, int outType) {
          d.padH < most && d.padW > -most && d.padW < most;
 }
 
+namespace {
 // 3 x 3 taps: the same with their own figures, fitted to 6 100 timings of 500
 // random layers (1 to 64 images of 7 to 112 squared, 32 to 960 channels) within 8
 // to 9 %; the choice by it is 1 % behind the best.
@@ -281,6 +282,7 @@ double threeEstimateUs(const DepthwiseDesc &d) {
                        (double(d.inH) * d.inW + double(d.outH) * d.outW);
   return f.call + std::sqrt(std::hypot(us * us, std::pow(bytes / f.rate, 2)));
 }
+} // namespace
 
 // What a strip and a band cost, fitted to 1700 timings of 130 random layers
 // (the choice by it is within 2 % of the best on average): a wave issues its

@@ -586,14 +586,6 @@ __global__ __launch_bounds__(kThreads) void igemmFusedKernel(IgemmFusedArgs m) {
       m.firstBlock[i + 1] - m.firstBlock[i]);
 }
 
-template <class Kernel>
-hipError_t raiseLdsLimit(Kernel kernel, int ldsBytes) {
-  // More than the 64 KB a kernel gets by default.
-  return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                             ldsBytes);
-}
-
 /// What to launch once the kernel's template arguments are known: one
 /// convolution ...
 struct LaunchOne {

@@ -525,5 +525,13 @@ igemmEpilogue(char *lds, const IgemmArgs &a, floatx16 (&acc)[2][BN / 64],
 }
 
 } // namespace
+/// More LDS than the 64 KB a kernel gets by default.
+template <class Kernel>
+hipError_t raiseLdsLimit(Kernel kernel, int ldsBytes) {
+  return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             ldsBytes);
+}
+
 } // namespace mxk
 #endif

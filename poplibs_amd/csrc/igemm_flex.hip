@@ -578,12 +578,6 @@ constexpr int flexStages(int mb, int nb, bool shared) {
                                              : 6;
 }
 
-template <class Kernel>
-hipError_t raiseLds(Kernel kernel, int bytes) {
-  return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-}
-
 struct FlexOne {
   const IgemmArgs &a;
   const void *in, *w, *bias;
@@ -605,7 +599,7 @@ struct FlexOne {
     constexpr int kLds = FlexShape<MB, NB, NS>::template ldsBytes<OutT>();
     static_assert(kLds * PER_CU <= 160 * 1024, "a CU's LDS");
     const auto kernel = &igemmFlexKernel<MB, NB, NS, PER_CU, SPLIT, OutT>;
-    static const hipError_t attr = raiseLds(kernel, kLds);
+    static const hipError_t attr = raiseLdsLimit(kernel, kLds);
     if (attr != hipSuccess)
       return attr;
     hipLaunchKernelGGL(kernel, dim3(uint32_t(blocks)), dim3(kThreads), kLds,
@@ -626,7 +620,7 @@ struct FlexFused {
       return hipSuccess;
     constexpr int kLds = FlexShape<MB, NB, NS>::template ldsBytes<__half>();
     const auto kernel = &igemmFlexFusedKernel<MB, NB, NS, PER_CU, __half>;
-    static const hipError_t attr = raiseLds(kernel, kLds);
+    static const hipError_t attr = raiseLdsLimit(kernel, kLds);
     if (attr != hipSuccess)
       return attr;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), kLds, stream, m);
