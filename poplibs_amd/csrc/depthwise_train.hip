@@ -171,7 +171,9 @@ struct BlockArgs {
 /// What bounds it is a wave's chain of instructions, 1 200 with two blocks of 5 x 5
 /// taps: with one block to a thread instead of two (5 x 5) or four (3 x 3), and no
 /// load under a condition of its own, 17 x 44 x 44, 400 channels, 5 x 5 17.8 -> 13.2
-/// us, 19 x 25 x 25, 40, 3 x 3 4.4 -> 2.8; 70 layers 1.32 times as fast.
+/// us, 19 x 25 x 25, 40, 3 x 3 4.4 -> 2.8; 70 layers 1.32 times as fast.  607 with
+/// three calls' tensors in turn 1.28 times, 3 x 3 layers of more than 100 MB 1.02
+/// (28; 15 x 71 x 71, 800 channels 35.3 -> 37.7, 26 x 78 x 78, 440 45.6 -> 41.7).
 template <int S, int K, int R, class OutT>
 __global__ __launch_bounds__(256, K == 5 ? 2 : 4) void
 depthwiseDilatedBlockKernel(
@@ -422,7 +424,8 @@ constexpr uint32_t kManyOutputs = 3500, kManyOutputsPerSlice = 25;
 /// 16 slices: 8.0 -> 3.2 us).  Their chain is eight times as long, which shows right
 /// behind the kernel that writes the slices: the line below is where both were level
 /// over 70 passes.
-/// WIDE: offsets beyond 31 bits.
+/// WIDE: offsets beyond 31 bits, which take 13 million outputs: those are one or
+/// two slices.
 template <class OutT, int PARTS, int COLUMNS, bool WIDE>
 __global__ __launch_bounds__(PARTS *COLUMNS) void depthwiseDeltaSumKernel(
     const float *__restrict__ partial, uint32_t slices, uint32_t taps,

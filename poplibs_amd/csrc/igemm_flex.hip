@@ -18,10 +18,11 @@
 // turn: 4096 x 4096 x 4096 118.2 -> 105.3 (256 x 256: 1.31 PFLOP/s), 1026 x 1080 x
 // 4604 23.7 -> 18.1 (192 x 128), N = 47, 44 x 44, 3 x 3 stride 2, 192 -> 136 24.1 ->
 // 18.1 (128 x 160), N = 68, 19 x 19, 3 x 3, 160 -> 160 21.8 -> 15.6 (resident patch).
-// What bounds it: a k-step of a 128 x 128 tile takes 0.30 us on a full chip with
+// What bounds it: a k-step of a 128 x 128 tile takes 0.27 us on a full chip with
 // neither loads nor LDS reads in it (512 cycles of MFMAs at the clock the chip's
-// power leaves), 0.38 with the reads, 0.42 with the loads, 0.52 with both; 1.16,
-// 1.25, 1.43 and 1.49 in one of 256 x 256.
+// power leaves), 0.37 with the reads, 0.42 with the loads, 0.51 with both; 1.14,
+// 1.28, 1.37 and 1.50 in one of 256 x 256, whose matrix pipe is busy 67 % of the
+// cycles at 1.81 GHz.
 #include "igemm_common.hpp"
 
 #include <algorithm>

@@ -567,10 +567,10 @@ __global__ __launch_bounds__(256) void biasUpdateKernel(
 /// outweighs up to 2 048 rows - 3 200 of 1 MB in all, 4 096 of a single line,
 /// but 1 024 of no whole vectors.  The call, host and all, us, on rows from
 /// memory and on rows just read, with this kernel and with two:
-///   halves   64 x 4 096   7.1, 4.6   6.8, 6.6     144 x 2 048  5.3, 4.1   6.5, 6.5
-///           144 x 3 072   7.2, 4.5   6.6, 6.6   1 024 x 2 048  5.8, 3.8   6.8, 6.6
-///         1 024 x 4 096  10.9, 4.9   7.2, 6.5   8 192 x 2 048  9.9, 4.8  11.1, 7.8
-///   floats  144 x 2 048   5.4, 4.0   6.7, 6.6   2 048 x 2 048  8.8, 4.0   8.7, 6.4
+///   halves   64 x 4 096   6.8, 4.7   6.4, 6.3     144 x 2 048  5.3, 3.9   6.4, 6.4
+///           144 x 3 136   7.3, 4.5   6.4, 6.5   1 024 x 2 048  8.8, 3.9   6.7, 6.5
+///         1 024 x 4 096  15.3, 5.0   7.0, 6.5   8 192 x 2 048 10.4, 4.9  10.8, 7.3
+///   floats  144 x 2 048   5.5, 4.9   6.5, 6.8   2 048 x 2 048  9.4, 3.9   8.2, 6.4
 /// In a layer's training step the rows are somewhere between: 16 images of
 /// 14 x 14, 1 x 1, 512 -> 1024 (3 136 rows) 55.1 us with this kernel, 52.4 with
 /// two, 64 of 8 x 8, 3 x 3, 256 -> 512 (4 096) 74.8 and 71.2, but 4 of 28 x 28,

@@ -520,7 +520,11 @@ std::size_t flexPartsColumns(std::size_t co, std::size_t blockN) {
 /// times as fast on average (1.17), one round of them 1.0075 (under 1), of 128 x
 /// 64 1.013 (1.01), resident patch of 16-pixel blocks 1.13 (1.15), of 32 1.03,
 /// pointwise layers 1.014 (1.02, one in seven slower); at the share 7 of 1 400 are
-/// slower by more than 3 %, the worst 0.85 times as fast, in brackets 190.
+/// slower by more than 3 %, the worst 0.85 times as fast, in brackets 190.  Of
+/// 1 105 other layers and products with three calls' tensors in turn, those that
+/// the rules below leave aside taken out: 1.25 (484), 1.04 (38), 1.16 (57), 1.30 (96),
+/// 1.38 (13), 1.23 (79), tiles of 256 x 192 and 256 x 256 1.19 and 1.14 (338); 13
+/// slower by more than 3 %, the worst 0.86.
 double flexShare(bool pointwise, unsigned patch, unsigned blockN,
                  unsigned stages) {
   return pointwise ? 0.9 : patch ? 0.82 : blockN == 64 || stages == 4 ? 0.85 : 0.88;
@@ -2241,9 +2245,9 @@ mxconv_plan makePlanWith(const ConvParams &params,
       // The phases of a zero-stuffed input, all with taps, in two rounds or more
       // of tiles of 128 x 128 that their channels fill badly: tiles of 160
       // channels where those cover them in 0.7 of the columns (N = 42, 35 x 35,
-      // 3 x 3 stride 2, 136 -> 80 backwards 14.4 -> 10.7 us; four such layers
-      // 1.24 to 1.34 times as fast), of 96 where those do in three quarters (N =
-      // 25, 57 x 57, 72 -> 200 20.5 -> 19.4; four 1.01 to 1.07).  Single taps,
+      // 3 x 3 stride 2, 136 -> 80 backwards 14.4 -> 10.7 us; 17 such layers 1.39
+      // times as fast), of 96 where those do in three quarters (N = 25, 57 x 57,
+      // 72 -> 200 20.5 -> 19.4; 55 1.16, the slowest two 0.93).  Single taps,
       // whose other phases write zeros, and fewer tiles gain nothing or lose (N =
       // 38, 27 x 27, 192 -> 56 7.4 -> 8.6).
       std::size_t tiles = 0;
