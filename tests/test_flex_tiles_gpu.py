@@ -293,11 +293,12 @@ def test_a_multi_convolution_in_one_launch(bias):
 @pytest.mark.parametrize("layers,shared", [
     # (batch, field, kernel, channels, stride): K in parts in front of tiles of 128
     # x 64 and behind them; in two shapes of its own; beside too many tiles to gain
-    # by it
+    # by it, or by enough
     ([(15, 22, 5, 248, 168, 1), (15, 22, 5, 248, 48, 1)], True),
     ([(15, 22, 5, 248, 48, 1), (15, 22, 5, 248, 168, 1)], True),
     ([(7, 22, 5, 392, 312, 1), (6, 21, 5, 392, 264, 1)], True),
     ([(7, 22, 5, 392, 312, 1), (15, 22, 5, 248, 168, 1)], False),
+    ([(19, 13, 5, 464, 280, 1), (8, 22, 5, 472, 200, 1)], False),
     ([(15, 22, 5, 248, 168, 1), (22, 27, 3, 352, 56, 1)], False)])
 def test_k_in_parts_shares_a_launch(layers, shared):
     """Sums of K in parts are rounded elsewhere than those of K whole: the bytes
