@@ -983,7 +983,13 @@ hipError_t prepare(const IgemmDesc &d, int inType, bool haveWorkspace,
   // Buffer addressing is 32-bit: the weights as a whole, the input from the
   // first image a tile reads (igemmAddressable; the planner keeps other
   // shapes away).
-  const uint64_t wBytes = uint64_t(d.groups) * a.coPadded * a.kPadded * eb;
+  // (rows of the weights beyond the buffer have vector offsets beyond it)
+  if (d.packedColumns && (d.flex || wide || d.groups != 1 ||
+                          d.packedColumns < d.outChansPerGroup))
+    return hipErrorInvalidValue;
+  const uint32_t columns =
+      d.packedColumns ? std::min(d.packedColumns, a.coPadded) : a.coPadded;
+  const uint64_t wBytes = uint64_t(d.groups) * columns * a.kPadded * eb;
   if (!igemmAddressable(d, inType) || wBytes >= kOutOfRange)
     return hipErrorInvalidConfiguration;
   a.imageBytes = uint32_t(uint64_t(d.inD) * d.inH * d.inW * d.groups *

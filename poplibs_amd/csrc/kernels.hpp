@@ -237,6 +237,10 @@ struct IgemmDesc {
   // 1 or 2: the kernel of tiles of 128, 192 or 256 pixels x 64 to 256 channels
   // in steps of 32 runs (igemmFlexTakes), 2 with two workgroups to a CU.
   uint32_t flex = 0;
+  // Columns that the packed weights hold where they were packed for tiles of
+  // another width (igemmKernel, one group; 0: whole tiles of blockN); those of a
+  // tile beyond them are read as zeros.
+  uint32_t packedColumns = 0;
   // Patch rows the tallest tile of the resident-patch kernel spans (igemmPatchMaxRows),
   // worked out once when the plan is made - it takes a walk over the tiles -
   // so that a launch does not repeat it; 0 = not known, work it out.

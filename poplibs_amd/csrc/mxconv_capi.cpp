@@ -1033,17 +1033,17 @@ mxconv_status mxconv_multi_fwd(size_t n, const mxconv_plan *const *plans,
     return (k + d.blockK - 1) / d.blockK;
   };
   // A plan of flexible tiles with K in parts can run in the tiles of another
-  // member as well: its packed weights hold whole tiles of 128 columns.  (Without
-  // that N = 15, 22 x 22, 248 channels, four layers, of which 5 x 5 -> 168 and -> 48
-  // share one, 64.8 us, 56.2 so.)
+  // member as well.  (Without that N = 15, 22 x 22, 248 channels, four layers, of
+  // which 5 x 5 -> 168 and -> 48 share one, 64.8 us, 56.2 so.)
   auto streams = [](const mxk::IgemmDesc &d) {
     return !d.small && !d.patch && !d.flex && d.blockM == 128;
   };
   auto adapts = [](const mxk::IgemmDesc &d) {
     return d.flex && d.splitK > 1 && d.groups == 1;
   };
-  auto asTile = [](mxk::IgemmDesc &d, const mxk::IgemmDesc &tile) {
+  auto asTile = [&](mxk::IgemmDesc &d, size_t i, const mxk::IgemmDesc &tile) {
     d.flex = 0;
+    d.packedColumns = uint32_t(plans[i]->coPadded);
     d.blockM = tile.blockM, d.blockN = tile.blockN, d.stages = tile.stages;
   };
   auto fusedItem = [&](size_t i, size_t slot, mxk::IgemmFusedItem &item) {
@@ -1099,10 +1099,10 @@ mxconv_status mxconv_multi_fwd(size_t n, const mxconv_plan *const *plans,
           if (done[j] || !fusedItem(j, 1, item))
             continue;
           if (adapts(plans[j]->igemm) && !fusable(group[0], item))
-            asTile(unsplit[1], narrow);
+            asTile(unsplit[1], j, narrow);
           if (!streams(unsplit[1]))
             continue;
-          asTile(unsplit[0], unsplit[1]);
+          asTile(unsplit[0], i, unsplit[1]);
           if (!fusable(group[0], item))
             unsplit[0] = own;
         }
@@ -1115,7 +1115,7 @@ mxconv_status mxconv_multi_fwd(size_t n, const mxconv_plan *const *plans,
         const bool other = adapt && adapts(plans[j]->igemm) &&
                            streams(unsplit[0]);
         if (other)
-          asTile(unsplit[members], unsplit[0]);
+          asTile(unsplit[members], j, unsplit[0]);
         if (!fusable(group[0], item))
           continue;
         adapted = adapted || other;

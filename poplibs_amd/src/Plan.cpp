@@ -507,13 +507,6 @@ double estimateBesideFlexPartsOfFewRows(unsigned blockN, std::size_t parts,
          f.partial * partialMB;
 }
 
-/// Columns of the packed weights of a product in flexible tiles with K in parts:
-/// whole tiles of 128 besides its own, so that it can share the launch of several
-/// convolutions in tiles of igemmKernel (mxconv_multi_fwd).
-std::size_t flexPartsColumns(std::size_t co, std::size_t blockN) {
-  return std::max((co + blockN - 1) / blockN * blockN, (co + 127) / 128 * 128);
-}
-
 /// igemmFlexKernel is taken where it is estimated at less than these shares of
 /// what is planned.  Over the layers of the fit, at the share and (in brackets)
 /// wherever the estimate is lower at all: tiles of 128 x 128, two to a CU, 1.155
@@ -1626,10 +1619,6 @@ mxconv_plan makePlanWith(const ConvParams &params,
       if (s.hasDepth() && s.inputDilated())
         parts = 1;
       g.splitK = uint32_t(parts);
-      if (g.flex && parts > 1 && p.numConvGroups == 1) {
-        plan.coPadded = flexPartsColumns(co, g.blockN);
-        plan.weightPackedElems = plan.coPadded * plan.kPadded;
-      }
       plan.workspaceBytes = mxk::igemmWorkspaceBytes(g);
       if (ciPadded != ci) {
         plan.paddedInputChans = ciPadded;
@@ -2490,7 +2479,7 @@ mxconv_plan makePlanWith(const ConvParams &params,
       }
       if (chosenTile.flex) {
         g = chosenTile;
-        plan.coPadded = flexPartsColumns(co, g.blockN);
+        plan.coPadded = (co + g.blockN - 1) / g.blockN * g.blockN;
         plan.kPadded = kSteps * 64;
         plan.weightPackedElems = plan.coPadded * plan.kPadded;
         plan.workspaceBytes = mxk::igemmWorkspaceBytes(g);

@@ -297,6 +297,8 @@ def test_a_multi_convolution_in_one_launch(bias):
     ([(15, 22, 5, 248, 168, 1), (15, 22, 5, 248, 48, 1)], True),
     ([(15, 22, 5, 248, 48, 1), (15, 22, 5, 248, 168, 1)], True),
     ([(7, 22, 5, 392, 312, 1), (6, 21, 5, 392, 264, 1)], True),
+    # (weights packed in 288 columns, read in 320)
+    ([(11, 30, 3, 424, 288, 2), (12, 36, 3, 376, 196, 2)], True),
     ([(7, 22, 5, 392, 312, 1), (15, 22, 5, 248, 168, 1)], False),
     ([(19, 13, 5, 464, 280, 1), (8, 22, 5, 472, 200, 1)], False),
     ([(15, 22, 5, 248, 168, 1), (22, 27, 3, 352, 56, 1)], False)])
@@ -355,14 +357,15 @@ def test_k_in_parts_shares_a_launch(layers, shared):
 
 
 @pytest.mark.parametrize("m,k,n", [(133, 4872, 5488), (450, 7416, 1400)])
-def test_packed_weights_of_parts_hold_whole_tiles_of_128(m, k, n):
+def test_packed_weights_of_parts_are_the_tile_s(m, k, n):
     from poplibs_amd import capi
     p = pa.matMulParams(pa.HALF, pa.HALF, 1, m, k, n)
     plan = pa.Plan(p)
     again = pa.Plan(p, {"planConstraints": plan.constraints()})
-    assert json.loads(plan.constraints())["gfx950"]["splitK"] > 1
+    named = json.loads(plan.constraints())["gfx950"]
+    assert named["splitK"] > 1
     rows = plan.buffer_bytes(capi.BUF_WEIGHTS_PACKED) // (-(-k // 64) * 128)
-    assert rows >= -(-n // 128) * 128
+    assert rows == -(-n // named["blockN"]) * named["blockN"]
     assert again.packs_like(plan)
 
 
